@@ -252,7 +252,7 @@ def vector_errors(hs, hd, ev_f, z_f, ev_s, z_s, complex_: bool, nsample: int = 2
 
 def measure(L, run, basis, kd, args, label: str, workload: str, full_checks: bool):
     """W warmup and K timed k-points in FP64 and in split precision, one
-    k-point with per-launch SYMV events, checks against the reference."""
+    k-point with per-launch events around the panel products, checks against the reference."""
     el, eu, nume = float(kd["EL"]), float(kd["EU"]), int(kd["NUME"])
     ctx = L.Lapw1(run)
     ctx.set_basis(basis)
@@ -291,7 +291,7 @@ def measure(L, run, basis, kd, args, label: str, workload: str, full_checks: boo
     tk = None
     if not args.no_kernel_timing:
         # one more k-point, outside the timed region, with per-launch events
-        # around the tridiagonalisation SYMV (its kernel-level roofline)
+        # around the band reduction's panel products (their kernel-level roofline)
         ctx.set_kernel_timing(True)
         ctx.calkpt(el, eu, nume)
         tk = dict(zip(names, ctx.timings()))
@@ -333,13 +333,12 @@ def measure(L, run, basis, kd, args, label: str, workload: str, full_checks: boo
         "k_hamilt_pw": ("valu", f_hamilt, t["hamilt_pw_kernel"], 1),
         "k_dgemm (HNS rank-K)": ("mfma", f_hns, t["hns_gemm"], 1),
     }
-    symv = "k_ztri_symv" if run.is_complex else "k_tri_symv"
     if tk is not None and tk["tri_symv_launches"] > 0:
-        # algorithmic bytes of the SYMV at step i: the lower triangle
-        # (diagonal included) of the trailing order m = n - i - 1
-        nsym = int(tk["tri_symv_launches"])
-        sym_bytes = sum(esz * m * (m + 1) / 2 for m in range(n - 1, n - 1 - nsym, -1))
-        kernels[symv] = ("hbm", sym_bytes, tk["tri_symv_total"], nsym)
+        # the products A V of the band reduction: order m = n - 32 p of the
+        # trailing matrix, 32 columns of V
+        npan = int(tk["tri_symv_launches"])
+        av_flops = sum(cx * 2.0 * 32 * float(n - 32 * p) ** 2 for p in range(1, npan + 1))
+        kernels["k_sb_av"] = ("mfma", av_flops, tk["tri_symv_total"], npan)
     kname, (bound, work, kms, nl) = max(kernels.items(), key=lambda kv: kv[1][2])
 
     def rate(bd, wk, ms_):
@@ -393,7 +392,7 @@ def main():
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-threads", type=int, default=min(16, os.cpu_count() or 1))
     ap.add_argument("--no-kernel-timing", action="store_true",
-                    help="skip the extra k-point with per-launch SYMV events (for profiler passes)")
+                    help="skip the extra k-point with per-launch events around the panel products (for profiler passes)")
     ap.add_argument("--split-slices", type=int, default=4,
                     help="INT8 digits per element for the split-precision pass (0: FP64 only)")
     ap.add_argument("--workload", choices=["c3", "c2"], default="c3",

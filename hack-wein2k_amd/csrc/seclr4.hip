@@ -13,8 +13,9 @@
 //   2. Reduction to standard form C = U^-T H U^-1 (DSCGST, dscgst.f:99-142):
 //      X = H W and C = W^T X as MFMA GEMMs (lower triangle of C; the tridiagonalisation reads and
 //      updates only the lower triangle).
-//   3. Householder tridiagonalisation (DSYTRD2, dsytrd2.f, lower; DLATRD
-//      panels of 32 columns, trailing rank-64 update on MFMA), DLARFG signs.
+//   3. Tridiagonalisation (DSYTRD2, dsytrd2.f, lower) in two stages: to
+//      bandwidth 32 by Householder panels and rank-64 updates on MFMA, then to
+//      tridiagonal form by bulge chasing (twostage.hip), DLARFG signs.
 //   4. Bisection (DSTEBZ2, RANGE='V', ORDER='B', ABSTOL=0, dstebz2.f:301-652):
 //      split points, per-block Gershgorin intervals, NWL (eigenvalues <= EL),
 //      block-ordered list capped at NUME; one thread per eigenvalue.
@@ -23,7 +24,7 @@
 //      (gap <= 1e-3 |T|_1) orthogonalised in order (block classical
 //      Gram-Schmidt, twice, on MFMA) and normalised with the largest
 //      component positive.
-//   6. Z = Q Zt with the reflectors in compact WY form (DORMTR), then the
+//   6. Z = Q1 Q2 Zt with the reflectors in compact WY form (DORMTR), then the
 //      selection sort of dsyevx2.f:381-400, then Z = U^-1 Z (DTRSM,
 //      seclr4.F:354) as a triangular MFMA GEMM with W = U^-1.
 // The arithmetic here is real FP64 throughout; the complex build (lapw1c)
@@ -36,9 +37,8 @@
 #include <utility>
 #include <vector>
 
-#include <hip/hip_ext.h>
-
 #include "seclr4_shared.h"
+#include "twostage.h"
 
 namespace w2k {
 
@@ -202,411 +202,6 @@ __global__ void k_fill(size_t cnt, double *p, double v)
 {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < cnt) p[i] = v;
-}
-
-// ------------------------------------------------------------------ tridiagonalisation
-// Panel of TNB columns (DLATRD, lower): the panel buffer P holds, for panel
-// column k, the reflector V(:,k) at column k, W(:,k) at column nb+k and a
-// second copy of V(:,k) at column 2nb+k, so that the trailing update
-// A -= V W^T + W V^T is one GEMM with operands P(:,0:2nb) and P(:,nb:3nb).
-// Per column i of the panel two multi-workgroup kernels run:
-//   k_tri_symv : DLARFG of column i (beta, tau, scal) from the norm partials,
-//                y = A(i+1:n, i+1:n) v as partial sums per column chunk, the
-//                dot products V^T v, W^T v and v^T y as partials, and V(:,k)
-//                written out (v = A(:,i) * scal, v(i+1) = 1);
-//   k_tri_col  : w = tau (y - W V^T v - V W^T v) - (tau/2)(w^T v) v written
-//                to W(:,k); the next column updated with the panel so far and
-//                the squared norm of its sub-subdiagonal part written as one
-//                partial per block.
-struct TriWork {
-  int n, p0, nb;
-  int lda;            // leading dimension of a (a multiple of 16: 128-byte aligned columns)
-  double *a;          // n x n, both triangles
-  double *P;          // n x 3 TNB panel buffer
-  double *d, *e, *tau, *scal;
-  double *part;       // nchunk x n SYMV partial sums
-  double *dots;       // tiles x 2 TNB partial V^T v, W^T v
-  double *vy;         // tiles x chunks partial v^T y
-  double *norm;       // blocks of the column update: partial squared norms
-  int *counter;       // unused by the real kernels
-};
-
-
-constexpr int COL_ROWS = 64;  // rows per block of the column update (one per lane)
-constexpr int COL_WAVES = 8;  // waves per block of the column update
-
-// DLARFG of column i on (A(i+1,i), A(i+2:n,i)), from the squared norm
-// partials of the column-update kernel; every wave of the SYMV evaluates it
-// with identical arithmetic (fixed-order sums), so no grid-wide step is
-// needed between the two kernels.  tri_norm_load issues the loads (first in
-// the wave, so that the reflector is formed while the tile is still on its
-// way); tri_reflector returns scal = 1/(alpha - beta).
-constexpr int NORM_B = 3;  // partials per lane loaded up front (n <= 64 NORM_B COL_ROWS)
-__device__ __forceinline__ void tri_norm_load(const TriWork &g, int i, int lane, double *x, double &alpha)
-{
-  const int nnorm = (g.n - i + COL_ROWS - 1) / COL_ROWS;  // blocks of the update of column i
-#pragma unroll
-  for (int u = 0; u < NORM_B; u++) x[u] = g.norm[min(lane + 64 * u, nnorm - 1)];
-  alpha = g.a[(size_t)g.lda * i + i + 1];
-}
-
-__device__ __forceinline__ double tri_reflector(const TriWork &g, int i, int lane, bool store, const double *x,
-                                                double alpha)
-{
-  const int nnorm = (g.n - i + COL_ROWS - 1) / COL_ROWS;
-  double xs = 0.0;
-#pragma unroll
-  for (int u = 0; u < NORM_B; u++) xs += (lane + 64 * u < nnorm) ? x[u] : 0.0;
-  for (int b = lane + 64 * NORM_B; b < nnorm; b += 64) xs += g.norm[b];
-  xs = wave_sum(xs);
-  xs = __shfl(xs, 0, 64);
-  const double xnorm = sqrt(xs);
-  double tau = 0.0, beta = alpha, scal = 0.0;
-  if (xnorm != 0.0) {
-    beta = -copysign(sqrt(alpha * alpha + xnorm * xnorm), alpha);
-    tau = (beta - alpha) / beta;
-    scal = 1.0 / (alpha - beta);
-  }
-  if (store && lane == 0) {
-    g.e[i] = beta;
-    g.tau[i] = tau;
-    g.scal[i] = scal;
-  }
-  return scal;
-}
-
-// y = A(r0:n, r0:n) v from the lower triangle only (A is symmetric): one
-// wave per 64 x 64 tile (I, J), J <= I, adds A_IJ v_J to the rows of tile I
-// and, for J < I, A_IJ^T v_I to the rows of tile J (column sums by a
-// wave-wide reduce-scatter, no LDS); a diagonal tile adds its lower part by
-// rows and its strict lower part by columns.  Row r of tile R receives
-// exactly one partial per tile index: from (R, J) at slot J <= R and from
-// (I, R) at slot I > R, so y(r) = sum over slots in a fixed order.  A tile
-// wave writes its partials into a block of its own, 128 doubles at bid * 128
-// (row sums, then column sums), so that consecutive waves write consecutive
-// memory (tiles x n vectors put every 512-byte segment in another place,
-// which costs the kernel's read stream more HBM time).  Every tile wave
-// writes its partial v^T y.  The nt waves after the
-// tiles each take one row block I: they write V(:,k) (v = A(:,i) * scal,
-// v(i+1) = 1) and the partial dot products V^T v, W^T v of the block's rows.
-__global__ __launch_bounds__(64, 3) void k_tri_symv(TriWork g, int i, int nt)
-{
-  const int n = g.n, lda = g.lda, r0 = i + 1, ii = i - g.p0, nb = g.nb;
-  const int base = r0 & ~15;  // tile grid origin: rows on 128-byte boundaries
-  const int lane = threadIdx.x;
-  const int nblk = nt * (nt + 1) / 2;
-  const int bid = blockIdx.x;
-  const double *ai = g.a + (size_t)lda * i;
-  double xn[NORM_B], alpha;
-  tri_norm_load(g, i, lane, xn, alpha);
-  if (bid >= nblk) {
-    // row block I, two waves: V column and V^T v (half 0), W^T v (half 1)
-    const int I = (bid - nblk) >> 1, half = (bid - nblk) & 1;
-    const int R = base + SYMV_T * I + lane;
-    const bool live = R >= r0 && R < n;
-    const int Rs = live ? R : r0;
-    const double a_r = ai[Rs];
-    double t[TNB];  // 32 values per wave keep the branch's registers at the tile loop's level
-    if (ii > 0) {
-#pragma unroll
-      for (int k = 0; k < TNB; k++) t[k] = g.P[(size_t)n * (half * nb + k) + Rs];
-    }
-    const double sc = tri_reflector(g, i, lane, false, xn, alpha);
-    const double vr = live ? (R == r0 ? 1.0 : a_r * sc) : 0.0;
-    if (live && half == 0) {
-      g.P[(size_t)n * ii + R] = vr;
-      g.P[(size_t)n * (2 * nb + ii) + R] = vr;
-    }
-    if (ii > 0) {
-      // t[k] = X(R,k) v(R) for k < ii, summed over the lanes: lanes 2q and
-      // 2q + 1 end with the sum of column q
-#pragma unroll
-      for (int k = 0; k < TNB; k++) {
-        const bool use = live && k < ii;
-        t[k] = use ? t[k] * vr : 0.0;
-      }
-      const double dq = wave_transpose_sum32x(t, lane);  // lanes 2k, 2k + 1: column k
-      if (!(lane & 1)) g.dots[(size_t)I * 2 * TNB + half * TNB + (lane >> 1)] = dq;
-    }
-    return;
-  }
-  // triangular block index -> (I, J), J <= I
-  int I = (int)((sqrt(8.0 * (double)bid + 1.0) - 1.0) * 0.5);
-  while ((I + 1) * (I + 2) / 2 <= bid) I++;
-  while (I * (I + 1) / 2 > bid) I--;
-  const int J = bid - I * (I + 1) / 2;
-  const int R = base + SYMV_T * I + lane;
-  const int C0 = base + SYMV_T * J;
-  const bool live = R >= r0 && R < n;
-  const bool off = (I != J);
-  const int m = min(SYMV_T, n - C0);
-  const int Rl = min(R, n - 1);  // the lane's row for the loads (in bounds)
-  // every load of the tile and of v is issued before the first use: clamped
-  // (in-bounds) addresses, values masked afterwards
-  const double a_c = ai[min(C0 + lane, n - 1)];
-  const double a_r = ai[Rl];
-  const double *ap = g.a + (size_t)Rl + (size_t)lda * C0;
-  double t[SYMV_T];
-#pragma unroll
-  for (int j = 0; j < SYMV_T; j++) t[j] = ap[(size_t)lda * min(j, m - 1)];
-  const double sc = tri_reflector(g, i, lane, bid == 0, xn, alpha);
-  const int c = C0 + lane;
-  const double vc = (c >= r0 && c < n) ? (c == r0 ? 1.0 : a_c * sc) : 0.0;  // v of the lane's column
-  const double vr = live ? (R == r0 ? 1.0 : a_r * sc) : 0.0;
-  if (m < SYMV_T || !live) {
-#pragma unroll
-    for (int j = 0; j < SYMV_T; j++) t[j] = (live && j < m) ? t[j] : 0.0;
-  }
-  // only the lower triangle of A is kept current (the trailing updates skip
-  // the upper one): a diagonal tile uses its lower part, by rows and (strictly
-  // below the diagonal) by columns
-  if (!off) {
-#pragma unroll
-    for (int j = 0; j < SYMV_T; j++) t[j] = (j <= lane) ? t[j] : 0.0;
-  }
-  // row sums: v(C0 + j) broadcast from lane j through scalar registers
-  const long long vcb = __double_as_longlong(vc);
-  const int vlo = (int)(unsigned)(vcb & 0xffffffffll), vhi = (int)(unsigned)((unsigned long long)vcb >> 32);
-  double y0 = 0.0, y1 = 0.0, y2 = 0.0, y3 = 0.0;
-#pragma unroll
-  for (int j = 0; j < SYMV_T; j += 4) {
-    double vj[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const unsigned lo = (unsigned)__builtin_amdgcn_readlane(vlo, j + u);
-      const unsigned hi = (unsigned)__builtin_amdgcn_readlane(vhi, j + u);
-      vj[u] = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-    }
-    y0 += t[j] * vj[0];
-    y1 += t[j + 1] * vj[1];
-    y2 += t[j + 2] * vj[2];
-    y3 += t[j + 3] * vj[3];
-  }
-  double yrow = (y0 + y1) + (y2 + y3);
-  if (!off) {
-#pragma unroll
-    for (int j = 0; j < SYMV_T; j++) t[j] = (j < lane) ? t[j] * vr : 0.0;
-    yrow += wave_transpose_sum(t, lane);  // column C0 + lane = row R of the strict lower part
-  }
-  if (live) g.part[(size_t)bid * 128 + lane] = yrow;
-  // v^T y over the tile: an off-diagonal tile adds v_I^T A_IJ v_J through its
-  // rows and the same number again through its columns
-  double vy = wave_sum(yrow * vr);
-  if (lane == 0) g.vy[bid] = off ? 2.0 * vy : vy;
-  if (off) {
-    double *pc = g.part + (size_t)bid * 128 + 64 + lane;
-    const bool st = lane < m && c >= r0;
-#pragma unroll
-    for (int j = 0; j < SYMV_T; j++) t[j] *= vr;
-    const double cs = wave_transpose_sum(t, lane);  // column C0 + lane of A_IJ^T v_I
-    if (st) *pc = cs;
-  }
-}
-
-// Finish W(:, fin - p0) (fin >= 0) and update column col (col >= 0) with the
-// panel so far (DLATRD); write the squared-norm partial of its
-// sub-subdiagonal part per block (DLARFG itself is evaluated by the next
-// SYMV's waves).  A block takes COL_ROWS = 64 consecutive rows, one per lane,
-// in each of its COL_WAVES waves, so that every load of a SYMV partial or a
-// panel column is one contiguous 512-byte row segment; the waves split the
-// SYMV partials (chunk w, w + 8, ...) and the panel columns (four each) and
-// their row sums meet in LDS.  Loads are issued in batches with clamped
-// indices and masked values, so that a batch is in flight at once.
-// offset of partial c of the rows of SYMV row block I (the lane's place in
-// the block at + l): the row sums of tile (I, c) for c <= I, else the column
-// sums of tile (c, I)
-__device__ __forceinline__ size_t tpart_off(int I, int c)
-{
-  return c <= I ? (size_t)(I * (I + 1) / 2 + c) * 128 : (size_t)(c * (c + 1) / 2 + I) * 128 + 64;
-}
-
-__global__ __launch_bounds__(64 * COL_WAVES) void k_tri_col(TriWork g, int fin, int col, int ntile, int nvy)
-{
-  constexpr int NT = 64 * COL_WAVES;   // threads
-  constexpr int KW = TNB / COL_WAVES;  // panel columns per wave
-  constexpr int YB = 16;               // SYMV-partial chunks per wave and batch
-  constexpr int VB = 10;               // first batch of v^T y pairs per thread (nvy <= 2 NT VB)
-  constexpr int DG = NT / 32;          // groups of the V^T v, W^T v sums (32 column pairs each)
-  constexpr int DB = 8;                // first batch of tiles per group (ntile <= DG DB)
-  const int n = g.n, p0 = g.p0, nb = g.nb, t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int nch = ntile;
-  const int rbase = fin >= 0 ? fin + 1 : col;
-  const int r = rbase + blockIdx.x * COL_ROWS + lane;
-  const bool live = r < n;
-  const int rs = live ? r : rbase;  // rbase < n: a safe row for dead lanes
-  const int ii = fin >= 0 ? fin - p0 : -1;
-  const int jj = col - p0;  // columns 0..jj-1 of the panel update column col
-  __shared__ double ab[2 * TNB];  // a_k = V_k^T v, b_k = W_k^T v
-  __shared__ double wc[TNB], vc[TNB];
-  __shared__ double dred[DG][2 * TNB];
-  __shared__ double red[3][COL_WAVES][COL_ROWS];  // per wave: y, z (W a + V b), a0
-  __shared__ double sh[2][COL_WAVES];
-  const double *V = g.P, *W = g.P + (size_t)n * nb;
-  double *ac = g.a + (size_t)g.lda * (col >= 0 ? col : 0);
-  // ---- per-block scalars: row col of the panel, v^T y, V^T v and W^T v
-  if (col >= 0 && t < jj) {
-    vc[t] = V[(size_t)n * t + col];
-    if (t < ii || fin < 0) wc[t] = W[(size_t)n * t + col];
-  }
-  if (fin >= 0) {
-    {
-      const int vlast = (nvy - 1) & ~1;  // the last pair (vy has one spare entry)
-      double2 xv[VB];
-#pragma unroll
-      for (int u = 0; u < VB; u++) xv[u] = *reinterpret_cast<const double2 *>(g.vy + min(2 * t + 2 * NT * u, vlast));
-      double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-      for (int u = 0; u < VB; u++) {
-        const int j = 2 * t + 2 * NT * u;
-        s0 += (j < nvy) ? xv[u].x : 0.0;
-        s1 += (j + 1 < nvy) ? xv[u].y : 0.0;
-      }
-      for (int j = 2 * t + 2 * NT * VB; j < nvy; j += 2 * NT) {
-        s0 += g.vy[j];
-        s1 += (j + 1 < nvy) ? g.vy[j + 1] : 0.0;
-      }
-      const double vs = wave_sum(s0 + s1);
-      if (lane == 0) sh[0][w] = vs;
-    }
-    if (col >= 0) {
-      double p = 0.0;
-      const int cl = col - (rbase & ~15);  // row col in row block 0 of the SYMV's grid
-      for (int c = t; c < nch; c += NT) p += g.part[tpart_off(0, c) + cl];
-      p = wave_sum(p);
-      if (lane == 0) sh[1][w] = p;
-    }
-    {
-      const int dq = t & 31, dp = t >> 5;
-      double s0 = 0.0, s1 = 0.0;
-      {
-        double2 xd[DB];
-#pragma unroll
-        for (int u = 0; u < DB; u++)
-          xd[u] = *reinterpret_cast<const double2 *>(g.dots + (size_t)min(dp + DG * u, ntile - 1) * 2 * TNB + 2 * dq);
-#pragma unroll
-        for (int u = 0; u < DB; u++) {
-          const bool k = dp + DG * u < ntile;
-          s0 += k ? xd[u].x : 0.0;
-          s1 += k ? xd[u].y : 0.0;
-        }
-      }
-      for (int b = dp + DG * DB; b < ntile; b += DG) {
-        const double2 x = *reinterpret_cast<const double2 *>(g.dots + (size_t)b * 2 * TNB + 2 * dq);
-        s0 += x.x;
-        s1 += x.y;
-      }
-      dred[dp][2 * dq] = s0;
-      dred[dp][2 * dq + 1] = s1;
-    }
-  }
-  // ---- this wave's share of the rows' sums
-  double kv[KW], kw[KW];  // V(r, k), W(r, k), k = KW w + u
-#pragma unroll
-  for (int u = 0; u < KW; u++) {
-    kv[u] = V[(size_t)n * (KW * w + u) + rs];
-    kw[u] = W[(size_t)n * (KW * w + u) + rs];
-  }
-  double y = 0.0;
-  if (fin >= 0) {
-    // the row's block and place in the SYMV's tile grid (origin rbase & ~15)
-    const int rg = rs - (rbase & ~15), I = rg >> 6, l = rg & 63;
-    for (int c0 = w; c0 < nch; c0 += COL_WAVES * YB) {
-      double xp[YB];
-#pragma unroll
-      for (int u = 0; u < YB; u++) xp[u] = g.part[tpart_off(I, min(c0 + COL_WAVES * u, nch - 1)) + l];
-#pragma unroll
-      for (int u = 0; u < YB; u++) y += (live && c0 + COL_WAVES * u < nch) ? xp[u] : 0.0;  // rows past n: never written
-    }
-  }
-  __syncthreads();
-  if (fin >= 0 && t < 2 * TNB) {
-    double q = 0.0;
-#pragma unroll
-    for (int p = 0; p < DG; p++) q += dred[p][t];
-    ab[t] = ((t & (TNB - 1)) < ii) ? q : 0.0;
-  }
-  __syncthreads();
-  {
-    double z = 0.0, a0 = 0.0;
-#pragma unroll
-    for (int u = 0; u < KW; u++) {
-      const int k = KW * w + u;
-      if (fin >= 0 && k < ii) z += kw[u] * ab[k] + kv[u] * ab[TNB + k];
-      // V(r,k) W(col,k) + W(r,k) V(col,k), k < jj, k != ii; panel columns
-      // k >= jj hold values of an earlier panel: selected away
-      const bool use = col >= 0 && k < jj && k != ii;
-      a0 += (use ? kv[u] : 0.0) * (use ? wc[min(k, TNB - 1)] : 0.0) +
-            (use ? kw[u] : 0.0) * (use ? vc[min(k, TNB - 1)] : 0.0);
-    }
-    red[0][w][lane] = y;
-    red[1][w][lane] = z;
-    red[2][w][lane] = a0;
-  }
-  __syncthreads();
-  // W(q, ii) = 0 above this kernel's rows
-  if (fin >= 0)
-    for (int q = blockIdx.x * NT + t; q < rbase; q += gridDim.x * NT) g.P[(size_t)n * (nb + ii) + q] = 0.0;
-  if (w != 0) return;
-  // ---- wave 0 finishes its 64 rows
-  double sy[3];
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    double sum = 0.0;
-#pragma unroll
-    for (int p = 0; p < COL_WAVES; p++) sum += red[a][p][lane];
-    sy[a] = sum;
-  }
-  double wr = 0.0, vii = 0.0, wcii = 0.0;  // W(r, ii), V(r, ii), W(col, ii)
-  if (fin >= 0) {
-    const double tauf = g.tau[fin];
-    vii = V[(size_t)n * ii + rs];
-    double vty = 0.0, scol = 0.0;
-#pragma unroll
-    for (int p = 0; p < COL_WAVES; p++) {
-      vty += sh[0][p];
-      scol += sh[1][p];
-    }
-    double ssum = 0.0;
-#pragma unroll
-    for (int k = 0; k < TNB; k++) ssum += ab[k] * ab[TNB + k];
-    const double alpha2 = -0.5 * tauf * tauf * (vty - 2.0 * ssum);
-    wr = tauf * (sy[0] - sy[1]) + alpha2 * vii;
-    if (live) g.P[(size_t)n * (nb + ii) + r] = wr;
-    if (col >= 0) {
-      // row col = fin + 1 of the same formula (v(col) = 1), in every lane
-      double corr = 0.0;
-      for (int k = 0; k < ii; k++) corr += wc[k] * ab[k] + vc[k] * ab[TNB + k];
-      wcii = tauf * (scol - corr) + alpha2;
-    }
-  }
-  if (col < 0) return;
-  double a = ac[rs] - sy[2];
-  if (fin >= 0) a -= vii * wcii + wr * vc[ii];
-  double nrm = 0.0;
-  if (live) {
-    ac[r] = a;
-    if (r == col) {
-      g.d[col] = a;
-      if (col == n - 1) {
-        g.tau[col] = 0.0;
-        g.scal[col] = 0.0;
-      }
-    }
-    if (r >= col + 2) nrm = a * a;
-  }
-  nrm = wave_sum(nrm);
-  if (lane == 0) g.norm[blockIdx.x] = nrm;
-}
-
-// reflectors of panel columns into A below the subdiagonal (read by the back-transform)
-__global__ void k_tri_store(TriWork g, int ncols)
-{
-  const int n = g.n;
-  const int k = blockIdx.y;
-  const int i = g.p0 + k;
-  const int r = i + 2 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= ncols || r >= n) return;
-  g.a[(size_t)r + (size_t)g.lda * i] = g.P[(size_t)n * k + r];
 }
 
 // ------------------------------------------------------------------ bisection
@@ -1126,7 +721,7 @@ __global__ __launch_bounds__(256) void k_normsign(int n, double *z, int ldz)
 }
 
 // ------------------------------------------------------------------ back-transforms
-// explicit panel of reflectors p0..p0+nb-1 (v(i+1)=1, v(i+2:n) from A) into vp
+// explicit panel of reflectors p0..p0+nb-1 of Q1 (v_i(i+BND) = 1, the rows below from A) into vp
 __global__ void k_vpanel(int n, int lda, int p0, int nb, const double *__restrict__ a, double *__restrict__ vp)
 {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1134,8 +729,8 @@ __global__ void k_vpanel(int n, int lda, int p0, int nb, const double *__restric
   if (r >= n || k >= nb) return;
   const int i = p0 + k;
   double v = 0.0;
-  if (r == i + 1) v = 1.0;
-  else if (r > i + 1) v = a[(size_t)r + (size_t)lda * i];
+  if (r == i + BND) v = 1.0;
+  else if (r > i + BND) v = a[(size_t)r + (size_t)lda * i];
   vp[(size_t)r + (size_t)n * k] = v;
 }
 
@@ -1288,22 +883,20 @@ __global__ void k_gather_cols(int n, int m, const int *__restrict__ perm, const 
 }
 
 // ------------------------------------------------------------------ driver
+size_t seclr4_doubles(size_t n, int cplx)
+{
+  // eleven pieces of at most n + 31, the panel buffer and tau
+  const size_t z = cplx ? 2 : 1;
+  return 11 * (n + 31) + z * (n + 3 * n * BND) + 128;
+}
+
 int seclr4_buffers(Ctx &c, int n, int cplx, Seclr4Bufs &B)
 {
   int rc;
-  const int nt = (n + SYMV_T - 1) / SYMV_T;
   const size_t z = cplx ? 2 : 1;
-  const size_t nts = (size_t)nt;
-  const size_t nnorm = nts + (size_t)n / COL_ROWS + 64;  // partial norms per block of 64 (complex) or 32 rows
-  // SYMV partials: 128 (real) or 256 (complex) per tile of the lower triangle
-  const size_t npart = cplx ? std::max(2 * nts * n, (size_t)128 * nts * (nts + 1))
-                            : std::max(nts * n, (size_t)64 * nts * (nts + 1));
-  const size_t small = (size_t)12 * n + z * 2 * n + z * 3 * (size_t)n * TNB + npart + z * nts * 2 * TNB +
-                       nts * (nts + 1) / 2 + 2 + nnorm + 64 + 32 * 24;
-  if ((rc = c.w_small.alloc(small))) return rc;
+  if ((rc = c.w_small.alloc(seclr4_doubles(n, cplx)))) return rc;
   if ((rc = c.w_int.alloc((size_t)6 * n + 32))) return rc;
   B.n = n;
-  B.nt = nt;
   B.cplx = cplx;
   double *p = c.w_small.p;
   auto take = [&](size_t cnt) {  // 256-byte aligned pieces
@@ -1312,13 +905,9 @@ int seclr4_buffers(Ctx &c, int n, int cplx, Seclr4Bufs &B)
     return q;
   };
   B.d = take(n); B.e = take(n); B.e2 = take(n);
-  B.tau = take(z * n); B.scal = take(z * n);
+  B.tau = take(z * n);
   B.wv = take(n);
-  B.P = take(z * 3 * (size_t)n * TNB);
-  B.part = take(npart);
-  B.tdots = take(z * nts * 2 * TNB);
-  B.tvy = take(nts * (nts + 1) / 2 + 2);
-  B.tnorm = take(nnorm);
+  B.P = take(z * 3 * (size_t)n * BND);
   B.bgl = take(n); B.bgu = take(n); B.batol = take(n); B.bnrm = take(n); B.xs = take(n);
   B.pivmin = take(1);
   // ints: [0,4) INFO, [4,12) counts, [12,16) grid-reduction tickets, then task arrays
@@ -1518,8 +1107,8 @@ int sort_eigen(Ctx &c, Seclr4Bufs &B, int m)
   return 0;
 }
 
-// Launch mode of the tridiagonalisation (2n kernel launches and n/32 GEMMs
-// with no host read-back): direct launches, or one HIP graph captured from
+// Launch mode of the tridiagonalisation (six launches per 32 columns with no
+// host read-back): direct launches, or one HIP graph captured from
 // them and replayed.  The choice is made per shape by measurement: the first
 // call with a given key (order, leading dimension and the buffers the
 // launches address) launches directly, the second captures the launches into
@@ -1531,7 +1120,8 @@ template <class F>
 static int tri_run(Ctx &c, hipStream_t s, int n, int lda, const double *a, bool kt, F &launch)
 {
   Ctx::TriGraph &tg = c.tri_graph;
-  const bool same = tg.n == n && tg.lda == lda && tg.a == a && tg.small == c.w_small.p && tg.ints == c.w_int.p;
+  const bool same = tg.n == n && tg.lda == lda && tg.a == a && tg.small == c.w_small.p && tg.ints == c.w_int.p &&
+                    tg.sb == c.w_sb.p && tg.v2 == c.w_a.p;
   if (same) {
     // the phase time of the previous call, by the mode it used
     if (tg.mode == 0) tg.direct_ms = c.last_ms[5];
@@ -1543,6 +1133,7 @@ static int tri_run(Ctx &c, hipStream_t s, int n, int lda, const double *a, bool 
     if (tg.exec) (void)hipGraphExecDestroy(tg.exec);
     tg = Ctx::TriGraph();
     tg.n = n; tg.lda = lda; tg.a = a; tg.small = c.w_small.p; tg.ints = c.w_int.p;
+    tg.sb = c.w_sb.p; tg.v2 = c.w_a.p;
   }
   tg.seen++;
   tg.mode = -1;
@@ -1585,7 +1176,7 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
   const size_t nn = (size_t)n * n;
   // workspaces: w_a = S/U, w_b = H full then C, w_c = W = U^-1, w_x = X.
   // H/C has its leading dimension rounded up to 16 so that its columns start
-  // on 128-byte boundaries (the tridiagonalisation SYMV reads aligned rows)
+  // on 128-byte boundaries (the band reduction reads aligned rows)
   const int lda = (n + 15) & ~15;
   if ((rc = c.w_a.alloc(nn)) || (rc = c.w_b.alloc((size_t)lda * n)) || (rc = c.w_c.alloc(nn))) return rc;
   double *U = c.w_a.p, *Hf = c.w_b.p, *W = c.w_c.p;
@@ -1594,7 +1185,7 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
   if ((rc = c.w_gk.alloc((size_t)1 << 22))) return rc;  // split-K partial products
   Seclr4Bufs B;
   if ((rc = seclr4_buffers(c, n, 0, B))) return rc;
-  double *d = B.d, *e = B.e, *tau = B.tau, *scal = B.scal, *P = B.P;
+  double *d = B.d, *e = B.e, *tau = B.tau, *P = B.P;
   int *info = B.info;
 
   W2K_HIP(hipEventRecord(c.ev[6], s));
@@ -1647,87 +1238,18 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
     if ((rc = dgemm(s, 'T', 'N', n, n, n, 1.0, W, n, X.p, n, 0.0, Hf, lda, 1, 2, 0))) return rc;
   }
   W2K_HIP(hipEventRecord(c.ev[8], s));
-  // ---- 3. tridiagonalisation of C (in Hf)
+  // ---- 3. tridiagonalisation of C (in Hf): band, then bulge chasing
   double *A = Hf;
-  int nsymv = 0;
+  SbArgs g;
+  if ((rc = sb_buffers(c, g, n, 0))) return rc;
+  g.lda = lda; g.ar = A; g.Pr = P; g.d = d; g.e = e; g.taur = tau;
+  g.V2r = U;  // U is not needed after the inversion
   {
-    // optional per-launch events around the SYMV (kernel-level roofline)
-    const bool kt = c.ktime != 0;
-    if (kt && c.kev.size() < (size_t)2 * n) {
-      const size_t old = c.kev.size();
-      c.kev.resize((size_t)2 * n);
-      for (size_t q = old; q < c.kev.size(); q++) W2K_HIP(hipEventCreate(&c.kev[q]));
-    }
-    TriWork g;
-    g.n = n; g.lda = lda; g.a = A; g.P = P; g.d = d; g.e = e; g.tau = tau; g.scal = scal;
-    g.part = B.part; g.dots = B.tdots; g.vy = B.tvy; g.norm = B.tnorm; g.counter = B.ticket;
-    // every launch of the phase (no host read-back in between)
-    auto launches = [&]() -> int {
-      nsymv = 0;
-      for (int p0 = 0; p0 < n; p0 += TNB) {
-        const int nb = std::min(TNB, n - p0);
-        g.p0 = p0;
-        g.nb = nb;
-        // reflector of the panel's first column (already updated by earlier panels)
-        hipLaunchKernelGGL(k_tri_col, dim3((n - p0 + COL_ROWS - 1) / COL_ROWS), dim3(64 * COL_WAVES), 0, s, g, -1, p0, 0,
-                           0);
-        W2K_STAGE(s, "k_tri_col");
-        int nref = 0;  // panel columns that carry a reflector
-        for (int k = 0; k < nb; k++) {
-          const int i = p0 + k;
-          if (i >= n - 1) break;
-          nref = k + 1;
-          const int rows = n - (i + 1);
-          const int base = (i + 1) & ~15;  // the SYMV's aligned tile origin
-          const int nt = (n - base + SYMV_T - 1) / SYMV_T, nblk = nt * (nt + 1) / 2;
-          // timed launches carry their events in the dispatch itself, so the
-          // duration is the kernel's own (no marker packets between launches)
-          if (kt) hipExtLaunchKernelGGL(k_tri_symv, dim3(nblk + 2 * nt), dim3(SYMV_T), 0, s, c.kev[2 * nsymv],
-                                        c.kev[2 * nsymv + 1], 0, g, i, nt);
-          else hipLaunchKernelGGL(k_tri_symv, dim3(nblk + 2 * nt), dim3(SYMV_T), 0, s, g, i, nt);
-          W2K_STAGE(s, "k_tri_symv");
-          nsymv++;
-          const int next = (k + 1 < nb) ? i + 1 : -1;
-          hipLaunchKernelGGL(k_tri_col, dim3((rows + COL_ROWS - 1) / COL_ROWS), dim3(64 * COL_WAVES), 0, s, g, i,
-                             next, nt, nblk);
-          W2K_STAGE(s, "k_tri_col");
-        }
-        if (nref > 0) {
-          hipLaunchKernelGGL(k_tri_store, dim3((n + 255) / 256, nref), dim3(256), 0, s, g, nref);
-          W2K_STAGE(s, "k_tri_store");
-        }
-        const int p1 = p0 + nb;
-        if (p1 < n) {
-          // A(p1:n, p1:n) -= [V W] [W V]^T, lower triangle
-          const int r = n - p1;
-          double *A1 = A + (size_t)p1 + (size_t)lda * p1;
-          int r2;
-          if ((r2 = dgemm(s, 'N', 'T', r, r, 2 * nb, -1.0, P + p1, n, P + (size_t)n * nb + p1, n, 1.0, A1, lda, 1)))
-            return r2;
-        }
-      }
-      return 0;
-    };
-    if ((rc = tri_run(c, s, n, lda, A, kt, launches))) return rc;
+    auto launches = [&]() -> int { return sb_reduce(c, s, g, 0); };
+    if ((rc = tri_run(c, s, n, lda, A, c.ktime != 0, launches))) return rc;
   }
   W2K_HIP(hipEventRecord(c.ev[9], s));
-  if (c.ktime) {
-    // [10] summed SYMV kernel time, [11] number of SYMV launches
-    W2K_HIP(hipStreamSynchronize(s));
-    double tot = 0.0;
-    int cntl = 0;
-    for (int q = 0; q < nsymv; q++) {
-      float ms = 0.f;
-      if (hipEventElapsedTime(&ms, c.kev[2 * q], c.kev[2 * q + 1]) != hipSuccess) {
-        (void)hipGetLastError();
-        break;
-      }
-      tot += ms;
-      cntl++;
-    }
-    c.last_ms[10] = tot;
-    c.last_ms[11] = cntl;
-  }
+  if ((rc = sb_take_times(c, s, n))) return rc;
   // ---- 4./5. bisection, inverse iteration, cluster orthogonalisation
   double *Zt = X.p;  // n x m
   int m = 0, nbelw = 0;
@@ -1737,7 +1259,8 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
   if ((rc = c.d_z.alloc((size_t)n * (m > 0 ? m : 1)))) return rc;
   W2K_HIP(hipEventRecord(c.ev[10], s));
   if (m > 0) {
-    // ---- 6. Z = Q Zt (reflectors of step 3, last panel first), sort, Z = W Z
+    // ---- 6. Z = Q1 Q2 Zt (reflectors of step 3, last first), sort, Z = W Z
+    if ((rc = sb_apply_q2(c, s, g, 0, m, Zt, nullptr, n))) return rc;
     // Blocks of BTNB reflectors, last block first.  The reflector panel V,
     // its Gram matrix and T (I - V T V^T) depend on the reflectors only, so
     // they are formed on the second stream up to two blocks ahead, in two
@@ -1756,7 +1279,7 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
     tbuf[1] = tbuf[0] + BTNB * BTNB;
     double *gm = tbuf[1] + BTNB * BTNB, *y1 = gm + BTNB * BTNB, *y2 = y1 + (size_t)BTNB * m;
     double *gws = y2 + (size_t)BTNB * m;
-    const int nref = n - 1;  // reflectors 0..n-2
+    const int nref = std::max(0, n - BND - 1);  // reflectors of Q1; v_i starts at row i + BND
     const int nblk = nref > 0 ? (nref + BTNB - 1) / BTNB : 0;
     hipStream_t sa = c.aux;
     auto p0_of = [&](int q) { return (nblk - 1 - q) * BTNB; };
@@ -1766,9 +1289,9 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
       hipLaunchKernelGGL(k_vpanel, dim3((n + 255) / 256, nb), dim3(256), 0, sa, n, lda, p0, nb, A, vbuf[u]);
       W2K_STAGE(sa, "k_vpanel");
       int r2;
-      // rows 0 .. p0 of the block's reflectors are zero: the products start at
-      // row p0+1 rounded down to 16 rows, which keeps the operands' 128-byte alignment
-      const int o = (p0 + 1) & ~15, nr = n - o;
+      // the block's reflectors are zero above row p0+BND: the products start at
+      // that row rounded down to 16 rows, which keeps the operands' 128-byte alignment
+      const int o = (p0 + BND) & ~15, nr = n - o;
       if ((r2 = dgemm(sa, 'T', 'N', nb, nb, nr, 1.0, vbuf[u] + o, n, vbuf[u] + o, n, 0.0, gm, nb, 0, 0, 0, gws,
                       GWS)))
         return r2;
@@ -1787,7 +1310,7 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
     for (int q = 0; q < nblk; q++) {
       const int u = q & 1, p0 = p0_of(q), nb = std::min(BTNB, nref - p0);
       W2K_HIP(hipStreamWaitEvent(s, c.bt_ready[u], 0));
-      const int o = (p0 + 1) & ~15, nr = n - o;  // the block's reflectors are zero above row p0+1
+      const int o = (p0 + BND) & ~15, nr = n - o;  // the block's reflectors are zero above row p0+1
       if ((rc = dgemm(s, 'T', 'N', nb, m, nr, 1.0, vbuf[u] + o, n, Zt + o, n, 0.0, y1, nb, 0, 0, 0, c.w_gk.p,
                       c.w_gk.n)))
         return rc;

@@ -19,9 +19,8 @@
 #include <functional>
 #include <vector>
 
-#include <hip/hip_ext.h>
-
 #include "seclr4_shared.h"
+#include "twostage.h"
 
 namespace w2k {
 
@@ -135,12 +134,6 @@ static int zgemm3(Ctx &c, hipStream_t s, char ta, char tb, int m, int n, int k, 
   hipLaunchKernelGGL(k_z3m_comb, gc, dim3(256), 0, s, m, n, T, alpha, beta, Cr, Ci, ldc, tri, 1);
   W2K_STAGE(s, "k_z3m_comb");
   return 0;
-}
-
-__device__ __forceinline__ void cmad(double ar, double ai, double br, double bi, double &cr, double &ci)
-{
-  cr += ar * br - ai * bi;
-  ci += ar * bi + ai * br;
 }
 
 // ------------------------------------------------------------------ set-up
@@ -342,545 +335,6 @@ __global__ void k_zmirror_lower(int n, double *Cr, double *Ci)
   Ci[up] = -Ci[lo];
 }
 
-// ------------------------------------------------------------------ tridiagonalisation
-// ZLATRD panels (lower), as the real build (seclr4.hip) with complex
-// arithmetic: V(:,k) at panel column k, W(:,k) at nb+k, V again at 2nb+k;
-// the SYMV adds A_IJ v_J to tile I and A_IJ^H v_I to tile J.
-struct ZTriWork {
-  int n, p0, nb;
-  double *ar, *ai;          // n x n Hermitian (both triangles)
-  double *Pr, *Pi;          // panel buffer n x 3 TNB
-  double *d, *e;            // real tridiagonal
-  double *taur, *taui;      // reflector scalars
-  double *scr, *sci;        // 1 / (alpha - beta)
-  double *part;             // SYMV partials: 256 per tile (zpart_off)
-  double *dotr, *doti;      // tiles x 2 TNB partial V^H v, W^H v
-  double *vy;               // partial Re(v^H y) per tile pair
-  double *norm;             // per block partial |x|^2
-  int *counter;
-};
-
-constexpr int ZCOL_ROWS = 64;  // rows per block of the column kernel (one per lane)
-
-// ZLARFG of column i on (A(i+1,i), A(i+2:n,i)) from the squared-norm
-// partials of the column kernel (one per block of its rows), evaluated by
-// every SYMV wave with the same fixed-order arithmetic (so no grid-wide step
-// separates the two kernels); the wave with store set writes E, TAU and the
-// scale 1/(alpha - beta) of v.
-__device__ __forceinline__ void ztri_reflector(const ZTriWork &g, int i, int lane, bool store, double &scr,
-                                               double &sci)
-{
-  const int n = g.n;
-  const int nnorm = (n - i + ZCOL_ROWS - 1) / ZCOL_ROWS;  // blocks of the column kernel
-  double x[4];
-#pragma unroll
-  for (int u = 0; u < 4; u++) x[u] = g.norm[min(lane + 64 * u, nnorm - 1)];
-  const double alr = g.ar[(size_t)n * i + i + 1], ali = g.ai[(size_t)n * i + i + 1];
-  double xs = 0.0;
-#pragma unroll
-  for (int u = 0; u < 4; u++) xs += (lane + 64 * u < nnorm) ? x[u] : 0.0;
-  for (int b = lane + 256; b < nnorm; b += 64) xs += g.norm[b];
-  xs = wave_sum(xs);
-  xs = __shfl(xs, 0, 64);
-  const double xnorm = sqrt(xs);
-  double taur = 0.0, taui = 0.0, beta = alr;
-  scr = 0.0;
-  sci = 0.0;
-  if (!(xnorm == 0.0 && ali == 0.0)) {
-    beta = -copysign(sqrt(alr * alr + ali * ali + xnorm * xnorm), alr);
-    taur = (beta - alr) / beta;
-    taui = -ali / beta;
-    const double zr = alr - beta, zi = ali, den = zr * zr + zi * zi;
-    scr = zr / den;
-    sci = -zi / den;
-  }
-  if (store && lane == 0) {
-    g.e[i] = beta;
-    g.taur[i] = taur;
-    g.taui[i] = taui;
-    g.scr[i] = scr;
-    g.sci[i] = sci;
-  }
-}
-
-// y = A(r0:n, r0:n) v for Hermitian A from the tiles on and below the
-// diagonal (one wave per 64 x 64 tile (I, J), J <= I): A_IJ v_J to the rows
-// of tile I and, for J < I, A_IJ^H v_I to the rows of tile J.  A tile is
-// taken in four quarters of 16 columns: the real and imaginary parts of a
-// quarter-row fill 32 of the lane's registers, row sums stay in the lane and
-// column sums use a wave-wide reduce-scatter (no LDS); v(C0 + j) reaches the
-// row sums from lane j by readlane.  The first quarter's loads are issued
-// before the reflector is formed and each further quarter's as soon as the
-// previous one has been reduced, so a tile wave always has a quarter in
-// flight.  The 4 nt waves after the tiles, four per row block, write V(:,k)
-// and the partial dot products V^H v, W^H v of the block's rows.
-//
-// Each tile wave writes its partial sums into a block of its own, 256
-// doubles at bid * 256: the row sums (Re, Im: 64 each), then the column sums
-// (Re, Im).  Consecutive waves so write consecutive memory.  The writes are
-// about 3% of the kernel's bytes but cost far more inside its read stream: on
-// the order-12445 trailing matrix the kernel takes 222 us without them, 268
-// us with the sums laid out as tiles x n vectors (every 512-byte segment in
-// another place) and 251 us with this layout.
-__device__ __forceinline__ double dbl_readlane(double v, int src)
-{
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b & 0xffffffffll), src);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)((unsigned long long)b >> 32), src);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// columns of the tile taken per step of the SYMV's tile loop (8-column steps
-// at four or five waves per SIMD measured slower on the 100-atom cell)
-constexpr int ZQC = 16;
-static_assert(ZQC == 16, "the column sums take 32 entries per step");
-
-__global__ __launch_bounds__(64, 3) void k_ztri_symv(ZTriWork g, int i, int nt)
-{
-  const int n = g.n, r0 = i + 1, ii = i - g.p0, nb = g.nb;
-  const int lane = threadIdx.x;
-  const int nblk = nt * (nt + 1) / 2;
-  const int bid = blockIdx.x;
-  const double *air = g.ar + (size_t)n * i, *aii = g.ai + (size_t)n * i;
-  // tile waves: the tile (I, J), J <= I, and its first 16 columns, loaded
-  // before the reflector is formed so that their latency overlaps it
-  const bool tile = bid < nblk;
-  int I = 0, J = 0;
-  if (tile) {
-    I = (int)((sqrt(8.0 * (double)bid + 1.0) - 1.0) * 0.5);
-    while ((I + 1) * (I + 2) / 2 <= bid) I++;
-    while (I * (I + 1) / 2 > bid) I--;
-    J = bid - I * (I + 1) / 2;
-  }
-  const int C0t = r0 + SYMV_T * J;
-  const int mt = min(SYMV_T, n - C0t);
-  const int Rlt = min(r0 + SYMV_T * I + lane, n - 1);
-  const double *apr = g.ar + (size_t)Rlt + (size_t)n * C0t, *api = g.ai + (size_t)Rlt + (size_t)n * C0t;
-  double q[2 * ZQC];  // q[j] = Re A(R, C0 + c0 + j), q[ZQC + j] = Im
-  if (tile) {
-#pragma unroll
-    for (int j = 0; j < ZQC; j++) {
-      const int jj = min(j, mt - 1);
-      q[j] = apr[(size_t)n * jj];
-      q[ZQC + j] = api[(size_t)n * jj];
-    }
-  }
-  double sr, si;
-  ztri_reflector(g, i, lane, bid == 0, sr, si);
-  // v(x): 1 at r0, A(x, i) (sr + i si) below it, 0 outside [r0, n)
-  auto vof = [&](int x, double &vr, double &vi) {
-    const int xc = min(max(x, r0), n - 1);
-    const double ar = air[xc], ai = aii[xc];
-    vr = 0.0;
-    vi = 0.0;
-    if (x == r0) {
-      vr = 1.0;
-    } else if (x > r0 && x < n) {
-      vr = ar * sr - ai * si;
-      vi = ar * si + ai * sr;
-    }
-  };
-  if (bid >= nblk) {
-    // four waves per row block: V then W, each Re then Im of conj(X(R,k)) v(R)
-    const int I = (bid - nblk) >> 2, pass = (bid - nblk) & 3;
-    const int R = r0 + SYMV_T * I + lane;
-    const bool live = R < n;
-    const int Rs = live ? R : r0;
-    double vrr, vri;
-    vof(R, vrr, vri);
-    if (pass == 0) {
-      double *Vr = g.Pr + (size_t)n * ii, *Vi = g.Pi + (size_t)n * ii;
-      double *V2r = g.Pr + (size_t)n * (2 * nb + ii), *V2i = g.Pi + (size_t)n * (2 * nb + ii);
-      if (live) { Vr[R] = vrr; Vi[R] = vri; V2r[R] = vrr; V2i[R] = vri; }
-      for (int q = I * SYMV_T + lane; q < r0; q += nt * SYMV_T) { Vr[q] = 0.0; Vi[q] = 0.0; V2r[q] = 0.0; V2i[q] = 0.0; }
-    }
-    if (ii > 0) {
-      double *dr = g.dotr + (size_t)I * 2 * TNB, *di = g.doti + (size_t)I * 2 * TNB;
-      const int half = pass >> 1, im = pass & 1;
-      const double *Xr = g.Pr + (size_t)n * (half * nb), *Xi = g.Pi + (size_t)n * (half * nb);
-      double t[TNB];  // 32 values per wave keep the branch's registers at the tile loop's level
-#pragma unroll
-      for (int k = 0; k < TNB; k++) {
-        const double ur = Xr[(size_t)n * k + Rs], ui = Xi[(size_t)n * k + Rs];
-        const bool use = live && k < ii;
-        t[k] = use ? (im ? ur * vri - ui * vrr : ur * vrr + ui * vri) : 0.0;
-      }
-      const double sq = wave_transpose_sum32x(t, lane);  // lanes 2k, 2k + 1: column k
-      if (!(lane & 1)) (im ? di : dr)[half * TNB + (lane >> 1)] = sq;
-    }
-    return;
-  }
-  const int R = r0 + SYMV_T * I + lane;
-  const int C0 = r0 + SYMV_T * J;
-  const bool live = R < n;
-  const bool off = (I != J);
-  const int m = min(SYMV_T, n - C0);
-  double vcr, vci, vrr, vri;
-  vof(C0 + lane, vcr, vci);  // v of the lane's column
-  vof(R, vrr, vri);          // v of the lane's row
-  double yr = 0.0, yi = 0.0, vyc = 0.0;
-  // a full off-diagonal tile (all 64 rows and columns inside the matrix)
-  // needs no masks; wave-uniform
-  const bool full = off && m == SYMV_T && r0 + SYMV_T * (I + 1) <= n;
-  // only the lower triangle of the trailing matrix is kept current: a
-  // diagonal tile uses its lower part by rows and its strict lower part by
-  // columns (A^H v), the column sums folded into the rows they belong to
-#pragma unroll 1
-  for (int c0 = 0; c0 < m; c0 += ZQC) {  // steps of ZQC columns (wave-uniform); q holds step c0
-    if (!full) {
-#pragma unroll
-      for (int j = 0; j < ZQC; j++) {
-        const bool ok = live && c0 + j < m && (off || c0 + j <= lane);
-        q[j] = ok ? q[j] : 0.0;
-        q[ZQC + j] = ok ? q[ZQC + j] : 0.0;
-      }
-    }
-    {
-      // four independent accumulator pairs (a chain of 8 multiply-adds
-      // instead of 32 per quarter), added in a fixed order
-      double ar[4] = {0.0, 0.0, 0.0, 0.0}, ai[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int j = 0; j < ZQC; j++)
-        cmad(q[j], q[ZQC + j], dbl_readlane(vcr, c0 + j), dbl_readlane(vci, c0 + j), ar[j & 3], ai[j & 3]);
-      yr += (ar[0] + ar[1]) + (ar[2] + ar[3]);
-      yi += (ai[0] + ai[1]) + (ai[2] + ai[3]);
-    }
-#pragma unroll
-    for (int j = 0; j < ZQC; j++) {  // conj(A(R,c)) v(R); the diagonal tile's diagonal only by rows
-      const bool use = off || c0 + j < lane;
-      const double ar = q[j], ai = q[ZQC + j];
-      q[j] = use ? ar * vrr + ai * vri : 0.0;
-      q[ZQC + j] = use ? ar * vri - ai * vrr : 0.0;
-    }
-    // lanes 2e and 2e + 1: entry e summed over the wave (Re of column e in
-    // lanes 0..31, Im of column e - 16 in lanes 32..63)
-    const double cs = wave_transpose_sum32x(q, lane);
-    if (c0 + ZQC < m) {  // the next step's columns (q is free again)
-#pragma unroll
-      for (int j = 0; j < ZQC; j++) {
-        const int jj = min(c0 + ZQC + j, m - 1);
-        q[j] = apr[(size_t)n * jj];
-        q[ZQC + j] = api[(size_t)n * jj];
-      }
-    }
-    if (off) {
-      const double co = xor32(cs, lane);  // the other part of the same column
-      const int cl = c0 + ((lane >> 1) & (ZQC - 1));
-      if (!(lane & 1) && cl < m) g.part[(size_t)bid * 256 + 128 + ((lane & 32) ? 64 : 0) + cl] = cs;
-      const double vcl_r = __shfl(vcr, cl, 64), vcl_i = __shfl(vci, cl, 64);
-      if (lane < 32 && !(lane & 1) && cl < m) vyc += vcl_r * cs + vcl_i * co;  // Re(conj(v_c) (A^H v)_c)
-    } else {
-      // column c0 + j of the tile is row C0 + c0 + j: lane c0 + j takes it
-      const int src = lane - c0;
-      const bool mine = src >= 0 && src < ZQC;
-      const double fr = __shfl(cs, mine ? 2 * src : 0, 64), fi = __shfl(cs, mine ? 32 + 2 * src : 32, 64);
-      if (mine) {
-        yr += fr;
-        yi += fi;
-      }
-    }
-  }
-  if (live) {
-    g.part[(size_t)bid * 256 + lane] = yr;
-    g.part[(size_t)bid * 256 + 64 + lane] = yi;
-  }
-  double vy = vrr * yr + vri * yi + vyc;  // Re(conj(v) y)
-  vy = wave_sum(vy);
-  if (lane == 0) g.vy[bid] = vy;
-}
-
-// Finish W(:, fin - p0) (fin >= 0) and update column col (col >= 0) with the
-// panel so far (ZLATRD); write the squared-norm partial of its
-// sub-subdiagonal part per block (ZLARFG itself is evaluated by the next
-// SYMV's waves).  A block takes ZCOL_ROWS = 64 consecutive rows, one per
-// lane, in each of its ZCOL_WAVES waves, so that every load of a SYMV partial
-// or a panel column is one contiguous 512-byte row segment; the waves split
-// the SYMV partials (chunk w, w + 8, ...) and the panel columns (four each)
-// and their row sums meet in LDS.  Loads are issued in batches with clamped
-// indices and masked values, so that a batch is in flight at once.
-constexpr int ZCOL_WAVES = 8;
-static_assert(ZCOL_ROWS == SYMV_T, "a column-kernel block reads the partials of one SYMV row block");
-
-// offset of partial c (c < nt) of the rows of SYMV row block I, Re (Im at
-// +64): the row sums of tile (I, c) for c <= I, else the column sums of tile
-// (c, I); the lane's row at + lane
-__device__ __forceinline__ size_t zpart_off(int I, int c)
-{
-  return c <= I ? (size_t)(I * (I + 1) / 2 + c) * 256 : (size_t)(c * (c + 1) / 2 + I) * 256 + 128;
-}
-
-__global__ __launch_bounds__(64 * ZCOL_WAVES) void k_ztri_col(ZTriWork g, int fin, int col, int ntile, int nch,
-                                                              int nvy)
-{
-  constexpr int NT = 64 * ZCOL_WAVES;   // threads
-  constexpr int KW = TNB / ZCOL_WAVES;  // panel columns per wave
-  constexpr int YB = 16;                // SYMV-partial chunks per wave and batch
-  constexpr int VB = 10;                // first batch of v^H y pairs per thread (nvy <= 2 NT VB)
-  constexpr int DG = NT / 32;           // groups of the V^H v, W^H v sums (32 column pairs each)
-  constexpr int DB = 8;                 // first batch of tiles per group (ntile <= DG DB)
-  const int n = g.n, p0 = g.p0, nb = g.nb, t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int rbase = fin >= 0 ? fin + 1 : col;
-  const int r = rbase + blockIdx.x * ZCOL_ROWS + lane;
-  const bool live = r < n;
-  const int rs = live ? r : rbase;
-  const int ii = fin >= 0 ? fin - p0 : -1;
-  const int jj = col - p0;
-  __shared__ double abr[2 * TNB], abi[2 * TNB];  // a_k = V_k^H v, b_k = W_k^H v
-  __shared__ double wcr[TNB], wci[TNB], vcr[TNB], vci[TNB];
-  __shared__ double dred[2][DG][2 * TNB];
-  __shared__ double red[6][ZCOL_WAVES][ZCOL_ROWS];  // per wave: y, z (W a + V b), a0 (re, im)
-  __shared__ double sh[3][ZCOL_WAVES];
-  const double *Vr = g.Pr, *Vi = g.Pi, *Wr = g.Pr + (size_t)n * nb, *Wi = g.Pi + (size_t)n * nb;
-  double *acr = g.ar + (size_t)n * (col >= 0 ? col : 0), *aci = g.ai + (size_t)n * (col >= 0 ? col : 0);
-  // ---- per-block scalars: column col of the panel, v^H y, V^H v and W^H v
-  if (col >= 0 && t < jj) {
-    vcr[t] = Vr[(size_t)n * t + col];
-    vci[t] = Vi[(size_t)n * t + col];
-    if (t < ii || fin < 0) {
-      wcr[t] = Wr[(size_t)n * t + col];
-      wci[t] = Wi[(size_t)n * t + col];
-    }
-  }
-  if (fin >= 0) {
-    // v^H y: every partial once, in pairs
-    {
-      const int vlast = (nvy - 1) & ~1;
-      double2 xv[VB];
-#pragma unroll
-      for (int u = 0; u < VB; u++) xv[u] = *reinterpret_cast<const double2 *>(g.vy + min(2 * t + 2 * NT * u, vlast));
-      double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-      for (int u = 0; u < VB; u++) {
-        const int j = 2 * t + 2 * NT * u;
-        s0 += (j < nvy) ? xv[u].x : 0.0;
-        s1 += (j + 1 < nvy) ? xv[u].y : 0.0;
-      }
-      for (int j = 2 * t + 2 * NT * VB; j < nvy; j += 2 * NT) {
-        s0 += g.vy[j];
-        s1 += (j + 1 < nvy) ? g.vy[j + 1] : 0.0;
-      }
-      const double vs = wave_sum(s0 + s1);
-      if (lane == 0) sh[0][w] = vs;
-    }
-    // row col's SYMV partials (for W(col, ii))
-    if (col >= 0) {
-      double pr = 0.0, pi = 0.0;
-      for (int c = t; c < nch; c += NT) {  // row col is row 0 of row block 0
-        const size_t o = zpart_off(0, c);
-        pr += g.part[o];
-        pi += g.part[o + 64];
-      }
-      pr = wave_sum(pr);
-      pi = wave_sum(pi);
-      if (lane == 0) {
-        sh[1][w] = pr;
-        sh[2][w] = pi;
-      }
-    }
-    // V^H v, W^H v: columns 2dq, 2dq + 1 of tiles dp, dp + DG, ...
-    {
-      const int dq = t & 31, dp = t >> 5;
-      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-      {
-        double2 xd[DB], zd[DB];
-#pragma unroll
-        for (int u = 0; u < DB; u++) {
-          const size_t o = (size_t)min(dp + DG * u, ntile - 1) * 2 * TNB + 2 * dq;
-          xd[u] = *reinterpret_cast<const double2 *>(g.dotr + o);
-          zd[u] = *reinterpret_cast<const double2 *>(g.doti + o);
-        }
-#pragma unroll
-        for (int u = 0; u < DB; u++) {
-          const bool k = dp + DG * u < ntile;
-          s0 += k ? xd[u].x : 0.0;
-          s1 += k ? xd[u].y : 0.0;
-          s2 += k ? zd[u].x : 0.0;
-          s3 += k ? zd[u].y : 0.0;
-        }
-      }
-      for (int b = dp + DG * DB; b < ntile; b += DG) {
-        const size_t o = (size_t)b * 2 * TNB + 2 * dq;
-        const double2 x = *reinterpret_cast<const double2 *>(g.dotr + o);
-        const double2 z = *reinterpret_cast<const double2 *>(g.doti + o);
-        s0 += x.x;
-        s1 += x.y;
-        s2 += z.x;
-        s3 += z.y;
-      }
-      dred[0][dp][2 * dq] = s0;
-      dred[0][dp][2 * dq + 1] = s1;
-      dred[1][dp][2 * dq] = s2;
-      dred[1][dp][2 * dq + 1] = s3;
-    }
-  }
-  // ---- this wave's share of the rows' sums
-  double kvr[KW], kvi[KW], kwr[KW], kwi[KW];  // V(r, k), W(r, k), k = KW w + u
-#pragma unroll
-  for (int u = 0; u < KW; u++) {
-    const size_t o = (size_t)n * (KW * w + u) + rs;
-    kvr[u] = Vr[o];
-    kvi[u] = Vi[o];
-    kwr[u] = Wr[o];
-    kwi[u] = Wi[o];
-  }
-  double yr = 0.0, yi = 0.0;
-  if (fin >= 0) {
-    for (int c0 = w; c0 < nch; c0 += ZCOL_WAVES * YB) {
-      double xr[YB], xi[YB];
-#pragma unroll
-      for (int u = 0; u < YB; u++) {
-        const size_t o = zpart_off(blockIdx.x, min(c0 + ZCOL_WAVES * u, nch - 1)) + lane;
-        xr[u] = g.part[o];
-        xi[u] = g.part[o + 64];
-      }
-#pragma unroll
-      for (int u = 0; u < YB; u++) {  // rows past n: never written, selected away
-        const bool k = live && c0 + ZCOL_WAVES * u < nch;
-        yr += k ? xr[u] : 0.0;
-        yi += k ? xi[u] : 0.0;
-      }
-    }
-  }
-  __syncthreads();
-  if (fin >= 0 && t < 2 * TNB) {
-    double qr = 0.0, qi = 0.0;
-#pragma unroll
-    for (int p = 0; p < DG; p++) {
-      qr += dred[0][p][t];
-      qi += dred[1][p][t];
-    }
-    const bool use = (t & (TNB - 1)) < ii;
-    abr[t] = use ? qr : 0.0;
-    abi[t] = use ? qi : 0.0;
-  }
-  __syncthreads();
-  {
-    double zr = 0.0, zi = 0.0, a0r = 0.0, a0i = 0.0;
-#pragma unroll
-    for (int u = 0; u < KW; u++) {
-      const int k = KW * w + u;
-      if (fin >= 0 && k < ii) {  // W(r,k) a_k + V(r,k) b_k
-        zr += kwr[u] * abr[k] - kwi[u] * abi[k] + kvr[u] * abr[TNB + k] - kvi[u] * abi[TNB + k];
-        zi += kwr[u] * abi[k] + kwi[u] * abr[k] + kvr[u] * abi[TNB + k] + kvi[u] * abr[TNB + k];
-      }
-      // V(r,k) conj(W(col,k)) + W(r,k) conj(V(col,k)), k < jj, k != ii; panel
-      // columns k >= jj hold values of an earlier panel (or never written
-      // memory): selected away, never multiplied by zero
-      const bool use = col >= 0 && k < jj && k != ii;
-      const double wcr_ = use ? wcr[min(k, TNB - 1)] : 0.0, wci_ = use ? wci[min(k, TNB - 1)] : 0.0;
-      const double vcr_ = use ? vcr[min(k, TNB - 1)] : 0.0, vci_ = use ? vci[min(k, TNB - 1)] : 0.0;
-      const double vr_ = use ? kvr[u] : 0.0, vi_ = use ? kvi[u] : 0.0;
-      const double wr_ = use ? kwr[u] : 0.0, wi_ = use ? kwi[u] : 0.0;
-      a0r += vr_ * wcr_ + vi_ * wci_ + wr_ * vcr_ + wi_ * vci_;
-      a0i += vi_ * wcr_ - vr_ * wci_ + wi_ * vcr_ - wr_ * vci_;
-    }
-    red[0][w][lane] = yr;
-    red[1][w][lane] = yi;
-    red[2][w][lane] = zr;
-    red[3][w][lane] = zi;
-    red[4][w][lane] = a0r;
-    red[5][w][lane] = a0i;
-  }
-  __syncthreads();
-  // W(q, ii) = 0 above this kernel's rows
-  if (fin >= 0) {
-    double *Wir = g.Pr + (size_t)n * (nb + fin - p0), *Wii = g.Pi + (size_t)n * (nb + fin - p0);
-    for (int q = blockIdx.x * NT + t; q < rbase; q += gridDim.x * NT) {
-      Wir[q] = 0.0;
-      Wii[q] = 0.0;
-    }
-  }
-  if (w != 0) return;
-  // ---- wave 0 finishes its 64 rows
-  double sy[6];
-#pragma unroll
-  for (int a = 0; a < 6; a++) {
-    double s = 0.0;
-#pragma unroll
-    for (int p = 0; p < ZCOL_WAVES; p++) s += red[a][p][lane];
-    sy[a] = s;
-  }
-  double wrr = 0.0, wri = 0.0, viir = 0.0, viii = 0.0, wciir = 0.0, wciii = 0.0;
-  if (fin >= 0) {
-    const double tr = g.taur[fin], ti = g.taui[fin];
-    viir = Vr[(size_t)n * ii + rs];
-    viii = Vi[(size_t)n * ii + rs];
-    double vty = 0.0;
-#pragma unroll
-    for (int p = 0; p < ZCOL_WAVES; p++) vty += sh[0][p];
-    double ssum = 0.0;
-#pragma unroll
-    for (int k = 0; k < TNB; k++) ssum += abr[k] * abr[TNB + k] + abi[k] * abi[TNB + k];
-    const double alpha2 = -0.5 * (tr * tr + ti * ti) * (vty - 2.0 * ssum);
-    const double yr_ = sy[0] - sy[2], yi_ = sy[1] - sy[3];
-    wrr = tr * yr_ - ti * yi_ + alpha2 * viir;
-    wri = tr * yi_ + ti * yr_ + alpha2 * viii;
-    double *Wir = g.Pr + (size_t)n * (nb + ii), *Wii = g.Pi + (size_t)n * (nb + ii);
-    if (live) {
-      Wir[r] = wrr;
-      Wii[r] = wri;
-    }
-    if (col >= 0) {
-      // row col = fin + 1 of the same formula (v(col) = 1), in every lane
-      double cr = 0.0, ci = 0.0;
-      for (int k = 0; k < ii; k++) {
-        cr += wcr[k] * abr[k] - wci[k] * abi[k] + vcr[k] * abr[TNB + k] - vci[k] * abi[TNB + k];
-        ci += wcr[k] * abi[k] + wci[k] * abr[k] + vcr[k] * abi[TNB + k] + vci[k] * abr[TNB + k];
-      }
-      double pr = 0.0, pi = 0.0;
-#pragma unroll
-      for (int p = 0; p < ZCOL_WAVES; p++) {
-        pr += sh[1][p];
-        pi += sh[2][p];
-      }
-      const double sr = pr - cr, si = pi - ci;
-      wciir = tr * sr - ti * si + alpha2;
-      wciii = tr * si + ti * sr;
-    }
-  }
-  if (col < 0) return;
-  double xr = acr[rs], xi = aci[rs];
-  {
-    double a0r = sy[4], a0i = sy[5];
-    if (fin >= 0) {  // k = ii: this kernel's W(r, ii) and W(col, ii)
-      const double vr_ = vcr[ii], vi_ = vci[ii];
-      a0r += viir * wciir + viii * wciii + wrr * vr_ + wri * vi_;
-      a0i += viii * wciir - viir * wciii + wri * vr_ - wrr * vi_;
-    }
-    xr -= a0r;
-    xi -= a0i;
-  }
-  double nrm = 0.0;
-  if (live && r >= col) {
-    if (r == col) xi = 0.0;
-    acr[r] = xr;
-    aci[r] = xi;
-    if (r == col) {
-      g.d[col] = xr;
-      if (col >= n - 1) {
-        g.taur[col] = 0.0;
-        g.taui[col] = 0.0;
-        g.scr[col] = 0.0;
-        g.sci[col] = 0.0;
-      }
-    }
-    if (r >= col + 2) nrm = xr * xr + xi * xi;
-  }
-  nrm = wave_sum(nrm);
-  if (lane == 0) g.norm[blockIdx.x] = nrm;
-}
-
-__global__ void k_ztri_store(ZTriWork g, int ncols)
-{
-  const int n = g.n;
-  const int k = blockIdx.y;
-  const int i = g.p0 + k;
-  const int r = i + 2 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= ncols || r >= n) return;
-  g.ar[(size_t)r + (size_t)n * i] = g.Pr[(size_t)n * k + r];
-  g.ai[(size_t)r + (size_t)n * i] = g.Pi[(size_t)n * k + r];
-}
-
 // ------------------------------------------------------------------ back-transforms
 __global__ void k_zvpanel(int n, int p0, int nb, const double *__restrict__ ar, const double *__restrict__ ai,
                           double *__restrict__ vr, double *__restrict__ vi)
@@ -890,8 +344,8 @@ __global__ void k_zvpanel(int n, int p0, int nb, const double *__restrict__ ar, 
   if (r >= n || k >= nb) return;
   const int i = p0 + k;
   double xr = 0.0, xi = 0.0;
-  if (r == i + 1) xr = 1.0;
-  else if (r > i + 1) { xr = ar[(size_t)r + (size_t)n * i]; xi = ai[(size_t)r + (size_t)n * i]; }
+  if (r == i + BND) xr = 1.0;
+  else if (r > i + BND) { xr = ar[(size_t)r + (size_t)n * i]; xi = ai[(size_t)r + (size_t)n * i]; }
   vr[(size_t)r + (size_t)n * k] = xr;
   vi[(size_t)r + (size_t)n * k] = xi;
 }
@@ -1049,82 +503,17 @@ int seclr4_complex(Ctx &c, double el, double eu, int nume, int *ne_out, int *nbe
     W2K_STAGE(s, "k_zmirror_lower");
   }
   W2K_HIP(hipEventRecord(c.ev[8], s));
-  // ---- 3. Hermitian tridiagonalisation of C (in H)
-  const int nts = B.nt;
-  ZTriWork g;
-  g.n = n; g.ar = Hr; g.ai = Hi;
-  g.Pr = B.P; g.Pi = B.P + (size_t)3 * n * TNB;
+  // ---- 3. Hermitian tridiagonalisation of C (in H): band, then bulge chasing
+  SbArgs g;
+  if ((rc = sb_buffers(c, g, n, 1))) return rc;
+  g.lda = n; g.ar = Hr; g.ai = Hi;
+  g.Pr = B.P; g.Pi = B.P + (size_t)3 * n * BND;
   g.d = B.d; g.e = B.e;
   g.taur = B.tau; g.taui = B.tau + n;
-  g.scr = B.scal; g.sci = B.scal + n;
-  g.part = B.part;
-  g.dotr = B.tdots; g.doti = B.tdots + (size_t)nts * 2 * TNB;
-  g.vy = B.tvy; g.norm = B.tnorm; g.counter = B.ticket;
-  // optional per-launch events around the SYMV (kernel-level roofline)
-  const bool kt = c.ktime != 0;
-  if (kt && c.kev.size() < (size_t)2 * n) {
-    const size_t old = c.kev.size();
-    c.kev.resize((size_t)2 * n);
-    for (size_t q = old; q < c.kev.size(); q++) W2K_HIP(hipEventCreate(&c.kev[q]));
-  }
-  int nsymv = 0;
-  for (int p0 = 0; p0 < n; p0 += TNB) {
-    const int nb = std::min(TNB, n - p0);
-    g.p0 = p0;
-    g.nb = nb;
-    hipLaunchKernelGGL(k_ztri_col, dim3((n - p0 + ZCOL_ROWS - 1) / ZCOL_ROWS), dim3(64 * ZCOL_WAVES), 0, s, g, -1, p0, 0,
-                       0, 0);
-    W2K_STAGE(s, "k_ztri_col");
-    int nref = 0;
-    for (int k = 0; k < nb; k++) {
-      const int i = p0 + k;
-      if (i >= n - 1) break;
-      nref = k + 1;
-      const int rows = n - (i + 1);
-      const int nt = (rows + SYMV_T - 1) / SYMV_T, nblk = nt * (nt + 1) / 2;
-      // timed launches carry their events in the dispatch itself
-      if (kt) hipExtLaunchKernelGGL(k_ztri_symv, dim3(nblk + 4 * nt), dim3(SYMV_T), 0, s, c.kev[2 * nsymv],
-                                    c.kev[2 * nsymv + 1], 0, g, i, nt);
-      else hipLaunchKernelGGL(k_ztri_symv, dim3(nblk + 4 * nt), dim3(SYMV_T), 0, s, g, i, nt);
-      W2K_STAGE(s, "k_ztri_symv");
-      nsymv++;
-      const int next = (k + 1 < nb) ? i + 1 : -1;
-      hipLaunchKernelGGL(k_ztri_col, dim3((rows + ZCOL_ROWS - 1) / ZCOL_ROWS), dim3(64 * ZCOL_WAVES), 0, s, g, i,
-                         next, nt, nt, nblk);
-      W2K_STAGE(s, "k_ztri_col");
-    }
-    if (nref > 0) {
-      hipLaunchKernelGGL(k_ztri_store, dim3((n + 255) / 256, nref), dim3(256), 0, s, g, nref);
-      W2K_STAGE(s, "k_ztri_store");
-    }
-    const int p1 = p0 + nb;
-    if (p1 < n) {
-      // A(p1:n, p1:n) -= [V W] [W V]^H, lower triangle
-      const int r = n - p1;
-      const size_t o1 = (size_t)p1 + (size_t)n * p1, ow = (size_t)n * nb + p1;
-      if ((rc = zgemm(s, 'N', 'C', r, r, 2 * nb, -1.0, g.Pr + p1, g.Pi + p1, n, g.Pr + ow, g.Pi + ow, n, 1.0, Hr + o1,
-                      Hi + o1, n, 1)))
-        return rc;
-    }
-  }
+  g.V2r = Ur; g.V2i = Ui;  // U is not needed after the inversion
+  if ((rc = sb_reduce(c, s, g, 1))) return rc;
   W2K_HIP(hipEventRecord(c.ev[9], s));
-  if (kt) {
-    // [10] summed SYMV kernel time, [11] number of SYMV launches
-    W2K_HIP(hipStreamSynchronize(s));
-    double tot = 0.0;
-    int cntl = 0;
-    for (int q = 0; q < nsymv; q++) {
-      float ms = 0.f;
-      if (hipEventElapsedTime(&ms, c.kev[2 * q], c.kev[2 * q + 1]) != hipSuccess) {
-        (void)hipGetLastError();
-        break;
-      }
-      tot += ms;
-      cntl++;
-    }
-    c.last_ms[10] = tot;
-    c.last_ms[11] = cntl;
-  }
+  if ((rc = sb_take_times(c, s, n))) return rc;
   // ---- 4./5. real tridiagonal eigenpairs (shared with the real build)
   double *Zt = Xr;  // n x m real, then the real part of Q Zt
   double *Zi = Xi;  // imaginary part of Q Zt
@@ -1139,6 +528,7 @@ int seclr4_complex(Ctx &c, double el, double eu, int nume, int *ne_out, int *nbe
     const size_t zc = (size_t)n * m;
     hipLaunchKernelGGL(k_zfill, dim3((unsigned)((zc + 255) / 256)), dim3(256), 0, s, zc, Zi, 0.0);
     W2K_STAGE(s, "k_zfill");
+    if ((rc = sb_apply_q2(c, s, g, 1, m, Zt, Zi, n))) return rc;
     // blocks of ZBT reflectors (the launches of a block, not its arithmetic,
     // set the pace at these orders: 64-reflector blocks halve them)
     constexpr int ZBT = 64;
@@ -1163,7 +553,7 @@ int seclr4_complex(Ctx &c, double el, double eu, int nume, int *ne_out, int *nbe
     q += 2 * ZBT * ZBT;
     double *y1r = q, *y1i = y1r + (size_t)ZBT * m, *y2r = y1i + (size_t)ZBT * m, *y2i = y2r + (size_t)ZBT * m;
     double *gws = y2i + (size_t)ZBT * m;
-    const int nref = n - 1;
+    const int nref = std::max(0, n - BND - 1);  // reflectors of Q1; v_i starts at row i + BND
     const int nblk = nref > 0 ? (nref + ZBT - 1) / ZBT : 0;
     hipStream_t sa = c.aux;
     auto p0_of = [&](int k) { return (nblk - 1 - k) * ZBT; };
@@ -1172,9 +562,9 @@ int seclr4_complex(Ctx &c, double el, double eu, int nume, int *ne_out, int *nbe
       if (k >= 2) W2K_HIP(hipStreamWaitEvent(sa, c.bt_used[u], 0));
       hipLaunchKernelGGL(k_zvpanel, dim3((n + 255) / 256, nb), dim3(256), 0, sa, n, p0, nb, Hr, Hi, vr[u], vi[u]);
       W2K_STAGE(sa, "k_zvpanel");
-      // rows 0 .. p0 of the block's reflectors are zero: the products start at
-      // row p0+1 rounded down to 16 rows, which keeps the operands' 128-byte alignment
-      const int o = (p0 + 1) & ~15, nr = n - o;
+      // the block's reflectors are zero above row p0+BND: the products start at
+      // that row rounded down to 16 rows, which keeps the operands' 128-byte alignment
+      const int o = (p0 + BND) & ~15, nr = n - o;
       int r2;
       if ((r2 = zgemm(sa, 'C', 'N', nb, nb, nr, 1.0, vr[u] + o, vi[u] + o, n, vr[u] + o, vi[u] + o, n, 0.0, gmr, gmi,
                       nb, 0, 0, 0, gws, GWS)))
@@ -1194,7 +584,7 @@ int seclr4_complex(Ctx &c, double el, double eu, int nume, int *ne_out, int *nbe
     }
     for (int k = 0; k < nblk; k++) {
       const int u = k & 1, p0 = p0_of(k), nb = std::min(ZBT, nref - p0);
-      const int o = (p0 + 1) & ~15, nr = n - o;  // the block's reflectors are zero above row p0+1
+      const int o = (p0 + BND) & ~15, nr = n - o;  // the block's reflectors are zero above row p0+BND
       W2K_HIP(hipStreamWaitEvent(s, c.bt_ready[u], 0));
       if ((rc = zgemm(s, 'C', 'N', nb, m, nr, 1.0, vr[u] + o, vi[u] + o, n, Zt + o, Zi + o, n, 0.0, y1r, y1i, nb, 0,
                       0, 0, ws, wsn)))

@@ -9,14 +9,6 @@
 namespace w2k {
 
 constexpr int NB = 64;      // Cholesky / inversion block
-constexpr int TNB = 32;     // tridiagonalisation panel
-constexpr int SYMV_T = 64;  // tile of the symmetric / Hermitian SYMV (one wave)
-
-__device__ __forceinline__ double wave_sum(double v)
-{
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
-}
 
 // v from the partner lane of a halving step with stride S: any lane that has
 // bit S flipped and the bits above S unchanged will do, so the short strides
@@ -40,60 +32,6 @@ __device__ __forceinline__ double bfly_partner(double v)
     }
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
   }
-}
-
-// One halving step of a wave-wide reduce-scatter: lanes with bit S set keep
-// entries S..2S-1, the others keep 0..S-1, and each adds the half that its
-// partner lane gives away.
-template <int S>
-__device__ __forceinline__ void bfly_step(double *t, int lane)
-{
-  const bool hi = (lane & S) != 0;
-#pragma unroll
-  for (int j = 0; j < S; j++) {
-    const double keep = hi ? t[j + S] : t[j];
-    const double send = hi ? t[j] : t[j + S];
-    t[j] = keep + bfly_partner<S>(send);
-  }
-}
-
-// t[0..63] per lane -> returns, in lane l, the sum over the 64 lanes of t[l]
-// (a transpose-and-sum in six halving steps, no LDS).  Overwrites t.
-__device__ __forceinline__ double wave_transpose_sum(double *t, int lane)
-{
-  bfly_step<32>(t, lane);
-  bfly_step<16>(t, lane);
-  bfly_step<8>(t, lane);
-  bfly_step<4>(t, lane);
-  bfly_step<2>(t, lane);
-  bfly_step<1>(t, lane);
-  return t[0];
-}
-
-// t[0..31] per lane -> returns, in lane l, the sum over the 64 lanes of
-// t[l % 32] (five halving steps within each 32-lane half, then the halves
-// added).  Overwrites t.
-__device__ __forceinline__ double wave_transpose_sum32(double *t, int lane)
-{
-  bfly_step<16>(t, lane);
-  bfly_step<8>(t, lane);
-  bfly_step<4>(t, lane);
-  bfly_step<2>(t, lane);
-  bfly_step<1>(t, lane);
-  return t[0] + __shfl_xor(t[0], 32, 64);
-}
-
-// t[0..15] per lane -> returns, in lane l, the sum over the 64 lanes of
-// t[l % 16] (four halving steps within each 16-lane group, then the groups
-// added).  Overwrites t.
-__device__ __forceinline__ double wave_transpose_sum16(double *t, int lane)
-{
-  bfly_step<8>(t, lane);
-  bfly_step<4>(t, lane);
-  bfly_step<2>(t, lane);
-  bfly_step<1>(t, lane);
-  const double s = t[0] + __shfl_xor(t[0], 16, 64);
-  return s + __shfl_xor(s, 32, 64);
 }
 
 // One halving step with the lane bit S of a permlane swap (S = 16: gfx950
@@ -168,21 +106,19 @@ __device__ __forceinline__ double wave_transpose_sum32x(double *t, int lane)
 // device work buffers of one SECLR4 call (carved from Ctx::w_small / w_int);
 // complex quantities are planar: real parts, then imaginary parts at +stride
 struct Seclr4Bufs {
-  int n = 0, nt = 0;        // order, SYMV tiles per dimension
+  int n = 0;                // order
   int cplx = 0;
   double *d, *e, *e2;       // tridiagonal (real in both builds), squared off-diagonals
-  double *tau, *scal;       // reflector scalars (complex: re[n], im[n])
+  double *tau;              // reflector scalars (complex: re[n], im[n])
   double *wv;               // eigenvalues (block order, then sorted)
-  double *P;                // panel buffer n x 3 TNB (complex: twice)
-  double *part;             // SYMV partials: 128 (complex 256) per tile of the lower triangle
-  double *tdots;            // nt x 2 TNB (complex: twice)
-  double *tvy;              // nt (nt + 1) / 2
-  double *tnorm;            // nt
+  double *P;                // panel buffer n x 3 BND (complex: twice)
   double *bgl, *bgu, *batol, *bnrm, *xs, *pivmin;
   int *info, *cnt, *ticket, *tblk, *tidx, *bstart, *bend, *cstart, *perm;
 };
 
-// allocate and carve the work buffers; zero INFO, counts and tickets
+// doubles of those buffers
+size_t seclr4_doubles(size_t n, int cplx);
+// allocate and carve the work buffers; zero INFO and counts
 int seclr4_buffers(Ctx &c, int n, int cplx, Seclr4Bufs &B);
 
 // bisection (window (el, eu], NUME cap, NBELW) on B.d/B.e, inverse iteration

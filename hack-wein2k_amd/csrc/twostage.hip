@@ -1,0 +1,1490 @@
+// Two-stage reduction of the standard-form matrix C to tridiagonal form, for
+// both builds (CX: complex Hermitian, planar; else real symmetric):
+//   1. C = Q1 B Q1^H, B of bandwidth BND: per BND columns a Householder QR of the
+//      panel below the band (k_sb_qr) and one rank-2 BND update of the trailing
+//      matrix, so that the matrix is read by products instead of by one
+//      matrix-vector product per column;
+//   2. B = Q2 T Q2^H by bulge chasing (k_sb_chase), T real tridiagonal;
+//   3. the vectors of T are multiplied by Q2 here (sb_apply_q2) and by Q1 in
+//      the drivers' back-transform.
+// The reference reduces column by column (dsytrd2.f, zheevx2.f:305-367); both
+// give an orthogonally similar T, so eigenvalues agree to rounding and
+// eigenvectors up to the phase that they are determined to.
+//
+// Column by column the matrix is read once per column (HBM bound at large
+// orders, 4.5 TB/s) through two dependent launches per column (12-24 us at
+// small ones).  Here a panel of BND columns takes six launches, the flops are
+// matrix products, and the serial part is 32 short exchanges per panel and
+// two steps per sweep.  Whole reduction, before -> now (Q2's application in
+// brackets): real N = 221 3.1 -> 1.8 ms, N = 731 10.7 -> 7.4, N = 5951 135 ->
+// 79 (+ 11); complex N = 251 5.4 -> 2.9, N = 1950 47 -> 28 (+ 2), N = 10880
+// 1018 -> 374 (+ 161).
+#include <algorithm>
+#include <cmath>
+
+#include <hip/hip_ext.h>
+
+#include "seclr4_shared.h"
+#include "twostage.h"
+
+namespace w2k {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// ------------------------------------------------------------------ device-wide words
+// Data exchanged between work-groups of a running kernel goes through relaxed
+// agent-scope accesses, which pass the XCDs' private L2 caches; a wave orders
+// its stores before a later flag with vm_drain().
+__device__ __forceinline__ double agent_ld(const double *p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int agent_ld(const int *p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_st(double *p, double v)
+{
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_st(int *p, int v)
+{
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// every vector memory access of this wave done (vmcnt = 0)
+__device__ __forceinline__ void vm_drain()
+{
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+// LDS written by this wave is read by its other lanes
+__device__ __forceinline__ void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Before FP64 MFMA results are read by another instruction: 64 clocks more
+// than the compiler leaves after the last MFMA.  It leaves 19 wait
+// states (16 passes + 3) after its issue; where that MFMA accumulates onto the
+// one just before it, whose end it has to wait for, item 3 of the result was
+// read three passes early.
+__device__ __forceinline__ void mfma_settle()
+{
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_sleep(1);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// sum over the 32 lanes of a half wave, in every lane
+__device__ __forceinline__ double sum32(double v)
+{
+  v = swap_sum<16>(v, v);
+  v += bfly_partner<8>(v);
+  v += bfly_partner<4>(v);
+  v += bfly_partner<2>(v);
+  return v + bfly_partner<1>(v);
+}
+
+// xLARFG of (alpha, x) with |x|^2 = ss: H = I - tau v v^H, H^H (alpha; x) =
+// (beta; 0), v = (1; scale x), beta real
+struct Reflector {
+  double beta, tr, ti, sr, si;
+};
+template <bool CX>
+__device__ __forceinline__ Reflector larfg(double ar, double ai, double ss)
+{
+#pragma clang fp contract(off)  // the same bits wherever it is inlined
+  Reflector h;
+  if (ss == 0.0 && (!CX || ai == 0.0)) {
+    h.beta = ar;
+    h.tr = h.ti = h.sr = h.si = 0.0;
+    return h;
+  }
+  const double nrm = sqrt(CX ? fma(ar, ar, fma(ai, ai, ss)) : fma(ar, ar, ss));
+  const double b = ar >= 0.0 ? -nrm : nrm;
+  h.beta = b;
+  const double rb = 1.0 / b, dr = ar - b;
+  h.tr = (b - ar) * rb;
+  if (CX) {
+    h.ti = -ai * rb;
+    const double rd = 1.0 / fma(dr, dr, ai * ai);
+    h.sr = dr * rd;
+    h.si = -ai * rd;
+  } else {
+    h.ti = h.si = 0.0;
+    h.sr = 1.0 / dr;
+  }
+  return h;
+}
+
+// ------------------------------------------------------------------ 1a. panel QR
+// "not yet written" in the exchange buffer: a NaN pattern that arithmetic does
+// not produce (a value with these bits is published as another NaN)
+constexpr long long SB_EMPTY = 0x7FF8DEADBEEF5A5All;
+constexpr int QR_ROWS = 256;          // rows of a block (one per thread)
+constexpr int SB_CLOSED = 1 << 30;    // registration word: no more work-groups
+constexpr long long QR_WAIT = 3000;   // registration wait, ticks of the 100 MHz counter (30 us)
+
+__global__ void k_sb_reset(double *exch, size_t cnt, int *sync)
+{
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < cnt) exch[i] = __longlong_as_double(SB_EMPTY);
+  if (i < 4) sync[i] = 0;
+}
+
+// values k of blocks b0, b0 + step, .. < nb summed in that order, each taken
+// once it has been written; eight loads in flight
+__device__ __forceinline__ double gather_sum(const double *ex, int b0, int step, int nb, size_t stride)
+{
+  double s = 0.0;
+  for (int b = b0; b < nb; b += 8 * step) {
+    double v[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int bb = b + q * step;
+      v[q] = bb < nb ? agent_ld(ex + (size_t)bb * stride) : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const int bb = b + q * step;
+      while (__double_as_longlong(v[q]) == SB_EMPTY) v[q] = agent_ld(ex + (size_t)bb * stride);
+      if (bb < nb) s += v[q];
+    }
+  }
+  return s;
+}
+
+// Householder QR of the panel A(r0:n, j0:j0+BND), r0 = j0 + BND: R and the
+// reflectors in place, V (unit lower trapezoidal, explicit) to P columns
+// 0..BND-1 and 2 BND..3 BND-1, tau, and G = V^H V above its diagonal.  One row
+// per thread with its BND columns in registers; per column one reduction over
+// all rows gives the norm, the products with the remaining columns and those
+// with the earlier reflectors (G), exchanged between the work-groups through
+// `exch`.  The columns sit rotated: entry k of a row is column j + k
+// (mod BND), earlier reflectors take the place of finished columns.
+//
+// Progress does not depend on all work-groups being resident: a work-group
+// registers when it starts, the first one closes the registration once all
+// have come or QR_WAIT has passed, later ones leave, and the registered ones
+// share the blocks (RES: each has one, held in registers; else all go through
+// memory), with the same sums in the same order either way.
+template <bool CX>
+struct QrShared {
+  static constexpr int NV = CX ? 2 * BND : BND, NG = QR_ROWS / NV;
+  double red[4][NV], piv[NV], cf[NV], part[NG][NV];
+  int share[2];
+};
+
+template <bool CX, bool RES>
+__device__ __forceinline__ void qr_panel(const SbArgs &g, int j0, int nblk, int idx, int np, QrShared<CX> &sh)
+{
+#pragma clang fp contract(off)  // both forms round alike
+  constexpr int NV = QrShared<CX>::NV, NG = QrShared<CX>::NG;
+  const int n = g.n, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r0 = j0 + BND, m = n - r0, nref = min(BND, m - 1);
+  double xr[BND], xi[CX ? BND : 1];
+  double *const pv = g.Pr, *const pvi = g.Pi;
+  // the row's columns in their rotated places at step j
+  auto load = [&](int b, int j) {
+    const int pr = b * QR_ROWS + tid;
+    const bool live = pr < m;
+    const size_t row = r0 + min(pr, m - 1);
+#pragma unroll
+    for (int k = 0; k < BND; k++) {
+      const bool old = k >= BND - j;
+      const size_t o = old ? row + (size_t)n * (j + k - BND) : row + (size_t)g.lda * (j0 + j + k);
+      const double vr = old ? pv[o] : g.ar[o];
+      xr[k] = live ? vr : 0.0;
+      if (CX) {
+        const double vi = old ? pvi[o] : g.ai[o];
+        xi[k] = live ? vi : 0.0;
+      }
+    }
+  };
+  if (RES) load(idx, 0);
+  for (int j = 0; j < nref; j++) {
+    double *const ex = g.exch + (size_t)j * (nblk + 1) * NV;
+    for (int b = idx; b < nblk; b += np) {
+      if (!RES) load(b, j);
+      const int pr = b * QR_ROWS + tid;
+      double t[BND];
+      const double ar = pr > j ? xr[0] : 0.0, ai = CX ? (pr > j ? xi[0] : 0.0) : 0.0;
+#pragma unroll
+      for (int k = 0; k < BND; k++) t[k] = CX ? fma(ar, xr[k], ai * xi[k]) : ar * xr[k];
+      const double s0 = wave_transpose_sum32x(t, lane);
+      if (!(lane & 1)) sh.red[wave][lane >> 1] = s0;
+      if (CX) {
+#pragma unroll
+        for (int k = 0; k < BND; k++) t[k] = fma(ar, xi[k], -(ai * xr[k]));
+        const double s1 = wave_transpose_sum32x(t, lane);
+        if (!(lane & 1)) sh.red[wave][BND + (lane >> 1)] = s1;
+      }
+      if (pr == j) {
+#pragma unroll
+        for (int k = 0; k < BND; k++) {
+          sh.piv[k] = xr[k];
+          if (CX) sh.piv[BND + k] = xi[k];
+        }
+      }
+      __syncthreads();
+      if (nblk > 1) {
+        if (tid < NV) {
+          double s = ((sh.red[0][tid] + sh.red[1][tid]) + sh.red[2][tid]) + sh.red[3][tid];
+          if (__double_as_longlong(s) == SB_EMPTY) s = __longlong_as_double(0x7FF8000000000000ll);
+          agent_st(ex + (size_t)b * NV + tid, s);
+          if (b == 0) {
+            double p = sh.piv[tid];
+            if (__double_as_longlong(p) == SB_EMPTY) p = __longlong_as_double(0x7FF8000000000000ll);
+            agent_st(ex + (size_t)nblk * NV + tid, p);
+          }
+        }
+        if (!RES) __syncthreads();  // red and piv are written again
+      }
+      if (RES) break;
+    }
+    // sum over the rows of conj(x_0) x_k
+    auto total = [&](int k) {
+      if (nblk == 1) return ((sh.red[0][k] + sh.red[1][k]) + sh.red[2][k]) + sh.red[3][k];
+      double s = sh.part[0][k];
+#pragma unroll
+      for (int q = 1; q < NG; q++) s += sh.part[q][k];
+      return s;
+    };
+    if (nblk > 1) {
+      const int k = tid % NV, grp = tid / NV;
+      sh.part[grp][k] = gather_sum(ex + k, grp, NG, nblk, NV);
+      if (grp == NG - 1) sh.piv[k] = gather_sum(ex + (size_t)nblk * NV + k, 0, 1, 1, NV);
+      __syncthreads();
+    }
+    const Reflector h = larfg<CX>(sh.piv[0], CX ? sh.piv[BND] : 0.0, total(0));
+    if (tid < BND) {
+      // v^H x_k = p_k + conj(scale) S_k
+      const double a = total(tid);
+      double wr, wi = 0.0;
+      if (CX) {
+        const double b = total(BND + tid);
+        wr = fma(h.sr, a, fma(h.si, b, sh.piv[tid]));
+        wi = fma(h.sr, b, fma(-h.si, a, sh.piv[BND + tid]));
+      } else {
+        wr = fma(h.sr, a, sh.piv[tid]);
+      }
+      const bool old = tid >= BND - j;  // an earlier reflector: G(i, j) = conj(v_j^H v_i)
+      if (old && idx == 0) {
+        g.G[j + tid - BND + BND * j] = wr;
+        if (CX) g.G[BND * BND + j + tid - BND + BND * j] = -wi;
+      }
+      sh.cf[tid] = old ? 0.0 : (CX ? fma(h.tr, wr, h.ti * wi) : h.tr * wr);  // conj(tau) w
+      if (CX) sh.cf[BND + tid] = old ? 0.0 : fma(h.tr, wi, -(h.ti * wr));
+      if (tid == 0 && idx == 0) {
+        g.taur[j0 + j] = h.tr;
+        if (CX) g.taui[j0 + j] = h.ti;
+      }
+    }
+    __syncthreads();
+    for (int b = idx; b < nblk; b += np) {
+      if (!RES) load(b, j);
+      const int pr = b * QR_ROWS + tid;
+      const double x0r = xr[0], x0i = CX ? xi[0] : 0.0;
+      double vr = pr > j ? (CX ? fma(h.sr, x0r, -(h.si * x0i)) : h.sr * x0r) : (pr == j ? 1.0 : 0.0);
+      double vi = CX && pr > j ? fma(h.sr, x0i, h.si * x0r) : 0.0;
+      if (pr >= m) vr = vi = 0.0;
+#pragma unroll
+      for (int k = 1; k < BND; k++) {
+        const double cr = sh.cf[k];
+        if (CX) {
+          const double ci = sh.cf[BND + k];
+          xr[k - 1] = fma(vi, ci, fma(-vr, cr, xr[k]));
+          xi[k - 1] = fma(-vi, cr, fma(-vr, ci, xi[k]));
+        } else {
+          xr[k - 1] = fma(-vr, cr, xr[k]);
+        }
+      }
+      xr[BND - 1] = vr;
+      if (CX) xi[BND - 1] = vi;
+      if (pr < m) {
+        const size_t row = r0 + pr;
+        const size_t oa = row + (size_t)g.lda * (j0 + j), op = row + (size_t)n * j;
+        g.ar[oa] = pr > j ? vr : (pr == j ? h.beta : x0r);
+        pv[op] = vr;
+        pv[op + (size_t)2 * BND * n] = vr;
+        if (CX) {
+          g.ai[oa] = pr > j ? vi : (pr == j ? 0.0 : x0i);
+          pvi[op] = vi;
+          pvi[op + (size_t)2 * BND * n] = vi;
+        }
+        if (!RES) {
+#pragma unroll
+          for (int k = 1; k < BND; k++) {
+            if (k >= BND - j) continue;
+            g.ar[row + (size_t)g.lda * (j0 + j + k)] = xr[k - 1];
+            if (CX) g.ai[row + (size_t)g.lda * (j0 + j + k)] = xi[k - 1];
+          }
+        }
+      }
+      if (RES) break;
+    }
+  }
+  // columns past the last reflector (short panels, one block): R as it is, V = 0
+  if (RES && nref < BND) {
+    if (tid < m) {
+#pragma unroll
+      for (int k = 0; k < BND; k++) {
+        const int j = nref + k;
+        if (j >= BND) continue;
+        const size_t row = r0 + tid, oa = row + (size_t)g.lda * (j0 + j), op = row + (size_t)n * j;
+        g.ar[oa] = xr[k];
+        pv[op] = 0.0;
+        pv[op + (size_t)2 * BND * n] = 0.0;
+        if (CX) {
+          g.ai[oa] = xi[k];
+          pvi[op] = 0.0;
+          pvi[op + (size_t)2 * BND * n] = 0.0;
+        }
+      }
+    }
+    if (tid >= nref && tid < BND && j0 + tid < n) {
+      g.taur[j0 + tid] = 0.0;
+      if (CX) g.taui[j0 + tid] = 0.0;
+    }
+  }
+}
+
+template <bool CX>
+__global__ __launch_bounds__(QR_ROWS) void k_sb_qr(SbArgs g, int j0)
+{
+  __shared__ QrShared<CX> sh;
+  const int tid = threadIdx.x, m = g.n - (j0 + BND);
+  const int nblk = (m + QR_ROWS - 1) / QR_ROWS;
+  int idx = 0, np = 1;
+  if (nblk > 1) {
+    if (tid == 0) {
+      const int old = __hip_atomic_fetch_add(g.sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      int me = old, cnt = 0;
+      if (old & SB_CLOSED) {
+        me = -1;
+      } else if (old == 0) {
+        const long long t0 = wall_clock64();
+        while (agent_ld(g.sync) < nblk && wall_clock64() - t0 < QR_WAIT) __builtin_amdgcn_s_sleep(1);
+        cnt = __hip_atomic_fetch_or(g.sync, SB_CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        agent_st(g.sync + 1, cnt);
+      } else {
+        while ((cnt = agent_ld(g.sync + 1)) == 0) __builtin_amdgcn_s_sleep(1);
+      }
+      sh.share[0] = me;
+      sh.share[1] = cnt;
+    }
+    __syncthreads();
+    idx = __builtin_amdgcn_readfirstlane(sh.share[0]);
+    np = __builtin_amdgcn_readfirstlane(sh.share[1]);
+    if (idx < 0) return;
+  }
+  if (np >= nblk) qr_panel<CX, true>(g, j0, nblk, idx, np, sh);
+  else qr_panel<CX, false>(g, j0, nblk, idx, np, sh);
+}
+
+// T of I - V T V^H from G = V^H V and tau: T(0:i, i) = -tau_i T(0:i, 0:i)
+// G(0:i, i), T(i, i) = tau_i; one wave, lanes r and r + 32 taking the even and
+// odd terms of row r
+template <bool CX>
+__device__ __forceinline__ void panel_t(const SbArgs &g, int j0, double (*tm)[BND][BND + 1], double (*gm)[BND][BND + 1])
+{
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, h = lane >> 5;
+  const int nref = min(BND, g.n - (j0 + BND) - 1);
+  for (int e = tid; e < BND * BND; e += blockDim.x) {
+    const int a = e % BND, b = e / BND;
+    const bool in = a < b && b < nref;
+    tm[0][a][b] = 0.0;
+    gm[0][a][b] = in ? g.G[e] : 0.0;
+    if (CX) {
+      tm[1][a][b] = 0.0;
+      gm[1][a][b] = in ? g.G[BND * BND + e] : 0.0;
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    for (int i = 0; i < nref; i++) {
+      const double tr = g.taur[j0 + i], ti = CX ? g.taui[j0 + i] : 0.0;
+      double ar = 0.0, ai = 0.0;
+#pragma unroll 4
+      for (int q = h; q < i; q += 2) {
+        const double a = tm[0][r][q], b = gm[0][q][i];
+        if (CX) {
+          const double a2 = tm[1][r][q], b2 = gm[1][q][i];
+          ar += a * b - a2 * b2;
+          ai += a * b2 + a2 * b;
+        } else {
+          ar += a * b;
+        }
+      }
+      ar += xor32(ar, lane);
+      if (CX) ai += xor32(ai, lane);
+      if (h == 0 && r <= i) {
+        tm[0][r][i] = r < i ? -(CX ? tr * ar - ti * ai : tr * ar) : tr;
+        if (CX) tm[1][r][i] = r < i ? -(tr * ai + ti * ar) : ti;
+      }
+      wave_sync();
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < BND * BND; e += blockDim.x) {
+    g.T[e] = tm[0][e % BND][e / BND];
+    if (CX) g.T[BND * BND + e] = tm[1][e % BND][e / BND];
+  }
+}
+
+// ------------------------------------------------------------------ 1b. Y = A V
+// Partial products of A(r0:n, r0:n) (lower triangle stored) with the panel V:
+// a work-group forms 64 rows of Y over one slice of K, four waves of 16 rows
+// each, operands swapped (D = V^T A^T) so that the 16 rows of a result lie
+// across lanes.  A goes from memory to registers (no wave shares it), one
+// 64-column slab ahead; V through LDS.  Lane group q takes k = 4q + s of a
+// 16-wide chunk at step s, which makes the transposed reads (k beyond the
+// row) 32 contiguous bytes per lane.
+constexpr int AV_K = 64, AV_LD = 36;
+
+// The block past the last row forms the panel's T meanwhile.
+template <bool CX>
+__global__ __launch_bounds__(256, 2) void k_sb_av(SbArgs g, int r0, int slab, int mp)
+{
+  constexpr int CP = CX ? 2 : 1;
+  __shared__ double lds[CP * AV_K * AV_LD];
+  static_assert(AV_K * AV_LD >= 2 * BND * (BND + 1), "T and G fit");
+  if ((int)blockIdx.x * 64 >= g.n - r0) {
+    if (blockIdx.y == 0)
+      panel_t<CX>(g, r0 - BND, reinterpret_cast<double(*)[BND][BND + 1]>(lds),
+                  reinterpret_cast<double(*)[BND][BND + 1]>(lds + CP * BND * (BND + 1)));
+    return;
+  }
+  double(*vs)[AV_K][AV_LD] = reinterpret_cast<double(*)[AV_K][AV_LD]>(lds);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int l16 = lane & 15, q4 = lane >> 4;
+  const int m = g.n - r0, n = g.n;
+  const int i0 = blockIdx.x * 64 + 16 * wave;  // first row of the wave
+  const int kb = blockIdx.y * slab * AV_K, ke = min(m, kb + slab * AV_K);
+  const double *ar = g.ar + (size_t)r0 + (size_t)g.lda * r0;
+  const double *ai = CX ? g.ai + (size_t)r0 + (size_t)g.lda * r0 : nullptr;
+  const int i = min(i0 + l16, m - 1);
+  double pr[16], pi[CX ? 16 : 1];
+  // chunk c, step s of slab k0: element (i, k), k = k0 + 16 c + 4 q4 + s, from
+  // the stored triangle (its conjugate where k > i)
+  auto loadA = [&](int k0) {
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int k = min(k0 + 16 * c + 4 * q4 + s, m - 1);
+        const bool up = k > i;
+        const size_t o = up ? (size_t)k + (size_t)g.lda * i : (size_t)i + (size_t)g.lda * k;
+        pr[4 * c + s] = ar[o];
+        if (CX) {
+          const double v = ai[o];
+          pi[4 * c + s] = up ? -v : (k == i ? 0.0 : v);
+        }
+      }
+  };
+  d4 yr[2], yi[CX ? 2 : 1];
+  for (int t = 0; t < 2; t++) {
+    yr[t] = d4{0.0, 0.0, 0.0, 0.0};
+    if (CX) yi[t] = d4{0.0, 0.0, 0.0, 0.0};
+  }
+  loadA(kb);
+  for (int k0 = kb; k0 < ke; k0 += AV_K) {
+    double br[16], bi[CX ? 16 : 1];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      br[q] = pr[q];
+      if (CX) bi[q] = pi[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      const int k = tid & 63, col = (tid >> 6) + 4 * c;
+      const bool ok = k0 + k < ke;
+      const size_t o = (size_t)(r0 + min(k0 + k, m - 1)) + (size_t)n * col;
+      const double v = g.Pr[o];
+      vs[0][k][col] = ok ? v : 0.0;
+      if (CX) {
+        const double w = g.Pi[o];
+        vs[1][k][col] = ok ? w : 0.0;
+      }
+    }
+    if (k0 + AV_K < ke) loadA(k0 + AV_K);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int k = 16 * c + 4 * q4 + s, e = 4 * c + s;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+          const double vr = vs[0][k][16 * t + l16];
+          yr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vr, br[e], yr[t], 0, 0, 0);
+          if (CX) {
+            const double vi = vs[1][k][16 * t + l16];
+            yr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-vi, bi[e], yr[t], 0, 0, 0);
+            yi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vi, br[e], yi[t], 0, 0, 0);
+            yi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vr, bi[e], yi[t], 0, 0, 0);
+          }
+        }
+      }
+  }
+  mfma_settle();
+  // D(c, i): lane i + 16 (c % 4), item c / 4
+  if (i0 + l16 < m) {
+    const size_t plane = (size_t)mp * BND;
+    double *out = g.part + (size_t)blockIdx.y * plane * (CX ? 2 : 1);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const size_t o = (size_t)(i0 + l16) + (size_t)mp * (16 * t + q4 + 4 * r);
+        out[o] = yr[t][r];
+        if (CX) out[plane + o] = yi[t][r];
+      }
+  }
+}
+
+// Z = (sum of the slices) T for 32 rows per work-group (fixed order), and the
+// work-group's part of V^H Z
+template <bool CX>
+__global__ __launch_bounds__(256) void k_sb_y(SbArgs g, int r0, int nz, int mp)
+{
+  constexpr int CP = CX ? 2 : 1;
+  __shared__ double ys[CP][32][BND + 1], vs[CP][32][BND + 1], ts[CP][BND][BND + 1], zs[CP][32][BND + 1];
+  const int tid = threadIdx.x, n = g.n, m = n - r0, t0 = blockIdx.x * 32;
+  const size_t plane = (size_t)mp * BND;
+  const int r = tid & 31, c0 = tid >> 5;
+  const bool ok = t0 + r < m;
+  const int rr = min(t0 + r, m - 1);
+  double ar[4] = {0.0, 0.0, 0.0, 0.0}, ai[4] = {0.0, 0.0, 0.0, 0.0};
+  const double *p = g.part + rr + (size_t)mp * c0;
+#pragma unroll 4
+  for (int z = 0; z < nz; z++) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      ar[q] += p[(size_t)mp * 8 * q];
+      if (CX) ai[q] += p[plane + (size_t)mp * 8 * q];
+    }
+    p += plane * CP;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int c = c0 + 8 * q;
+    const size_t ov = (size_t)(r0 + rr) + (size_t)n * c;
+    const double vr = g.Pr[ov];
+    ys[0][r][c] = ok ? ar[q] : 0.0;
+    vs[0][r][c] = ok ? vr : 0.0;
+    ts[0][r][c] = g.T[r + BND * c];
+    if (CX) {
+      const double vi = g.Pi[ov];
+      ys[1][r][c] = ok ? ai[q] : 0.0;
+      vs[1][r][c] = ok ? vi : 0.0;
+      ts[1][r][c] = g.T[BND * BND + r + BND * c];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; q++) ar[q] = ai[q] = 0.0;
+#pragma unroll 4
+  for (int a = 0; a < BND; a++) {
+    const double yr = ys[0][r][a], yi = CX ? ys[CP - 1][r][a] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const double tr = ts[0][a][c0 + 8 * q];
+      ar[q] += yr * tr;
+      if (CX) {
+        const double ti = ts[CP - 1][a][c0 + 8 * q];
+        ar[q] -= yi * ti;
+        ai[q] += yr * ti + yi * tr;
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int c = c0 + 8 * q;
+    const size_t ov = (size_t)(r0 + rr) + (size_t)n * c;
+    zs[0][r][c] = ar[q];
+    if (ok) g.Yr[ov] = ar[q];
+    if (CX) {
+      zs[CP - 1][r][c] = ai[q];
+      if (ok) g.Yi[ov] = ai[q];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; q++) ar[q] = ai[q] = 0.0;
+#pragma unroll 4
+  for (int x = 0; x < 32; x++) {
+    const double vr = vs[0][x][r], vi = CX ? vs[CP - 1][x][r] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const double zr = zs[0][x][c0 + 8 * q];
+      ar[q] += vr * zr;
+      if (CX) {
+        const double zi = zs[CP - 1][x][c0 + 8 * q];
+        ar[q] += vi * zi;
+        ai[q] += vr * zi - vi * zr;
+      }
+    }
+  }
+  double *out = g.spart + (size_t)blockIdx.x * BND * BND * CP;
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int e = r + BND * (c0 + 8 * q);
+    out[e] = ar[q];
+    if (CX) out[BND * BND + e] = ai[q];
+  }
+}
+
+// S = V^H Z from its parts, 32 entries per work-group (fixed order)
+__global__ __launch_bounds__(256) void k_sb_s(SbArgs g, int nwg, int stride)
+{
+  __shared__ double red[8][33];
+  const int tid = threadIdx.x, e = tid & 31, grp = tid >> 5;
+  const double *p = g.spart + (size_t)blockIdx.x * 32 + e;
+  double s = 0.0;
+#pragma unroll 8
+  for (int w = grp; w < nwg; w += 8) s += p[(size_t)w * stride];
+  red[grp][e] = s;
+  __syncthreads();
+  if (tid < 32) {
+    s = red[0][tid];
+#pragma unroll
+    for (int q = 1; q < 8; q++) s += red[q][tid];
+    g.S[blockIdx.x * 32 + tid] = s;
+  }
+}
+
+// W = Z - 1/2 V (T^H S) (P columns BND..2 BND-1), which makes the update
+// Q^H A Q = A - V W^H - W V^H; also clears the exchange buffer of the next
+// panel's QR
+template <bool CX>
+__global__ __launch_bounds__(256) void k_sb_w(SbArgs g, int r0, size_t nexch)
+{
+  constexpr int CP = CX ? 2 : 1;
+  __shared__ double vs[CP][32][BND + 1], ts[CP][BND][BND + 1], ss[CP][BND][BND + 1], mm[CP][BND][BND + 1];
+  const int tid = threadIdx.x, n = g.n, m = n - r0, t0 = blockIdx.x * 32;
+  const int r = tid & 31, c0 = tid >> 5;
+  for (size_t i = (size_t)blockIdx.x * 256 + tid; i < nexch; i += (size_t)gridDim.x * 256)
+    g.exch[i] = __longlong_as_double(SB_EMPTY);
+  if (blockIdx.x == 0 && tid < 4) g.sync[tid] = 0;
+  const size_t row = r0 + min(t0 + r, m - 1);
+  double zr[4], zi[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int c = c0 + 8 * q;
+    const size_t o = row + (size_t)n * c;
+    zr[q] = g.Yr[o];
+    vs[0][r][c] = g.Pr[o];
+    ts[0][r][c] = g.T[r + BND * c];
+    ss[0][r][c] = g.S[r + BND * c];
+    if (CX) {
+      zi[q] = g.Yi[o];
+      vs[CP - 1][r][c] = g.Pi[o];
+      ts[CP - 1][r][c] = g.T[BND * BND + r + BND * c];
+      ss[CP - 1][r][c] = g.S[BND * BND + r + BND * c];
+    }
+  }
+  __syncthreads();
+  double ar[4] = {0.0, 0.0, 0.0, 0.0}, ai[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+  for (int a = 0; a < BND; a++) {  // T^H S
+    const double tr = ts[0][a][r], ti = CX ? ts[CP - 1][a][r] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const double sr = ss[0][a][c0 + 8 * q];
+      ar[q] += tr * sr;
+      if (CX) {
+        const double si = ss[CP - 1][a][c0 + 8 * q];
+        ar[q] += ti * si;
+        ai[q] += tr * si - ti * sr;
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    mm[0][r][c0 + 8 * q] = -0.5 * ar[q];
+    if (CX) mm[CP - 1][r][c0 + 8 * q] = -0.5 * ai[q];
+  }
+  __syncthreads();
+#pragma unroll 4
+  for (int a = 0; a < BND; a++) {
+    const double vr = vs[0][r][a], vi = CX ? vs[CP - 1][r][a] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const double mr = mm[0][a][c0 + 8 * q];
+      zr[q] += vr * mr;
+      if (CX) {
+        const double mi = mm[CP - 1][a][c0 + 8 * q];
+        zr[q] -= vi * mi;
+        zi[q] += vr * mi + vi * mr;
+      }
+    }
+  }
+  if (t0 + r < m) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const size_t o = row + (size_t)n * (BND + c0 + 8 * q);
+      g.Pr[o] = zr[q];
+      if (CX) g.Pi[o] = zi[q];
+    }
+  }
+}
+
+// ------------------------------------------------------------------ 2. bulge chasing
+// band storage: column j at ab + BLD j, entry (i, j) at offset i - j (0..BLD-1)
+constexpr int BLD = 2 * BND;
+constexpr int CHASE_DONE = 1 << 30;
+
+template <bool CX>
+__global__ void k_sb_band(SbArgs g)
+{
+  const int o = threadIdx.x & (BLD - 1), j = blockIdx.x * (blockDim.x / BLD) + threadIdx.x / BLD;
+  if (j >= g.n) return;
+  const bool in = o <= BND && j + o < g.n;
+  const size_t a = (size_t)min(j + o, g.n - 1) + (size_t)g.lda * j, d = (size_t)BLD * j + o;
+  g.ab[d] = in ? g.ar[a] : 0.0;
+  if (CX) g.ab[(size_t)BLD * g.n + d] = in && o > 0 ? g.ai[a] : 0.0;
+  if (o == 0) {
+    g.prog[j] = 0;
+    if (j == 0) {
+      g.prog[g.n] = 0;  // sweep ticket
+      if (g.n == 1) g.d[0] = g.ar[0];
+    }
+  }
+}
+
+// t[0..NC-1] per lane, summed over the 32 lanes of each half: lane l returns
+// entry (l & 31) >> SH, SH = 5 - log2(NC)
+template <int NC>
+__device__ __forceinline__ double half_reduce(double *t, int lane)
+{
+  static_assert(NC == 16 || NC == 8 || NC == 4, "columns per lane");
+#pragma unroll
+  for (int j = 0; j < NC / 2; j++) t[j] = swap_sum<16>(t[j], t[j + NC / 2]);
+  bfly_step_h<8, NC / 4>(t, lane);
+  if constexpr (NC >= 8) bfly_step_h<4, NC / 8>(t, lane);
+  else t[0] += bfly_partner<4>(t[0]);
+  if constexpr (NC >= 16) bfly_step_h<2, 1>(t, lane);
+  else t[0] += bfly_partner<2>(t[0]);
+  return t[0] + bfly_partner<1>(t[0]);
+}
+
+// Sweep s reduces column s of the band and chases the bulge that this makes
+// down the matrix.  Rows R_t = s + 1 + BND t .. (BND of them); step t applies
+// the reflector of R_t to the diagonal block D = A(R_t, R_t) from both sides
+// and to C = A(R_t+1, R_t) from the right, and forms the reflector of R_t+1
+// from C's first column and applies it to C from the left.  Step t of sweep s
+// needs steps up to t + 1 of sweep s - 1 (C's last entry is what that step
+// leaves of its first column), so sweeps follow each other two steps apart.
+// A work-group takes whole sweeps in order from a ticket: the oldest
+// unfinished sweep always has a running work-group and waits for nothing, so
+// no residency is assumed.  NW waves share a step: lane (r, h) of wave w holds
+// row r, columns (2 w + h) NC .. of D (mirrored) and C.
+template <bool CX, int NW>
+__global__ __launch_bounds__(64 * NW) void k_sb_chase(SbArgs g)
+{
+  constexpr int NC = 16 / NW, CP = CX ? 2 : 1;
+  __shared__ double yz[2][CP][2 * NW][BND], xc[CP][BND];
+  __shared__ double vb[NW][CP][BND], ub[NW][CP][BND], gb[NW][CP][BND];
+  __shared__ int tick;
+  const int n = g.n, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 31, h = lane >> 5, j0 = (2 * wave + h) * NC;
+  double *const abr = g.ab, *const abi = g.ab + (size_t)BLD * n;
+  const int nsweep = n - 1;
+  const bool first = wave == 0 && h == 0;  // lanes that hold column 0
+  // one work-item takes the ticket; a barrier stands on both sides of it, so
+  // that no lane runs ahead with the old one
+  auto ticket = [&]() {
+    return __hip_atomic_fetch_add(g.prog + n, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (tid == 0) tick = ticket();
+  __syncthreads();
+  int s = __builtin_amdgcn_readfirstlane(tick);
+  while (s < nsweep) {
+    auto wait = [&](int need) {
+      if (s > 0)
+        while (agent_ld(g.prog + s - 1) < need) __builtin_amdgcn_s_sleep(1);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    };
+    wait(2);
+    double dr[NC], di[CX ? NC : 1], cr[NC], ci[CX ? NC : 1];
+    // D and C of the step whose rows start at c0 (L and L2 rows)
+    auto load = [&](int c0) {
+      const int L = min(BND, n - c0), L2 = min(BND, n - c0 - BND);
+#pragma unroll
+      for (int q = 0; q < NC; q++) {
+        const int j = j0 + q;
+        const int hi = max(r, j), lo = min(r, j);
+        const bool okd = hi < L, okc = r < L2;
+        const size_t od = okd ? (size_t)(hi - lo) + (size_t)BLD * (c0 + lo) : 0;
+        const size_t oc = okc ? (size_t)(BND + r - j) + (size_t)BLD * (c0 + j) : 0;
+        const double a = agent_ld(abr + od), c = agent_ld(abr + oc);
+        dr[q] = okd ? a : 0.0;
+        cr[q] = okc ? c : 0.0;
+        if (CX) {
+          const double a2 = agent_ld(abi + od), c2 = agent_ld(abi + oc);
+          di[q] = okd && r != j ? (r > j ? a2 : -a2) : 0.0;
+          ci[q] = okc ? c2 : 0.0;
+        }
+      }
+    };
+    int c0 = s + 1;
+    double vr, vi = 0.0, tr, ti;  // v(r) and tau of the step's reflector
+    {
+      const int L = min(BND, n - c0);
+      const bool ok = r < L;
+      const size_t o = (size_t)BLD * s + (ok ? 1 + r : 0);
+      double x = agent_ld(abr + o), x2 = CX ? agent_ld(abi + o) : 0.0;
+      const double dg = agent_ld(abr + (size_t)BLD * s);
+      load(c0);
+      x = ok ? x : 0.0;
+      x2 = ok ? x2 : 0.0;
+      const double ss = sum32(r > 0 ? (CX ? x * x + x2 * x2 : x * x) : 0.0);
+      const double ar = __shfl(x, 0, 64), ai = CX ? __shfl(x2, 0, 64) : 0.0;
+      const Reflector f = larfg<CX>(ar, ai, ss);
+      vr = r == 0 ? 1.0 : (CX ? f.sr * x - f.si * x2 : f.sr * x);
+      if (CX) vi = r == 0 ? 0.0 : f.sr * x2 + f.si * x;
+      tr = f.tr;
+      ti = f.ti;
+      if (first && ok) {
+        g.V2r[(size_t)c0 + r + (size_t)n * s] = vr;
+        if (CX) g.V2i[(size_t)c0 + r + (size_t)n * s] = vi;
+      }
+      if (tid == 0) {
+        g.d[s] = dg;
+        g.e[s] = f.beta;
+        g.tau2[s] = tr;
+        if (CX) g.tau2[g.ntau2 + s] = ti;
+      }
+    }
+    for (int t = 0;; t++) {
+      const int L = min(BND, n - c0), L2 = min(BND, n - c0 - BND);
+      // v at this lane's columns
+      if (h == 0) {
+        vb[wave][0][r] = vr;
+        if (CX) vb[wave][1][r] = vi;
+      }
+      wave_sync();
+      double vj[NC], vji[CX ? NC : 1];
+#pragma unroll
+      for (int q = 0; q < NC; q++) {
+        vj[q] = vb[wave][0][j0 + q];
+        if (CX) vji[q] = vb[wave][1][j0 + q];
+      }
+      // y = D v, z = C v
+      double yr = 0.0, yi = 0.0, zr = 0.0, zi = 0.0;
+#pragma unroll
+      for (int q = 0; q < NC; q++) {
+        yr += dr[q] * vj[q];
+        zr += cr[q] * vj[q];
+        if (CX) {
+          yr -= di[q] * vji[q];
+          yi += dr[q] * vji[q] + di[q] * vj[q];
+          zr -= ci[q] * vji[q];
+          zi += cr[q] * vji[q] + ci[q] * vj[q];
+        }
+      }
+      yz[0][0][2 * wave + h][r] = yr;
+      yz[1][0][2 * wave + h][r] = zr;
+      if (CX) {
+        yz[0][CP - 1][2 * wave + h][r] = yi;
+        yz[1][CP - 1][2 * wave + h][r] = zi;
+      }
+      __syncthreads();
+      yr = zr = yi = zi = 0.0;
+#pragma unroll
+      for (int q = 0; q < 2 * NW; q++) {
+        yr += yz[0][0][q][r];
+        zr += yz[1][0][q][r];
+        if (CX) {
+          yi += yz[0][CP - 1][q][r];
+          zi += yz[1][CP - 1][q][r];
+        }
+      }
+      // C <- C - tau z v^H
+      const double tzr = CX ? tr * zr - ti * zi : tr * zr, tzi = CX ? tr * zi + ti * zr : 0.0;
+#pragma unroll
+      for (int q = 0; q < NC; q++) {
+        if (CX) {
+          cr[q] = fma(-tzi, vji[q], fma(-tzr, vj[q], cr[q]));
+          ci[q] = fma(tzr, vji[q], fma(-tzi, vj[q], ci[q]));
+        } else {
+          cr[q] = fma(-tzr, vj[q], cr[q]);
+        }
+      }
+      if (first) {
+        xc[0][r] = cr[0];
+        if (CX) xc[CP - 1][r] = ci[0];
+      }
+      // u = tau y - 1/2 |tau|^2 (v^H y) v;  D <- D - u v^H - v u^H
+      const double p = sum32(CX ? vr * yr + vi * yi : vr * yr);
+      const double hp = 0.5 * p * (CX ? tr * tr + ti * ti : tr * tr);
+      const double ur = (CX ? tr * yr - ti * yi : tr * yr) - hp * vr;
+      const double ui = CX ? tr * yi + ti * yr - hp * vi : 0.0;
+      if (h == 0) {
+        ub[wave][0][r] = ur;
+        if (CX) ub[wave][CP - 1][r] = ui;
+      }
+      wave_sync();
+#pragma unroll
+      for (int q = 0; q < NC; q++) {
+        const double uj = ub[wave][0][j0 + q];
+        if (CX) {
+          const double uji = ub[wave][CP - 1][j0 + q];
+          dr[q] = fma(-vi, uji, fma(-vr, uj, fma(-ui, vji[q], fma(-ur, vj[q], dr[q]))));
+          di[q] = fma(vr, uji, fma(-vi, uj, fma(ur, vji[q], fma(-ui, vj[q], di[q]))));
+        } else {
+          dr[q] = fma(-vr, uj, fma(-ur, vj[q], dr[q]));
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < NC; q++) {
+        const int j = j0 + q;
+        if (r >= j && r < L) {
+          const size_t o = (size_t)(r - j) + (size_t)BLD * (c0 + j);
+          agent_st(abr + o, dr[q]);
+          if (CX) agent_st(abi + o, r == j ? 0.0 : di[q]);
+          if (r == 0 && s == n - 2) g.d[n - 1] = dr[q];
+        }
+      }
+      if (L2 <= 0) break;
+      __syncthreads();
+      // reflector of the next rows from C's first column, applied from the left
+      const double x = xc[0][r], x2 = CX ? xc[CP - 1][r] : 0.0;
+      const double ss = sum32(r > 0 ? (CX ? x * x + x2 * x2 : x * x) : 0.0);
+      const Reflector f = larfg<CX>(xc[0][0], CX ? xc[CP - 1][0] : 0.0, ss);
+      vr = r == 0 ? 1.0 : (CX ? f.sr * x - f.si * x2 : f.sr * x);
+      if (CX) vi = r == 0 ? 0.0 : f.sr * x2 + f.si * x;
+      tr = f.tr;
+      ti = f.ti;
+      double tq[NC];
+#pragma unroll
+      for (int q = 0; q < NC; q++) tq[q] = CX ? vr * cr[q] + vi * ci[q] : vr * cr[q];
+      constexpr int SH = NC == 16 ? 1 : NC == 8 ? 2 : 3;
+      const double g0 = half_reduce<NC>(tq, lane);
+      if (!(r & ((1 << SH) - 1))) gb[wave][0][h * NC + (r >> SH)] = g0;
+      if (CX) {
+#pragma unroll
+        for (int q = 0; q < NC; q++) tq[q] = vr * ci[q] - vi * cr[q];
+        const double g1 = half_reduce<NC>(tq, lane);
+        if (!(r & ((1 << SH) - 1))) gb[wave][CP - 1][h * NC + (r >> SH)] = g1;
+      }
+      wave_sync();
+      const double wr = CX ? tr * vr + ti * vi : tr * vr, wi = CX ? tr * vi - ti * vr : 0.0;  // conj(tau) v
+#pragma unroll
+      for (int q = 0; q < NC; q++) {
+        const double gr = gb[wave][0][h * NC + q];
+        if (CX) {
+          const double gi = gb[wave][CP - 1][h * NC + q];
+          cr[q] = fma(wi, gi, fma(-wr, gr, cr[q]));
+          ci[q] = fma(-wi, gr, fma(-wr, gi, ci[q]));
+        } else {
+          cr[q] = fma(-wr, gr, cr[q]);
+        }
+      }
+      // column 0 is (beta, 0, ..)
+      if (first) {
+        cr[0] = r == 0 ? f.beta : 0.0;
+        if (CX) ci[0] = 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < NC; q++) {
+        const int j = j0 + q;
+        if (r < L2) {
+          const size_t o = (size_t)(BND + r - j) + (size_t)BLD * (c0 + j);
+          agent_st(abr + o, cr[q]);
+          if (CX) agent_st(abi + o, ci[q]);
+        }
+      }
+      const int c1 = c0 + BND;
+      if (first && r < L2) {
+        g.V2r[(size_t)c1 + r + (size_t)n * s] = vr;
+        if (CX) g.V2i[(size_t)c1 + r + (size_t)n * s] = vi;
+      }
+      if (tid == 0) {
+        g.tau2[(size_t)(t + 1) * n + s] = tr;
+        if (CX) g.tau2[g.ntau2 + (size_t)(t + 1) * n + s] = ti;
+      }
+      vm_drain();
+      __syncthreads();
+      if (tid == 0) agent_st(g.prog + s, t + 1);
+      c0 = c1;
+      wait(t + 3);
+      load(c0);
+    }
+    vm_drain();
+    __syncthreads();
+    if (tid == 0) {
+      agent_st(g.prog + s, CHASE_DONE);
+      tick = ticket();
+    }
+    __syncthreads();
+    s = __builtin_amdgcn_readfirstlane(tick);
+  }
+}
+
+// ------------------------------------------------------------------ 3. Q2 times vectors
+// The reflectors of BND consecutive sweeps at one step are a block I - V T V^H
+// on 2 BND - 1 rows (V a parallelogram): k_sb_frag forms V and -V T of every
+// block in the order in which k_sb_q2's lanes read them as MFMA operands.
+// Block (group, t) of ntg groups: groups 0..gr-1 have ntg, ntg - 1, .. blocks.
+__device__ __forceinline__ size_t frag_block(int ntg, int gr, int t)
+{
+  return (size_t)gr * ntg - (size_t)gr * (gr - 1) / 2 + t;
+}
+constexpr int FRAG = 4096;  // doubles of a block per plane: 32 + 32 operand fragments of 64
+
+template <bool CX>
+__global__ __launch_bounds__(256) void k_sb_frag(SbArgs g, int ntg, int nsync)
+{
+  __shared__ double v[CX ? 2 : 1][64][BND + 1], gm[CX ? 2 : 1][BND][BND + 1], tm[CX ? 2 : 1][BND][BND + 1];
+  const int gr = blockIdx.y, t = blockIdx.x, tid = threadIdx.x, n = g.n;
+  // the ticket and progress words of k_sb_q2
+  for (int i = (gr * ntg + t) * 256 + tid; i < nsync; i += ntg * ntg * 256) g.q2sync[i] = 0;
+  if (gr + t >= ntg) return;
+  const int s0 = gr * BND, w0 = s0 + 1 + BND * t;
+  for (int e = tid; e < 64 * BND; e += 256) {
+    const int x = e & 63, i = e >> 6;
+    const bool in = x >= i && x < i + BND && w0 + x < n && s0 + i <= n - 2;
+    const size_t o = in ? (size_t)(w0 + x) + (size_t)n * (s0 + i) : 0;
+    v[0][x][i] = in ? g.V2r[o] : 0.0;
+    if (CX) v[1][x][i] = in ? g.V2i[o] : 0.0;
+  }
+  for (int e = tid; e < BND * BND; e += 256) {
+    tm[0][e & 31][e >> 5] = 0.0;
+    if (CX) tm[1][e & 31][e >> 5] = 0.0;
+  }
+  __syncthreads();
+  {
+    const int a = tid & 31;
+    double sr[4] = {0.0, 0.0, 0.0, 0.0}, si[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int x = 0; x < 64; x++) {
+      const double ar = v[0][x][a], ai = CX ? v[1][x][a] : 0.0;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int b = (tid >> 5) + 8 * q;
+        const double br = v[0][x][b];
+        if (CX) {
+          const double bi = v[1][x][b];
+          sr[q] += ar * br + ai * bi;
+          si[q] += ar * bi - ai * br;
+        } else {
+          sr[q] += ar * br;
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      gm[0][a][(tid >> 5) + 8 * q] = sr[q];
+      if (CX) gm[1][a][(tid >> 5) + 8 * q] = si[q];
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const int lane = tid & 31;
+    for (int i = 0; i < BND; i++) {
+      const bool in = s0 + i <= n - 2 && w0 + i < n;
+      const size_t o = in ? (size_t)t * n + s0 + i : 0;
+      const double tr = in ? g.tau2[o] : 0.0, ti = CX && in ? g.tau2[g.ntau2 + o] : 0.0;
+      double ar = 0.0, ai = 0.0;
+      for (int q = 0; q < i; q++) {
+        const double a = tm[0][lane][q], b = gm[0][q][i];
+        if (CX) {
+          const double a2 = tm[1][lane][q], b2 = gm[1][q][i];
+          ar += a * b - a2 * b2;
+          ai += a * b2 + a2 * b;
+        } else {
+          ar += a * b;
+        }
+      }
+      if (tid < 32 && lane <= i) {
+        tm[0][lane][i] = lane < i ? -(CX ? tr * ar - ti * ai : tr * ar) : tr;
+        if (CX) tm[1][lane][i] = lane < i ? -(tr * ai + ti * ar) : ti;
+      }
+      wave_sync();
+    }
+  }
+  __syncthreads();
+  double *out = g.frag + frag_block(ntg, gr, t) * FRAG * (CX ? 2 : 1);
+  // V: fragment (w, mt, k): lane (l, q) holds row 16 w + 4 q + k, column 16 mt + l
+  for (int e = tid; e < 2048; e += 256) {
+    const int lane = e & 63, f = e >> 6, k = f & 3, mt = (f >> 2) & 1, w = f >> 3;
+    const int x = 16 * w + 4 * (lane >> 4) + k, c = 16 * mt + (lane & 15);
+    out[e] = v[0][x][c];
+    if (CX) out[FRAG + e] = v[1][x][c];
+  }
+  // -V T: fragment (w, s): lane (l, q) holds row 16 w + 4 (l % 4) + l / 4, column 4 s + q
+  for (int e = tid; e < 2048; e += 256) {
+    const int lane = e & 63, f = e >> 6, s = f & 7, w = f >> 3, l = lane & 15;
+    const int x = 16 * w + 4 * (l & 3) + (l >> 2), c = 4 * s + (lane >> 4);
+    double ar = 0.0, ai = 0.0;
+    for (int q = 0; q <= c; q++) {
+      ar += v[0][x][q] * tm[0][q][c];
+      if (CX) {
+        ar -= v[1][x][q] * tm[1][q][c];
+        ai += v[0][x][q] * tm[1][q][c] + v[1][x][q] * tm[0][q][c];
+      }
+    }
+    out[2048 + e] = -ar;
+    if (CX) out[FRAG + 2048 + e] = -ai;
+  }
+}
+
+// Z <- Q2 Z.  A task is one group of sweeps on a slab of 16 columns of Z: its
+// blocks slide down the rows.  A wave holds 16 of the window's 64 rows as MFMA
+// accumulators (lane (l, q): column l, rows 4 q + k in item k), which are at
+// once the operand of V^H Z; the four partial V^H Z meet in LDS.  The window
+// moves by 32 rows, so two waves keep their rows and the other two store
+// theirs and take the next 32.  Rows and operands are loaded a step ahead and
+// rows stored a step late, so that no step waits for memory it has just asked.
+//
+// The groups of a slab follow each other (the last group first) a few steps
+// apart, which keeps the chip busy where there are few slabs: work-groups take
+// tasks in order from a ticket, so the group that a task waits for has started
+// before it, and every Q2_FLAG steps a task publishes how many it has done.
+constexpr int Q2_FLAG = 4;
+
+template <bool CX>
+__global__ __launch_bounds__(256, CX ? 1 : 2) void k_sb_q2(SbArgs g, int ntg, int mcol, double *__restrict__ Zr,
+                                                           double *__restrict__ Zi, int ldz)
+{
+  constexpr int CP = CX ? 2 : 1;
+  __shared__ double yp[2][CP][4][8][64];
+  __shared__ int tick;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l = lane & 15, q4 = lane >> 4;
+  const int n = g.n, nslab = (mcol + 15) / 16, ntask = nslab * ntg;
+  int *const done = g.q2sync + 1;  // steps done of (group from the last, slab)
+  auto ticket = [&]() { return __hip_atomic_fetch_add(g.q2sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  if (tid == 0) tick = ticket();
+  __syncthreads();
+  int task = __builtin_amdgcn_readfirstlane(tick);
+  while (task < ntask) {
+    const int gi = task / nslab, slab = task - gi * nslab, gr = ntg - 1 - gi, nt = gi + 1;
+    const int col = slab * 16 + l;
+    const bool okc = col < mcol;
+    const size_t zc = (size_t)ldz * min(col, mcol - 1);
+    int seen = gi == 0 ? CHASE_DONE : 0;
+    // rows of window t are final once the group after this one has done step t
+    auto ready = [&](int t) {
+      while (seen < t + 1) {
+        seen = agent_ld(done + (size_t)(gi - 1) * nslab + slab);
+        if (seen < t + 1) __builtin_amdgcn_s_sleep(1);
+      }
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    };
+    auto zload = [&](int row0, d4 &a, d4 &b) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const size_t o = zc + min(row0 + 4 * q4 + k, n - 1);
+        a[k] = agent_ld(Zr + o);
+        if (CX) b[k] = agent_ld(Zi + o);
+      }
+    };
+    auto zmask = [&](int row0, d4 &a, d4 &b) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const bool ok = okc && row0 + 4 * q4 + k < n;
+        a[k] = ok ? a[k] : 0.0;
+        if (CX) b[k] = ok ? b[k] : 0.0;
+      }
+    };
+    auto zstore = [&](int row0, const d4 &a, const d4 &b) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int row = row0 + 4 * q4 + k;
+        if (okc && row < n) {
+          agent_st(Zr + zc + row, a[k]);
+          if (CX) agent_st(Zi + zc + row, b[k]);
+        }
+      }
+    };
+    struct Ops {
+      double a[8], t[8], ai[CX ? 8 : 1], ti[CX ? 8 : 1];
+    };
+    auto fetch = [&](Ops &o, int t, int role) {
+      const double *f = g.frag + frag_block(ntg, gr, t) * FRAG * CP + (size_t)role * 512 + lane;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        o.a[k] = f[k * 64];
+        o.t[k] = f[2048 + k * 64];
+        if (CX) {
+          o.ai[k] = f[FRAG + k * 64];
+          o.ti[k] = f[FRAG + 2048 + k * 64];
+        }
+      }
+    };
+    int role = wave, w0 = gr * BND + 1, pend = -1;  // pend: first row of the tile to be stored
+    d4 zr, zi, sr, si;
+    ready(0);
+    zload(w0 + 16 * role, zr, zi);
+    Ops oa, ob;
+    fetch(oa, 0, role);
+    zmask(w0 + 16 * role, zr, zi);
+    auto step = [&](const Ops &o, Ops &next, int t) {
+      // what the last step asked for has come; then, in this order so that no
+      // wait below includes a younger access: rows, operands, stores
+      vm_drain();
+      const bool more = t + 1 < nt, leave = role < 2 && more;
+      d4 nr, ni;
+      if (leave) {
+        ready(t + 1);
+        zload(w0 + 64 + 16 * role, nr, ni);
+      }
+      fetch(next, more ? t + 1 : t, (role + 2) & 3);
+      if (pend >= 0) zstore(pend, sr, si);
+      // partial V^H Z over this wave's rows
+      d4 yr[2], yi[2];
+#pragma unroll
+      for (int mt = 0; mt < 2; mt++) {
+        yr[mt] = d4{0.0, 0.0, 0.0, 0.0};
+        yi[mt] = d4{0.0, 0.0, 0.0, 0.0};
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++) {
+          yr[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[4 * mt + k], zr[k], yr[mt], 0, 0, 0);
+          if (CX) {
+            yi[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[4 * mt + k], zi[k], yi[mt], 0, 0, 0);
+            yr[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.ai[4 * mt + k], zi[k], yr[mt], 0, 0, 0);
+            yi[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(-o.ai[4 * mt + k], zr[k], yi[mt], 0, 0, 0);
+          }
+        }
+      mfma_settle();
+      const int par = t & 1;
+#pragma unroll
+      for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          yp[par][0][role][4 * mt + k][lane] = yr[mt][k];
+          if (CX) yp[par][CP - 1][role][4 * mt + k][lane] = yi[mt][k];
+        }
+      const bool flag = t % Q2_FLAG == Q2_FLAG - 1;
+      if (flag) vm_drain();  // the tiles of the steps before this one are stored
+      __syncthreads();
+      if (flag && tid == 0) agent_st(done + (size_t)gi * nslab + slab, t);
+      // Z -= (V T) (V^H Z), in two accumulator chains
+      d4 z2 = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 8; s++) {
+        double a = yp[par][0][0][s][lane], b = 0.0;
+        if (CX) b = yp[par][CP - 1][0][s][lane];
+#pragma unroll
+        for (int w = 1; w < 4; w++) {
+          a += yp[par][0][w][s][lane];
+          if (CX) b += yp[par][CP - 1][w][s][lane];
+        }
+        if (CX || !(s & 1)) zr = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], a, zr, 0, 0, 0);
+        else z2 = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], a, z2, 0, 0, 0);
+        if (CX) {
+          zi = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], b, zi, 0, 0, 0);
+          zr = __builtin_amdgcn_mfma_f64_16x16x4f64(-o.ti[s], b, zr, 0, 0, 0);
+          zi = __builtin_amdgcn_mfma_f64_16x16x4f64(o.ti[s], a, zi, 0, 0, 0);
+        }
+      }
+      mfma_settle();
+      if (!CX) zr += z2;
+      pend = -1;
+      if (more) {
+        if (leave) {
+          pend = w0 + 16 * role;
+          sr = zr;
+          zr = nr;
+          if (CX) {
+            si = zi;
+            zi = ni;
+          }
+          zmask(w0 + 64 + 16 * role, zr, zi);
+        }
+        role = (role + 2) & 3;
+        w0 += BND;
+      }
+    };
+    for (int t = 0; t < nt; t += 2) {
+      step(oa, ob, t);
+      if (t + 1 < nt) step(ob, oa, t + 1);
+    }
+    zstore(w0 + 16 * role, zr, zi);
+    vm_drain();
+    __syncthreads();
+    if (tid == 0) {
+      agent_st(done + (size_t)gi * nslab + slab, CHASE_DONE);
+      tick = ticket();
+    }
+    __syncthreads();
+    task = __builtin_amdgcn_readfirstlane(tick);
+  }
+}
+
+// ------------------------------------------------------------------ host side
+static size_t up32(size_t x) { return (x + 31) & ~(size_t)31; }
+
+static int av_slices(int m, int &slab)
+{
+  const int tiles = (m + 63) / 64;
+  int z = std::max(1, std::min(1024 / tiles, tiles));
+  slab = (tiles + z - 1) / z;
+  return (tiles + slab - 1) / slab;
+}
+
+size_t sb_doubles(int n, int cplx, size_t *ints)
+{
+  const size_t cp = cplx ? 2 : 1, tiles = (n + 63) / 64, nblk = (n + QR_ROWS - 1) / QR_ROWS;
+  const size_t ntg = (n - 1 + BND - 1) / BND;
+  if (ints) *ints = (size_t)n + 1 + 8;
+  return up32(std::max(tiles, std::min((size_t)1024, tiles * tiles)) * 64 * BND * cp) + up32((size_t)n * BND * cp) +
+         up32((size_t)(n + 31) / 32 * BND * BND * cp) + 3 * up32(BND * BND * cp) + up32((nblk + 1) * BND * BND * cp) + up32((size_t)BLD * n * cp) +
+         up32((size_t)n * (ntg + 1) * cp);
+}
+
+static size_t q2_words(int n, size_t m) { return (m + 15) / 16 * ((n - 1 + BND - 1) / BND) + 1; }
+
+size_t sb_frag_doubles(int n, size_t m, int cplx)
+{
+  const size_t ntg = (n - 1 + BND - 1) / BND;
+  return ntg * (ntg + 1) / 2 * FRAG * (cplx ? 2 : 1) + (q2_words(n, m) + 1) / 2;
+}
+
+int sb_buffers(Ctx &c, SbArgs &g, int n, int cplx)
+{
+  size_t ni = 0;
+  int rc;
+  const size_t nd = sb_doubles(n, cplx, &ni);
+  if ((rc = c.w_sb.alloc(nd)) || (rc = c.w_sbi.alloc(ni))) return rc;
+  const size_t cp = cplx ? 2 : 1, tiles = (n + 63) / 64, nblk = (n + QR_ROWS - 1) / QR_ROWS;
+  const size_t ntg = (n - 1 + BND - 1) / BND;
+  double *p = c.w_sb.p;
+  auto take = [&](size_t k) {
+    double *q = p;
+    p += up32(k);
+    return q;
+  };
+  g.n = n;
+  g.part = take(std::max(tiles, std::min((size_t)1024, tiles * tiles)) * 64 * BND * cp);
+  g.Yr = take((size_t)n * BND * cp);
+  g.Yi = g.Yr + (size_t)n * BND;
+  g.spart = take((size_t)(n + 31) / 32 * BND * BND * cp);
+  g.T = take(BND * BND * cp);
+  g.G = take(BND * BND * cp);
+  g.S = take(BND * BND * cp);
+  g.exch = take((nblk + 1) * BND * BND * cp);
+  g.ab = take((size_t)BLD * n * cp);
+  g.tau2 = take((size_t)n * (ntg + 1) * cp);
+  g.ntau2 = (size_t)n * (ntg + 1);
+  g.prog = c.w_sbi.p;
+  g.sync = c.w_sbi.p + n + 1;
+  return 0;
+}
+
+// events around every k_sb_av launch while kernel timing is on (carried by the
+// dispatch itself, so that a duration is the kernel's own)
+int sb_take_times(Ctx &c, hipStream_t s, int n)
+{
+  if (!c.ktime) return 0;
+  W2K_HIP(hipStreamSynchronize(s));
+  double tot = 0.0;
+  int cnt = 0;
+  for (int j0 = 0; n - j0 - BND >= 2; j0 += BND) {
+    float ms = 0.f;
+    if (hipEventElapsedTime(&ms, c.kev[2 * cnt], c.kev[2 * cnt + 1]) != hipSuccess) {
+      (void)hipGetLastError();
+      break;
+    }
+    tot += ms;
+    cnt++;
+  }
+  c.last_ms[10] = tot;
+  c.last_ms[11] = cnt;
+  return 0;
+}
+
+template <bool CX>
+static int reduce(Ctx &c, hipStream_t s, SbArgs &g)
+{
+  const int n = g.n, cp = CX ? 2 : 1;
+  int rc;
+  const bool kt = c.ktime != 0;
+  while (kt && c.kev.size() < (size_t)2 * (n / BND + 1)) {
+    hipEvent_t e;
+    W2K_HIP(hipEventCreate(&e));
+    c.kev.push_back(e);
+  }
+  int panel = 0;
+  auto nexch = [&](int m) { return (size_t)((m + QR_ROWS - 1) / QR_ROWS + 1) * BND * BND * cp; };
+  if (n - BND >= 2) {
+    const size_t k = nexch(n - BND);
+    hipLaunchKernelGGL(k_sb_reset, dim3((unsigned)((k + 255) / 256)), dim3(256), 0, s, g.exch, k, g.sync);
+    W2K_STAGE(s, "k_sb_reset");
+  }
+  for (int j0 = 0; n - j0 - BND >= 2; j0 += BND) {
+    const int r0 = j0 + BND, m = n - r0;
+    hipLaunchKernelGGL((k_sb_qr<CX>), dim3((m + QR_ROWS - 1) / QR_ROWS), dim3(QR_ROWS), 0, s, g, j0);
+    W2K_STAGE(s, "k_sb_qr");
+    int slab = 1;
+    const int nz = av_slices(m, slab), tiles = (m + 63) / 64;
+    const int nwg = (m + 31) / 32;
+    if (kt)
+      hipExtLaunchKernelGGL((k_sb_av<CX>), dim3(tiles + 1, nz), dim3(256), 0, s, c.kev[2 * panel], c.kev[2 * panel + 1],
+                            0, g, r0, slab, tiles * 64);
+    else hipLaunchKernelGGL((k_sb_av<CX>), dim3(tiles + 1, nz), dim3(256), 0, s, g, r0, slab, tiles * 64);
+    panel++;
+    W2K_STAGE(s, "k_sb_av");
+    hipLaunchKernelGGL((k_sb_y<CX>), dim3(nwg), dim3(256), 0, s, g, r0, nz, tiles * 64);
+    W2K_STAGE(s, "k_sb_y");
+    hipLaunchKernelGGL(k_sb_s, dim3(BND * cp), dim3(256), 0, s, g, nwg, BND * BND * cp);
+    W2K_STAGE(s, "k_sb_s");
+    hipLaunchKernelGGL((k_sb_w<CX>), dim3(nwg), dim3(256), 0, s, g, r0, nexch(m));
+    W2K_STAGE(s, "k_sb_w");
+    // A(r0:n, r0:n) -= [V W] [W V]^H, lower triangle
+    const size_t o = (size_t)r0 + (size_t)g.lda * r0, ow = (size_t)n * BND + r0;
+    if (CX)
+      rc = zgemm_fused(s, 'N', 'C', m, m, 2 * BND, -1.0, g.Pr + r0, g.Pi + r0, n, g.Pr + ow, g.Pi + ow, n, 1.0, g.ar + o,
+                       g.ai + o, g.lda, 1);
+    else rc = dgemm(s, 'N', 'T', m, m, 2 * BND, -1.0, g.Pr + r0, n, g.Pr + ow, n, 1.0, g.ar + o, g.lda, 1);
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL((k_sb_band<CX>), dim3((n + 3) / 4), dim3(4 * BLD), 0, s, g);
+  W2K_STAGE(s, "k_sb_band");
+  if (n > 1) {
+    // about one sweep in flight per 2 BND columns
+    const int nwg = std::min(256, n / (2 * BND) + 1);
+    hipLaunchKernelGGL((k_sb_chase<CX, 4>), dim3(nwg), dim3(256), 0, s, g);
+    W2K_STAGE(s, "k_sb_chase");
+  }
+  return 0;
+}
+
+int sb_reduce(Ctx &c, hipStream_t s, SbArgs &g, int cplx)
+{
+  return cplx ? reduce<true>(c, s, g) : reduce<false>(c, s, g);
+}
+
+template <bool CX>
+static int apply_q2(hipStream_t s, SbArgs &g, int m, double *Zr, double *Zi, int ldz)
+{
+  const int ntg = (g.n - 1 + BND - 1) / BND;
+  if (ntg == 0 || m == 0) return 0;
+  const size_t words = q2_words(g.n, m);
+  hipLaunchKernelGGL((k_sb_frag<CX>), dim3(ntg, ntg), dim3(256), 0, s, g, ntg, (int)words);
+  W2K_STAGE(s, "k_sb_frag");
+  const int nwg = (int)std::min(words - 1, (size_t)512);
+  hipLaunchKernelGGL((k_sb_q2<CX>), dim3(nwg), dim3(256), 0, s, g, ntg, m, Zr, Zi, ldz);
+  W2K_STAGE(s, "k_sb_q2");
+  return 0;
+}
+
+int sb_apply_q2(Ctx &c, hipStream_t s, SbArgs &g, int cplx, int m, double *Zr, double *Zi, int ldz)
+{
+  int rc;
+  if ((rc = c.w_frag.alloc(sb_frag_doubles(g.n, m, cplx)))) return rc;
+  g.frag = c.w_frag.p;
+  const size_t ntg = (g.n - 1 + BND - 1) / BND;
+  g.q2sync = reinterpret_cast<int *>(g.frag + ntg * (ntg + 1) / 2 * FRAG * (cplx ? 2 : 1));
+  return cplx ? apply_q2<true>(s, g, m, Zr, Zi, ldz) : apply_q2<false>(s, g, m, Zr, Zi, ldz);
+}
+
+}  // namespace w2k

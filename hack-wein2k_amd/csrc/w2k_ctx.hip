@@ -11,6 +11,8 @@
 #include <thread>
 
 #include "w2k_internal.h"
+#include "seclr4_shared.h"
+#include "twostage.h"
 #include "../../include/w2k_lapw1_test.h"
 
 // Scratch of w2k_seclr4_noalloc: every SECLR4 workspace of that entry point
@@ -412,12 +414,14 @@ void drop_kpoint_state(Ctx &c)
 {
   DBuf<double> *bufs[] = {&c.d_kvec, &c.d_hs, &c.d_hsdiag, &c.d_al, &c.d_bl, &c.d_cs, &c.d_theta, &c.d_colcoef,
                           &c.d_hnsL, &c.d_hnsR, &c.h_small, &c.h_re, &c.h_im, &c.d_eig, &c.d_z, &c.w_a,
-                          &c.w_b, &c.w_c, &c.w_v, &c.w_x, &c.w_small, &c.w_fac, &c.w_bt, &c.w_cl, &c.w_gk, &c.w_3m};
+                          &c.w_b, &c.w_c, &c.w_v, &c.w_x, &c.w_small, &c.w_fac, &c.w_bt, &c.w_cl, &c.w_gk, &c.w_3m,
+                          &c.w_sb, &c.w_frag};
   for (DBuf<double> *b : bufs) b->release();
   c.d_kzz.release();
   c.h_int.release();
   c.w_int.release();
   c.w_piv.release();
+  c.w_sbi.release();
   c.w_dig.release();
   if (c.tri_graph.exec) (void)hipGraphExecDestroy(c.tri_graph.exec);
   c.tri_graph = Ctx::TriGraph();
@@ -550,14 +554,12 @@ static void *noalloc_scratch(int device)
 // seclr4_complex, seclr4_buffers and tridiag_eigen, each rounded to 256 bytes
 static size_t noalloc_bytes(size_t n, size_t m, int cplx)
 {
-  const size_t z = cplx ? 2 : 1, lda = (n + 15) & ~(size_t)15, nt = (n + 63) / 64;
+  const size_t z = cplx ? 2 : 1, lda = (n + 15) & ~(size_t)15;
   auto r = [](size_t doubles) { return (doubles * 8 + 255) & ~(size_t)255; };
   size_t b = 0;
   b += cplx ? 4 * r(2 * n * n) : 3 * r(n * n) + r(lda * n);                  // U, H/C, W, X
   b += r((size_t)1 << 22);                                                   // split-K partials
-  const size_t npart = cplx ? std::max(2 * nt * n, 128 * nt * (nt + 1)) : std::max(nt * n, 64 * nt * (nt + 1));
-  b += r(12 * n + z * 2 * n + z * 3 * n * 32 + npart + z * nt * 64 + nt * (nt + 1) / 2 + 2 + nt + n / 32 +
-         64 + 64 + 768);                                                     // tridiagonal work
+  b += r(seclr4_doubles(n, cplx));                                           // tridiagonal work
   b += r((6 * n + 32 + 1) / 2);                                              // ints
   b += r(m + 1);                                                             // eigenvalues
   const size_t zp = ((n + 2) / 2) * 2 * m;
@@ -565,6 +567,9 @@ static size_t noalloc_bytes(size_t n, size_t m, int cplx)
   b += r(2 * n * 64 + 2 * 64 * 64 + m * 64 + m + 1);                         // clusters
   b += r(z * n * (m + 1));                                                   // Z
   b += cplx ? r(2 * (2 * n + 3 * 64 + 2 * m) * 64 + 64 * 64 * 64) : r((2 * n + 2 * m + 3 * 128) * 128 + 32 * 128 * 128);
+  size_t nint = 0;
+  b += r(sb_doubles((int)n, cplx, &nint)) + r(sb_frag_doubles((int)n, m, cplx));   // two-stage tridiagonalisation
+  b += r((nint + 1) / 2);
   return b;
 }
 
@@ -741,8 +746,8 @@ int w2k_seclr4_noalloc(w2k_ctx *x, int n, double *hs, double *hsdiag, double el,
   // and restored afterwards; HS/HSDIAG are the caller's buffers, every
   // workspace and the eigenpairs come from the scratch
   DBuf<double> *dbufs[] = {&c.d_hs, &c.d_hsdiag, &c.d_eig, &c.d_z, &c.w_a, &c.w_b, &c.w_c, &c.w_v, &c.w_x,
-                           &c.w_small, &c.w_fac, &c.w_bt, &c.w_cl, &c.w_gk};
-  DBuf<int> *ibufs[] = {&c.w_int, &c.w_piv};
+                           &c.w_small, &c.w_fac, &c.w_bt, &c.w_cl, &c.w_gk, &c.w_sb, &c.w_frag};
+  DBuf<int> *ibufs[] = {&c.w_int, &c.w_piv, &c.w_sbi};
   constexpr int ND = sizeof(dbufs) / sizeof(dbufs[0]), NI = sizeof(ibufs) / sizeof(ibufs[0]);
   DBuf<double> dsave[ND];
   DBuf<int> isave[NI];

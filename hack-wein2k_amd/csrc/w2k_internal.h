@@ -181,13 +181,16 @@ struct Ctx {
   DBuf<double> w_bt;    // back-transform panel work
   DBuf<double> w_cl;    // cluster orthogonalisation work
   DBuf<double> w_gk;    // split-K GEMM partial products
+  DBuf<double> w_sb;    // two-stage tridiagonalisation: panel sums, band, reflector scalars
+  DBuf<int> w_sbi;      // its progress and registration words
+  DBuf<double> w_frag;  // operands of the second stage's reflector blocks
   DBuf<double> w_3m;    // three-product complex GEMM: Re + Im of both operands, one real product
   // launch mode of the tridiagonalisation, chosen per shape by measurement:
   // direct launches or one captured HIP graph replayed (seclr4.hip)
   int graphs = 0;  // 1: capture and replay where it measures faster (off by default)
   struct TriGraph {
     int n = -1, lda = 0;  // key: order, leading dimension and the buffers the launches address
-    const void *a = nullptr, *small = nullptr, *ints = nullptr;
+    const void *a = nullptr, *small = nullptr, *ints = nullptr, *sb = nullptr, *v2 = nullptr;
     hipGraphExec_t exec = nullptr;
     int seen = 0;      // calls with this key
     int mode = -1;     // last call: 0 direct, 1 replay, 2 capture and replay, -1 none
@@ -202,7 +205,7 @@ struct Ctx {
   // timing
   hipEvent_t ev[W2K_NEVENTS];
   double last_ms[W2K_NTIMINGS] = {0};
-  // per-launch timing of the tridiagonalisation SYMV (off unless requested)
+  // per-launch timing of the tridiagonalisation's panel products (off unless requested)
   int ktime = 0;
   std::vector<hipEvent_t> kev;
 };

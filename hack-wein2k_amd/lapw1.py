@@ -530,7 +530,8 @@ class Lapw1:
                     "tri_launch_mode")
 
     def set_kernel_timing(self, on: bool):
-        """Per-launch events around the tridiagonalisation SYMV kernels."""
+        """Per-launch events around the tridiagonalisation's products of the
+        trailing matrix with a panel (the tri_symv timings)."""
         self._chk("w2k_set_kernel_timing", self.lib.w2k_set_kernel_timing(self.ctx, int(bool(on))))
 
     def set_graphs(self, on: bool):

@@ -337,21 +337,22 @@ int w2k_sync(w2k_ctx *ctx);
  * [3] Cholesky, [4] reduction to standard form, [5] tridiagonalisation,
  * [6] bisection + inverse iteration, [7] back-transforms, [8] the HAMILT
  * plane-wave pair kernel alone, [9] the HNS rank-K GEMM alone, [10] the
- * summed time of the tridiagonalisation SYMV kernels and [11] their number of
- * launches (both only while per-launch timing is on), [12] the launch mode of
+ * summed time of the tridiagonalisation's products of the trailing matrix with
+ * a panel of 32 reflectors and [11] their number of launches (both only while
+ * per-launch timing is on), [12] the launch mode of
  * the last tridiagonalisation (0 direct launches, 1 replay of a captured HIP
  * graph, 2 capture and replay; see w2k_set_graphs).  At most n values are
  * written. */
 int w2k_last_timings(w2k_ctx *ctx, double *ms, int n);
 
-/* Per-launch HIP events around the tridiagonalisation SYMV kernels (slots
+/* Per-launch HIP events around the tridiagonalisation's panel products (slots
  * [10], [11] of w2k_last_timings); off by default since the events add a
  * little time between launches.  No counterpart in the reference. */
 int w2k_set_kernel_timing(w2k_ctx *ctx, int on);
 
 /* Launch mode of the tridiagonalisation (off by default): with on = 1 the
- * library captures the phase's launches (two kernels per column and one GEMM
- * per 32-column panel, no host read-back) into a HIP graph on the second
+ * library captures the phase's launches (six per 32-column panel and the bulge
+ * chasing, no host read-back) into a HIP graph on the second
  * call with the same order and buffers, replays it on the third, and keeps
  * replaying only if that replay measured faster than the direct launches;
  * on = 0 always launches directly.  Results are the same either way.  The

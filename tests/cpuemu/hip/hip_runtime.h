@@ -228,6 +228,37 @@ inline int __ffsll(unsigned long long x) { return __builtin_ffsll((long long)x);
 #define __builtin_amdgcn_ds_swizzle(v, p) emu::wave_swizzle((v), (p))
 #define __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, x, y, z) emu::wave_mfma_f64((a), (b), (c))
 #define __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, x, y, z) emu::wave_mfma_i8((a), (b), (c))
+// device-scope words: one work-item runs at a time, so plain accesses
+#define __HIP_MEMORY_SCOPE_AGENT 4
+#define __hip_atomic_load(p, o, sc) (*(p))
+#define __hip_atomic_store(p, v, o, sc) ((void)(*(p) = (v)))
+template <class T>
+inline T emu_fetch_add(T *p, T v)
+{
+  const T o = *p;
+  *p = o + v;
+  return o;
+}
+template <class T>
+inline T emu_fetch_or(T *p, T v)
+{
+  const T o = *p;
+  *p = o | v;
+  return o;
+}
+#define __hip_atomic_fetch_add(p, v, o, sc) emu_fetch_add((p), (v))
+#define __hip_atomic_fetch_or(p, v, o, sc) emu_fetch_or((p), (v))
+#define __builtin_amdgcn_s_waitcnt(x) ((void)0)
+#define __builtin_amdgcn_s_sleep(x) ((void)0)
+#define __builtin_amdgcn_sched_barrier(x) ((void)0)
+#define __builtin_amdgcn_fence(...) ((void)0)
+#define __builtin_amdgcn_wave_barrier() ((void)emu::wave_ballot(1))
+// blocks run one after another: a wait for another block ends at its time limit
+inline long long wall_clock64()
+{
+  static thread_local long long t = 0;
+  return t += 1000000;
+}
 #define __builtin_amdgcn_rcp(x) (1.0 / (x))
 #define __builtin_amdgcn_rsq(x) (1.0 / std::sqrt(x))
 
