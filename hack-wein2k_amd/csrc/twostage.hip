@@ -16,9 +16,9 @@
 // small ones).  Here a panel of BND columns takes six launches, the flops are
 // matrix products, and the serial part is 32 short exchanges per panel and
 // two steps per sweep.  Whole reduction, before -> now (Q2's application in
-// brackets): real N = 221 3.1 -> 1.8 ms, N = 731 10.7 -> 7.4, N = 5951 135 ->
-// 79 (+ 11); complex N = 251 5.4 -> 2.9, N = 1950 47 -> 28 (+ 2), N = 10880
-// 1018 -> 374 (+ 161).
+// brackets): real N = 221 3.1 -> 1.3 ms, N = 731 10.7 -> 5.3, N = 5951 135 ->
+// 64 (+ 11); complex N = 251 5.4 -> 2.6, N = 1950 47 -> 26 (+ 2), N = 10880
+// 1018 -> 360 (+ 161).
 #include <algorithm>
 #include <cmath>
 
@@ -88,6 +88,38 @@ __device__ __forceinline__ double sum32(double v)
   return v + bfly_partner<1>(v);
 }
 
+// the value of one lane, the same for all
+__device__ __forceinline__ double lane_value(double v, int lane)
+{
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+// the lower and the upper half wave's value, in every lane
+__device__ __forceinline__ void swap_halves(double v, double &lower, double &upper)
+{
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)((unsigned long long)b >> 32);
+  const auto x = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto y = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  lower = __longlong_as_double((long long)((unsigned long long)y[0] << 32 | x[0]));
+  upper = __longlong_as_double((long long)((unsigned long long)y[1] << 32 | x[1]));
+}
+// t[0..N-1] per lane, summed over the 32 lanes of each half: lane l returns
+// entry (l & 31) / (32 / N), N = 4 or 8
+template <int N>
+__device__ __forceinline__ double half_sums(double *t, int lane)
+{
+  static_assert(N == 4 || N == 8, "entries");
+#pragma unroll
+  for (int j = 0; j < N / 2; j++) t[j] = swap_sum<16>(t[j], t[j + N / 2]);
+  bfly_step_h<8, N / 4>(t, lane);
+  if constexpr (N == 8) bfly_step_h<4, N / 8>(t, lane);
+  else t[0] += bfly_partner<4>(t[0]);
+  t[0] += bfly_partner<2>(t[0]);
+  return t[0] + bfly_partner<1>(t[0]);
+}
+
 // xLARFG of (alpha, x) with |x|^2 = ss: H = I - tau v v^H, H^H (alpha; x) =
 // (beta; 0), v = (1; scale x), beta real
 struct Reflector {
@@ -103,19 +135,46 @@ __device__ __forceinline__ Reflector larfg(double ar, double ai, double ss)
     h.tr = h.ti = h.sr = h.si = 0.0;
     return h;
   }
-  const double nrm = sqrt(CX ? fma(ar, ar, fma(ai, ai, ss)) : fma(ar, ar, ss));
-  const double b = ar >= 0.0 ? -nrm : nrm;
-  h.beta = b;
-  const double rb = 1.0 / b, dr = ar - b;
-  h.tr = (b - ar) * rb;
+  // norm and 1 / norm by Goldschmidt's iteration from the hardware's estimate
+  // (two rounds and a correction: rounding error only), the library's
+  // functions outside its range
+  const double x = CX ? fma(ar, ar, fma(ai, ai, ss)) : fma(ar, ar, ss);
+  double nrm, inv;
+  if (x > 1.0e-280 && x < 1.0e280) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double q = x * y, hh = 0.5 * y;
+    double e = fma(-q, hh, 0.5);
+    q = fma(q, e, q);
+    hh = fma(hh, e, hh);
+    e = fma(-q, hh, 0.5);
+    q = fma(q, e, q);
+    hh = fma(hh, e, hh);
+    nrm = fma(fma(-q, q, x), hh, q);
+    inv = 2.0 * fma(hh, fma(-nrm, 2.0 * hh, 1.0), hh);
+  } else {
+    nrm = sqrt(x);
+    inv = 1.0 / nrm;
+  }
+  const double a = fabs(ar), d = a + nrm;  // alpha - beta = +-d + i alpha_i
+  const double den = CX ? fma(d, d, ai * ai) : d;
+  double rd;
+  if (den > 1.0e-280 && den < 1.0e280) {
+    rd = __builtin_amdgcn_rcp(den);
+    rd = fma(rd, fma(-den, rd, 1.0), rd);
+    rd = fma(rd, fma(-den, rd, 1.0), rd);
+  } else {
+    rd = 1.0 / den;
+  }
+  const bool neg = ar < 0.0;
+  h.beta = neg ? nrm : -nrm;
+  h.tr = fma(a, inv, 1.0);
   if (CX) {
-    h.ti = -ai * rb;
-    const double rd = 1.0 / fma(dr, dr, ai * ai);
-    h.sr = dr * rd;
+    h.ti = (neg ? -ai : ai) * inv;
+    h.sr = (neg ? -d : d) * rd;
     h.si = -ai * rd;
   } else {
     h.ti = h.si = 0.0;
-    h.sr = 1.0 / dr;
+    h.sr = neg ? -rd : rd;
   }
   return h;
 }
@@ -737,65 +796,96 @@ __global__ __launch_bounds__(256) void k_sb_w(SbArgs g, int r0, size_t nexch)
 // ------------------------------------------------------------------ 2. bulge chasing
 // band storage: column j at ab + BLD j, entry (i, j) at offset i - j (0..BLD-1)
 constexpr int BLD = 2 * BND;
+constexpr int BPAD = 4 * BND;  // columns of zeros after the band's last one
 constexpr int CHASE_DONE = 1 << 30;
+constexpr int CHASE_KD = 3, CHASE_KZ = 2;  // sweeps per work-group (real, complex)
 
 template <bool CX>
 __global__ void k_sb_band(SbArgs g)
 {
   const int o = threadIdx.x & (BLD - 1), j = blockIdx.x * (blockDim.x / BLD) + threadIdx.x / BLD;
-  if (j >= g.n) return;
+  if (j >= g.n + BPAD) return;
   const bool in = o <= BND && j + o < g.n;
-  const size_t a = (size_t)min(j + o, g.n - 1) + (size_t)g.lda * j, d = (size_t)BLD * j + o;
+  const size_t a = in ? (size_t)(j + o) + (size_t)g.lda * j : 0, d = (size_t)BLD * j + o;
   g.ab[d] = in ? g.ar[a] : 0.0;
-  if (CX) g.ab[(size_t)BLD * g.n + d] = in && o > 0 ? g.ai[a] : 0.0;
-  if (o == 0) {
-    g.prog[j] = 0;
-    if (j == 0) {
-      g.prog[g.n] = 0;  // sweep ticket
-      if (g.n == 1) g.d[0] = g.ar[0];
-    }
-  }
+  if (CX) g.ab[(size_t)BLD * (g.n + BPAD) + d] = in && o > 0 ? g.ai[a] : 0.0;
+  if (o == 0 && j <= g.n) g.prog[j] = 0;  // the last one: the sweeps' ticket
 }
 
-// t[0..NC-1] per lane, summed over the 32 lanes of each half: lane l returns
-// entry (l & 31) >> SH, SH = 5 - log2(NC)
-template <int NC>
-__device__ __forceinline__ double half_reduce(double *t, int lane)
+template <class T>
+__device__ __forceinline__ T *byte_at(T *p, unsigned bytes)
 {
-  static_assert(NC == 16 || NC == 8 || NC == 4, "columns per lane");
-#pragma unroll
-  for (int j = 0; j < NC / 2; j++) t[j] = swap_sum<16>(t[j], t[j + NC / 2]);
-  bfly_step_h<8, NC / 4>(t, lane);
-  if constexpr (NC >= 8) bfly_step_h<4, NC / 8>(t, lane);
-  else t[0] += bfly_partner<4>(t[0]);
-  if constexpr (NC >= 16) bfly_step_h<2, 1>(t, lane);
-  else t[0] += bfly_partner<2>(t[0]);
-  return t[0] + bfly_partner<1>(t[0]);
+  return (T *)((std::conditional_t<std::is_const_v<T>, const char, char> *)p + bytes);
 }
+
+constexpr int CNC = 4;  // columns per lane of a sweep's four waves
 
 // Sweep s reduces column s of the band and chases the bulge that this makes
 // down the matrix.  Rows R_t = s + 1 + BND t .. (BND of them); step t applies
 // the reflector of R_t to the diagonal block D = A(R_t, R_t) from both sides
 // and to C = A(R_t+1, R_t) from the right, and forms the reflector of R_t+1
-// from C's first column and applies it to C from the left.  Step t of sweep s
-// needs steps up to t + 1 of sweep s - 1 (C's last entry is what that step
-// leaves of its first column), so sweeps follow each other two steps apart.
-// A work-group takes whole sweeps in order from a ticket: the oldest
-// unfinished sweep always has a running work-group and waits for nothing, so
-// no residency is assumed.  NW waves share a step: lane (r, h) of wave w holds
-// row r, columns (2 w + h) NC .. of D (mirrored) and C.
-template <bool CX, int NW>
-__global__ __launch_bounds__(64 * NW) void k_sb_chase(SbArgs g)
+// from C's first column and applies it to C from the left: it reads and
+// writes the band's columns R_t.  Step t of sweep s needs the steps up to
+// t + 1 of sweep s - 1 (C's last entry is what that step leaves of its first
+// column), so sweeps follow each other two steps apart; step -1 forms the
+// reflector of R_0 from column s.
+//
+// What a sweep costs is that distance: two steps, and the way of the columns
+// through memory (drain, flag, poll, load: about 3 us).  So a work-group runs
+// K consecutive sweeps, four waves each, in step: at tick k sweep w of the
+// group does its step k - 2 w, and hands its columns to the next sweep through
+// LDS (two steps' columns, the older ones read at the start of the tick in
+// which they are overwritten).  Only the first sweep reads the band from
+// memory, a tick ahead, and only the last writes it, publishing its progress a
+// tick late, so that neither waits for memory within a tick.
+//
+// A step itself is bound by the chain of its operations and, with K waves on
+// each SIMD, by their issue.  Two barriers a step: between the waves' shares
+// of D v and C v and their sums, and before the next sweep reads; what follows
+// the sums is done by every wave for itself.  The band has columns of zeros
+// after the last one, and sweeps and steps past the matrix' end run on those:
+// no step has an edge.  Reduction as a whole with one sweep per work-group and
+// three barriers a step -> as here: real N = 731 7.4 -> 5.3 ms, N = 5951 79 ->
+// 64; complex N = 251 2.9 -> 2.6, N = 1950 28.2 -> 25.8.  K = 2, 3, 4 take
+// 5.5, 5.3, 5.5 (N = 731) and 69, 64, 63 ms (N = 5951), complex K = 1, 2, 3
+// 3.2, 2.6, 2.5 (N = 251) and 30.8, 25.8, 26.4 ms (N = 1950).
+//
+// A work-group takes groups of sweeps in order from a ticket: the oldest
+// unfinished group always has a running work-group and waits for nothing, so
+// no residency is assumed.  Lane (r, h) of wave w of a sweep holds row r,
+// columns (2 w + h) CNC .. of D (mirrored) and C.
+template <bool CX, int K>
+__global__ __launch_bounds__(256 * K) void k_sb_chase(SbArgs g)
 {
-  constexpr int NC = 16 / NW, CP = CX ? 2 : 1;
-  __shared__ double yz[2][CP][2 * NW][BND], xc[CP][BND];
-  __shared__ double vb[NW][CP][BND], ub[NW][CP][BND], gb[NW][CP][BND];
+  constexpr int CP = CX ? 2 : 1;
+  // columns of a sweep's last two steps for the next sweep; column 64 repeats
+  // column 0, so that 32 columns from an odd place on lie in one piece
+  constexpr int RING = (2 * BND + 1) * BLD;
+  __shared__ double ring[K > 1 ? K - 1 : 1][CP][K > 1 ? RING : 1];
+  __shared__ double yz[K][CP][4][2 * BND], xc[K][CP][BND];  // y and z of a wave, side by side
+  // the same values from each of a sweep's waves
+  __shared__ __align__(16) double vb[K][CP][BND], ub[K][CP][BND], gb[K][CP][BND];
   __shared__ int tick;
-  const int n = g.n, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = lane & 31, h = lane >> 5, j0 = (2 * wave + h) * NC;
-  double *const abr = g.ab, *const abi = g.ab + (size_t)BLD * n;
-  const int nsweep = n - 1;
+  const int n = g.n, tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 8), wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
+  const int r = lane & 31, h = lane >> 5, j0 = (2 * wave + h) * CNC;
+  const int ngroup = (n + K - 1) / K;
   const bool first = wave == 0 && h == 0;  // lanes that hold column 0
+  const bool lead = (tid & 255) == 0;
+  const size_t plane = (size_t)BLD * (n + BPAD);
+  // places in the band (bytes from the step's first column): entry (r, j0 + q)
+  // of D below the diagonal at ob + QS q, of C CS further; D mirrored at od[q]
+  constexpr unsigned QS = 8 * (BLD - 1), CS = 8 * BND;
+  const unsigned ob = 8 * (r + (BLD - 1) * j0);
+  unsigned od[CNC];
+#pragma unroll
+  for (int q = 0; q < CNC; q++) {
+    const int j = j0 + q;
+    od[q] = 8 * (r >= j ? r + (BLD - 1) * j : j + (BLD - 1) * r);
+  }
+  // what no sweep writes there (entry (31, j < 31) of the next sweep's C) is zero
+  if constexpr (K > 1)
+    for (int i = tid; i < (K - 1) * CP * RING; i += 256 * K) (&ring[0][0][0])[i] = 0.0;
   // one work-item takes the ticket; a barrier stands on both sides of it, so
   // that no lane runs ahead with the old one
   auto ticket = [&]() {
@@ -803,227 +893,270 @@ __global__ __launch_bounds__(64 * NW) void k_sb_chase(SbArgs g)
   };
   if (tid == 0) tick = ticket();
   __syncthreads();
-  int s = __builtin_amdgcn_readfirstlane(tick);
-  while (s < nsweep) {
+  int grp = __builtin_amdgcn_readfirstlane(tick);
+  while (grp < ngroup) {
+    const int s = grp * K + w;
+    // steps of the group's first sweep, and one of zeros
+    const int nst = (n - 1 - grp * K + BND - 1) / BND + 1, ntick = nst + 2 * (K - 1);
+    auto flag = [&]() { return grp > 0 ? agent_ld(g.prog + grp - 1) : CHASE_DONE; };
     auto wait = [&](int need) {
-      if (s > 0)
-        while (agent_ld(g.prog + s - 1) < need) __builtin_amdgcn_s_sleep(1);
+      while (__builtin_amdgcn_readfirstlane(flag()) < need) __builtin_amdgcn_s_sleep(1);
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
     };
-    wait(2);
-    double dr[NC], di[CX ? NC : 1], cr[NC], ci[CX ? NC : 1];
-    // D and C of the step whose rows start at c0 (L and L2 rows)
-    auto load = [&](int c0) {
-      const int L = min(BND, n - c0), L2 = min(BND, n - c0 - BND);
+    double dr[CNC], di[CX ? CNC : 1], cr[CNC], ci[CX ? CNC : 1];    // D and C of the step
+    double pd[CNC], pdi[CX ? CNC : 1], pc[CNC], pci[CX ? CNC : 1];  // of the next one (first sweep)
+    double vj[CNC], vji[CX ? CNC : 1];                              // v at this lane's columns
+    double vr = 0.0, vi = 0.0, tr = 0.0, ti = 0.0;                  // v(r) and tau of the step's reflector
+    int done = 0;                                                   // steps to publish (last sweep)
+    int seen = 0;                                                   // progress of the group before (first sweep)
+    // raw D and C of the step whose rows start at c0, from the band
+    auto fetch = [&](int c0) {
+      const double *b = g.ab + (size_t)BLD * c0;
 #pragma unroll
-      for (int q = 0; q < NC; q++) {
-        const int j = j0 + q;
-        const int hi = max(r, j), lo = min(r, j);
-        const bool okd = hi < L, okc = r < L2;
-        const size_t od = okd ? (size_t)(hi - lo) + (size_t)BLD * (c0 + lo) : 0;
-        const size_t oc = okc ? (size_t)(BND + r - j) + (size_t)BLD * (c0 + j) : 0;
-        const double a = agent_ld(abr + od), c = agent_ld(abr + oc);
-        dr[q] = okd ? a : 0.0;
-        cr[q] = okc ? c : 0.0;
+      for (int q = 0; q < CNC; q++) {
+        pd[q] = agent_ld(byte_at(b, od[q]));
+        pc[q] = agent_ld(byte_at(b, ob) + (CS + QS * q) / 8);
         if (CX) {
-          const double a2 = agent_ld(abi + od), c2 = agent_ld(abi + oc);
-          di[q] = okd && r != j ? (r > j ? a2 : -a2) : 0.0;
-          ci[q] = okc ? c2 : 0.0;
+          pdi[q] = agent_ld(byte_at(b + plane, od[q]));
+          pci[q] = agent_ld(byte_at(b + plane, ob) + (CS + QS * q) / 8);
         }
       }
     };
-    int c0 = s + 1;
-    double vr, vi = 0.0, tr, ti;  // v(r) and tau of the step's reflector
-    {
-      const int L = min(BND, n - c0);
-      const bool ok = r < L;
-      const size_t o = (size_t)BLD * s + (ok ? 1 + r : 0);
-      double x = agent_ld(abr + o), x2 = CX ? agent_ld(abi + o) : 0.0;
-      const double dg = agent_ld(abr + (size_t)BLD * s);
-      load(c0);
-      x = ok ? x : 0.0;
-      x2 = ok ? x2 : 0.0;
-      const double ss = sum32(r > 0 ? (CX ? x * x + x2 * x2 : x * x) : 0.0);
-      const double ar = __shfl(x, 0, 64), ai = CX ? __shfl(x2, 0, 64) : 0.0;
-      const Reflector f = larfg<CX>(ar, ai, ss);
-      vr = r == 0 ? 1.0 : (CX ? f.sr * x - f.si * x2 : f.sr * x);
-      if (CX) vi = r == 0 ? 0.0 : f.sr * x2 + f.si * x;
+    // the reflector of x (rows c1 + r), its sum of squares below the first
+    // known: v and tau; v to this lane's columns, v and tau to memory
+    auto reflect = [&](int c1, int t1, double x, double x2, double ss) {
+      const Reflector f = larfg<CX>(lane_value(x, 0), CX ? lane_value(x2, 0) : 0.0, ss);
+      vr = r == 0 ? 1.0 : (CX ? fma(f.sr, x, -(f.si * x2)) : f.sr * x);
+      if (CX) vi = r == 0 ? 0.0 : fma(f.sr, x2, f.si * x);
       tr = f.tr;
       ti = f.ti;
-      if (first && ok) {
-        g.V2r[(size_t)c0 + r + (size_t)n * s] = vr;
-        if (CX) g.V2i[(size_t)c0 + r + (size_t)n * s] = vi;
-      }
-      if (tid == 0) {
-        g.d[s] = dg;
-        g.e[s] = f.beta;
-        g.tau2[s] = tr;
-        if (CX) g.tau2[g.ntau2 + s] = ti;
-      }
-    }
-    for (int t = 0;; t++) {
-      const int L = min(BND, n - c0), L2 = min(BND, n - c0 - BND);
-      // v at this lane's columns
       if (h == 0) {
-        vb[wave][0][r] = vr;
-        if (CX) vb[wave][1][r] = vi;
+        vb[w][0][r] = vr;
+        if (CX) vb[w][CP - 1][r] = vi;
       }
-      wave_sync();
-      double vj[NC], vji[CX ? NC : 1];
-#pragma unroll
-      for (int q = 0; q < NC; q++) {
-        vj[q] = vb[wave][0][j0 + q];
-        if (CX) vji[q] = vb[wave][1][j0 + q];
-      }
-      // y = D v, z = C v
-      double yr = 0.0, yi = 0.0, zr = 0.0, zi = 0.0;
-#pragma unroll
-      for (int q = 0; q < NC; q++) {
-        yr += dr[q] * vj[q];
-        zr += cr[q] * vj[q];
-        if (CX) {
-          yr -= di[q] * vji[q];
-          yi += dr[q] * vji[q] + di[q] * vj[q];
-          zr -= ci[q] * vji[q];
-          zi += cr[q] * vji[q] + ci[q] * vj[q];
+      if (first && s < n - 1 && c1 + r < n) {
+        const size_t o = (size_t)c1 + (size_t)n * s;
+        (g.V2r + o)[r] = vr;
+        if (CX) (g.V2i + o)[r] = vi;
+        if (r == 0) {
+          const size_t o2 = (size_t)t1 * n + s;
+          g.tau2[o2] = tr;
+          if (CX) g.tau2[g.ntau2 + o2] = ti;
         }
       }
-      yz[0][0][2 * wave + h][r] = yr;
-      yz[1][0][2 * wave + h][r] = zr;
-      if (CX) {
-        yz[0][CP - 1][2 * wave + h][r] = yi;
-        yz[1][CP - 1][2 * wave + h][r] = zi;
+      return f.beta;
+    };
+    for (int k = -1; k < ntick; k++) {
+      const int t = k - 2 * w, c0 = s + 1 + BND * t;
+      const bool act = t >= 0 && t < nst;
+      if (act) {
+        if (w > 0) {
+          // the columns that the sweep before left, one further on
+          const double *b = ring[w > 0 ? w - 1 : 0][0] + ((t & 1) * BND + 1) * BLD;
+          const double *b2 = ring[w > 0 ? w - 1 : 0][CP - 1] + ((t & 1) * BND + 1) * BLD;
+#pragma unroll
+          for (int q = 0; q < CNC; q++) {
+            dr[q] = *byte_at(b, od[q]);
+            cr[q] = byte_at(b, ob)[(CS + QS * q) / 8];
+            if (CX) {
+              di[q] = *byte_at(b2, od[q]);
+              ci[q] = byte_at(b2, ob)[(CS + QS * q) / 8];
+            }
+          }
+        } else {
+          // C's last row holds one entry, in its last column; what memory has
+          // for the others is older than the bulge
+#pragma unroll
+          for (int q = 0; q < CNC; q++) {
+            const bool okc = r < BND - 1 || j0 + q == BND - 1;
+            dr[q] = pd[q];
+            cr[q] = okc ? pc[q] : 0.0;
+            if (CX) {
+              di[q] = pdi[q];
+              ci[q] = okc ? pci[q] : 0.0;
+            }
+          }
+        }
+        if (CX)
+#pragma unroll
+          for (int q = 0; q < CNC; q++) di[q] = r < j0 + q ? -di[q] : di[q];
+        if (first) {
+          xc[w][0][r] = cr[0];
+          if (CX) xc[w][CP - 1][r] = ci[0];
+        }
+        // y = D v, z = C v: this wave's eight columns
+        double yr = 0.0, yi = 0.0, zr = 0.0, zi = 0.0;
+#pragma unroll
+        for (int q = 0; q < CNC; q++) {
+          vj[q] = vb[w][0][j0 + q];
+          if (CX) vji[q] = vb[w][CP - 1][j0 + q];
+          yr = fma(dr[q], vj[q], yr);
+          zr = fma(cr[q], vj[q], zr);
+          if (CX) {
+            yr = fma(-di[q], vji[q], yr);
+            yi = fma(di[q], vj[q], fma(dr[q], vji[q], yi));
+            zr = fma(-ci[q], vji[q], zr);
+            zi = fma(ci[q], vj[q], fma(cr[q], vji[q], zi));
+          }
+        }
+        // lanes of the lower half take y, of the upper half z
+        yz[w][0][wave][lane] = swap_sum<32>(yr, zr);
+        if (CX) yz[w][CP - 1][wave][lane] = swap_sum<32>(yi, zi);
+      }
+      if (done) vm_drain();
+      __syncthreads();
+      if (done && lead) agent_st(g.prog + grp, done);
+      done = 0;
+      if (w == 0 && t + 1 < nst) {
+        if (__builtin_amdgcn_readfirstlane(seen) < t + 3) wait(t + 3);
+        fetch(c0 + BND);
+        seen = flag();
+      }
+      if (act) {
+        double a = 0.0, a2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          a += yz[w][0][q][lane];
+          if (CX) a2 += yz[w][CP - 1][q][lane];
+        }
+        double yr, zr, yi = 0.0, zi = 0.0;
+        swap_halves(a, yr, zr);
+        if (CX) swap_halves(a2, yi, zi);
+        // C's first column after C <- C - tau z v^H (v(0) = 1)
+        const double tzr = CX ? fma(tr, zr, -(ti * zi)) : tr * zr, tzi = CX ? fma(tr, zi, ti * zr) : 0.0;
+        const double x = xc[w][0][r] - tzr, x2 = CX ? xc[w][CP - 1][r] - tzi : 0.0;
+        // v^H y in the lower half, the new column's sum of squares in the upper
+        const double py = CX ? fma(vr, yr, vi * yi) : vr * yr;
+        const double px = r > 0 ? (CX ? fma(x, x, x2 * x2) : x * x) : 0.0;
+        const double sums = sum32(h ? px : py);
+        const double p = lane_value(sums, 0), ss = lane_value(sums, 32);
+        // u = tau y - 1/2 |tau|^2 (v^H y) v;  D <- D - u v^H - v u^H
+        const double hp = 0.5 * p * (CX ? fma(tr, tr, ti * ti) : tr * tr);
+        const double ur = fma(-hp, vr, CX ? fma(tr, yr, -(ti * yi)) : tr * yr);
+        const double ui = CX ? fma(-hp, vi, fma(tr, yi, ti * yr)) : 0.0;
+        if (h == 0) {
+          ub[w][0][r] = ur;
+          if (CX) ub[w][CP - 1][r] = ui;
+        }
+#pragma unroll
+        for (int q = 0; q < CNC; q++) {
+          if (CX) {
+            cr[q] = fma(-tzi, vji[q], fma(-tzr, vj[q], cr[q]));
+            ci[q] = fma(tzr, vji[q], fma(-tzi, vj[q], ci[q]));
+            dr[q] = fma(-ui, vji[q], fma(-ur, vj[q], dr[q]));
+            di[q] = fma(ur, vji[q], fma(-ui, vj[q], di[q]));
+          } else {
+            cr[q] = fma(-tzr, vj[q], cr[q]);
+            dr[q] = fma(-ur, vj[q], dr[q]);
+          }
+        }
+        const double v0r = vr, v0i = vi;
+        // reflector of the next rows, applied to C from the left
+        const double beta = reflect(c0 + BND, t + 1, x, x2, ss);
+        double tq[CP * CNC];
+#pragma unroll
+        for (int q = 0; q < CNC; q++) {
+          tq[q] = CX ? fma(vr, cr[q], vi * ci[q]) : vr * cr[q];
+          if (CX) tq[CP * CNC - CNC + q] = fma(vr, ci[q], -(vi * cr[q]));
+        }
+        const double gs = half_sums<CP * CNC>(tq, lane);
+        constexpr int SH = CX ? 2 : 3;
+        if (!(r & ((1 << SH) - 1))) gb[w][r >> 4 & (CP - 1)][j0 + ((r >> SH) & (CNC - 1))] = gs;
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < CNC; q++) {
+          const double uj = ub[w][0][j0 + q];
+          if (CX) {
+            const double uji = ub[w][CP - 1][j0 + q];
+            dr[q] = fma(-v0i, uji, fma(-v0r, uj, dr[q]));
+            di[q] = fma(v0r, uji, fma(-v0i, uj, di[q]));
+            if (r == j0 + q) di[q] = 0.0;
+          } else {
+            dr[q] = fma(-v0r, uj, dr[q]);
+          }
+        }
+        // conj(tau) v
+        const double wr = CX ? fma(tr, vr, ti * vi) : tr * vr, wi = CX ? fma(tr, vi, -(ti * vr)) : 0.0;
+#pragma unroll
+        for (int q = 0; q < CNC; q++) {
+          const double gr = gb[w][0][j0 + q];
+          if (CX) {
+            const double gi = gb[w][CP - 1][j0 + q];
+            cr[q] = fma(wi, gi, fma(-wr, gr, cr[q]));
+            ci[q] = fma(-wi, gr, fma(-wr, gi, ci[q]));
+          } else {
+            cr[q] = fma(-wr, gr, cr[q]);
+          }
+        }
+        if (first) {  // column 0 is (beta, 0, ..)
+          cr[0] = r == 0 ? beta : 0.0;
+          if (CX) ci[0] = 0.0;
+        }
+        // leave the columns
+        if (w == K - 1) {
+          double *const b = byte_at(g.ab + (ptrdiff_t)BLD * c0, ob), *const b2 = byte_at(g.ab + plane + (ptrdiff_t)BLD * c0, ob);
+#pragma unroll
+          for (int q = 0; q < CNC; q++) {
+            if (r >= j0 + q) {
+              agent_st(b + QS / 8 * q, dr[q]);
+              if (CX) agent_st(b2 + QS / 8 * q, di[q]);
+            }
+            agent_st(b + (CS + QS * q) / 8, cr[q]);
+            if (CX) agent_st(b2 + (CS + QS * q) / 8, ci[q]);
+          }
+          done = t + 1;
+        } else {
+          double *const b = byte_at(ring[w < K - 1 ? w : 0][0] + (t & 1) * BND * BLD, ob);
+          double *const b2 = byte_at(ring[w < K - 1 ? w : 0][CP - 1] + (t & 1) * BND * BLD, ob);
+#pragma unroll
+          for (int q = 0; q < CNC; q++) {
+            if (r >= j0 + q) {
+              b[QS / 8 * q] = dr[q];
+              if (CX) b2[QS / 8 * q] = di[q];
+            }
+            b[(CS + QS * q) / 8] = cr[q];
+            if (CX) b2[(CS + QS * q) / 8] = ci[q];
+          }
+          if (first && !(t & 1)) {
+            b[2 * BND * BLD] = dr[0];
+            b[2 * BND * BLD + BND] = cr[0];
+            if (CX) {
+              b2[2 * BND * BLD] = di[0];
+              b2[2 * BND * BLD + BND] = ci[0];
+            }
+          }
+        }
+      } else if (t == -1) {
+        // column s: d, e and the reflector of R_0
+        const int o = 1 + r;
+        double x, x2 = 0.0, dg;
+        if (w == 0) {
+          const double *b = g.ab + (size_t)BLD * s;
+          x = agent_ld(b + o);
+          if (CX) x2 = agent_ld(b + plane + o);
+          dg = agent_ld(b);
+          vm_drain();  // here, so that no later step waits for registers of these loads
+        } else {
+          x = ring[w > 0 ? w - 1 : 0][0][o];
+          if (CX) x2 = ring[w > 0 ? w - 1 : 0][CP - 1][o];
+          dg = ring[w > 0 ? w - 1 : 0][0][0];
+        }
+        const double beta = reflect(s + 1, 0, x, x2, sum32(r > 0 ? (CX ? fma(x, x, x2 * x2) : x * x) : 0.0));
+        if (lead && s < n) {
+          g.d[s] = dg;
+          if (s < n - 1) g.e[s] = beta;
+        }
       }
       __syncthreads();
-      yr = zr = yi = zi = 0.0;
-#pragma unroll
-      for (int q = 0; q < 2 * NW; q++) {
-        yr += yz[0][0][q][r];
-        zr += yz[1][0][q][r];
-        if (CX) {
-          yi += yz[0][CP - 1][q][r];
-          zi += yz[1][CP - 1][q][r];
-        }
-      }
-      // C <- C - tau z v^H
-      const double tzr = CX ? tr * zr - ti * zi : tr * zr, tzi = CX ? tr * zi + ti * zr : 0.0;
-#pragma unroll
-      for (int q = 0; q < NC; q++) {
-        if (CX) {
-          cr[q] = fma(-tzi, vji[q], fma(-tzr, vj[q], cr[q]));
-          ci[q] = fma(tzr, vji[q], fma(-tzi, vj[q], ci[q]));
-        } else {
-          cr[q] = fma(-tzr, vj[q], cr[q]);
-        }
-      }
-      if (first) {
-        xc[0][r] = cr[0];
-        if (CX) xc[CP - 1][r] = ci[0];
-      }
-      // u = tau y - 1/2 |tau|^2 (v^H y) v;  D <- D - u v^H - v u^H
-      const double p = sum32(CX ? vr * yr + vi * yi : vr * yr);
-      const double hp = 0.5 * p * (CX ? tr * tr + ti * ti : tr * tr);
-      const double ur = (CX ? tr * yr - ti * yi : tr * yr) - hp * vr;
-      const double ui = CX ? tr * yi + ti * yr - hp * vi : 0.0;
-      if (h == 0) {
-        ub[wave][0][r] = ur;
-        if (CX) ub[wave][CP - 1][r] = ui;
-      }
-      wave_sync();
-#pragma unroll
-      for (int q = 0; q < NC; q++) {
-        const double uj = ub[wave][0][j0 + q];
-        if (CX) {
-          const double uji = ub[wave][CP - 1][j0 + q];
-          dr[q] = fma(-vi, uji, fma(-vr, uj, fma(-ui, vji[q], fma(-ur, vj[q], dr[q]))));
-          di[q] = fma(vr, uji, fma(-vi, uj, fma(ur, vji[q], fma(-ui, vj[q], di[q]))));
-        } else {
-          dr[q] = fma(-vr, uj, fma(-ur, vj[q], dr[q]));
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < NC; q++) {
-        const int j = j0 + q;
-        if (r >= j && r < L) {
-          const size_t o = (size_t)(r - j) + (size_t)BLD * (c0 + j);
-          agent_st(abr + o, dr[q]);
-          if (CX) agent_st(abi + o, r == j ? 0.0 : di[q]);
-          if (r == 0 && s == n - 2) g.d[n - 1] = dr[q];
-        }
-      }
-      if (L2 <= 0) break;
-      __syncthreads();
-      // reflector of the next rows from C's first column, applied from the left
-      const double x = xc[0][r], x2 = CX ? xc[CP - 1][r] : 0.0;
-      const double ss = sum32(r > 0 ? (CX ? x * x + x2 * x2 : x * x) : 0.0);
-      const Reflector f = larfg<CX>(xc[0][0], CX ? xc[CP - 1][0] : 0.0, ss);
-      vr = r == 0 ? 1.0 : (CX ? f.sr * x - f.si * x2 : f.sr * x);
-      if (CX) vi = r == 0 ? 0.0 : f.sr * x2 + f.si * x;
-      tr = f.tr;
-      ti = f.ti;
-      double tq[NC];
-#pragma unroll
-      for (int q = 0; q < NC; q++) tq[q] = CX ? vr * cr[q] + vi * ci[q] : vr * cr[q];
-      constexpr int SH = NC == 16 ? 1 : NC == 8 ? 2 : 3;
-      const double g0 = half_reduce<NC>(tq, lane);
-      if (!(r & ((1 << SH) - 1))) gb[wave][0][h * NC + (r >> SH)] = g0;
-      if (CX) {
-#pragma unroll
-        for (int q = 0; q < NC; q++) tq[q] = vr * ci[q] - vi * cr[q];
-        const double g1 = half_reduce<NC>(tq, lane);
-        if (!(r & ((1 << SH) - 1))) gb[wave][CP - 1][h * NC + (r >> SH)] = g1;
-      }
-      wave_sync();
-      const double wr = CX ? tr * vr + ti * vi : tr * vr, wi = CX ? tr * vi - ti * vr : 0.0;  // conj(tau) v
-#pragma unroll
-      for (int q = 0; q < NC; q++) {
-        const double gr = gb[wave][0][h * NC + q];
-        if (CX) {
-          const double gi = gb[wave][CP - 1][h * NC + q];
-          cr[q] = fma(wi, gi, fma(-wr, gr, cr[q]));
-          ci[q] = fma(-wi, gr, fma(-wr, gi, ci[q]));
-        } else {
-          cr[q] = fma(-wr, gr, cr[q]);
-        }
-      }
-      // column 0 is (beta, 0, ..)
-      if (first) {
-        cr[0] = r == 0 ? f.beta : 0.0;
-        if (CX) ci[0] = 0.0;
-      }
-#pragma unroll
-      for (int q = 0; q < NC; q++) {
-        const int j = j0 + q;
-        if (r < L2) {
-          const size_t o = (size_t)(BND + r - j) + (size_t)BLD * (c0 + j);
-          agent_st(abr + o, cr[q]);
-          if (CX) agent_st(abi + o, ci[q]);
-        }
-      }
-      const int c1 = c0 + BND;
-      if (first && r < L2) {
-        g.V2r[(size_t)c1 + r + (size_t)n * s] = vr;
-        if (CX) g.V2i[(size_t)c1 + r + (size_t)n * s] = vi;
-      }
-      if (tid == 0) {
-        g.tau2[(size_t)(t + 1) * n + s] = tr;
-        if (CX) g.tau2[g.ntau2 + (size_t)(t + 1) * n + s] = ti;
-      }
-      vm_drain();
-      __syncthreads();
-      if (tid == 0) agent_st(g.prog + s, t + 1);
-      c0 = c1;
-      wait(t + 3);
-      load(c0);
     }
     vm_drain();
     __syncthreads();
     if (tid == 0) {
-      agent_st(g.prog + s, CHASE_DONE);
+      agent_st(g.prog + grp, CHASE_DONE);
       tick = ticket();
     }
     __syncthreads();
-    s = __builtin_amdgcn_readfirstlane(tick);
+    grp = __builtin_amdgcn_readfirstlane(tick);
   }
 }
 
@@ -1337,7 +1470,7 @@ size_t sb_doubles(int n, int cplx, size_t *ints)
   const size_t ntg = (n - 1 + BND - 1) / BND;
   if (ints) *ints = (size_t)n + 1 + 8;
   return up32(std::max(tiles, std::min((size_t)1024, tiles * tiles)) * 64 * BND * cp) + up32((size_t)n * BND * cp) +
-         up32((size_t)(n + 31) / 32 * BND * BND * cp) + 3 * up32(BND * BND * cp) + up32((nblk + 1) * BND * BND * cp) + up32((size_t)BLD * n * cp) +
+         up32((size_t)(n + 31) / 32 * BND * BND * cp) + 3 * up32(BND * BND * cp) + up32((nblk + 1) * BND * BND * cp) + up32((size_t)BLD * (n + BPAD) * cp) +
          up32((size_t)n * (ntg + 1) * cp);
 }
 
@@ -1372,7 +1505,7 @@ int sb_buffers(Ctx &c, SbArgs &g, int n, int cplx)
   g.G = take(BND * BND * cp);
   g.S = take(BND * BND * cp);
   g.exch = take((nblk + 1) * BND * BND * cp);
-  g.ab = take((size_t)BLD * n * cp);
+  g.ab = take((size_t)BLD * (n + BPAD) * cp);
   g.tau2 = take((size_t)n * (ntg + 1) * cp);
   g.ntau2 = (size_t)n * (ntg + 1);
   g.prog = c.w_sbi.p;
@@ -1447,14 +1580,13 @@ static int reduce(Ctx &c, hipStream_t s, SbArgs &g)
     else rc = dgemm(s, 'N', 'T', m, m, 2 * BND, -1.0, g.Pr + r0, n, g.Pr + ow, n, 1.0, g.ar + o, g.lda, 1);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL((k_sb_band<CX>), dim3((n + 3) / 4), dim3(4 * BLD), 0, s, g);
+  hipLaunchKernelGGL((k_sb_band<CX>), dim3((n + BPAD + 3) / 4), dim3(4 * BLD), 0, s, g);
   W2K_STAGE(s, "k_sb_band");
-  if (n > 1) {
-    // about one sweep in flight per 2 BND columns
-    const int nwg = std::min(256, n / (2 * BND) + 1);
-    hipLaunchKernelGGL((k_sb_chase<CX, 4>), dim3(nwg), dim3(256), 0, s, g);
-    W2K_STAGE(s, "k_sb_chase");
-  }
+  // groups in flight: one per 2 K + 2 steps
+  constexpr int K = CX ? CHASE_KZ : CHASE_KD;
+  const int nwg = std::min(256, n / (BND * (2 * K + 2)) + 2);
+  hipLaunchKernelGGL((k_sb_chase<CX, K>), dim3(nwg), dim3(256 * K), 0, s, g);
+  W2K_STAGE(s, "k_sb_chase");
   return 0;
 }
 
