@@ -9,8 +9,8 @@
 // over the logarithmic mesh r_k = RO exp(DH (k-1)), the normalisation by
 // 1/sqrt(RINT13(u, u)), the energy derivative by the difference of the
 // functions at E -+ DELE (DELE = 2e-3 Hartree, scaled by 0.25/DELE), its
-// orthogonalisation to u, and RINT13's Simpson sum with the mesh points
-// multiplied out one by one.
+// orthogonalisation to u, and RINT13's Simpson sum (as a weighted sum over the
+// mesh).
 #include <algorithm>
 #include <cmath>
 #include <tuple>
@@ -30,218 +30,326 @@ struct AtparArgs {
   const int *loor;                     // [a][LOMAXP]
   double *fn;                          // [a][l < nslmax][4][jrid]: A1, B1, AE1, BE1
   double *fnlo;                        // [a][l <= lomax][2][jrid]: A1LO, B1LO
-  double *work;                        // [a][l][2][jrid]: A, B of OUTWIN
+  double *work;                        // [a][l][AT_ROWS][jrid]: A, B of OUTWIN per energy; weights
   double *out;                         // [a][l][6]: P, DP, PE, DPE, PEI, E used
   double *outlo;                       // [a][l][4]: PLO, DPLO, PI12LO, PE12LO
 };
 
-// OUTWIN (outwin.f:20-112): A (large) and B (small, times c/2) components,
-// value and slope of u/r at the sphere boundary
-__device__ void outwin(bool rel, const double *v, double rnot, double dh, int jri, double eh, double fl, double z,
-                       double *A, double *B, double &val, double &slo)
+// OUTWIN (outwin.f:20-112) is a recurrence along the mesh.  All that its step
+// needs besides the functions themselves is formed beforehand, for AT_CH mesh
+// points and AT_NE energies at once: U and Y of outwin.f:73-80 (X = -DH) and
+// 1 / DET, whose rounding error goes along: with one rounding more per point
+// the difference of the functions at E -+ DELE would lose a digit's fraction.
+constexpr int AT_NE = 4;    // energies E - DELE, E + DELE, E and the local orbital's
+constexpr int AT_CH = 64;   // mesh points formed at a time
+constexpr int AT_PF = 4;    // mesh points whose operands are read at a time
+constexpr int AT_NC = 4;    // 1 / DET in two parts, U, Y
+constexpr int AT_NT = 64 * (1 + AT_NE);
+constexpr int AT_ROWS = 2 * AT_NE + 1;  // rows of an (atom, l): A and B of each energy, RINT13's weights
+
+struct AtparShared {
+  double __attribute__((aligned(16))) c[2][AT_CH + 2 * AT_PF][AT_NE][AT_NC];  // of this piece of the mesh and the next
+  double f[2][2][AT_CH][AT_NE];  // A, B of this piece and the one before
+  double red[2][AT_NT / 64][3];
+  double end[2][AT_NE], norm[AT_NE];  // value and slope at the boundary; 1 / sqrt of the norm
+};
+
+// OUTWIN's coefficients at mesh point k; of the first three points A, B and
+// their derivatives instead (outwin.f:49-60)
+__device__ __forceinline__ void outwin_coef(bool rel, double v, double rnot, double dh, double eh, double fl, double z,
+                                            int k, double *o)
 {
-  const double e = eh * 2.0;
-  const double zz = z + z;
-  double c = 2.0 * 137.0359895;
-  if (!rel) c = 1.0e10;
+  const double e = eh * 2.0, zz = z + z, c = rel ? 2.0 * 137.0359895 : 1.0e10;
   const double fllp1 = fl * (fl + 1.0);
-  const double r83sq = 64.0 / 9.0, r1 = 1.0 / 9.0, r2 = -5.0 * r1, r3 = 19.0 * r1, h83 = 8.0 / 3.0;
-  const double g0 = 1.0;
-  double s, sf, f0;
-  if (z < 0.9) {
-    s = fl + 1.0;
-    sf = fl;
-    f0 = fl / c;
-  } else {
-    const double aa = zz / c;
-    s = sqrt(fllp1 + 1.0 - aa * aa);
-    sf = s;
-    f0 = g0 * (s - 1.0) / aa;
+  const double r = rnot * exp(dh * (double)k), drdi = dh * r;
+  if (k < 3) {
+    const bool bare = z < 0.9;
+    const double aa = zz / c, s0 = sqrt(fllp1 + 1.0 - aa * aa);
+#pragma unroll 1
+    for (int q = 0; q < 2; q++) {
+      const double s = !bare ? s0 : q == 0 ? fl + 1.0 : fl;
+      const double f0 = q == 0 ? 1.0 : bare ? fl / c : (s0 - 1.0) / aa;
+      o[q] = pow(r, s) * f0;
+      o[2 + q] = drdi * o[q] * s / r;
+    }
+    return;
   }
-  double d1[3], d2[3];
-  for (int k = 0; k < 3; k++) {
-    const double r = rnot * exp(dh * (double)k);
-    const double drdi = dh * r;
-    A[k] = pow(r, s) * g0;
-    B[k] = pow(r, sf) * f0;
-    d1[k] = drdi * A[k] * s / r;
-    d2[k] = drdi * B[k] * sf / r;
-  }
-  double dg1 = d1[0], dg2 = d1[1], dg3 = d1[2], df1 = d2[0], df2 = d2[1], df3 = d2[2];
-  double a_prev = A[2], b_prev = B[2];
-  for (int k = 3; k < jri; k++) {
-    const double r = rnot * exp(dh * (double)k);
-    const double drdi = dh * r;
-    const double phi = (e - 2.0 * v[k] / r) * drdi / c;
-    const double u = drdi * c + phi;
-    const double x = -drdi / r;
-    const double y = -fllp1 * x * x / u + phi;
-    const double det = r83sq - x * x + u * y;
-    const double b11 = a_prev * h83 + r1 * dg1 + r2 * dg2 + r3 * dg3;
-    const double b22 = b_prev * h83 + r1 * df1 + r2 * df2 + r3 * df3;
-    const double ak = (b11 * (h83 - x) + b22 * u) / det;
-    const double bk = (b22 * (h83 + x) - b11 * y) / det;
-    A[k] = ak;
-    B[k] = bk;
-    dg1 = dg2; dg2 = dg3; dg3 = u * bk - x * ak;
-    df1 = df2; df2 = df3; df3 = x * bk - y * ak;
-    a_prev = ak;
-    b_prev = bk;
-  }
-  for (int k = 0; k < jri; k++) B[k] = B[k] * c / 2.0;
-  const double rj = rnot * exp(dh * (double)(jri - 1));
-  val = A[jri - 1] / rj;
-  slo = dg3 / (dh * rj);
-  slo = (slo - val) / rj;
+  const double phi = (e - 2.0 * v / r) * drdi / c;
+  const double u = drdi * c + phi, x = -dh;
+  const double y = -fllp1 * x * x / u + phi;
+  const double det = 64.0 / 9.0 - x * x + u * y, inv = 1.0 / det;
+  o[0] = inv;
+  o[1] = inv * fma(-det, inv, 1.0);
+  o[2] = u;
+  o[3] = y;
 }
 
-// RINT13 (rint13.f:28-62): integral of c1 a x + c2 b y over the mesh
-template <class F>
-__device__ double rint13_of(double rnot, double dx, int jri, F f)
+// RINT13 (rint13.f:28-62) as a weighted sum: weight of mesh point k (0-based)
+__device__ __forceinline__ double rint13_w(double rnot, double dx, int jri, int k)
 {
-  const double d = exp(dx);
-  int j = 3 - (jri % 2);  // 1-based
-  const int j1 = j - 1;
-  double r = rnot * pow(d, (double)(j - 1));
-  const double r1 = r / d;
-  double z4 = 0.0, z2 = 0.0;
-  for (;;) {
-    z4 = z4 + r * f(j - 1);
-    if (z4 == 0.0) z4 = 2.0e-55;
-    r = r * d;
-    j = j + 1;
-    if (j >= jri) break;
-    z2 = z2 + r * f(j - 1);
-    r = r * d;
-    j = j + 1;
-  }
-  const double p1 = rnot * f(0);
-  const double p2 = r1 * f(j1 - 1);
-  double s = 2 * z2 + 4 * z4 + r * f(j - 1) + p2;
-  s = (dx * s + p1) / 3.0;
-  if (j1 > 1) s = s + 0.5 * dx * (p1 + p2);
-  return s;
+  const double r = rnot * exp(dx * (double)k);
+  const int k0 = 2 - jri % 2;  // first point of weight 4
+  double w = k == jri - 1 ? r * dx / 3.0 : k >= k0 ? ((k - k0) & 1 ? 2.0 : 4.0) * r * dx / 3.0 : 0.0;
+  if (k == k0 - 1) w = r * dx / 3.0 + (k0 > 1 ? 0.5 * dx * r : 0.0);
+  if (k == 0) w += rnot / 3.0 + (k0 > 1 ? 0.5 * dx * rnot : 0.0);
+  return w;
 }
+// RINT13 leaves no sum at zero (rint13.f:37)
+__device__ __forceinline__ double rint13_nonzero(double s, double dx) { return s == 0.0 ? dx * (4.0 * 2.0e-55) / 3.0 : s; }
 
-__device__ double rint13(double c1, double c2, const double *a, const double *b, const double *x, const double *y,
-                         double rnot, double dx, int jri)
+__device__ __forceinline__ double wave_sum(double v)
 {
-  return rint13_of(rnot, dx, jri, [&](int k) { return c1 * a[k] * x[k] + c2 * b[k] * y[k]; });
+#pragma unroll 1
+  for (int m = 32; m; m >>= 1) v += __shfl_xor(v, m, 64);
+  return v;
 }
 
-// one thread per (atom type, l): atpar.f:212-289 and, for l <= LOMAX with a
+// sums over the block of N values each; `slot` alternates between calls
+template <int N>
+__device__ __forceinline__ void block_sums(AtparShared &sh, int &slot, double (&s)[N])
+{
+  for (int q = 0; q < N; q++) {
+    s[q] = wave_sum(s[q]);
+    if ((threadIdx.x & 63) == 0) sh.red[slot][threadIdx.x >> 6][q] = s[q];
+  }
+  __syncthreads();
+  for (int q = 0; q < N; q++) {
+    s[q] = 0.0;
+#pragma unroll 1
+    for (int w = 0; w < AT_NT / 64; w++) s[q] += sh.red[slot][w][q];
+  }
+  slot ^= 1;
+}
+
+// one block per (atom type, l): atpar.f:212-289 and, for l <= LOMAX with a
 // local-orbital function, atpar.f:297-330.  The functions of l < NSLMAX are
-// kept (fn, fnlo); those of higher l go to the thread's scratch rows.
-__global__ void k_atpar_l(AtparArgs g, double *__restrict__ scratch)
+// kept (fn, fnlo).
+//
+// Bound by the recurrences' chain (six dependent FP64 operations a mesh point,
+// three or four functions an l) and by the fetch of code that runs once, far
+// from any throughput: so the functions of an l run in lanes of one wave, side
+// by side, their operands read from LDS ahead, while the other four
+// waves form what the next 64 points need (one energy each, a point per lane:
+// an exponential and four divisions a point) and write back the last 64; and
+// the integrals are weighted sums in three loops.  One work-item per l did all
+// of it in turn.  64 atom types, 781 points, 11 l: 3.75 ->
+// 0.18 ms.
+__global__ __launch_bounds__(AT_NT, 4) void k_atpar_l(AtparArgs g)
 {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int a = t / g.nt, l = t % g.nt;
-  if (a >= g.nat) return;
+  __shared__ AtparShared sh;
+  const int l = blockIdx.x, a = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool rel = g.rel != 0;
   const double c1 = 1.0, c2 = rel ? 1.0 / (137.0359895 * 137.0359895) : 1.0e-22;
   const double dele = 2.0e-3, delei = 0.25 / dele;
+  const double cl = rel ? 2.0 * 137.0359895 : 1.0e10;
   const int jri = g.jrj[a];
   const double rnot = g.ro[a], dx = g.dh[a], z = g.zz[a];
   const double *v = g.vr + (size_t)a * g.jrid;
-  double *A = g.work + ((size_t)(a * g.nt + l) * 2) * g.jrid, *B = A + g.jrid;
-  double *A1 = (l < g.nslmax) ? g.fn + ((size_t)(a * g.nslmax + l) * 4) * g.jrid
-                              : scratch + ((size_t)(a * g.nt + l) * 4) * g.jrid;
-  double *B1 = A1 + g.jrid, *AE = A1 + 2 * (size_t)g.jrid, *BE = A1 + 3 * (size_t)g.jrid;
+  const size_t ld = g.jrid;
+  double *const work = g.work + (size_t)(a * g.nt + l) * AT_ROWS * ld, *const wt = work + 2 * AT_NE * ld;
   const double fl = (double)l;
+  const bool lo = l <= g.lomax && g.loor[a * (g.lomax + 1) + l];
+  const double elo = lo ? g.elo[a * (g.lomax + 1) + l] / 2.0 : 0.0;
   double ei = g.e[(size_t)a * g.lmaxd + l] / 2.0;
-  double P = 0, DP = 0, PE = 0, DPE = 0, PEI = 0;
+  int slot = 0;
+  double *const A1 = l < g.nslmax ? g.fn + ((size_t)(a * g.nslmax + l) * 4) * ld : nullptr;
+  double *const ALO = lo ? g.fnlo + ((size_t)(a * (g.lomax + 1) + l) * 2) * ld : nullptr;
   for (int pass = 0; pass < 2; pass++) {
-    double uvb, duvb, uve, duve, uv, duv;
-    outwin(rel, v, rnot, dx, jri, ei - dele, fl, z, A, B, uvb, duvb);
-    double ovlp = rint13(c1, c2, A, B, A, B, rnot, dx, jri);
-    double trx = 1.0 / sqrt(ovlp);
-    for (int m = 0; m < jri; m++) { AE[m] = trx * A[m]; BE[m] = trx * B[m]; }
-    uvb = trx * uvb;
-    duvb = trx * duvb;
-    outwin(rel, v, rnot, dx, jri, ei + dele, fl, z, A, B, uve, duve);
-    ovlp = rint13(c1, c2, A, B, A, B, rnot, dx, jri);
-    trx = 1.0 / sqrt(ovlp);
-    uve = delei * (trx * uve - uvb);
-    duve = delei * (trx * duve - duvb);
-    for (int m = 0; m < jri; m++) {
-      AE[m] = delei * (trx * A[m] - AE[m]);
-      BE[m] = delei * (trx * B[m] - BE[m]);
+    const int ne = lo ? AT_NE : AT_NE - 1;
+    const int nch = (jri + AT_CH - 1) / AT_CH;
+    // the chain's state, one energy per lane of wave 0
+    double a0 = 0, b0 = 0, dg1 = 0, dg2 = 0, dg3 = 0, df1 = 0, df2 = 0, df3 = 0;
+#pragma unroll 1
+    for (int ch = -1; ch <= nch; ch++) {
+      if (wave > 0) {
+        const int en = wave - 1, k = (ch + 1) * AT_CH + lane, kp = (ch - 1) * AT_CH + lane;
+        if (en < ne && k < jri) {
+          const double eh = en == 0 ? ei - dele : en == 1 ? ei + dele : en == 2 ? ei : elo;
+          outwin_coef(rel, v[k], rnot, dx, eh, fl, z, k, sh.c[(ch + 1) & 1][lane][en]);
+        }
+        if (en < ne && ch > 0 && kp < jri) {
+          work[2 * en * ld + kp] = sh.f[(ch - 1) & 1][0][lane][en];
+          work[(2 * en + 1) * ld + kp] = sh.f[(ch - 1) & 1][1][lane][en] * cl / 2.0;
+          if (en == 0) wt[kp] = rint13_w(rnot, dx, jri, kp);
+        }
+      } else if (ch >= 0 && ch < nch && lane < ne) {
+        const double h83 = 8.0 / 3.0, r1 = 1.0 / 9.0, r2 = -5.0 * r1, r3 = 19.0 * r1, x = -dx;
+        const double(&c)[AT_CH + 2 * AT_PF][AT_NE][AT_NC] = sh.c[ch & 1];
+        double(&f)[2][AT_CH][AT_NE] = sh.f[ch & 1];
+        const int k1 = min(AT_CH, jri - ch * AT_CH);
+        int k = 0;
+        if (ch == 0) {
+#pragma unroll 1
+          for (; k < 3; k++) {
+            a0 = c[k][lane][0];
+            b0 = c[k][lane][1];
+            dg1 = dg2; dg2 = dg3; dg3 = c[k][lane][2];
+            df1 = df2; df2 = df3; df3 = c[k][lane][3];
+            f[0][k][lane] = a0;
+            f[1][k][lane] = b0;
+          }
+        }
+        // AT_PF points a turn, their operands read a turn ahead (past the
+        // piece's end from rows that hold nothing yet, and not used)
+        double o[AT_PF][AT_NC], p[AT_PF][AT_NC];
+        auto read = [&](double(&o)[AT_PF][AT_NC], int k) {
+#pragma unroll
+          for (int m = 0; m < AT_PF; m++)
+#pragma unroll
+            for (int q = 0; q < AT_NC; q++) o[m][q] = c[k + m][lane][q];
+        };
+        auto points = [&](const double(&o)[AT_PF][AT_NC]) {
+#pragma unroll
+          for (int m = 0; m < AT_PF; m++, k++) {
+            if (k == k1) break;
+            const double b11 = a0 * h83 + (r1 * dg1 + r2 * dg2) + r3 * dg3;
+            const double b22 = b0 * h83 + (r1 * df1 + r2 * df2) + r3 * df3;
+            const double u = o[m][2], y = o[m][3];
+            a0 = b11 * (h83 - x) + b22 * u;
+            b0 = b22 * (h83 + x) - b11 * y;
+            a0 = fma(a0, o[m][0], a0 * o[m][1]);
+            b0 = fma(b0, o[m][0], b0 * o[m][1]);
+            dg1 = dg2; dg2 = dg3; dg3 = u * b0 - x * a0;
+            df1 = df2; df2 = df3; df3 = x * b0 - y * a0;
+            f[0][k][lane] = a0;
+            f[1][k][lane] = b0;
+          }
+        };
+        read(o, k);
+#pragma unroll 1
+        while (k < k1) {
+          read(p, k + AT_PF);
+          points(o);
+          if (k == k1) break;
+          read(o, k + AT_PF);
+          points(p);
+        }
+        if (ch == nch - 1) {
+          const double rj = rnot * exp(dx * (double)(jri - 1)), val = a0 / rj;
+          sh.end[0][lane] = val;
+          sh.end[1][lane] = (dg3 / (dx * rj) - val) / rj;
+        }
+      }
+      __syncthreads();
     }
-    outwin(rel, v, rnot, dx, jri, ei, fl, z, A, B, uv, duv);
-    ovlp = rint13(c1, c2, A, B, A, B, rnot, dx, jri);
-    trx = 1.0 / sqrt(ovlp);
-    P = trx * uv;
-    DP = trx * duv;
-    for (int m = 0; m < jri; m++) { A1[m] = trx * A[m]; B1[m] = trx * B[m]; }
-    const double cross = rint13(c1, c2, A1, B1, AE, BE, rnot, dx, jri);
-    const double tr = -cross;
-    for (int m = 0; m < jri; m++) { AE[m] = AE[m] + tr * A1[m]; BE[m] = BE[m] + tr * B1[m]; }
-    PE = uve + tr * P;
-    DPE = duve + tr * DP;
-    PEI = rint13(c1, c2, AE, BE, AE, BE, rnot, dx, jri);
+    // norms (atpar.f:222-262), a wave for each energy
+    if (wave < ne) {
+      const double *A = work + 2 * wave * ld, *B = A + ld;
+      double s = 0.0;
+#pragma unroll 4
+      for (int k = lane; k < jri; k += 64) s += wt[k] * (c1 * A[k] * A[k] + c2 * B[k] * B[k]);
+      s = wave_sum(s);
+      if (lane == 0) sh.norm[wave] = 1.0 / sqrt(rint13_nonzero(s, dx));
+    }
+    __syncthreads();
+    const double tr1 = sh.norm[0], tr2 = sh.norm[1], tr3 = sh.norm[2], trx = lo ? sh.norm[3] : 0.0;
+    const double P = tr3 * sh.end[0][2], DP = tr3 * sh.end[1][2];
+    // the normalised function and its energy derivative, made orthogonal to it
+    double s1[1] = {0.0};
+#pragma unroll 1
+    for (int k = tid; k < jri; k += AT_NT) {
+      const double A = tr3 * work[4 * ld + k], B = tr3 * work[5 * ld + k];
+      const double AE = delei * (tr2 * work[2 * ld + k] - tr1 * work[k]);
+      const double BE = delei * (tr2 * work[3 * ld + k] - tr1 * work[ld + k]);
+      s1[0] += wt[k] * (c1 * A * AE + c2 * B * BE);
+    }
+    block_sums(sh, slot, s1);
+    const double tr = -rint13_nonzero(s1[0], dx);
+    const double PE = delei * (tr2 * sh.end[0][1] - tr1 * sh.end[0][0]) + tr * P;
+    const double DPE = delei * (tr2 * sh.end[1][1] - tr1 * sh.end[1][0]) + tr * DP;
     // a function almost zero at the boundary: the energy is lowered by
     // 0.05 Ry and the l is done again, once (atpar.f:281-290)
     if (pass == 0 && fabs(P) < 1.0e-3) {
       ei = (g.e[(size_t)a * g.lmaxd + l] - 0.05) / 2.0;
       continue;
     }
+    double s3[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int k = tid; k < jri; k += AT_NT) {
+      const double A = tr3 * work[4 * ld + k], B = tr3 * work[5 * ld + k];
+      const double AE = delei * (tr2 * work[2 * ld + k] - tr1 * work[k]) + tr * A;
+      const double BE = delei * (tr2 * work[3 * ld + k] - tr1 * work[ld + k]) + tr * B;
+      s3[0] += wt[k] * (c1 * AE * AE + c2 * BE * BE);
+      if (A1) {
+        A1[k] = A;
+        A1[ld + k] = B;
+        A1[2 * ld + k] = AE;
+        A1[3 * ld + k] = BE;
+      }
+      if (lo) {
+        const double AL = trx * work[6 * ld + k], BL = trx * work[7 * ld + k];
+        ALO[k] = AL;
+        ALO[ld + k] = BL;
+        s3[1] += wt[k] * (c1 * A * AL + c2 * B * BL);
+        s3[2] += wt[k] * (c1 * AE * AL + c2 * BE * BL);
+      }
+    }
+    block_sums(sh, slot, s3);
+    if (tid == 0) {
+      double *o = g.out + (size_t)(a * g.nt + l) * 6;
+      o[0] = P; o[1] = DP; o[2] = PE; o[3] = DPE; o[4] = rint13_nonzero(s3[0], dx); o[5] = 2.0 * ei;
+      if (lo) {
+        double *q = g.outlo + (size_t)(a * (g.lomax + 1) + l) * 4;
+        q[0] = trx * sh.end[0][3];
+        q[1] = trx * sh.end[1][3];
+        q[2] = rint13_nonzero(s3[1], dx);
+        q[3] = rint13_nonzero(s3[2], dx);
+      }
+    }
     break;
-  }
-  double *o = g.out + (size_t)(a * g.nt + l) * 6;
-  o[0] = P; o[1] = DP; o[2] = PE; o[3] = DPE; o[4] = PEI; o[5] = 2.0 * ei;
-  if (l <= g.lomax && g.loor[a * (g.lomax + 1) + l]) {
-    double uv, duv;
-    outwin(rel, v, rnot, dx, jri, g.elo[a * (g.lomax + 1) + l] / 2.0, fl, z, A, B, uv, duv);
-    const double ovlp = rint13(c1, c2, A, B, A, B, rnot, dx, jri);
-    const double trx = 1.0 / sqrt(ovlp);
-    double *ALO = g.fnlo + ((size_t)(a * (g.lomax + 1) + l) * 2) * g.jrid, *BLO = ALO + g.jrid;
-    for (int m = 0; m < jri; m++) { ALO[m] = trx * A[m]; BLO[m] = trx * B[m]; }
-    double *q = g.outlo + (size_t)(a * (g.lomax + 1) + l) * 4;
-    q[0] = trx * uv;
-    q[1] = trx * duv;
-    q[2] = rint13(c1, c2, A1, B1, ALO, BLO, rnot, dx, jri);
-    q[3] = rint13(c1, c2, AE, BE, ALO, BLO, rnot, dx, jri);
   }
 }
 
-// one thread per (atom type, l0, lm, lp) triple that the coupling list reads:
-// VNS1..3 and, for l0 <= LOMAX, the local-orbital integrals (atpar.f:489-552)
+// one wave per (atom type, l0, lm, lp) triple that the coupling list reads:
+// VNS1..3 and, for l0 <= LOMAX, the local-orbital integrals (atpar.f:489-552),
+// all of them in one pass over the mesh.  64 atom types, 781 points: 563 us
+// with one work-item per triple -> 20 us.
 struct VnsTriple {
   int a, l0, lm, lp;
 };
 
-__global__ void k_atpar_vns(int ntrip, const VnsTriple *__restrict__ trip, AtparArgs g, const double *__restrict__ vlm,
-                            int lmmxd, double *__restrict__ res)
+__global__ __launch_bounds__(256) void k_atpar_vns(int ntrip, const VnsTriple *__restrict__ trip, AtparArgs g,
+                                                   const double *__restrict__ vlm, int lmmxd, double *__restrict__ res)
 {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64, lane = threadIdx.x & 63;
   if (t >= ntrip) return;
   const VnsTriple q = trip[t];
   const bool rel = g.rel != 0;
   const double c1 = 1.0, c2 = rel ? 1.0 / (137.0359895 * 137.0359895) : 1.0e-22;
   const int jri = g.jrj[q.a];
-  const double rnot = g.ro[q.a], dx = g.dh[q.a];
-  const double *V = vlm + ((size_t)q.a * lmmxd + q.lm) * g.jrid;
-  const double *f0 = g.fn + ((size_t)(q.a * g.nslmax + q.l0) * 4) * g.jrid;
-  const double *fp = g.fn + ((size_t)(q.a * g.nslmax + q.lp) * 4) * g.jrid;
-  const double *A1 = f0, *B1 = f0 + g.jrid, *AE1 = f0 + 2 * (size_t)g.jrid, *BE1 = f0 + 3 * (size_t)g.jrid;
-  const double *A1p = fp, *B1p = fp + g.jrid, *AE1p = fp + 2 * (size_t)g.jrid, *BE1p = fp + 3 * (size_t)g.jrid;
-  double *o = res + (size_t)t * 6;
-  // VNS1 = <u_l0 V u_lp>, VNS2 = <ue V ue>, VNS3 = <u_l0 V ue_lp>
-  o[0] = rint13_of(rnot, dx, jri, [&](int k) { return c1 * (A1[k] * V[k]) * A1p[k] + c2 * (B1[k] * V[k]) * B1p[k]; });
-  o[1] = rint13_of(rnot, dx, jri,
-                   [&](int k) { return c1 * (AE1[k] * V[k]) * AE1p[k] + c2 * (BE1[k] * V[k]) * BE1p[k]; });
-  o[2] = rint13_of(rnot, dx, jri, [&](int k) { return c1 * (A1[k] * V[k]) * AE1p[k] + c2 * (B1[k] * V[k]) * BE1p[k]; });
-  o[3] = o[4] = o[5] = 0.0;
-  if (q.l0 <= g.lomax && g.loor[q.a * (g.lomax + 1) + q.l0]) {
-    const double *L0 = g.fnlo + ((size_t)(q.a * (g.lomax + 1) + q.l0) * 2) * g.jrid, *L0b = L0 + g.jrid;
-    o[3] = rint13_of(rnot, dx, jri, [&](int k) { return c1 * (L0[k] * V[k]) * A1p[k] + c2 * (L0b[k] * V[k]) * B1p[k]; });
-    o[4] =
-        rint13_of(rnot, dx, jri, [&](int k) { return c1 * (L0[k] * V[k]) * AE1p[k] + c2 * (L0b[k] * V[k]) * BE1p[k]; });
-    if (q.lp <= g.lomax && g.loor[q.a * (g.lomax + 1) + q.lp]) {
-      const double *Lp = g.fnlo + ((size_t)(q.a * (g.lomax + 1) + q.lp) * 2) * g.jrid, *Lpb = Lp + g.jrid;
-      o[5] =
-          rint13_of(rnot, dx, jri, [&](int k) { return c1 * (L0[k] * V[k]) * Lp[k] + c2 * (L0b[k] * V[k]) * Lpb[k]; });
-    }
+  const double dx = g.dh[q.a];
+  const size_t ld = g.jrid;
+  const double *wt = g.work + ((size_t)q.a * g.nt * AT_ROWS + 2 * AT_NE) * ld;  // l = 0's row
+  const double *V = vlm + ((size_t)q.a * lmmxd + q.lm) * ld;
+  const double *f0 = g.fn + ((size_t)(q.a * g.nslmax + q.l0) * 4) * ld;
+  const double *fp = g.fn + ((size_t)(q.a * g.nslmax + q.lp) * 4) * ld;
+  const bool lo0 = q.l0 <= g.lomax && g.loor[q.a * (g.lomax + 1) + q.l0];
+  const bool lop = lo0 && q.lp <= g.lomax && g.loor[q.a * (g.lomax + 1) + q.lp];
+  // without a local orbital the integrals that are not wanted read u instead
+  const double *L0 = lo0 ? g.fnlo + ((size_t)(q.a * (g.lomax + 1) + q.l0) * 2) * ld : f0;
+  const double *Lp = lop ? g.fnlo + ((size_t)(q.a * (g.lomax + 1) + q.lp) * 2) * ld : fp;
+  // VNS1 = <u_l0 V u_lp>, VNS2 = <ue V ue>, VNS3 = <u_l0 V ue_lp>, and with the
+  // local orbitals <lo V u>, <lo V ue>, <lo V lo>
+  auto f = [&](int k, double(&y)[6]) {
+    const double A = f0[k] * V[k], B = f0[ld + k] * V[k], AE = f0[2 * ld + k] * V[k], BE = f0[3 * ld + k] * V[k];
+    const double Ap = fp[k], Bp = fp[ld + k], AEp = fp[2 * ld + k], BEp = fp[3 * ld + k];
+    const double L = L0[k] * V[k], Lb = L0[ld + k] * V[k];
+    y[0] = c1 * A * Ap + c2 * B * Bp;
+    y[1] = c1 * AE * AEp + c2 * BE * BEp;
+    y[2] = c1 * A * AEp + c2 * B * BEp;
+    y[3] = c1 * L * Ap + c2 * Lb * Bp;
+    y[4] = c1 * L * AEp + c2 * Lb * BEp;
+    y[5] = c1 * L * Lp[k] + c2 * Lb * Lp[ld + k];
+  };
+  double z[6] = {};
+  for (int k = lane; k < jri; k += 64) {
+    double y[6];
+    f(k, y);
+    for (int m = 0; m < 6; m++) z[m] += wt[k] * y[m];
+  }
+  for (int m = 0; m < 6; m++) {
+    const double s = rint13_nonzero(wave_sum(z[m]), dx);
+    if (lane == 0) res[(size_t)t * 6 + m] = m < 3 || (m < 5 ? lo0 : lop) ? s : 0.0;
   }
 }
 
@@ -401,7 +509,7 @@ int atpar(Ctx &c, const w2k_radial_desc *rd, double *const out[16])
       loor[a * W2K_LOMAXP + l] = R.loor[l + W2K_LOMAXP * a] ? 1 : 0;
       if (il > 0) elo[a * W2K_LOMAXP + l] = R.elo[l + W2K_LOMAXP * ((il - 1) + W2K_NLOAT * (size_t)a)];
     }
-  DBuf<double> d_vr, d_e, d_elo, d_work, d_out, d_outlo, d_scr;
+  DBuf<double> d_vr, d_e, d_elo, d_work, d_out, d_outlo;
   DBuf<int> d_loor;
   if ((rc = put(R.d_at_jrj, rd->jrj, nat, s)) || (rc = put(R.d_at_ro, rd->ro, nat, s)) ||
       (rc = put(R.d_at_dh, rd->dh, nat, s)) || (rc = put(R.d_at_zz, rd->zz, nat, s)) ||
@@ -410,7 +518,7 @@ int atpar(Ctx &c, const w2k_radial_desc *rd, double *const out[16])
     return rc;
   if ((rc = R.d_at_fn.alloc((size_t)nat * W2K_NSLMAX * 4 * jrid)) ||
       (rc = R.d_at_fnlo.alloc((size_t)nat * W2K_LOMAXP * 2 * jrid)) ||
-      (rc = d_work.alloc((size_t)nat * nt * 2 * jrid)) || (rc = d_scr.alloc((size_t)nat * nt * 4 * jrid)) ||
+      (rc = d_work.alloc((size_t)nat * nt * AT_ROWS * jrid)) ||
       (rc = d_out.alloc((size_t)nat * nt * 6)) || (rc = d_outlo.alloc((size_t)nat * W2K_LOMAXP * 4)))
     return rc;
   W2K_HIP(hipMemsetAsync(R.d_at_fnlo.p, 0, sizeof(double) * R.d_at_fnlo.n, s));
@@ -424,7 +532,7 @@ int atpar(Ctx &c, const w2k_radial_desc *rd, double *const out[16])
   g.out = d_out.p;
   g.outlo = d_outlo.p;
   const int nth = nat * nt;
-  hipLaunchKernelGGL(k_atpar_l, dim3((nth + 63) / 64), dim3(64), 0, s, g, d_scr.p);
+  hipLaunchKernelGGL(k_atpar_l, dim3(nt, nat), dim3(AT_NT), 0, s, g);
   W2K_STAGE(s, "k_atpar_l");
   std::vector<double> o((size_t)nth * 6), olo((size_t)nat * W2K_LOMAXP * 4);
   W2K_HIP(hipMemcpyAsync(o.data(), d_out.p, sizeof(double) * o.size(), hipMemcpyDeviceToHost, s));
@@ -440,7 +548,7 @@ int atpar(Ctx &c, const w2k_radial_desc *rd, double *const out[16])
         (rc = put(d_vlm, rd->vlm, (size_t)jrid * rd->lmmxd * nat, s)) || (rc = d_res.alloc(trip.size() * 6)))
       return rc;
     const int ntr = (int)trip.size();
-    hipLaunchKernelGGL(k_atpar_vns, dim3((ntr + 63) / 64), dim3(64), 0, s, ntr,
+    hipLaunchKernelGGL(k_atpar_vns, dim3((ntr + 3) / 4), dim3(256), 0, s, ntr,
                        reinterpret_cast<const VnsTriple *>(d_trip.p), g, d_vlm.p, rd->lmmxd, d_res.p);
     W2K_STAGE(s, "k_atpar_vns");
     vres.resize(trip.size() * 6);
