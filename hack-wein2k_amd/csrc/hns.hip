@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "mfma.h"
 #include "special.h"
 #include "w2k_internal.h"
 
@@ -41,11 +42,13 @@ struct HnsArgs {
   int nlo;
 };
 
-// ALM/BLM/CLM(i, L0M0) of row i and equivalent atom e (hns.F:160-259):
-// 4 pi R^2 sqrt(1/Omega) i^L0 e^{2 pi i G_i.tau} conj Y_L0M0(R k_i) times
-// {AL, BL, 0} (plane-wave rows) or {ALO, BLO, CLO} (the LO rows of that
-// atom, l and jlo)
-__device__ __forceinline__ void hns_alm(const HnsArgs &g, int i, int e, int a, cd *alm, cd *blm, cd *clm)
+// of row i and equivalent atom e (hns.F:160-259): put(lm, t) with
+// t = 4 pi R^2 sqrt(1/Omega) i^L0 e^{2 pi i G_i.tau} conj Y_L0M0(R k_i), and
+// before the lm of an l put_l(l, fa, fb, fc): ALM/BLM/CLM(i, L0M0) are t times
+// {AL, BL, 0} (plane-wave rows) or {ALO, BLO, CLO} (the LO rows of that atom,
+// l and jlo; zero for others)
+template <class FL, class F>
+__device__ __forceinline__ void hns_alm(const HnsArgs &g, int i, int e, int a, FL put_l, F put)
 {
   const int n = g.n;
   const double r = g.rmt[a];
@@ -61,11 +64,9 @@ __device__ __forceinline__ void hns_alm(const HnsArgs &g, int i, int e, int a, c
   double cilr = 1.0, cili = 0.0;
   for (int l0 = 0; l0 < g.nnsl; l0++) {
     double fa = 0.0, fb = 0.0, fc = 0.0;
-    bool on = false;
     if (i < g.nv) {
       fa = g.al[i + (size_t)n * (l0 + (size_t)g.lt * a)];
       fb = g.bl[i + (size_t)n * (l0 + (size_t)g.lt * a)];
-      on = true;
     } else if (l0 <= W2K_LOMAX) {
       for (int jlo = 0; jlo < W2K_NLOAT; jlo++) {
         const int *rr = g.lorow + 2 * (l0 + W2K_LOMAXP * (jlo + W2K_NLOAT * a));
@@ -73,19 +74,15 @@ __device__ __forceinline__ void hns_alm(const HnsArgs &g, int i, int e, int a, c
         if (rr[0] >= 0 && qq >= rr[0] && qq <= rr[1]) {
           const double *ab = g.loabc + 3 * (l0 + W2K_LOMAXP * (jlo + W2K_NLOAT * a));
           fa = ab[0]; fb = ab[1]; fc = ab[2];
-          on = true;
         }
       }
     }
+    put_l(l0, fa, fb, fc);
     for (int m0 = -l0; m0 <= l0; m0++, lm++) {
-      if (!on) { alm[lm] = {0, 0}; blm[lm] = {0, 0}; clm[lm] = {0, 0}; continue; }
       // (CIL*PHS) * conj(YL)
       const cd cp = cmul({cilr, cili}, {phr, phi});
       const cd t = cmul(cp, conj(yl[lm]));
-      const double ar = rhoatm * t.re, ai = rhoatm * t.im;
-      alm[lm] = {fa * ar, fa * ai};
-      blm[lm] = {fb * ar, fb * ai};
-      clm[lm] = {fc * ar, fc * ai};
+      put(lm, cd{rhoatm * t.re, rhoatm * t.im});
     }
     const double t = cilr;  // CIL = CIL * i
     cilr = -cili;
@@ -93,65 +90,125 @@ __device__ __forceinline__ void hns_alm(const HnsArgs &g, int i, int e, int a, c
   }
 }
 
-// one thread per (row i, equivalent atom e)
+// The operands of the update, for one equivalent atom and 64 rows a block.
+// With z = [Re, Im] of ALM and BLM (and CLM) of a row, its A2, -A2I.. are the
+// real products W z of a 4 LINDEX x 4 NNSL^2 matrix that the coupling
+// coefficients give:
+//   Re sum T conj(X) = sum (T.re, T.im).(X.re, X.im),
+//  -Im sum T conj(X) = sum (-T.im, T.re).(X.re, X.im),
+// on the matrix cores: a 16 x 16 tile holds four k of A2, -A2I, B2, -B2I by 16
+// rows, one step of its inner dimension is one p with ALM and BLM's parts.
+// CLM is zero in plane-wave rows and C2 used in LO rows only: the blocks that
+// hold such rows have one step more per p, and C2's tiles.  A wave takes every
+// fourth tile for all 64 rows.  Bound by the operands' stores at large sizes,
+// by the chain (Y_lm, then 25 dependent steps) at small ones; one work-item
+// per row and atom spent LINDEX NNSL^2 36 multiply-adds on scalar loads: N =
+// 3861, 100 atoms 3.25 -> 0.68 ms (0.9 GB stored), one atom 0.24 -> 0.03 ms.
+constexpr int HP_ROWS = 64, HP_LD = HP_ROWS + 16;  // row length: the four parts' rows two by two on other banks
+
 template <bool CPX>
-__global__ __launch_bounds__(64) void k_hns_prep(HnsArgs g)
+__global__ __launch_bounds__(256) void k_hns_prep(HnsArgs g)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int e = blockIdx.y;
-  if (i >= g.n) return;
-  const int a = g.atom_of[e];
-  const int lidx = g.lindex[a];
+  __shared__ double za[W2K_NSL2][2][HP_LD];      // t of a row and lm
+  __shared__ double zf[W2K_NSLMAX][3][HP_LD];    // AL, BL, CL of a row and l
+  const int e = blockIdx.y, i0 = blockIdx.x * HP_ROWS;
+  const int a = g.atom_of[e], lidx = g.lindex[a];
   if (lidx == 0) return;
-  const int n = g.n;
-  cd alm[W2K_NSL2], blm[W2K_NSL2], clm[W2K_NSL2];
-  hns_alm(g, i, e, a, alm, blm, clm);
-  const bool lorow = (i >= g.nv);
-  const int q = i - g.nv;
-  const int kb = g.koff[e];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = g.n, np = g.nnsl * g.nnsl;
+  const bool lo = i0 + HP_ROWS > g.nv && n > g.nv;  // the block has LO rows
+  if (wave == 0) {
+    if (i0 + lane < n) {
+      hns_alm(g, i0 + lane, e, a,
+              [&](int l, double fa, double fb, double fc) {
+                zf[l][0][lane] = fa;
+                zf[l][1][lane] = fb;
+                zf[l][2][lane] = fc;
+              },
+              [&](int lm, cd t) {
+                za[lm][0][lane] = t.re;
+                za[lm][1][lane] = t.im;
+              });
+    } else {
+      for (int l = 0; l < g.nnsl; l++) zf[l][0][lane] = zf[l][1][lane] = zf[l][2][lane] = 0.0;
+      for (int p = 0; p < np; p++) za[p][0][lane] = za[p][1][lane] = 0.0;
+    }
+  }
+  __syncthreads();
+  const size_t ldL = (size_t)n, ldC = (size_t)g.nlo, KT = g.ktot, kb = g.koff[e];
+  const int *lm0 = g.lm0_of + a * W2K_NSL2;
+  {
+    // A1, B1 (and C1): wave = part of [Re A, Im A, Re B, Im B]
+    const int i = i0 + lane, q = i - g.nv;
+    for (int k = 0; k < lidx; k++) {
+      const int p = lm0[k];
+      int l = 0;
+      while ((l + 1) * (l + 1) <= p) l++;
+      const double f = zf[l][wave >> 1][lane], re = za[p][0][lane], im = za[p][1][lane];
+      const size_t c = kb + k;
+      if (i < n) {
+        g.R[i + ldL * (c + wave * KT)] = f * (wave & 1 ? im : re);
+        if (CPX) g.R2[i + ldL * (c + wave * KT)] = wave & 1 ? -(f * re) : f * im;
+        if (lo && q >= 0 && wave < 2) {
+          const double fc = zf[l][2][lane];
+          g.RC[q + ldC * (c + wave * KT)] = fc * (wave ? im : re);
+          if (CPX) g.RC2[q + ldC * (c + wave * KT)] = wave ? -(fc * re) : fc * im;
+        }
+      }
+    }
+  }
   const double *T = g.tcoef + (size_t)a * W2K_NSL2 * W2K_NSL2 * 18;
-  const size_t ldL = (size_t)n, ldC = (size_t)g.nlo;
-  const int KT = g.ktot;
-  for (int k = 0; k < lidx; k++) {
-    const int lk = g.lm0_of[a * W2K_NSL2 + k];
-    double a2r = 0, a2i = 0, b2r = 0, b2i = 0, c2r = 0, c2i = 0;
-    const int np = g.nnsl * g.nnsl;
-    for (int p = 0; p < np; p++) {
-      const double *t = T + ((size_t)k * W2K_NSL2 + p) * 18;
-      const cd A = conj(alm[p]), B = conj(blm[p]), Cc = conj(clm[p]);
-      // A2 += TUU A + TDU B + TUU21 C ; B2 += TUD A + TDD B + TUD21 C ; C2 += TUU12 A + TDU12 B + TUU22 C
-      a2r += t[0] * A.re - t[1] * A.im + t[2] * B.re - t[3] * B.im + t[4] * Cc.re - t[5] * Cc.im;
-      a2i += t[0] * A.im + t[1] * A.re + t[2] * B.im + t[3] * B.re + t[4] * Cc.im + t[5] * Cc.re;
-      b2r += t[6] * A.re - t[7] * A.im + t[8] * B.re - t[9] * B.im + t[10] * Cc.re - t[11] * Cc.im;
-      b2i += t[6] * A.im + t[7] * A.re + t[8] * B.im + t[9] * B.re + t[10] * Cc.im + t[11] * Cc.re;
-      c2r += t[12] * A.re - t[13] * A.im + t[14] * B.re - t[15] * B.im + t[16] * Cc.re - t[17] * Cc.im;
-      c2i += t[12] * A.im + t[13] * A.re + t[14] * B.im + t[15] * B.re + t[16] * Cc.im + t[17] * Cc.re;
+  const int l16 = lane & 15, part = lane >> 4;       // part of z: Re A, Im A, Re B, Im B
+  const int ntab = (4 * lidx + 15) / 16, ntile = ntab + (lo ? (2 * lidx + 15) / 16 : 0);
+  for (int tile = wave; tile < ntile; tile += 4) {
+    // this lane's row of W: k, m (A2, B2, C2) and part of the output
+    const bool tc = tile >= ntab;
+    const int o = (tc ? tile - ntab : tile) * 16 + l16;
+    const int k = tc ? o >> 1 : o >> 2, m = tc ? 2 : (o >> 1) & 1, oi = o & 1;
+    const bool on = k < lidx;
+    const double sg = !on ? 0.0 : oi && !(part & 1) ? -1.0 : 1.0;
+    const double *w = T + (size_t)(on ? k : 0) * W2K_NSL2 * 18 + 6 * m + 2 * (part >> 1) + (oi ^ (part & 1));
+    const double *wc = T + (size_t)(on ? k : 0) * W2K_NSL2 * 18 + 6 * m + 4 + (oi ^ (part & 1));
+    const double sgc = part < 2 ? sg : 0.0;
+    d4 acc[4] = {};
+#pragma unroll
+    for (int l = 0; l < W2K_NSLMAX; l++) {
+      if (l >= g.nnsl) break;
+      double wl[2 * W2K_NSLMAX - 1], f[4], fc[4];
+#pragma unroll
+      for (int q = 0; q < 2 * l + 1; q++) wl[q] = sg * w[(l * l + q) * 18];
+#pragma unroll
+      for (int b = 0; b < 4; b++) f[b] = zf[l][part >> 1][16 * b + l16];
+#pragma unroll
+      for (int q = 0; q < 2 * l + 1; q++)
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+          acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(wl[q], f[b] * za[l * l + q][part & 1][16 * b + l16], acc[b], 0, 0, 0);
+      if (lo) {
+#pragma unroll
+        for (int q = 0; q < 2 * l + 1; q++) wl[q] = sgc * wc[(l * l + q) * 18];
+#pragma unroll
+        for (int b = 0; b < 4; b++) fc[b] = zf[l][2][16 * b + l16];
+#pragma unroll
+        for (int q = 0; q < 2 * l + 1; q++)
+#pragma unroll
+          for (int b = 0; b < 4; b++)
+            acc[b] =
+                __builtin_amdgcn_mfma_f64_16x16x4f64(wl[q], fc[b] * za[l * l + q][part & 1][16 * b + l16], acc[b], 0, 0, 0);
+      }
     }
-    const cd a1 = alm[lk], b1 = blm[lk], c1 = clm[lk];
-    // columns: block 0 A, block 1 A (imag), block 2 B, block 3 B (imag)
-    const size_t c0 = (size_t)(kb + k);
-    g.L[i + ldL * (c0 + 0 * (size_t)KT)] = a2r;
-    g.L[i + ldL * (c0 + 1 * (size_t)KT)] = -a2i;
-    g.L[i + ldL * (c0 + 2 * (size_t)KT)] = b2r;
-    g.L[i + ldL * (c0 + 3 * (size_t)KT)] = -b2i;
-    g.R[i + ldL * (c0 + 0 * (size_t)KT)] = a1.re;
-    g.R[i + ldL * (c0 + 1 * (size_t)KT)] = a1.im;
-    g.R[i + ldL * (c0 + 2 * (size_t)KT)] = b1.re;
-    g.R[i + ldL * (c0 + 3 * (size_t)KT)] = b1.im;
-    if (CPX) {
-      g.R2[i + ldL * (c0 + 0 * (size_t)KT)] = a1.im;
-      g.R2[i + ldL * (c0 + 1 * (size_t)KT)] = -a1.re;
-      g.R2[i + ldL * (c0 + 2 * (size_t)KT)] = b1.im;
-      g.R2[i + ldL * (c0 + 3 * (size_t)KT)] = -b1.re;
-    }
-    if (lorow) {
-      g.LC[q + ldC * (c0 + 0 * (size_t)KT)] = c2r;
-      g.LC[q + ldC * (c0 + 1 * (size_t)KT)] = -c2i;
-      g.RC[q + ldC * (c0 + 0 * (size_t)KT)] = c1.re;
-      g.RC[q + ldC * (c0 + 1 * (size_t)KT)] = c1.im;
-      if (CPX) {
-        g.RC2[q + ldC * (c0 + 0 * (size_t)KT)] = c1.im;
-        g.RC2[q + ldC * (c0 + 1 * (size_t)KT)] = -c1.re;
+    mfma_settle();
+    // lane: row l16 of each 16, outputs part + 4 j of the tile
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      const int i = i0 + 16 * b + l16;
+      if (i >= n || (tc && i < g.nv)) continue;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int oo = (tc ? tile - ntab : tile) * 16 + part + 4 * j, kk = tc ? oo >> 1 : oo >> 2;
+        if (kk >= lidx) continue;
+        if (tc) g.LC[(i - g.nv) + ldC * (kb + kk + (oo & 1) * KT)] = acc[b][j];
+        else g.L[i + ldL * (kb + kk + (oo & 3) * KT)] = acc[b][j];
       }
     }
   }
@@ -171,17 +228,17 @@ __global__ void k_add_cplx_lower(int n, int off, int ld, const double *__restric
 }
 
 // kernel arguments of the HNS stage over the context's buffers
-static HnsArgs hns_args(Ctx &c, int ktot, const int *d_koff)
+static HnsArgs hns_args(Ctx &c)
 {
   RunDev &R = c.run();
   const int n = c.n, nlo = c.nlo, ndf = R.ndf;
-  const int cpx = R.is_complex;
+  const int cpx = R.is_complex, ktot = R.ktot;
   const size_t kcols = (size_t)4 * ktot;
   const size_t lcsz = (size_t)(nlo > 0 ? nlo : 1) * 2 * ktot;
   HnsArgs g;
   g.n = n; g.nv = c.nv; g.nnsl = R.nnsl; g.lt = R.ltop; g.ndf = ndf;
   g.kv = c.d_kvec.p; g.cs = c.d_cs.p; g.al = c.d_al.p; g.bl = c.d_bl.p;
-  g.atom_of = R.d_atom_of.p; g.lindex = R.d_lindex.p; g.koff = d_koff; g.lm0_of = R.d_lm0_of.p;
+  g.atom_of = R.d_atom_of.p; g.lindex = R.d_lindex.p; g.koff = R.d_koff.p; g.lm0_of = R.d_lm0_of.p;
   g.tcoef = R.d_tcoef.p; g.lorow = R.d_lorow.p; g.loabc = R.d_loabc.p;
   g.rotij = R.d_rotij.p; g.rotloc = R.d_rotloc.p; g.rmt = R.d_rmt.p; g.vi = R.vi;
   g.ktot = ktot;
@@ -202,12 +259,7 @@ int hns(Ctx &c)
   const int n = c.n, nlo = c.nlo, ndf = R.ndf;
   const int cpx = R.is_complex;
   hipStream_t s = c.stream;
-  int ktot = 0;
-  std::vector<int> koff(ndf);
-  for (int e = 0; e < ndf; e++) {
-    koff[e] = ktot;
-    ktot += R.lindex[R.atom_of[e]];
-  }
+  const int ktot = R.ktot;
   if (ktot == 0) return 0;
   int rc;
   const size_t kcols = (size_t)4 * ktot;
@@ -215,19 +267,11 @@ int hns(Ctx &c)
   if ((rc = c.d_hnsR.alloc((size_t)n * kcols * (cpx ? 2 : 1)))) return rc;
   const size_t lcsz = (size_t)(nlo > 0 ? nlo : 1) * 2 * ktot;
   if ((rc = c.h_small.alloc(lcsz * (cpx ? 3 : 2)))) return rc;
-  int *d_koff;
-  if ((rc = c.h_int.alloc(ndf))) return rc;
-  d_koff = c.h_int.p;
-  W2K_HIP(hipMemcpyAsync(d_koff, koff.data(), sizeof(int) * ndf, hipMemcpyHostToDevice, s));
-  W2K_HIP(hipStreamSynchronize(s));  // koff is a host temporary
-  HnsArgs g = hns_args(c, ktot, d_koff);
-  // atoms without non-spherical terms leave their columns untouched: clear
-  W2K_HIP(hipMemsetAsync(c.d_hnsL.p, 0, sizeof(double) * (size_t)n * kcols, s));
-  W2K_HIP(hipMemsetAsync(c.d_hnsR.p, 0, sizeof(double) * (size_t)n * kcols * (cpx ? 2 : 1), s));
-  W2K_HIP(hipMemsetAsync(c.h_small.p, 0, sizeof(double) * lcsz * (cpx ? 3 : 2), s));
-  dim3 grid((n + 63) / 64, ndf);
-  if (cpx) hipLaunchKernelGGL(k_hns_prep<true>, grid, dim3(64), 0, s, g);
-  else hipLaunchKernelGGL(k_hns_prep<false>, grid, dim3(64), 0, s, g);
+  // every entry of the operands is written
+  HnsArgs g = hns_args(c);
+  dim3 grid((n + HP_ROWS - 1) / HP_ROWS, ndf);
+  if (cpx) hipLaunchKernelGGL(k_hns_prep<true>, grid, dim3(256), 0, s, g);
+  else hipLaunchKernelGGL(k_hns_prep<false>, grid, dim3(256), 0, s, g);
   W2K_STAGE(s, "k_hns_prep");
   const int K4 = (int)kcols, K2 = 2 * ktot;
   const int sl = c.hns_slices;
@@ -288,15 +332,21 @@ __global__ __launch_bounds__(64) void k_alm_store(HnsArgs g, int np, double *__r
   const int e = blockIdx.y;
   if (i >= g.n) return;
   const int a = g.atom_of[e];
-  cd t[3][W2K_NSL2];
-  hns_alm(g, i, e, a, t[0], t[1], t[2]);
-  const size_t n = (size_t)g.n;
-  for (int x = 0; x < 3; x++)
-    for (int p = 0; p < np; p++) {
-      const size_t o = (((size_t)e * 3 + x) * np + p) * n + i;
-      xlm[2 * o] = t[x][p].re;
-      xlm[2 * o + 1] = t[x][p].im;
-    }
+  const size_t n = (size_t)g.n, step = 2 * (size_t)np * n;
+  double *o = xlm + 2 * ((size_t)e * 3 * np * n + i);
+  double f[3];
+  hns_alm(g, i, e, a,
+          [&](int, double fa, double fb, double fc) {
+            f[0] = fa;
+            f[1] = fb;
+            f[2] = fc;
+          },
+          [&](int lm, cd t) {
+            for (int x = 0; x < 3; x++) {
+              o[x * step + 2 * n * lm] = f[x] * t.re;
+              o[x * step + 2 * n * lm + 1] = f[x] * t.im;
+            }
+          });
 }
 
 // w Gamma on the lower triangle: off-diagonal doubled, the diagonal's
@@ -414,12 +464,7 @@ int adjoint_vns(Ctx &c, const double *f_host, double *const gout[6])
   const size_t nvlo = (size_t)LOP2 * R.lmmxd * W2K_NSLMAX * nat;
   for (int q = 0; q < 6; q++)
     if (gout[q]) std::fill(gout[q], gout[q] + (q < 3 ? nvns : nvlo), 0.0);
-  int ktot = 0;
-  std::vector<int> koff(ndf);
-  for (int e = 0; e < ndf; e++) {
-    koff[e] = ktot;
-    ktot += R.lindex[R.atom_of[e]];
-  }
+  const int ktot = R.ktot;
   if (ktot == 0 || ne == 0) return 0;
   if (!c.have_hns_ops) return W2K_ESTATE;
   int rc;
@@ -442,12 +487,7 @@ int adjoint_vns(Ctx &c, const double *f_host, double *const gout[6])
   if ((rc = c.w_c.alloc((cpx ? 2 : 1) * (psz + pcsz)))) return rc;
   double *P1 = c.w_c.p, *P2 = cpx ? P1 + psz : nullptr;
   double *PC1 = P1 + (cpx ? 2 : 1) * psz, *PC2 = cpx ? PC1 + pcsz : nullptr;
-  int *d_koff;
-  if ((rc = c.w_int.alloc(ndf))) return rc;
-  d_koff = c.w_int.p;
-  W2K_HIP(hipMemcpyAsync(d_koff, koff.data(), sizeof(int) * ndf, hipMemcpyHostToDevice, s));
-  W2K_HIP(hipStreamSynchronize(s));  // koff is a host temporary
-  HnsArgs g = hns_args(c, ktot, d_koff);
+  HnsArgs g = hns_args(c);
   if ((rc = dgemm(s, 'N', 'N', n, (int)kcols, n, 1.0, Gr, n, g.R, n, 0.0, P1, n, 0, 2, 0))) return rc;
   if (cpx && (rc = dgemm(s, 'N', 'N', n, (int)kcols, n, 1.0, Gi, n, g.R, n, 0.0, P2, n, 0, 2, 0))) return rc;
   if (nlo > 0) {
@@ -466,7 +506,7 @@ int adjoint_vns(Ctx &c, const double *f_host, double *const gout[6])
   W2K_HIP(hipMemsetAsync(c.w_fac.p, 0, sizeof(double) * xsz, s));
   AdjXArgs xa;
   xa.n = n; xa.nv = nv; xa.nlo = nlo; xa.np = np; xa.ktot = ktot;
-  xa.atom_of = R.d_atom_of.p; xa.lindex = R.d_lindex.p; xa.koff = d_koff;
+  xa.atom_of = R.d_atom_of.p; xa.lindex = R.d_lindex.p; xa.koff = R.d_koff.p;
   xa.xlm = c.w_x.p; xa.p1 = P1; xa.p2 = P2; xa.pc1 = PC1; xa.pc2 = PC2; xa.cpx = cpx; xa.x = c.w_fac.p;
   hipLaunchKernelGGL(k_adj_x, dim3(ndf, 9), dim3(256), 0, s, xa);
   W2K_STAGE(s, "k_adj_x");

@@ -24,12 +24,11 @@
 
 #include <hip/hip_ext.h>
 
+#include "mfma.h"
 #include "seclr4_shared.h"
 #include "twostage.h"
 
 namespace w2k {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------ device-wide words
 // Data exchanged between work-groups of a running kernel goes through relaxed
@@ -64,18 +63,6 @@ __device__ __forceinline__ void wave_sync()
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Before FP64 MFMA results are read by another instruction: 64 clocks more
-// than the compiler leaves after the last MFMA.  It leaves 19 wait
-// states (16 passes + 3) after its issue; where that MFMA accumulates onto the
-// one just before it, whose end it has to wait for, item 3 of the result was
-// read three passes early.
-__device__ __forceinline__ void mfma_settle()
-{
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_sleep(1);
-  __builtin_amdgcn_sched_barrier(0);
 }
 
 // sum over the 32 lanes of a half wave, in every lane

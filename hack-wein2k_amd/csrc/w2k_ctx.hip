@@ -362,6 +362,14 @@ int run_upload(Ctx &c, const w2k_run_desc *r)
     if ((rc = upload(R.d_lm0_of, R.lm0_of.data(), R.lm0_of.size(), s))) return rc;
     if ((rc = upload(R.d_lindex, R.lindex.data(), R.lindex.size(), s))) return rc;
   }
+  // first column of each equivalent atom in the operands of the HNS update
+  std::vector<int> koff(ndf);
+  R.ktot = 0;
+  for (int e = 0; e < ndf; e++) {
+    koff[e] = R.ktot;
+    R.ktot += R.lindex[R.atom_of[e]];
+  }
+  if ((rc = upload(R.d_koff, koff.data(), koff.size(), s))) return rc;
   W2K_HIP(hipStreamSynchronize(s));
   return 0;
 }
@@ -418,7 +426,6 @@ void drop_kpoint_state(Ctx &c)
                           &c.w_sb, &c.w_frag};
   for (DBuf<double> *b : bufs) b->release();
   c.d_kzz.release();
-  c.h_int.release();
   c.w_int.release();
   c.w_piv.release();
   c.w_sbi.release();

@@ -121,6 +121,8 @@ struct RunDev {
   DBuf<int> d_lm0_of;
   DBuf<double> d_tcoef;             // [a][25][25][9][2]
   DBuf<int> d_lindex;
+  int ktot = 0;         // sum over the equivalent atoms of lindex
+  DBuf<int> d_koff;     // that sum before each of them
   // LO columns in HAMILT order (hamilt.F:495-552): a, l, jlo, jeqo, mo1, nnlo, first_eq, mult
   int nlo_cols = 0;
   std::vector<int> locol;
@@ -163,7 +165,6 @@ struct Ctx {
   // HNS work
   DBuf<double> d_hnsL, d_hnsR;  // rank-update operands
   DBuf<double> h_small;         // LO-block operands
-  DBuf<int> h_int;              // per-atom column offsets
   DBuf<double> h_re, h_im;      // complex build: planar products
   int have_hns_ops = 0;         // L/R operands of the last HNS are valid (same basis)
   int hns_slices = 0;           // 0: FP64 rank-K update; 3..7: INT8 digit slices (split precision)
