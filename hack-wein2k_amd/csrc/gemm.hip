@@ -42,32 +42,124 @@ struct GemmArgs {
   int atri, btri;    // op(A): 1 upper / 2 lower; op(B): 1 upper / 2 lower
 };
 
-// element (i, kk) of op(A), zero outside the matrix or outside its triangle
-__device__ __forceinline__ double load_opA(const GemmArgs &g, int i, int kk)
+// One slab of an operand for a tile: ROWS rows (of op(A); columns of op(B)) from
+// r0 on by BK steps of k, by 256 work-items; T: k is the contiguous index.
+// What varies over the work-items is a 32-bit offset that stays the same from
+// slab to slab, so that a load costs no vector arithmetic: the kernels spent
+// most of the time that the MFMAs left on 64-bit addresses, clamps and masks.
+// Rows past the matrix are read as its last row (they enter only outputs that
+// are not written); only a slab that ends past kend or crosses the operand's
+// triangle (mode 1: zero for k < row, 2: zero for k > row) goes element by
+// element.
+template <int T, int ROWS>
+struct Slab {
+  static constexpr int C = ROWS / 16, STEP = 256 / ROWS;
+  unsigned off[C];
+  __device__ __forceinline__ static int row(int r) { return T ? (threadIdx.x >> 4) + 16 * r : threadIdx.x & (ROWS - 1); }
+  __device__ __forceinline__ static int step(int r) { return T ? threadIdx.x & 15 : threadIdx.x / ROWS + STEP * r; }
+  __device__ __forceinline__ void init(int ld, int r0, int nrow)
+  {
+#pragma unroll
+    for (int r = 0; r < C; r++) {
+      const unsigned i = min(row(r), nrow - 1 - r0);
+      off[r] = 8 * (T ? step(r) + (unsigned)ld * i : i + (unsigned)ld * step(r));
+    }
+  }
+  __device__ __forceinline__ static const double *base(const double *X, int ld, int r0, int k0)
+  {
+    return T ? X + k0 + (size_t)ld * r0 : X + r0 + (size_t)ld * k0;
+  }
+  __device__ __forceinline__ static bool whole(int r0, int k0, int kend, int mode)
+  {
+    return k0 + BK <= kend && (mode != 1 || k0 >= r0 + ROWS - 1) && (mode != 2 || k0 + BK - 1 <= r0);
+  }
+  __device__ __forceinline__ void load(const double *p, double (&v)[C]) const
+  {
+#pragma unroll
+    for (int r = 0; r < C; r++) v[r] = *(const double *)((const char *)p + off[r]);
+  }
+  __device__ __forceinline__ static void load_part(const double *X, int ld, int r0, int nrow, int k0, int kend, int mode,
+                                                   double (&v)[C])
+  {
+#pragma unroll
+    for (int r = 0; r < C; r++) {
+      const int i = r0 + row(r), kk = k0 + step(r);
+      const bool ok = kk < kend && (mode != 1 || kk >= i) && (mode != 2 || kk <= i);
+      const int ic = min(i, nrow - 1), kc = min(kk, kend - 1);
+      const double x = X[T ? (size_t)kc + (size_t)ld * ic : (size_t)ic + (size_t)ld * kc];
+      v[r] = ok ? x : 0.0;
+    }
+  }
+  __device__ __forceinline__ static void store(double *s, int pitch, const double (&v)[C])
+  {
+#pragma unroll
+    for (int r = 0; r < C; r++) s[step(r) * pitch + row(r)] = v[r];
+  }
+};
+// Output tiles (mt x nt of them; tri 1: those with I >= J, 2: I <= J) in the order
+// that the work-groups take them: strips of eight tile columns, row by row, and
+// each XCD (work-groups go to them in turn) a contiguous eighth of that, so that
+// what runs on an XCD at a time shares rows and columns in its L2.  Tiles
+// outside a triangle have no work-group: launched as a square grid whose other
+// half left at once, the lower triangle of 31 x 31 tiles put 66 tiles on one
+// XCD's 64 places and took two turns (5.4 instead of 2.7 ms).  With a
+// triangular operand the work of a tile depends on its place, and the order is
+// plain.
+constexpr int STRIP = 8, XCDS = 8;
+__host__ __device__ inline int tile_count(int mt, int nt, int tri)
 {
-  if (i >= g.m || kk >= g.k) return 0.0;
-  if (g.atri == 1 && kk < i) return 0.0;
-  if (g.atri == 2 && kk > i) return 0.0;
-  return g.ta ? g.A[(size_t)kk + (size_t)g.lda * i] : g.A[(size_t)i + (size_t)g.lda * kk];
+  if (tri == 0) return mt * nt;
+  const int R = tri == 1 ? mt : nt, C = min(tri == 1 ? nt : mt, R);
+  return C * R - C * (C - 1) / 2;
 }
-__device__ __forceinline__ double load_opB(const GemmArgs &g, int kk, int j)
+__device__ __forceinline__ void tile_at(int id, int mt, int nt, int tri, bool spread, int &I, int &J)
 {
-  if (j >= g.n || kk >= g.k) return 0.0;
-  if (g.btri == 1 && kk > j) return 0.0;
-  if (g.btri == 2 && kk < j) return 0.0;
-  return g.tb ? g.B[(size_t)j + (size_t)g.ldb * kk] : g.B[(size_t)kk + (size_t)g.ldb * j];
+  if (spread) {
+    const int T = tile_count(mt, nt, tri), x = id % XCDS, q = id / XCDS;
+    id = x * (T / XCDS) + min(x, T % XCDS) + q;
+  }
+  const int R = tri == 2 ? nt : mt, C = tri == 2 ? mt : nt;  // tri 2: of the transposed triangle
+  for (int c = 0; c < C; c += STRIP) {
+    const int w = min(STRIP, C - c);
+    const int top = tri ? min(w, max(R - c, 0)) : 0;       // rows of 1, 2, .. tiles
+    const int tt = top * (top + 1) / 2, rows = tri ? max(R - c - top, 0) : R;
+    const int cnt = tt + rows * w;
+    if (id >= cnt) {
+      id -= cnt;
+      continue;
+    }
+    if (id < tt) {
+      int t = 0;
+      while (id > t) id -= ++t;
+      I = c + t;
+      J = c + id;
+    } else {
+      id -= tt;
+      I = (tri ? c + top : 0) + id / w;
+      J = c + id % w;
+    }
+    break;
+  }
+  if (tri == 2) {
+    const int t = I;
+    I = J;
+    J = t;
+  }
 }
 
-template <bool SPLIT>
+// the triangle of op(B) in terms of its columns
+__device__ __forceinline__ int btri_mode(int btri) { return btri == 1 ? 2 : btri == 2 ? 1 : 0; }
+
+template <bool SPLIT, int TA, int TB>
 __global__ __launch_bounds__(256) void k_dgemm(GemmArgs g)
 {
   __shared__ double As[2][BK][BM + PAD];
   __shared__ double Bs[2][BK][BN + PAD];
   const int tid = threadIdx.x;
-  const int i0 = blockIdx.x * BM, j0 = blockIdx.y * BN;
-  // output-triangle tile skip
-  if (g.tri == 1 && i0 + BM - 1 < j0) return;
-  if (g.tri == 2 && j0 + BN - 1 < i0) return;
+  int i0, j0;
+  tile_at(blockIdx.x, (g.m + BM - 1) / BM, (g.n + BN - 1) / BN, g.tri, !g.atri && !g.btri, i0, j0);
+  i0 *= BM;
+  j0 *= BN;
   // k range from operand structure
   int kbeg = 0, kend = g.k;
   if (g.atri == 1) kbeg = max(kbeg, i0);
@@ -88,34 +180,41 @@ __global__ __launch_bounds__(256) void k_dgemm(GemmArgs g)
   for (int a = 0; a < 2; a++)
     for (int b = 0; b < 2; b++) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
 
-  // with a K split, elements past this slice's end read as zero
-  GemmArgs gl = g;
-  if (SPLIT) gl.k = min(g.k, kend);
-  // register staging for the global loads of one slab: 4 A + 4 B per thread
+  // C (beta != 0) is read before the K loop, from clamped addresses, so that
+  // its loads overlap the products instead of following them
+  double pc[2][2][4];
+  if (!SPLIT && g.beta != 0.0) {
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        const int i = min(i0 + wi + 16 * a + li, g.m - 1);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int j = min(j0 + wj + 16 * b + lk + 4 * r, g.n - 1);
+          pc[a][b][r] = g.C[(size_t)i + (size_t)g.ldc * j];
+        }
+      }
+  }
+  const int bmode = btri_mode(g.btri);
+  Slab<TA, BM> sa;
+  Slab<!TB, BN> sb;
+  sa.init(g.lda, i0, g.m);
+  sb.init(g.ldb, j0, g.n);
   double ra[4], rb[4];
   auto gload = [&](int k0) {
-    if (!g.ta) {  // 64 rows contiguous per k column
-      for (int r = 0; r < 4; r++) ra[r] = load_opA(gl, i0 + (tid & 63), k0 + (tid >> 6) + 4 * r);
-    } else {      // 16 k contiguous per row
-      for (int r = 0; r < 4; r++) ra[r] = load_opA(gl, i0 + (tid >> 4) + 16 * r, k0 + (tid & 15));
-    }
-    if (g.tb) {   // 64 columns contiguous per k row
-      for (int r = 0; r < 4; r++) rb[r] = load_opB(gl, k0 + (tid >> 6) + 4 * r, j0 + (tid & 63));
-    } else {      // 16 k contiguous per column
-      for (int r = 0; r < 4; r++) rb[r] = load_opB(gl, k0 + (tid & 15), j0 + (tid >> 4) + 16 * r);
+    const double *pa = sa.base(g.A, g.lda, i0, k0), *pb = sb.base(g.B, g.ldb, j0, k0);
+    if (sa.whole(i0, k0, kend, g.atri) && sb.whole(j0, k0, kend, bmode)) {
+      sa.load(pa, ra);
+      sb.load(pb, rb);
+    } else {
+      sa.load_part(g.A, g.lda, i0, g.m, k0, kend, g.atri, ra);
+      sb.load_part(g.B, g.ldb, j0, g.n, k0, kend, bmode, rb);
     }
   };
   auto sstore = [&](int buf) {
-    if (!g.ta) {
-      for (int r = 0; r < 4; r++) As[buf][(tid >> 6) + 4 * r][tid & 63] = ra[r];
-    } else {
-      for (int r = 0; r < 4; r++) As[buf][tid & 15][(tid >> 4) + 16 * r] = ra[r];
-    }
-    if (g.tb) {
-      for (int r = 0; r < 4; r++) Bs[buf][(tid >> 6) + 4 * r][tid & 63] = rb[r];
-    } else {
-      for (int r = 0; r < 4; r++) Bs[buf][tid & 15][(tid >> 4) + 16 * r] = rb[r];
-    }
+    sa.store(&As[buf][0][0], BM + PAD, ra);
+    sb.store(&Bs[buf][0][0], BN + PAD, rb);
   };
 
   if (kbeg < kend) {
@@ -133,7 +232,7 @@ __global__ __launch_bounds__(256) void k_dgemm(GemmArgs g)
         for (int b = 0; b < 2; b++) bv[b] = Bs[buf][kq + lk][wj + 16 * b + li];
         for (int a = 0; a < 2; a++)
           for (int b = 0; b < 2; b++)
-            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
+            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[b], av[a], acc[a][b], 0, 0, 0);
       }
       if (more) {
         sstore(buf ^ 1);
@@ -142,13 +241,14 @@ __global__ __launch_bounds__(256) void k_dgemm(GemmArgs g)
       }
     }
   }
-  // epilogue: lane holds rows lane/16 + 4r (r = 0..3), column lane%16 of each
-  // 16x16 block (v_mfma_f64_16x16x4_f64 result layout, checked on gfx950)
+  // epilogue: an MFMA result has rows lane/16 + 4r (r = 0..3), column lane%16
+  // of each 16x16 block; with op(B) as the first operand these are columns and
+  // row of C, so that sixteen lanes write 128 contiguous bytes
   for (int a = 0; a < 2; a++) {
     for (int b = 0; b < 2; b++) {
-      const int j = j0 + wj + 16 * b + li;
+      const int i = i0 + wi + 16 * a + li;
       for (int r = 0; r < 4; r++) {
-        const int i = i0 + wi + 16 * a + lk + 4 * r;
+        const int j = j0 + wj + 16 * b + lk + 4 * r;
         if (i >= g.m || j >= g.n) continue;
         if (g.tri == 1 && i < j) continue;
         if (g.tri == 2 && i > j) continue;
@@ -156,10 +256,9 @@ __global__ __launch_bounds__(256) void k_dgemm(GemmArgs g)
           g.ws[((size_t)blockIdx.z * g.n + j) * g.m + i] = acc[a][b][r];
           continue;
         }
-        double *cp = g.C + (size_t)i + (size_t)g.ldc * j;
         double v = g.alpha * acc[a][b][r];
-        if (g.beta != 0.0) v += g.beta * *cp;
-        *cp = v;
+        if (g.beta != 0.0) v += g.beta * pc[a][b][r];
+        g.C[(size_t)i + (size_t)g.ldc * j] = v;
       }
     }
   }
@@ -167,10 +266,8 @@ __global__ __launch_bounds__(256) void k_dgemm(GemmArgs g)
 
 // Large products: tile 128x128x16, 256 threads = 4 wave64 in a 2x2
 // arrangement, each wave a 64x64 block of sixteen 16x16 MFMA accumulators
-// (eight operand reads from LDS per sixteen MFMAs).  The transposes are
-// template parameters, and every global load is unconditional (indices
-// clamped into the matrix, the value masked afterwards) so that a slab's
-// loads are issued together; LDS double-buffered as above.
+// (eight operand reads from LDS per sixteen MFMAs); LDS double-buffered as
+// above.
 constexpr int LM = 128, LN = 128, LK = 16;
 
 template <int TA, int TB>
@@ -179,9 +276,10 @@ __global__ __launch_bounds__(256, 2) void k_dgemm_big(GemmArgs g)
   __shared__ double As[2][LK][LM + PAD];
   __shared__ double Bs[2][LK][LN + PAD];
   const int tid = threadIdx.x;
-  const int i0 = blockIdx.x * LM, j0 = blockIdx.y * LN;
-  if (g.tri == 1 && i0 + LM - 1 < j0) return;
-  if (g.tri == 2 && j0 + LN - 1 < i0) return;
+  int i0, j0;
+  tile_at(blockIdx.x, (g.m + LM - 1) / LM, (g.n + LN - 1) / LN, g.tri, !g.atri && !g.btri, i0, j0);
+  i0 *= LM;
+  j0 *= LN;
   int kbeg = 0, kend = g.k;
   if (g.atri == 1) kbeg = max(kbeg, i0);
   if (g.atri == 2) kend = min(kend, i0 + LM);
@@ -198,45 +296,25 @@ __global__ __launch_bounds__(256, 2) void k_dgemm_big(GemmArgs g)
 #pragma unroll
     for (int b = 0; b < 4; b++) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
 
-  // this thread's eight elements of each operand per slab: op(A)(ia, ka + step),
-  // op(B)(kb + step, jb) with the step along k (no transpose) or the row / column
-  const int ia = TA ? i0 + (tid >> 4) : i0 + (tid & 127);
-  const int ka = TA ? (tid & 15) : (tid >> 7);
-  const int jb = TB ? j0 + (tid & 127) : j0 + (tid >> 4);
-  const int kb = TB ? (tid >> 7) : (tid & 15);
+  const int bmode = btri_mode(g.btri);
+  Slab<TA, LM> sa;
+  Slab<!TB, LN> sb;
+  sa.init(g.lda, i0, g.m);
+  sb.init(g.ldb, j0, g.n);
   double ra[8], rb[8];
   auto gload = [&](int k0) {
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-      const int i = TA ? ia + 16 * r : ia;
-      const int kk = TA ? k0 + ka : k0 + ka + 2 * r;
-      bool ok = i < g.m && kk < kend;
-      if (g.atri == 1) ok = ok && kk >= i;
-      if (g.atri == 2) ok = ok && kk <= i;
-      const int ic = min(i, g.m - 1), kc = min(kk, g.k - 1);
-      const double v = TA ? g.A[(size_t)kc + (size_t)g.lda * ic] : g.A[(size_t)ic + (size_t)g.lda * kc];
-      ra[r] = ok ? v : 0.0;
-    }
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-      const int j = TB ? jb : jb + 16 * r;
-      const int kk = TB ? k0 + kb + 2 * r : k0 + kb;
-      bool ok = j < g.n && kk < kend;
-      if (g.btri == 1) ok = ok && kk <= j;
-      if (g.btri == 2) ok = ok && kk >= j;
-      const int jc = min(j, g.n - 1), kc = min(kk, g.k - 1);
-      const double v = TB ? g.B[(size_t)jc + (size_t)g.ldb * kc] : g.B[(size_t)kc + (size_t)g.ldb * jc];
-      rb[r] = ok ? v : 0.0;
+    const double *pa = sa.base(g.A, g.lda, i0, k0), *pb = sb.base(g.B, g.ldb, j0, k0);
+    if (sa.whole(i0, k0, kend, g.atri) && sb.whole(j0, k0, kend, bmode)) {
+      sa.load(pa, ra);
+      sb.load(pb, rb);
+    } else {
+      sa.load_part(g.A, g.lda, i0, g.m, k0, kend, g.atri, ra);
+      sb.load_part(g.B, g.ldb, j0, g.n, k0, kend, bmode, rb);
     }
   };
   auto sstore = [&](int buf) {
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-      if (TA) As[buf][ka][(tid >> 4) + 16 * r] = ra[r];
-      else As[buf][ka + 2 * r][tid & 127] = ra[r];
-      if (TB) Bs[buf][kb + 2 * r][tid & 127] = rb[r];
-      else Bs[buf][kb][(tid >> 4) + 16 * r] = rb[r];
-    }
+    sa.store(&As[buf][0][0], LM + PAD, ra);
+    sb.store(&Bs[buf][0][0], LN + PAD, rb);
   };
 
   if (kbeg < kend) {
@@ -258,7 +336,7 @@ __global__ __launch_bounds__(256, 2) void k_dgemm_big(GemmArgs g)
         for (int a = 0; a < 4; a++)
 #pragma unroll
           for (int b = 0; b < 4; b++)
-            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
+            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[b], av[a], acc[a][b], 0, 0, 0);
       }
       if (more) {
         sstore(buf ^ 1);
@@ -267,24 +345,31 @@ __global__ __launch_bounds__(256, 2) void k_dgemm_big(GemmArgs g)
       }
     }
   }
-  // epilogue: as in k_dgemm (lane holds rows lane/16 + 4r, column lane%16)
+  // epilogue: as in k_dgemm; C
+  // (beta != 0) sixteen entries at a time, from clamped addresses
 #pragma unroll
-  for (int a = 0; a < 4; a++) {
+  for (int b = 0; b < 4; b++) {
+    double pc[4][4];
+    if (g.beta != 0.0) {
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-      const int j = j0 + wj + 16 * b + li;
+      for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          pc[a][r] = g.C[(size_t)min(i0 + wi + 16 * a + li, g.m - 1) +
+                         (size_t)g.ldc * min(j0 + wj + 16 * b + lk + 4 * r, g.n - 1)];
+    }
+#pragma unroll
+    for (int a = 0; a < 4; a++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int i = i0 + wi + 16 * a + lk + 4 * r;
+        const int i = i0 + wi + 16 * a + li, j = j0 + wj + 16 * b + lk + 4 * r;
         if (i >= g.m || j >= g.n) continue;
         if (g.tri == 1 && i < j) continue;
         if (g.tri == 2 && i > j) continue;
-        double *cp = g.C + (size_t)i + (size_t)g.ldc * j;
         double v = g.alpha * acc[a][b][r];
-        if (g.beta != 0.0) v += g.beta * *cp;
-        *cp = v;
+        if (g.beta != 0.0) v += g.beta * pc[a][r];
+        g.C[(size_t)i + (size_t)g.ldc * j] = v;
       }
-    }
   }
 }
 
@@ -332,9 +417,10 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(ZGemmArgs g)
   __shared__ double Ar_s[2][BK][BM + PAD], Ai_s[2][BK][BM + PAD];
   __shared__ double Br_s[2][BK][BN + PAD], Bi_s[2][BK][BN + PAD];
   const int tid = threadIdx.x;
-  const int i0 = blockIdx.x * BM, j0 = blockIdx.y * BN;
-  if (g.tri == 1 && i0 + BM - 1 < j0) return;
-  if (g.tri == 2 && j0 + BN - 1 < i0) return;
+  int i0, j0;
+  tile_at(blockIdx.x, (g.m + BM - 1) / BM, (g.n + BN - 1) / BN, g.tri, true, i0, j0);
+  i0 *= BM;
+  j0 *= BN;
   const int lane = tid & 63, wave = tid >> 6;
   const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
   const int li = lane & 15, lk = lane >> 4;
@@ -346,10 +432,10 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(ZGemmArgs g)
     for (int a = 0; a < 2; a++)
 #pragma unroll
       for (int b = 0; b < 2; b++) {
-        const int j = min(j0 + wj + 16 * b + li, g.n - 1);
+        const int i = min(i0 + wi + 16 * a + li, g.m - 1);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          const int i = min(i0 + wi + 16 * a + lk + 4 * r, g.m - 1);
+          const int j = min(j0 + wj + 16 * b + lk + 4 * r, g.n - 1);
           const size_t o = (size_t)i + (size_t)g.ldc * j;
           pcr[a][b][r] = g.Cr[o];
           pci[a][b][r] = g.Ci[o];
@@ -362,43 +448,38 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(ZGemmArgs g)
       cr[a][b] = d4{0.0, 0.0, 0.0, 0.0};
       ci[a][b] = d4{0.0, 0.0, 0.0, 0.0};
     }
-  // this thread's four elements of each operand per slab (rows or k steps as
-  // in k_dgemm), loaded unconditionally from clamped addresses and masked
+  // both planes of an operand lie alike: one set of offsets
+  Slab<TA, BM> sa;
+  Slab<!TB, BN> sb;
+  sa.init(g.lda, i0, g.m);
+  sb.init(g.ldb, j0, g.n);
   double rar[4], rai[4], rbr[4], rbi[4];
   auto gload = [&](int k0) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int i = TA ? i0 + (tid >> 4) + 16 * r : i0 + (tid & 63);
-      const int kk = TA ? k0 + (tid & 15) : k0 + (tid >> 6) + 4 * r;
-      const bool ok = i < g.m && kk < g.k;
-      const int ic = min(i, g.m - 1), kc = min(kk, g.k - 1);
-      const size_t o = TA ? (size_t)kc + (size_t)g.lda * ic : (size_t)ic + (size_t)g.lda * kc;
-      const double vr = g.Ar[o], vi = g.Ai[o];
-      rar[r] = ok ? vr : 0.0;
-      rai[r] = ok ? g.sa * vi : 0.0;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int j = TB ? j0 + (tid & 63) : j0 + (tid >> 4) + 16 * r;
-      const int kk = TB ? k0 + (tid >> 6) + 4 * r : k0 + (tid & 15);
-      const bool ok = j < g.n && kk < g.k;
-      const int jc = min(j, g.n - 1), kc = min(kk, g.k - 1);
-      const size_t o = TB ? (size_t)jc + (size_t)g.ldb * kc : (size_t)kc + (size_t)g.ldb * jc;
-      const double vr = g.Br[o], vi = g.Bi[o];
-      rbr[r] = ok ? vr : 0.0;
-      rbi[r] = ok ? g.sb * vi : 0.0;
+    const double *par = sa.base(g.Ar, g.lda, i0, k0), *pai = sa.base(g.Ai, g.lda, i0, k0);
+    const double *pbr = sb.base(g.Br, g.ldb, j0, k0), *pbi = sb.base(g.Bi, g.ldb, j0, k0);
+    if (k0 + BK <= g.k) {
+      sa.load(par, rar);
+      sa.load(pai, rai);
+      sb.load(pbr, rbr);
+      sb.load(pbi, rbi);
+    } else {
+      sa.load_part(g.Ar, g.lda, i0, g.m, k0, g.k, 0, rar);
+      sa.load_part(g.Ai, g.lda, i0, g.m, k0, g.k, 0, rai);
+      sb.load_part(g.Br, g.ldb, j0, g.n, k0, g.k, 0, rbr);
+      sb.load_part(g.Bi, g.ldb, j0, g.n, k0, g.k, 0, rbi);
     }
   };
+  // the imaginary parts signed for conjugation
   auto sstore = [&](int buf) {
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int ka = TA ? (tid & 15) : (tid >> 6) + 4 * r, ia = TA ? (tid >> 4) + 16 * r : (tid & 63);
-      Ar_s[buf][ka][ia] = rar[r];
-      Ai_s[buf][ka][ia] = rai[r];
-      const int kb = TB ? (tid >> 6) + 4 * r : (tid & 15), jb = TB ? (tid & 63) : (tid >> 4) + 16 * r;
-      Br_s[buf][kb][jb] = rbr[r];
-      Bi_s[buf][kb][jb] = rbi[r];
+      rai[r] *= g.sa;
+      rbi[r] *= g.sb;
     }
+    sa.store(&Ar_s[buf][0][0], BM + PAD, rar);
+    sa.store(&Ai_s[buf][0][0], BM + PAD, rai);
+    sb.store(&Br_s[buf][0][0], BN + PAD, rbr);
+    sb.store(&Bi_s[buf][0][0], BN + PAD, rbi);
   };
   if (g.k > 0) {
     gload(0);
@@ -420,12 +501,16 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(ZGemmArgs g)
           bi[b] = Bi_s[buf][kq + lk][wj + 16 * b + li];
           nbi[b] = -bi[b];
         }
+        // the two products of an accumulator eight MFMAs apart
         for (int a = 0; a < 2; a++)
           for (int b = 0; b < 2; b++) {
-            cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[a], br[b], cr[a][b], 0, 0, 0);
-            cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[a], nbi[b], cr[a][b], 0, 0, 0);
-            ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[a], bi[b], ci[a][b], 0, 0, 0);
-            ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[a], br[b], ci[a][b], 0, 0, 0);
+            cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(br[b], ar[a], cr[a][b], 0, 0, 0);
+            ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bi[b], ar[a], ci[a][b], 0, 0, 0);
+          }
+        for (int a = 0; a < 2; a++)
+          for (int b = 0; b < 2; b++) {
+            cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(nbi[b], ai[a], cr[a][b], 0, 0, 0);
+            ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(br[b], ai[a], ci[a][b], 0, 0, 0);
           }
       }
       if (more) {
@@ -437,9 +522,9 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(ZGemmArgs g)
   }
   for (int a = 0; a < 2; a++) {
     for (int b = 0; b < 2; b++) {
-      const int j = j0 + wj + 16 * b + li;
+      const int i = i0 + wi + 16 * a + li;
       for (int r = 0; r < 4; r++) {
-        const int i = i0 + wi + 16 * a + lk + 4 * r;
+        const int j = j0 + wj + 16 * b + lk + 4 * r;
         if (i >= g.m || j >= g.n) continue;
         if (g.tri == 1 && i < j) continue;
         if (g.tri == 2 && i > j) continue;
@@ -468,9 +553,10 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_split(ZGemmArgs g, int kslice,
   __shared__ double Ar_s[2][BK][BM + PAD], Ai_s[2][BK][BM + PAD];
   __shared__ double Br_s[2][BK][BN + PAD], Bi_s[2][BK][BN + PAD];
   const int tid = threadIdx.x;
-  const int i0 = blockIdx.x * BM, j0 = blockIdx.y * BN;
-  if (g.tri == 1 && i0 + BM - 1 < j0) return;
-  if (g.tri == 2 && j0 + BN - 1 < i0) return;
+  int i0, j0;
+  tile_at(blockIdx.x, (g.m + BM - 1) / BM, (g.n + BN - 1) / BN, g.tri, true, i0, j0);
+  i0 *= BM;
+  j0 *= BN;
   const int lane = tid & 63, wave = tid >> 6;
   const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
   const int li = lane & 15, lk = lane >> 4;
@@ -481,43 +567,38 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_split(ZGemmArgs g, int kslice,
       cr[a][b] = d4{0.0, 0.0, 0.0, 0.0};
       ci[a][b] = d4{0.0, 0.0, 0.0, 0.0};
     }
-  // this thread's four elements of each operand per slab (rows or k steps as
-  // in k_dgemm), loaded unconditionally from clamped addresses and masked
+  // both planes of an operand lie alike: one set of offsets
+  Slab<TA, BM> sa;
+  Slab<!TB, BN> sb;
+  sa.init(g.lda, i0, g.m);
+  sb.init(g.ldb, j0, g.n);
   double rar[4], rai[4], rbr[4], rbi[4];
   auto gload = [&](int k0) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int i = TA ? i0 + (tid >> 4) + 16 * r : i0 + (tid & 63);
-      const int kk = TA ? k0 + (tid & 15) : k0 + (tid >> 6) + 4 * r;
-      const bool ok = i < g.m && kk < kend;
-      const int ic = min(i, g.m - 1), kc = min(kk, g.k - 1);
-      const size_t o = TA ? (size_t)kc + (size_t)g.lda * ic : (size_t)ic + (size_t)g.lda * kc;
-      const double vr = g.Ar[o], vi = g.Ai[o];
-      rar[r] = ok ? vr : 0.0;
-      rai[r] = ok ? g.sa * vi : 0.0;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int j = TB ? j0 + (tid & 63) : j0 + (tid >> 4) + 16 * r;
-      const int kk = TB ? k0 + (tid >> 6) + 4 * r : k0 + (tid & 15);
-      const bool ok = j < g.n && kk < kend;
-      const int jc = min(j, g.n - 1), kc = min(kk, g.k - 1);
-      const size_t o = TB ? (size_t)jc + (size_t)g.ldb * kc : (size_t)kc + (size_t)g.ldb * jc;
-      const double vr = g.Br[o], vi = g.Bi[o];
-      rbr[r] = ok ? vr : 0.0;
-      rbi[r] = ok ? g.sb * vi : 0.0;
+    const double *par = sa.base(g.Ar, g.lda, i0, k0), *pai = sa.base(g.Ai, g.lda, i0, k0);
+    const double *pbr = sb.base(g.Br, g.ldb, j0, k0), *pbi = sb.base(g.Bi, g.ldb, j0, k0);
+    if (k0 + BK <= kend) {
+      sa.load(par, rar);
+      sa.load(pai, rai);
+      sb.load(pbr, rbr);
+      sb.load(pbi, rbi);
+    } else {
+      sa.load_part(g.Ar, g.lda, i0, g.m, k0, kend, 0, rar);
+      sa.load_part(g.Ai, g.lda, i0, g.m, k0, kend, 0, rai);
+      sb.load_part(g.Br, g.ldb, j0, g.n, k0, kend, 0, rbr);
+      sb.load_part(g.Bi, g.ldb, j0, g.n, k0, kend, 0, rbi);
     }
   };
+  // the imaginary parts signed for conjugation
   auto sstore = [&](int buf) {
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int ka = TA ? (tid & 15) : (tid >> 6) + 4 * r, ia = TA ? (tid >> 4) + 16 * r : (tid & 63);
-      Ar_s[buf][ka][ia] = rar[r];
-      Ai_s[buf][ka][ia] = rai[r];
-      const int kb = TB ? (tid >> 6) + 4 * r : (tid & 15), jb = TB ? (tid & 63) : (tid >> 4) + 16 * r;
-      Br_s[buf][kb][jb] = rbr[r];
-      Bi_s[buf][kb][jb] = rbi[r];
+      rai[r] *= g.sa;
+      rbi[r] *= g.sb;
     }
+    sa.store(&Ar_s[buf][0][0], BM + PAD, rar);
+    sa.store(&Ai_s[buf][0][0], BM + PAD, rai);
+    sb.store(&Br_s[buf][0][0], BN + PAD, rbr);
+    sb.store(&Bi_s[buf][0][0], BN + PAD, rbi);
   };
   if (kbeg < kend) {
     gload(kbeg);
@@ -539,12 +620,16 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_split(ZGemmArgs g, int kslice,
           bi[b] = Bi_s[buf][kq + lk][wj + 16 * b + li];
           nbi[b] = -bi[b];
         }
+        // the two products of an accumulator eight MFMAs apart
         for (int a = 0; a < 2; a++)
           for (int b = 0; b < 2; b++) {
-            cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[a], br[b], cr[a][b], 0, 0, 0);
-            cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[a], nbi[b], cr[a][b], 0, 0, 0);
-            ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[a], bi[b], ci[a][b], 0, 0, 0);
-            ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[a], br[b], ci[a][b], 0, 0, 0);
+            cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(br[b], ar[a], cr[a][b], 0, 0, 0);
+            ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bi[b], ar[a], ci[a][b], 0, 0, 0);
+          }
+        for (int a = 0; a < 2; a++)
+          for (int b = 0; b < 2; b++) {
+            cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(nbi[b], ai[a], cr[a][b], 0, 0, 0);
+            ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(br[b], ai[a], ci[a][b], 0, 0, 0);
           }
       }
       if (more) {
@@ -557,9 +642,9 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_split(ZGemmArgs g, int kslice,
   // raw sums of this K slice (no triangle: the split needs a full output)
   for (int a = 0; a < 2; a++) {
     for (int b = 0; b < 2; b++) {
-      const int j = j0 + wj + 16 * b + li;
+      const int i = i0 + wi + 16 * a + li;
       for (int r = 0; r < 4; r++) {
-        const int i = i0 + wi + 16 * a + lk + 4 * r;
+        const int j = j0 + wj + 16 * b + lk + 4 * r;
         if (i >= g.m || j >= g.n) continue;
         const size_t o = ((size_t)blockIdx.z * g.n + j) * g.m + i;
         wsr[o] = cr[a][b][r];
@@ -609,6 +694,7 @@ int zgemm_fused(hipStream_t s, char ta, char tb, int m, int n, int k, double alp
   // slices, partial sums in ws (two planes of m x n per slice)
   constexpr int ksl = W2K_ZSPLIT_KMIN / 2;
   const long tiles = (long)grid.x * grid.y;
+  grid = dim3(tile_count(grid.x, grid.y, tri));
   if (ws && tri == 0 && tiles < 256 && k >= W2K_ZSPLIT_KMIN) {
     int nz = (int)std::min<long>((k + ksl - 1) / ksl, std::max<long>(1, 1024 / tiles));
     nz = (int)std::min<size_t>((size_t)nz, wsn / ((size_t)2 * m * n));
@@ -674,11 +760,20 @@ bool tuning_on()
 }
 }  // namespace
 
+template <bool SPLIT>
+static void launch_dgemm(hipStream_t s, const GemmArgs &g, dim3 grid)
+{
+  if (!g.ta && !g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, 0, 0>), grid, dim3(256), 0, s, g);
+  else if (g.ta && !g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, 1, 0>), grid, dim3(256), 0, s, g);
+  else if (!g.ta && g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, 0, 1>), grid, dim3(256), 0, s, g);
+  else hipLaunchKernelGGL((k_dgemm<SPLIT, 1, 1>), grid, dim3(256), 0, s, g);
+}
+
 // variant 0: 64x64 tiles, 1: 128x128 tiles
 static int launch_tiles(hipStream_t s, const GemmArgs &g, int variant)
 {
   if (variant == 1) {
-    dim3 gb((g.m + LM - 1) / LM, (g.n + LN - 1) / LN);
+    const dim3 gb(tile_count((g.m + LM - 1) / LM, (g.n + LN - 1) / LN, g.tri));
     if (!g.ta && !g.tb) hipLaunchKernelGGL((k_dgemm_big<0, 0>), gb, dim3(256), 0, s, g);
     else if (g.ta && !g.tb) hipLaunchKernelGGL((k_dgemm_big<1, 0>), gb, dim3(256), 0, s, g);
     else if (!g.ta && g.tb) hipLaunchKernelGGL((k_dgemm_big<0, 1>), gb, dim3(256), 0, s, g);
@@ -686,8 +781,7 @@ static int launch_tiles(hipStream_t s, const GemmArgs &g, int variant)
     W2K_STAGE(s, "k_dgemm_big");
     return 0;
   }
-  dim3 grid((g.m + BM - 1) / BM, (g.n + BN - 1) / BN);
-  hipLaunchKernelGGL(k_dgemm<false>, grid, dim3(256), 0, s, g);
+  launch_dgemm<false>(s, g, dim3(tile_count((g.m + BM - 1) / BM, (g.n + BN - 1) / BN, g.tri)));
   W2K_STAGE(s, "k_dgemm");
   return 0;
 }
@@ -739,8 +833,8 @@ int dgemm(hipStream_t s, char ta, char tb, int m, int n, int k, double alpha, co
       g.kslice = ((k + nz - 1) / nz + BK - 1) / BK * BK;
       nz = (k + g.kslice - 1) / g.kslice;
       g.ws = ws;
-      grid.z = nz;
-      hipLaunchKernelGGL(k_dgemm<true>, grid, dim3(256), 0, s, g);
+      grid = dim3(tile_count(grid.x, grid.y, tri), 1, nz);
+      launch_dgemm<true>(s, g, grid);
       W2K_STAGE(s, "k_dgemm<split>");
       hipLaunchKernelGGL(k_splitk_reduce, dim3((m + 255) / 256, n), dim3(256), 0, s, m, n, nz, ws, alpha, beta, C,
                          ldc, tri);
