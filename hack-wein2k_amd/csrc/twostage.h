@@ -26,6 +26,7 @@ struct SbArgs {
   size_t ntau2 = 0;
   int *prog = nullptr;                      // finished steps per sweep; entry n: the next sweep
   double *frag = nullptr;                   // operands of the Q2 blocks
+  double *zb = nullptr;                     // vectors between the groups of Q2, 16 columns side by side
   int *q2sync = nullptr;                    // ticket and progress of their application
 };
 

@@ -17,8 +17,8 @@
 // matrix products, and the serial part is 32 short exchanges per panel and
 // two steps per sweep.  Whole reduction, before -> now (Q2's application in
 // brackets): real N = 221 3.1 -> 1.3 ms, N = 731 10.7 -> 5.3, N = 5951 135 ->
-// 64 (+ 11); complex N = 251 5.4 -> 2.6, N = 1950 47 -> 26 (+ 2), N = 10880
-// 1018 -> 360 (+ 161).
+// 60 (+ 6); complex N = 251 5.4 -> 2.5, N = 1950 47 -> 25 (+ 2), N = 10880
+// 1018 -> 325 (+ 84).
 #include <algorithm>
 #include <cmath>
 
@@ -1254,10 +1254,16 @@ __global__ __launch_bounds__(256) void k_sb_frag(SbArgs g, int ntg, int nsync)
   }
 }
 
+// rows of the blocked copy of Z (the last window reaches past the matrix)
+__host__ __device__ constexpr size_t q2_rows(int n) { return (size_t)n + 2 * BND; }
+
 // Z <- Q2 Z.  A task is one group of sweeps on a slab of 16 columns of Z: its
 // blocks slide down the rows.  A wave holds 16 of the window's 64 rows as MFMA
 // accumulators (lane (l, q): column l, rows 4 q + k in item k), which are at
-// once the operand of V^H Z; the four partial V^H Z meet in LDS.  The window
+// once the operand of V^H Z; the four partial V^H Z meet in LDS.  Between the
+// groups Z lives in a copy with 16 columns side by side, row after row, so that
+// such an item is four full lines; the first group that touches a row takes it
+// from Z, the last one puts it back.  The window
 // moves by 32 rows, so two waves keep their rows and the other two store
 // theirs and take the next 32.  Rows and operands are loaded a step ahead and
 // rows stored a step late, so that no step waits for memory it has just asked.
@@ -1267,60 +1273,97 @@ __global__ __launch_bounds__(256) void k_sb_frag(SbArgs g, int ntg, int nsync)
 // tasks in order from a ticket, so the group that a task waits for has started
 // before it, and every Q2_FLAG steps a task publishes how many it has done.
 constexpr int Q2_FLAG = 4;
+// From this many columns on a step's rate counts and not its length: two
+// work-groups a CU instead of one (complex N = 10886, m = 2177 205 -> 169 ms for
+// the whole back-transform; N = 1951, m = 195 6.2 -> 6.6 ms), and real tasks take
+// two sets of columns, which halves what the operands' loads move (N = 5940,
+// m = 1188 14.4 -> 13.4; N = 731, m = 88 0.87 -> 0.96 ms).
+constexpr int Q2_WIDE = 512;
 
-template <bool CX>
-__global__ __launch_bounds__(256, CX ? 1 : 2) void k_sb_q2(SbArgs g, int ntg, int mcol, double *__restrict__ Zr,
+template <bool CX, int NC>
+__global__ __launch_bounds__(256, 2) void k_sb_q2(SbArgs g, int ntg, int mcol, double *__restrict__ Zr,
                                                            double *__restrict__ Zi, int ldz)
 {
   constexpr int CP = CX ? 2 : 1;
-  __shared__ double yp[2][CP][4][8][64];
+  __shared__ double yp[2][CP][NC][4][8][64];
   __shared__ int tick;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l = lane & 15, q4 = lane >> 4;
-  const int n = g.n, nslab = (mcol + 15) / 16, ntask = nslab * ntg;
+  const int n = g.n, nslab = (mcol + 16 * NC - 1) / (16 * NC), ntask = nslab * ntg;
   int *const done = g.q2sync + 1;  // steps done of (group from the last, slab)
+  const size_t zrows = q2_rows(n), zplane = zrows * (size_t)nslab * NC * 16;
+  const int zo = 64 * q4 + l;  // this lane's place in four rows, 4 q4 rows on
   auto ticket = [&]() { return __hip_atomic_fetch_add(g.q2sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
   if (tid == 0) tick = ticket();
   __syncthreads();
   int task = __builtin_amdgcn_readfirstlane(tick);
   while (task < ntask) {
     const int gi = task / nslab, slab = task - gi * nslab, gr = ntg - 1 - gi, nt = gi + 1;
-    const int col = slab * 16 + l;
-    const bool okc = col < mcol;
-    const size_t zc = (size_t)ldz * min(col, mcol - 1);
+    double *const zb = g.zb + (size_t)slab * NC * 16 * zrows;
     int seen = gi == 0 ? CHASE_DONE : 0;
-    // rows of window t are final once the group after this one has done step t
+    // rows of window t are final once the group after this one has done step
+    // t; its progress is read a step ahead
+    int peek = 0;
+    auto progress = [&]() { return gi > 0 ? agent_ld(done + (size_t)(gi - 1) * nslab + slab) : CHASE_DONE; };
     auto ready = [&](int t) {
       while (seen < t + 1) {
-        seen = agent_ld(done + (size_t)(gi - 1) * nslab + slab);
+        seen = __builtin_amdgcn_readfirstlane(progress());
         if (seen < t + 1) __builtin_amdgcn_s_sleep(1);
       }
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
     };
-    auto zload = [&](int row0, d4 &a, d4 &b) {
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const size_t o = zc + min(row0 + 4 * q4 + k, n - 1);
-        a[k] = agent_ld(Zr + o);
-        if (CX) b[k] = agent_ld(Zi + o);
-      }
+    // four rows of each set of columns
+    struct Rows {
+      d4 r[NC], i[CX ? NC : 1];
     };
-    auto zmask = [&](int row0, d4 &a, d4 &b) {
+    // rows that no group has touched yet, from Z
+    auto zfirst = [&](int row0, Rows &z) {
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const bool ok = okc && row0 + 4 * q4 + k < n;
-        a[k] = ok ? a[k] : 0.0;
-        if (CX) b[k] = ok ? b[k] : 0.0;
-      }
-    };
-    auto zstore = [&](int row0, const d4 &a, const d4 &b) {
+      for (int c = 0; c < NC; c++) {
+        const int col = (slab * NC + c) * 16 + l;
+        const size_t zc = (size_t)ldz * min(col, mcol - 1);
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const int row = row0 + 4 * q4 + k;
-        if (okc && row < n) {
-          agent_st(Zr + zc + row, a[k]);
-          if (CX) agent_st(Zi + zc + row, b[k]);
+        for (int k = 0; k < 4; k++) {
+          const int row = row0 + 4 * q4 + k;
+          const size_t o = zc + min(row, n - 1);
+          const bool ok = col < mcol && row < n;
+          const double x = Zr[o], y = CX ? Zi[o] : 0.0;
+          z.r[c][k] = ok ? x : 0.0;
+          if (CX) z.i[c][k] = ok ? y : 0.0;
         }
       }
+    };
+    auto zload = [&](int row0, Rows &z) {
+#pragma unroll
+      for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const double *p = zb + (size_t)c * 16 * zrows + 16 * (size_t)(row0 + k);
+          z.r[c][k] = agent_ld(p + zo);
+          if (CX) z.i[c][k] = agent_ld(p + zplane + zo);
+        }
+    };
+    auto zstore = [&](int row0, const Rows &z) {
+      if (gr > 0) {
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            double *p = zb + (size_t)c * 16 * zrows + 16 * (size_t)(row0 + k);
+            agent_st(p + zo, z.r[c][k]);
+            if (CX) agent_st(p + zplane + zo, z.i[c][k]);
+          }
+        return;
+      }
+#pragma unroll
+      for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int col = (slab * NC + c) * 16 + l, row = row0 + 4 * q4 + k;
+          if (col < mcol && row < n) {
+            Zr[(size_t)ldz * col + row] = z.r[c][k];
+            if (CX) Zi[(size_t)ldz * col + row] = z.i[c][k];
+          }
+        }
     };
     struct Ops {
       double a[8], t[8], ai[CX ? 8 : 1], ti[CX ? 8 : 1];
@@ -1338,87 +1381,105 @@ __global__ __launch_bounds__(256, CX ? 1 : 2) void k_sb_q2(SbArgs g, int ntg, in
       }
     };
     int role = wave, w0 = gr * BND + 1, pend = -1;  // pend: first row of the tile to be stored
-    d4 zr, zi, sr, si;
+    Rows z, st;
     ready(0);
-    zload(w0 + 16 * role, zr, zi);
+    if (gi == 0 || role < 2) zfirst(w0 + 16 * role, z);
+    else zload(w0 + 16 * role, z);
     Ops oa, ob;
     fetch(oa, 0, role);
-    zmask(w0 + 16 * role, zr, zi);
     auto step = [&](const Ops &o, Ops &next, int t) {
       // what the last step asked for has come; then, in this order so that no
       // wait below includes a younger access: rows, operands, stores
       vm_drain();
+      seen = max(seen, __builtin_amdgcn_readfirstlane(peek));
       const bool more = t + 1 < nt, leave = role < 2 && more;
-      d4 nr, ni;
+      Rows nx;
       if (leave) {
         ready(t + 1);
-        zload(w0 + 64 + 16 * role, nr, ni);
+        zload(w0 + 64 + 16 * role, nx);
       }
+      peek = progress();
       fetch(next, more ? t + 1 : t, (role + 2) & 3);
-      if (pend >= 0) zstore(pend, sr, si);
+      if (pend >= 0) zstore(pend, st);
       // partial V^H Z over this wave's rows
-      d4 yr[2], yi[2];
+      d4 yr[NC][2], yi[NC][2];
 #pragma unroll
-      for (int mt = 0; mt < 2; mt++) {
-        yr[mt] = d4{0.0, 0.0, 0.0, 0.0};
-        yi[mt] = d4{0.0, 0.0, 0.0, 0.0};
-      }
-#pragma unroll
-      for (int k = 0; k < 4; k++)
+      for (int c = 0; c < NC; c++)
 #pragma unroll
         for (int mt = 0; mt < 2; mt++) {
-          yr[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[4 * mt + k], zr[k], yr[mt], 0, 0, 0);
-          if (CX) {
-            yi[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[4 * mt + k], zi[k], yi[mt], 0, 0, 0);
-            yr[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.ai[4 * mt + k], zi[k], yr[mt], 0, 0, 0);
-            yi[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(-o.ai[4 * mt + k], zr[k], yi[mt], 0, 0, 0);
-          }
+          yr[c][mt] = d4{0.0, 0.0, 0.0, 0.0};
+          yi[c][mt] = d4{0.0, 0.0, 0.0, 0.0};
         }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+          for (int mt = 0; mt < 2; mt++) {
+            yr[c][mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[4 * mt + k], z.r[c][k], yr[c][mt], 0, 0, 0);
+            if (CX) yi[c][mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[4 * mt + k], z.i[c][k], yi[c][mt], 0, 0, 0);
+          }
+        if (CX)
+#pragma unroll
+          for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+              yr[c][mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.ai[4 * mt + k], z.i[c][k], yr[c][mt], 0, 0, 0);
+              yi[c][mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(-o.ai[4 * mt + k], z.r[c][k], yi[c][mt], 0, 0, 0);
+            }
+      }
       mfma_settle();
       const int par = t & 1;
 #pragma unroll
-      for (int mt = 0; mt < 2; mt++)
+      for (int c = 0; c < NC; c++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          yp[par][0][role][4 * mt + k][lane] = yr[mt][k];
-          if (CX) yp[par][CP - 1][role][4 * mt + k][lane] = yi[mt][k];
-        }
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            yp[par][0][c][role][4 * mt + k][lane] = yr[c][mt][k];
+            if (CX) yp[par][CP - 1][c][role][4 * mt + k][lane] = yi[c][mt][k];
+          }
       const bool flag = t % Q2_FLAG == Q2_FLAG - 1;
       if (flag) vm_drain();  // the tiles of the steps before this one are stored
       __syncthreads();
       if (flag && tid == 0) agent_st(done + (size_t)gi * nslab + slab, t);
-      // Z -= (V T) (V^H Z), in two accumulator chains
+      // Z -= (V T) (V^H Z), for one real set of columns in two accumulator chains
+      constexpr bool TWO = !CX && NC == 1;
       d4 z2 = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int s = 0; s < 8; s++) {
-        double a = yp[par][0][0][s][lane], b = 0.0;
-        if (CX) b = yp[par][CP - 1][0][s][lane];
+        double a[NC], b[NC];
 #pragma unroll
-        for (int w = 1; w < 4; w++) {
-          a += yp[par][0][w][s][lane];
-          if (CX) b += yp[par][CP - 1][w][s][lane];
+        for (int c = 0; c < NC; c++) {
+          a[c] = yp[par][0][c][0][s][lane];
+          if (CX) b[c] = yp[par][CP - 1][c][0][s][lane];
+#pragma unroll
+          for (int w = 1; w < 4; w++) {
+            a[c] += yp[par][0][c][w][s][lane];
+            if (CX) b[c] += yp[par][CP - 1][c][w][s][lane];
+          }
         }
-        if (CX || !(s & 1)) zr = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], a, zr, 0, 0, 0);
-        else z2 = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], a, z2, 0, 0, 0);
-        if (CX) {
-          zi = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], b, zi, 0, 0, 0);
-          zr = __builtin_amdgcn_mfma_f64_16x16x4f64(-o.ti[s], b, zr, 0, 0, 0);
-          zi = __builtin_amdgcn_mfma_f64_16x16x4f64(o.ti[s], a, zi, 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          if (TWO && (s & 1)) z2 = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], a[c], z2, 0, 0, 0);
+          else z.r[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], a[c], z.r[c], 0, 0, 0);
+          if (CX) z.i[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.t[s], b[c], z.i[c], 0, 0, 0);
         }
+        if (CX)
+#pragma unroll
+          for (int c = 0; c < NC; c++) {
+            z.r[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(-o.ti[s], b[c], z.r[c], 0, 0, 0);
+            z.i[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.ti[s], a[c], z.i[c], 0, 0, 0);
+          }
       }
       mfma_settle();
-      if (!CX) zr += z2;
+      if (TWO) z.r[0] += z2;
       pend = -1;
       if (more) {
         if (leave) {
           pend = w0 + 16 * role;
-          sr = zr;
-          zr = nr;
-          if (CX) {
-            si = zi;
-            zi = ni;
-          }
-          zmask(w0 + 64 + 16 * role, zr, zi);
+          st = z;
+          z = nx;
         }
         role = (role + 2) & 3;
         w0 += BND;
@@ -1428,7 +1489,7 @@ __global__ __launch_bounds__(256, CX ? 1 : 2) void k_sb_q2(SbArgs g, int ntg, in
       step(oa, ob, t);
       if (t + 1 < nt) step(ob, oa, t + 1);
     }
-    zstore(w0 + 16 * role, zr, zi);
+    zstore(w0 + 16 * role, z);
     vm_drain();
     __syncthreads();
     if (tid == 0) {
@@ -1463,10 +1524,12 @@ size_t sb_doubles(int n, int cplx, size_t *ints)
 
 static size_t q2_words(int n, size_t m) { return (m + 15) / 16 * ((n - 1 + BND - 1) / BND) + 1; }
 
+static size_t q2_cols(size_t m) { return (m + 31) / 32 * 32; }
+
 size_t sb_frag_doubles(int n, size_t m, int cplx)
 {
   const size_t ntg = (n - 1 + BND - 1) / BND;
-  return ntg * (ntg + 1) / 2 * FRAG * (cplx ? 2 : 1) + (q2_words(n, m) + 1) / 2;
+  return (ntg * (ntg + 1) / 2 * FRAG + q2_rows(n) * q2_cols(m)) * (cplx ? 2 : 1) + (q2_words(n, m) + 1) / 2;
 }
 
 int sb_buffers(Ctx &c, SbArgs &g, int n, int cplx)
@@ -1590,8 +1653,9 @@ static int apply_q2(hipStream_t s, SbArgs &g, int m, double *Zr, double *Zi, int
   const size_t words = q2_words(g.n, m);
   hipLaunchKernelGGL((k_sb_frag<CX>), dim3(ntg, ntg), dim3(256), 0, s, g, ntg, (int)words);
   W2K_STAGE(s, "k_sb_frag");
-  const int nwg = (int)std::min(words - 1, (size_t)512);
-  hipLaunchKernelGGL((k_sb_q2<CX>), dim3(nwg), dim3(256), 0, s, g, ntg, m, Zr, Zi, ldz);
+  const int nwg = (int)std::min(words - 1, (size_t)(m >= Q2_WIDE ? 512 : 256));
+  if (!CX && m >= Q2_WIDE) hipLaunchKernelGGL((k_sb_q2<false, 2>), dim3(nwg), dim3(256), 0, s, g, ntg, m, Zr, Zi, ldz);
+  else hipLaunchKernelGGL((k_sb_q2<CX, 1>), dim3(nwg), dim3(256), 0, s, g, ntg, m, Zr, Zi, ldz);
   W2K_STAGE(s, "k_sb_q2");
   return 0;
 }
@@ -1602,7 +1666,8 @@ int sb_apply_q2(Ctx &c, hipStream_t s, SbArgs &g, int cplx, int m, double *Zr, d
   if ((rc = c.w_frag.alloc(sb_frag_doubles(g.n, m, cplx)))) return rc;
   g.frag = c.w_frag.p;
   const size_t ntg = (g.n - 1 + BND - 1) / BND;
-  g.q2sync = reinterpret_cast<int *>(g.frag + ntg * (ntg + 1) / 2 * FRAG * (cplx ? 2 : 1));
+  g.zb = g.frag + ntg * (ntg + 1) / 2 * FRAG * (cplx ? 2 : 1);
+  g.q2sync = reinterpret_cast<int *>(g.zb + q2_rows(g.n) * q2_cols(m) * (cplx ? 2 : 1));
   return cplx ? apply_q2<true>(s, g, m, Zr, Zi, ldz) : apply_q2<false>(s, g, m, Zr, Zi, ldz);
 }
 
