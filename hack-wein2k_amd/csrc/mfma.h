@@ -1,4 +1,4 @@
-// FP64 matrix-core helpers.
+// FP64 matrix-core and wave helpers.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -17,6 +17,22 @@ __device__ __forceinline__ void mfma_settle()
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_sleep(1);
   __builtin_amdgcn_sched_barrier(0);
+}
+
+// LDS written by this wave is read by its other lanes
+__device__ __forceinline__ void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the value of one lane, the same for all
+__device__ __forceinline__ double lane_value(double v, int lane)
+{
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
 
 }  // namespace w2k

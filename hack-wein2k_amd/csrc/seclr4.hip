@@ -37,6 +37,7 @@
 #include <utility>
 #include <vector>
 
+#include "chol_leaf.h"
 #include "seclr4_shared.h"
 #include "twostage.h"
 
@@ -84,27 +85,6 @@ __global__ void k_prep(int n, int ldh, const double *__restrict__ hs, const doub
   }
 }
 
-// 1/sqrt(x), x > 0: the hardware estimate refined by two Newton steps
-// y <- y + y (1/2 - (x/2) y^2) (a few ulp)
-__device__ __forceinline__ double rsqrt_nr(double x)
-{
-  double y = __builtin_amdgcn_rsq(x);
-  const double h = 0.5 * x;
-  double e = fma(-h * y, y, 0.5);
-  y = fma(y, e, y);
-  e = fma(-h * y, y, 0.5);
-  return fma(y, e, y);
-}
-
-// v of lane `src` (a wave-uniform lane index) in every lane
-__device__ __forceinline__ double lane_bcast(double v, int src)
-{
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b & 0xffffffffll), src);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)((unsigned long long)b >> 32), src);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
 // X = M^-1 of an N x N (N <= 64) upper triangular M held in LDS (M(r,q) at
 // sm[q LD + r]) by one wave, with dinv[r] = 1/M(r,r): lane c < N ends with
 // column c of X in x[0..N-1] (x[r] = 0 for r > c).  Rows from the bottom:
@@ -134,68 +114,35 @@ __device__ __forceinline__ void wave_trtri(const double *sm, const double *dinv,
 }
 
 // Cholesky S_kk = U^T U of the kb x kb diagonal block at (k0,k0) (upper) and
-// the inverse of its factor, by one wave: U over the block of a, U^-1 into
-// the same block of w (zeros below the diagonal).  Lane c holds column c in
-// registers; step j takes the pivot from lane j, scales row j by the inverse
-// square root of the pivot and broadcasts the row through LDS for the rank-1
-// update (rows below the diagonal of a column are carried along unused).  A
-// block smaller than 64 is padded with the identity.  A non-positive pivot
-// sets *info = k0 + j + 1 for the first such j (DPOTRF's INFO) and is taken
-// as 1 so that the arithmetic stays finite.  Loads and stores go through LDS
-// so that they are coalesced along the columns.
-__global__ __launch_bounds__(64) void k_chol_diag(int n, int k0, int kb, double *__restrict__ a,
-                                                  double *__restrict__ w, int *__restrict__ info)
+// the inverse of its factor: U over the block of a, U^-1 into the same block
+// of w (zeros below the diagonal).  A non-positive pivot sets *info = k0 + j +
+// 1 for the first such j (DPOTRF's INFO) and is taken as 1 so that the
+// arithmetic stays finite.  38 -> 20 us.
+__global__ __launch_bounds__(256) void k_chol_diag(int n, int k0, int kb, double *__restrict__ a,
+                                                   double *__restrict__ w, int *__restrict__ info)
 {
-  constexpr int LD = NB + 1;
-  __shared__ double sm[NB * LD];  // sm[c LD + r] = block element (r, c)
-  __shared__ double urow[2][NB];
-  __shared__ double dinv[NB];
-  const int lane = threadIdx.x;
+  __shared__ Leaf<false> s;
+  const int r = threadIdx.x & 63, g = threadIdx.x >> 6;
   {
-    // all 64 loads in flight together (clamped addresses, masked values)
-    double ld[NB];
-    const int rl = min(lane, kb - 1);
+    // all loads in flight together (clamped addresses, masked values)
+    double ld[16];
 #pragma unroll
-    for (int c = 0; c < NB; c++) ld[c] = a[(size_t)(k0 + rl) + (size_t)n * (k0 + min(c, kb - 1))];
+    for (int q = 0; q < 16; q++) ld[q] = a[(size_t)(k0 + min(r, kb - 1)) + (size_t)n * (k0 + min(g + 4 * q, kb - 1))];
 #pragma unroll
-    for (int c = 0; c < NB; c++) sm[c * LD + lane] = (lane <= c && c < kb) ? ld[c] : (lane == c ? 1.0 : 0.0);
+    for (int q = 0; q < 16; q++) {
+      const int c = g + 4 * q;
+      s.m[0][r][c] = r <= c && c < kb ? ld[q] : (r == c ? 1.0 : 0.0);
+    }
   }
   __syncthreads();
-  double v[NB];
-#pragma unroll
-  for (int r = 0; r < NB; r++) v[r] = sm[lane * LD + r];
-  int first = 0;
-#pragma unroll
-  for (int j = 0; j < NB; j++) {
-    const double ajj = lane_bcast(v[j], j);
-    const bool ok = ajj > 0.0;
-    first = (!ok && first == 0) ? j + 1 : first;
-    v[j] *= rsqrt_nr(ok ? ajj : 1.0);
-    urow[j & 1][lane] = v[j];
-    __syncthreads();
-    double u[NB];
-#pragma unroll
-    for (int r = j + 1; r < NB; r++) u[r] = urow[j & 1][r];
-#pragma unroll
-    for (int r = j + 1; r < NB; r++) v[r] = fma(-u[r], v[j], v[r]);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < NB; r++) sm[lane * LD + r] = (r <= lane) ? v[r] : 0.0;
-  __syncthreads();
-  for (int c = 0; c < kb; c++)
-    if (lane <= c) a[(size_t)(k0 + lane) + (size_t)n * (k0 + c)] = sm[c * LD + lane];
-  dinv[lane] = 1.0 / sm[lane * LD + lane];
-  __syncthreads();
-  double x[NB];
-  wave_trtri<NB, LD>(sm, dinv, lane, x);
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < NB; r++) sm[lane * LD + r] = (r <= lane) ? x[r] : 0.0;
-  __syncthreads();
-  if (lane < kb)
-    for (int c = 0; c < kb; c++) w[(size_t)(k0 + lane) + (size_t)n * (k0 + c)] = sm[c * LD + lane];
-  if (lane == 0 && first != 0 && *info == 0) *info = k0 + first;
+  const int first = chol_leaf<false>(s, [](double p) { return p > 0.0; });
+  if (r < kb)
+    for (int c = g; c < kb; c += 4) {
+      const size_t o = (size_t)(k0 + r) + (size_t)n * (k0 + c);
+      if (r <= c) a[o] = s.m[0][r][c];
+      w[o] = s.x[0][r][c];
+    }
+  if (threadIdx.x == 0 && first != 0 && *info == 0) *info = k0 + first;
 }
 
 __global__ void k_fill(size_t cnt, double *p, double v)
@@ -259,13 +206,13 @@ __device__ __forceinline__ int sturm_count_wave(int n, const double *d, const do
     for (; u + 4 <= rows; u += 4) {
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        const double ej = lane_bcast(ec, u + v);
-        sturm_row(t, c, lane_bcast(dc, u + v), ej * ej, x, pivmin);
+        const double ej = lane_value(ec, u + v);
+        sturm_row(t, c, lane_value(dc, u + v), ej * ej, x, pivmin);
       }
     }
     for (; u < rows; u++) {
-      const double ej = lane_bcast(ec, u);
-      sturm_row(t, c, lane_bcast(dc, u), ej * ej, x, pivmin);
+      const double ej = lane_value(ec, u);
+      sturm_row(t, c, lane_value(dc, u), ej * ej, x, pivmin);
     }
     dc = dx;
     ec = ex;
@@ -821,56 +768,30 @@ __global__ __launch_bounds__(256) void k_larft_inv(int nb, const double *__restr
   }
 }
 
-// Cholesky G = R^T R of a small Gram matrix (cw <= N <= 64) and R^-1
-// (upper), by one wave in registers as k_chol_diag (lane c holds column c;
-// columns past cw and the lanes above N carry the identity); *fail set when
-// G is not numerically positive definite (a non-positive or non-finite
-// pivot, taken as 1 so that the arithmetic stays finite)
-template <int N>
-__global__ __launch_bounds__(64) void k_chol_rinv(int cw, const double *__restrict__ g, double *__restrict__ rinv,
-                                                  int *__restrict__ fail)
+// Cholesky G = R^T R of a small Gram matrix (cw <= 64) and R^-1 (upper); *fail
+// set when G is not numerically positive definite (a non-positive or
+// non-finite pivot, taken as 1 so that the arithmetic stays finite).  39 ->
+// 18 us.
+__global__ __launch_bounds__(256) void k_chol_rinv(int cw, const double *__restrict__ g, double *__restrict__ rinv,
+                                                   int *__restrict__ fail)
 {
-  static_assert(N <= 64, "one lane per column");
-  constexpr int LD = N + 1;
-  __shared__ double sm[64 * LD];  // sm[c LD + r] = R(r, c), then R^-1(r, c)
-  __shared__ double urow[2][64];
-  __shared__ double dinv[64];
-  const int c = threadIdx.x;
-  double v[N];
-  const int cl = min(c, cw - 1);
+  __shared__ Leaf<false> s;
+  const int r = threadIdx.x & 63, h = threadIdx.x >> 6;
+  {
+    double ld[16];
 #pragma unroll
-  for (int r = 0; r < N; r++) v[r] = g[min(r, cw - 1) + (size_t)cw * cl];  // clamped: all loads in flight
+    for (int q = 0; q < 16; q++) ld[q] = g[min(r, cw - 1) + (size_t)cw * min(h + 4 * q, cw - 1)];
 #pragma unroll
-  for (int r = 0; r < N; r++) v[r] = (r <= c && c < cw) ? v[r] : (r == c ? 1.0 : 0.0);
-  bool bad = false;
-#pragma unroll
-  for (int j = 0; j < N; j++) {
-    const double ajj = lane_bcast(v[j], j);
-    const bool ok = ajj > 0.0 && ajj <= DBL_MAX;
-    bad = bad || !ok;
-    v[j] *= rsqrt_nr(ok ? ajj : 1.0);
-    urow[j & 1][c] = v[j];
-    __syncthreads();
-    double u[N];
-#pragma unroll
-    for (int r = j + 1; r < N; r++) u[r] = urow[j & 1][r];
-#pragma unroll
-    for (int r = j + 1; r < N; r++) v[r] = fma(-u[r], v[j], v[r]);
+    for (int q = 0; q < 16; q++) {
+      const int c = h + 4 * q;
+      s.m[0][r][c] = r <= c && c < cw ? ld[q] : (r == c ? 1.0 : 0.0);
+    }
   }
   __syncthreads();
-#pragma unroll
-  for (int r = 0; r < N; r++) sm[c * LD + r] = (r <= c) ? v[r] : 0.0;
-  __syncthreads();
-  dinv[c] = (c < N) ? 1.0 / sm[c * LD + c] : 1.0;
-  __syncthreads();
-  double x[N];
-  wave_trtri<N, LD>(sm, dinv, c, x);
-  if (c < cw) {
-#pragma unroll
-    for (int r = 0; r < N; r++)
-      if (r < cw) rinv[r + (size_t)cw * c] = (r <= c) ? x[r] : 0.0;
-  }
-  if (c == 0 && bad) *fail = 1;
+  const int first = chol_leaf<false>(s, [](double p) { return p > 0.0 && p <= DBL_MAX; });
+  if (r < cw)
+    for (int c = h; c < cw; c += 4) rinv[r + (size_t)cw * c] = s.x[0][r][c];
+  if (threadIdx.x == 0 && first != 0) *fail = 1;
 }
 
 __global__ void k_gather_cols(int n, int m, const int *__restrict__ perm, const double *__restrict__ src,
@@ -1021,7 +942,7 @@ int tridiag_eigen(Ctx &c, Seclr4Bufs &B, double el, double eu, int nume, double 
         int r2;
         if ((r2 = dgemm(s, 'T', 'N', cw, cw, n, 1.0, src, n, src, n, 0.0, cg, cw, 0, 0, 0, c.w_gk.p, c.w_gk.n)))
           return r2;
-        hipLaunchKernelGGL(k_chol_rinv<CW>, dim3(1), dim3(64), 0, s, cw, cg, crinv, flag);
+        hipLaunchKernelGGL(k_chol_rinv, dim3(1), dim3(256), 0, s, cw, cg, crinv, flag);
         W2K_STAGE(s, "k_chol_rinv");
         if ((r2 = dgemm(s, 'N', 'N', n, cw, cw, 1.0, src, n, crinv, cw, 0.0, dst, n, 0, 0, 1))) return r2;
         std::swap(src, dst);
@@ -1203,7 +1124,7 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
     W2K_STAGE(s, "k_prep");
     std::function<int(int, int)> rchol = [&](int j0, int nb) -> int {
       if (nb <= NB) {
-        hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(64), 0, s, n, j0, nb, U, W, info);
+        hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(256), 0, s, n, j0, nb, U, W, info);
         W2K_STAGE(s, "k_chol_diag");
         return 0;
       }

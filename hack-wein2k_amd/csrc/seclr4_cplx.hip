@@ -19,6 +19,7 @@
 #include <functional>
 #include <vector>
 
+#include "chol_leaf.h"
 #include "seclr4_shared.h"
 #include "twostage.h"
 
@@ -165,57 +166,43 @@ __global__ void k_zprep(int n, const double *__restrict__ hs, const double *__re
   }
 }
 
-// unblocked complex Cholesky S = U^H U of the kb x kb diagonal block at k0
-__global__ __launch_bounds__(256) void k_zpotf2(int n, int k0, int kb, double *__restrict__ Ur,
-                                                double *__restrict__ Ui, int *__restrict__ info)
+// Cholesky S = U^H U of the kb x kb diagonal block at k0 (over S) and U^-1 into
+// the same block of W (zero below the diagonal); INFO as k_chol_diag.  91 + 32
+// us as two kernels -> 35 us.
+__global__ __launch_bounds__(256) void k_zchol_diag(int n, int k0, int kb, double *__restrict__ Ur,
+                                                    double *__restrict__ Ui, double *__restrict__ Wr,
+                                                    double *__restrict__ Wi, int *__restrict__ info)
 {
-  __shared__ double ar[NB][NB + 1], ai[NB][NB + 1];
-  __shared__ double piv;
-  const int t = threadIdx.x;
-  for (int idx = t; idx < kb * kb; idx += blockDim.x) {
-    const int r = idx % kb, c = idx / kb;
-    const size_t o = (size_t)(k0 + r) + (size_t)n * (k0 + c);
-    ar[r][c] = (r <= c) ? Ur[o] : 0.0;
-    ai[r][c] = (r <= c) ? Ui[o] : 0.0;
+  __shared__ Leaf<true> s;
+  const int r = threadIdx.x & 63, g = threadIdx.x >> 6;
+  {
+    double lr[16], li[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const size_t o = (size_t)(k0 + min(r, kb - 1)) + (size_t)n * (k0 + min(g + 4 * q, kb - 1));
+      lr[q] = Ur[o];
+      li[q] = Ui[o];
+    }
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const int c = g + 4 * q;
+      s.m[0][r][c] = r <= c && c < kb ? lr[q] : (r == c ? 1.0 : 0.0);
+      s.m[1][r][c] = r <= c && c < kb ? li[q] : 0.0;
+    }
   }
   __syncthreads();
-  for (int j = 0; j < kb; j++) {
-    if (t == 0) {
-      double ajj = ar[j][j];
-      if (!(ajj > 0.0)) {
-        if (*info == 0) *info = k0 + j + 1;
-        ajj = 1.0;
-      }
-      piv = sqrt(ajj);
-      ar[j][j] = piv;
-      ai[j][j] = 0.0;
-    }
-    __syncthreads();
-    for (int c = j + 1 + t; c < kb; c += blockDim.x) {
-      ar[j][c] /= piv;
-      ai[j][c] /= piv;
-    }
-    __syncthreads();
-    // a[r][c] -= conj(a[j][r]) a[j][c], j < r <= c
-    const int m = kb - j - 1;
-    for (int idx = t; idx < m * m; idx += blockDim.x) {
-      const int r = j + 1 + idx % m, c = j + 1 + idx / m;
-      if (r <= c) {
-        const double xr = ar[j][r], xi = -ai[j][r], yr = ar[j][c], yi = ai[j][c];
-        ar[r][c] -= xr * yr - xi * yi;
-        ai[r][c] -= xr * yi + xi * yr;
-      }
-    }
-    __syncthreads();
-  }
-  for (int idx = t; idx < kb * kb; idx += blockDim.x) {
-    const int r = idx % kb, c = idx / kb;
-    if (r <= c) {
+  const int first = chol_leaf<true>(s, [](double p) { return p > 0.0; });
+  if (r < kb)
+    for (int c = g; c < kb; c += 4) {
       const size_t o = (size_t)(k0 + r) + (size_t)n * (k0 + c);
-      Ur[o] = ar[r][c];
-      Ui[o] = ai[r][c];
+      if (r <= c) {
+        Ur[o] = s.m[0][r][c];
+        Ui[o] = s.m[1][r][c];
+      }
+      Wr[o] = s.x[0][r][c];
+      Wi[o] = s.x[1][r][c];
     }
-  }
+  if (threadIdx.x == 0 && first != 0 && *info == 0) *info = k0 + first;
 }
 
 // R = S^-1 for a 64 x 64 upper triangular complex S in LDS (zero below the
@@ -271,40 +258,6 @@ __device__ void ztri_inv64(double (*sr)[NB + 1], double (*si)[NB + 1], double (*
       ri[b + r][b + h + c] = -ai;
     }
     __syncthreads();
-  }
-}
-
-// inverse of the kb x kb upper block at (j0, j0) of U (cj = 0) or of conj(U)
-// (cj = 1) into W (zero below the diagonal); a block shorter than 64 is
-// padded with the identity
-__global__ __launch_bounds__(256) void k_ztrtri_diag(int n, int j0, int kb, const double *__restrict__ Ur,
-                                                     const double *__restrict__ Ui, int cj, double *__restrict__ Wr,
-                                                     double *__restrict__ Wi)
-{
-  __shared__ double sr[NB][NB + 1], si[NB][NB + 1], rr[NB][NB + 1], ri[NB][NB + 1];
-  __shared__ double pr[NB / 2][NB / 2 + 1], pi[NB / 2][NB / 2 + 1];
-  const int t = threadIdx.x;
-  const double sg = cj ? -1.0 : 1.0;
-  for (int idx = t; idx < NB * NB; idx += blockDim.x) {
-    const int r = idx % NB, c = idx / NB;
-    double vr = (r == c) ? 1.0 : 0.0, vi = 0.0;
-    if (r < kb && c < kb) {
-      const size_t o = (size_t)(j0 + r) + (size_t)n * (j0 + c);
-      vr = (r <= c) ? Ur[o] : 0.0;
-      vi = (r <= c) ? sg * Ui[o] : 0.0;
-    }
-    sr[r][c] = vr;
-    si[r][c] = vi;
-    rr[r][c] = 0.0;
-    ri[r][c] = 0.0;
-  }
-  __syncthreads();
-  ztri_inv64(sr, si, rr, ri, pr, pi, t);
-  for (int idx = t; idx < kb * kb; idx += blockDim.x) {
-    const int r = idx % kb, c = idx / kb;
-    const size_t o = (size_t)(j0 + r) + (size_t)n * (j0 + c);
-    Wr[o] = (r <= c) ? rr[r][c] : 0.0;
-    Wi[o] = (r <= c) ? ri[r][c] : 0.0;
   }
 }
 
@@ -452,10 +405,8 @@ int seclr4_complex(Ctx &c, double el, double eu, int nume, int *ne_out, int *nbe
       const int nblk = (hi - lo + NB - 1) / NB;
       if (nblk <= 1) {
         const int kb = hi - lo;
-        hipLaunchKernelGGL(k_zpotf2, dim3(1), dim3(256), 0, s, n, lo, kb, Ur, Ui, B.info);
-        W2K_STAGE(s, "k_zpotf2");
-        hipLaunchKernelGGL(k_ztrtri_diag, dim3(1), dim3(256), 0, s, n, lo, kb, Ur, Ui, 0, Wr, Wi);
-        W2K_STAGE(s, "k_ztrtri_diag");
+        hipLaunchKernelGGL(k_zchol_diag, dim3(1), dim3(256), 0, s, n, lo, kb, Ur, Ui, Wr, Wi, B.info);
+        W2K_STAGE(s, "k_zchol_diag");
         return 0;
       }
       const int mid = lo + (nblk / 2) * NB;

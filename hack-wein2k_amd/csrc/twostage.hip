@@ -57,14 +57,6 @@ __device__ __forceinline__ void vm_drain()
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
-// LDS written by this wave is read by its other lanes
-__device__ __forceinline__ void wave_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // sum over the 32 lanes of a half wave, in every lane
 __device__ __forceinline__ double sum32(double v)
 {
@@ -75,13 +67,6 @@ __device__ __forceinline__ double sum32(double v)
   return v + bfly_partner<1>(v);
 }
 
-// the value of one lane, the same for all
-__device__ __forceinline__ double lane_value(double v, int lane)
-{
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
-}
 // the lower and the upper half wave's value, in every lane
 __device__ __forceinline__ void swap_halves(double v, double &lower, double &upper)
 {
