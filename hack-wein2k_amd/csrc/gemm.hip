@@ -150,8 +150,8 @@ __device__ __forceinline__ void tile_at(int id, int mt, int nt, int tri, bool sp
 // the triangle of op(B) in terms of its columns
 __device__ __forceinline__ int btri_mode(int btri) { return btri == 1 ? 2 : btri == 2 ? 1 : 0; }
 
-template <bool SPLIT, int TA, int TB>
-__global__ __launch_bounds__(256) void k_dgemm(GemmArgs g)
+template <bool SPLIT, bool DEEP, int TA, int TB>
+__global__ __launch_bounds__(256, 2) void k_dgemm(GemmArgs g)
 {
   __shared__ double As[2][BK][BM + PAD];
   __shared__ double Bs[2][BK][BN + PAD];
@@ -201,45 +201,78 @@ __global__ __launch_bounds__(256) void k_dgemm(GemmArgs g)
   Slab<!TB, BN> sb;
   sa.init(g.lda, i0, g.m);
   sb.init(g.ldb, j0, g.n);
-  double ra[4], rb[4];
-  auto gload = [&](int k0) {
-    const double *pa = sa.base(g.A, g.lda, i0, k0), *pb = sb.base(g.B, g.ldb, j0, k0);
-    if (sa.whole(i0, k0, kend, g.atri) && sb.whole(j0, k0, kend, bmode)) {
-      sa.load(pa, ra);
-      sb.load(pb, rb);
+  // A slab's MFMAs are shorter than its way from memory.  Where few work-groups
+  // share a CU (DEEP), slabs are asked for two ahead
+  struct Regs {
+    double a[4], b[4];
+  };
+  auto whole = [&](int k0) { return sa.whole(i0, k0, kend, g.atri) && sb.whole(j0, k0, kend, bmode); };
+  auto load = [&](int k0, Regs &x) {
+    sa.load(sa.base(g.A, g.lda, i0, k0), x.a);
+    sb.load(sb.base(g.B, g.ldb, j0, k0), x.b);
+  };
+  auto load_any = [&](int k0, Regs &x) {
+    if (whole(k0)) {
+      load(k0, x);
     } else {
-      sa.load_part(g.A, g.lda, i0, g.m, k0, kend, g.atri, ra);
-      sb.load_part(g.B, g.ldb, j0, g.n, k0, kend, bmode, rb);
+      sa.load_part(g.A, g.lda, i0, g.m, k0, kend, g.atri, x.a);
+      sb.load_part(g.B, g.ldb, j0, g.n, k0, kend, bmode, x.b);
     }
   };
-  auto sstore = [&](int buf) {
-    sa.store(&As[buf][0][0], BM + PAD, ra);
-    sb.store(&Bs[buf][0][0], BN + PAD, rb);
+  auto sstore = [&](int buf, const Regs &x) {
+    sa.store(&As[buf][0][0], BM + PAD, x.a);
+    sb.store(&Bs[buf][0][0], BN + PAD, x.b);
+  };
+  auto products = [&](int buf) {
+#pragma unroll
+    for (int kq = 0; kq < BK; kq += 4) {
+      double av[2], bv[2];
+      for (int a = 0; a < 2; a++) av[a] = As[buf][kq + lk][wi + 16 * a + li];
+      for (int b = 0; b < 2; b++) bv[b] = Bs[buf][kq + lk][wj + 16 * b + li];
+      for (int a = 0; a < 2; a++)
+        for (int b = 0; b < 2; b++)
+          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[b], av[a], acc[a][b], 0, 0, 0);
+    }
   };
 
   if (kbeg < kend) {
-    gload(kbeg);
-    sstore(0);
+    Regs x, y;
+    int buf = 0, k = kbeg;  // the slab in LDS
+    load_any(k, x);
+    sstore(0, x);
     __syncthreads();
-    int buf = 0;
-    for (int k0 = kbeg; k0 < kend; k0 += BK) {
-      const bool more = (k0 + BK < kend);
-      if (more) gload(k0 + BK);
-#pragma unroll
-      for (int kq = 0; kq < BK; kq += 4) {
-        double av[2], bv[2];
-        for (int a = 0; a < 2; a++) av[a] = As[buf][kq + lk][wi + 16 * a + li];
-        for (int b = 0; b < 2; b++) bv[b] = Bs[buf][kq + lk][wj + 16 * b + li];
-        for (int a = 0; a < 2; a++)
-          for (int b = 0; b < 2; b++)
-            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[b], av[a], acc[a][b], 0, 0, 0);
-      }
-      if (more) {
-        sstore(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
+    auto advance = [&](const Regs &x) {
+      products(buf);
+      sstore(buf ^ 1, x);
+      __syncthreads();
+      buf ^= 1;
+      k += BK;
+    };
+    while (k + BK < kend) {
+      if (DEEP && whole(k + BK) && whole(k + 2 * BK)) {
+        // nothing conditional between a slab's loads and their use: the wait
+        // for a slab is then not one for the slab after it
+        load(k + BK, x);
+        for (;;) {
+          if (!whole(k + 2 * BK)) {
+            advance(x);
+            break;
+          }
+          load(k + 2 * BK, y);
+          advance(x);
+          if (!whole(k + 2 * BK)) {
+            advance(y);
+            break;
+          }
+          load(k + 2 * BK, x);
+          advance(y);
+        }
+      } else {
+        load_any(k + BK, x);
+        advance(x);
       }
     }
+    products(buf);
   }
   // epilogue: an MFMA result has rows lane/16 + 4r (r = 0..3), column lane%16
   // of each 16x16 block; with op(B) as the first operand these are columns and
@@ -760,13 +793,25 @@ bool tuning_on()
 }
 }  // namespace
 
+template <bool SPLIT, bool DEEP>
+static void launch_dgemm_as(hipStream_t s, const GemmArgs &g, dim3 grid)
+{
+  if (!g.ta && !g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, DEEP, 0, 0>), grid, dim3(256), 0, s, g);
+  else if (g.ta && !g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, DEEP, 1, 0>), grid, dim3(256), 0, s, g);
+  else if (!g.ta && g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, DEEP, 0, 1>), grid, dim3(256), 0, s, g);
+  else hipLaunchKernelGGL((k_dgemm<SPLIT, DEEP, 1, 1>), grid, dim3(256), 0, s, g);
+}
+// Slabs two ahead up to two work-groups a CU and from eight slabs on: 200^3 18.2
+// -> 14.8 us; with more work-groups the
+// registers cost more than the waits (lower triangle of 5951, K = 64 79 -> 93
+// us; one ahead 69), and with few slabs there is nothing to run ahead of (64 x 731 x 64 7.2
+// -> 9.0 us)
 template <bool SPLIT>
 static void launch_dgemm(hipStream_t s, const GemmArgs &g, dim3 grid)
 {
-  if (!g.ta && !g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, 0, 0>), grid, dim3(256), 0, s, g);
-  else if (g.ta && !g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, 1, 0>), grid, dim3(256), 0, s, g);
-  else if (!g.ta && g.tb) hipLaunchKernelGGL((k_dgemm<SPLIT, 0, 1>), grid, dim3(256), 0, s, g);
-  else hipLaunchKernelGGL((k_dgemm<SPLIT, 1, 1>), grid, dim3(256), 0, s, g);
+  const int slabs = ((SPLIT ? g.kslice : g.k) + BK - 1) / BK;
+  if ((long)grid.x * grid.z <= 512 && slabs >= 8) launch_dgemm_as<SPLIT, true>(s, g, grid);
+  else launch_dgemm_as<SPLIT, false>(s, g, grid);
 }
 
 // variant 0: 64x64 tiles, 1: 128x128 tiles
