@@ -10,12 +10,17 @@
 //                loops 230 (hamilt.F:386-424) times (2l+1)*VIFPR4
 //   k_hamilt_pw  the pair loop 260.  One wave = 64 rows x C columns.  The
 //                Legendre polynomials of its pairs stay in registers, the
-//                per-column coefficients are wave-uniform (scalar loads), the
-//                per-row tables (AL, BL, cos/sin) are coalesced vector loads.
+//                per-column coefficients of a type are spread over the wave's
+//                lanes (one coalesced load, a type ahead) and handed out by
+//                readlane, the per-row tables (AL, BL, cos/sin) are coalesced
+//                vector loads.  With scalar loads for the coefficients the
+//                waits for them bound the kernel: 100 atoms, N = 3461 6.5 ->
+//                3.9 ms, 64 atoms, N = 5684 9.3 -> 6.4 ms.
 //                The step function Theta(G_J-G_I) (loops 160-180) is summed per
 //                group of equal sphere radii, so the pair loop evaluates one
 //                sincos per distinct RMT rather than one per atom.
 //   k_hamilt_lo  the LO columns (hamilt.F:475-815), one thread per (row, LO column)
+#include "mfma.h"
 #include "special.h"
 #include "w2k_internal.h"
 
@@ -195,6 +200,22 @@ __global__ __launch_bounds__(256) void k_hamilt_pw(PwArgs g)
     thr[c] = 0.0; thi[c] = 0.0;
   }
 
+  // the wave's 4 LT C column coefficients of a type, spread over its lanes, a
+  // type ahead; handed out by readlane
+  constexpr int NCF = 4 * LT * C, NU = (NCF + 63) / 64;
+  unsigned cfo[NU];
+  double cfc[NU], cfn[NU];
+#pragma unroll
+  for (int u = 0; u < NU; u++) {
+    const int k = min(lane + 64 * u, NCF - 1), c = k / 4 % C;
+    cfo[u] = ((unsigned)(k / (4 * C)) * g.nv + (i0 + c < g.nv ? i0 + c : i0)) * 4 + k % 4;
+  }
+  auto fetch = [&](int a) {
+    const double *cf = g.coef + (size_t)a * g.lt * g.nv * 4;
+#pragma unroll
+    for (int u = 0; u < NU; u++) cfn[u] = cf[cfo[u]];
+  };
+  fetch(g.aorder[0]);
   int pa = 0;
   for (int gi = 0; gi < g.ngrp; gi++) {
     const int pend = g.grp_end[gi];
@@ -203,6 +224,9 @@ __global__ __launch_bounds__(256) void k_hamilt_pw(PwArgs g)
     for (int c = 0; c < C; c++) { pr[c] = 0.0; pim[c] = 0.0; }
     for (; pa < pend; pa++) {
       const int a = g.aorder[pa];
+#pragma unroll
+      for (int u = 0; u < NU; u++) cfc[u] = cfn[u];
+      fetch(g.aorder[min(pa + 1, g.nat - 1)]);
       // phase factors PHASE(J,a) = sum_eq exp(2 pi i (G_J - G_I).tau), hamilt.F:199-243
       double phr[C], phi[C];
 #pragma unroll
@@ -227,15 +251,14 @@ __global__ __launch_bounds__(256) void k_hamilt_pw(PwArgs g)
       for (int c = 0; c < C; c++) { t1[c] = 0.0; t2[c] = 0.0; }
       const double *alr = g.al + (size_t)n * g.lt * a;
       const double *blr = g.bl + (size_t)n * g.lt * a;
-      const double *cf = g.coef + (size_t)a * g.lt * g.nv * 4;
 #pragma unroll
       for (int l = 0; l < LT; l++) {
         const double aj = alr[(size_t)n * l + jj], bj = blr[(size_t)n * l + jj];
-        const double *cl = cf + ((size_t)l * g.nv + i0) * 4;
 #pragma unroll
         for (int c = 0; c < C; c++) {
-          const int cc = (i0 + c < g.nv) ? c : 0;
-          const double sa = cl[4 * cc], sb = cl[4 * cc + 1], ha = cl[4 * cc + 2], hb = cl[4 * cc + 3];
+          const int k = 4 * (C * l + c);
+          const double sa = lane_value(cfc[k / 64], k % 64), sb = lane_value(cfc[(k + 1) / 64], (k + 1) % 64);
+          const double ha = lane_value(cfc[(k + 2) / 64], (k + 2) % 64), hb = lane_value(cfc[(k + 3) / 64], (k + 3) % 64);
           t2[c] += P[c][l] * (aj * sa + bj * sb);
           t1[c] += P[c][l] * (aj * ha + bj * hb);
         }
@@ -408,15 +431,23 @@ __global__ __launch_bounds__(256) void k_hamilt_lo(LoArgs g)
 }
 
 // ------------------------------------------------------------------ driver
+template <int LT, int C, bool CPX>
+static void launch_pw_as(const PwArgs &a, hipStream_t s)
+{
+  const dim3 grid((a.nv + 63) / 64, (a.nv + 4 * C - 1) / (4 * C));
+  hipLaunchKernelGGL((k_hamilt_pw<LT, C, CPX>), grid, dim3(256), 0, s, a);
+}
+
+// Columns per wave: with four a wave's row loads serve more pairs, with two
+// there are more waves.  Complex C = 2 -> 4: 100 atoms, N = 3461 4.2 -> 3.9 ms, 8
+// atoms, N = 1951 0.15 -> 0.17 ms; real C = 3 -> 4: 64 atoms, N = 5684 7.1 -> 6.4
+// ms, small cells alike
 template <int LT, bool CPX>
 static void launch_pw(const PwArgs &a, hipStream_t s)
 {
-  // columns per wave: the largest count whose registers still allow three
-  // waves per SIMD (measured on the 64-atom cell: C = 3 takes 9.4 ms, C = 4
-  // at two waves per SIMD 13.3 ms)
-  constexpr int C = CPX ? 2 : 3;
-  dim3 grid((a.nv + 63) / 64, (a.nv + 4 * C - 1) / (4 * C));
-  hipLaunchKernelGGL((k_hamilt_pw<LT, C, CPX>), grid, dim3(256), 0, s, a);
+  if constexpr (CPX)
+    if (a.nv < 2560) return launch_pw_as<LT, 2, CPX>(a, s);
+  launch_pw_as<LT, 4, CPX>(a, s);
 }
 
 template <bool CPX>
