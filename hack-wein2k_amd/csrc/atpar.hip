@@ -509,8 +509,9 @@ int atpar(Ctx &c, const w2k_radial_desc *rd, double *const out[16])
       loor[a * W2K_LOMAXP + l] = R.loor[l + W2K_LOMAXP * a] ? 1 : 0;
       if (il > 0) elo[a * W2K_LOMAXP + l] = R.elo[l + W2K_LOMAXP * ((il - 1) + W2K_NLOAT * (size_t)a)];
     }
-  DBuf<double> d_vr, d_e, d_elo, d_work, d_out, d_outlo;
-  DBuf<int> d_loor;
+  DBuf<double> &d_vr = c.at_d[0], &d_e = c.at_d[1], &d_elo = c.at_d[2], &d_work = c.at_d[3], &d_out = c.at_d[4];
+  DBuf<double> &d_outlo = c.at_d[5];
+  DBuf<int> &d_loor = c.at_i[0];
   if ((rc = put(R.d_at_jrj, rd->jrj, nat, s)) || (rc = put(R.d_at_ro, rd->ro, nat, s)) ||
       (rc = put(R.d_at_dh, rd->dh, nat, s)) || (rc = put(R.d_at_zz, rd->zz, nat, s)) ||
       (rc = put(d_vr, rd->vr, (size_t)jrid * nat, s)) || (rc = put(d_e, R.e.data(), R.e.size(), s)) ||
@@ -521,8 +522,8 @@ int atpar(Ctx &c, const w2k_radial_desc *rd, double *const out[16])
       (rc = d_work.alloc((size_t)nat * nt * AT_ROWS * jrid)) ||
       (rc = d_out.alloc((size_t)nat * nt * 6)) || (rc = d_outlo.alloc((size_t)nat * W2K_LOMAXP * 4)))
     return rc;
-  W2K_HIP(hipMemsetAsync(R.d_at_fnlo.p, 0, sizeof(double) * R.d_at_fnlo.n, s));
-  W2K_HIP(hipMemsetAsync(d_outlo.p, 0, sizeof(double) * d_outlo.n, s));
+  W2K_HIP(hipMemsetAsync(R.d_at_fnlo.p, 0, sizeof(double) * nat * W2K_LOMAXP * 2 * jrid, s));
+  W2K_HIP(hipMemsetAsync(d_outlo.p, 0, sizeof(double) * nat * W2K_LOMAXP * 4, s));
   AtparArgs g = atpar_args(R);
   g.vr = d_vr.p;
   g.e = d_e.p;
@@ -542,8 +543,8 @@ int atpar(Ctx &c, const w2k_radial_desc *rd, double *const out[16])
   std::vector<double> vres;
   if (rd->vlm && !R.hns_terms.empty()) {
     trip = vns_triples(R);
-    DBuf<int> d_trip;
-    DBuf<double> d_vlm, d_res;
+    DBuf<int> &d_trip = c.at_i[1];
+    DBuf<double> &d_vlm = c.at_d[6], &d_res = c.at_d[7];
     if ((rc = put(d_trip, reinterpret_cast<const int *>(trip.data()), trip.size() * 4, s)) ||
         (rc = put(d_vlm, rd->vlm, (size_t)jrid * rd->lmmxd * nat, s)) || (rc = d_res.alloc(trip.size() * 6)))
       return rc;

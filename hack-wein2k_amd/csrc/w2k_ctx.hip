@@ -425,6 +425,8 @@ void drop_kpoint_state(Ctx &c)
                           &c.w_b, &c.w_c, &c.w_v, &c.w_x, &c.w_small, &c.w_fac, &c.w_bt, &c.w_cl, &c.w_gk, &c.w_3m,
                           &c.w_sb, &c.w_frag};
   for (DBuf<double> *b : bufs) b->release();
+  for (DBuf<double> &b : c.at_d) b.release();
+  for (DBuf<int> &b : c.at_i) b.release();
   c.d_kzz.release();
   c.w_int.release();
   c.w_piv.release();

@@ -184,6 +184,10 @@ struct Ctx {
   DBuf<double> w_gk;    // split-K GEMM partial products
   DBuf<double> w_sb;    // two-stage tridiagonalisation: panel sums, band, reflector scalars
   DBuf<int> w_sbi;      // its progress and registration words
+  // ATPAR: potential, energies (two), work rows, results (two), V_LM, integrals;
+  // LO flags, coupling triples
+  DBuf<double> at_d[8];
+  DBuf<int> at_i[2];
   DBuf<double> w_frag;  // operands of the second stage's reflector blocks
   DBuf<double> w_3m;    // three-product complex GEMM: Re + Im of both operands, one real product
   // launch mode of the tridiagonalisation, chosen per shape by measurement:
