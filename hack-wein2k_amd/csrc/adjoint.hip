@@ -63,28 +63,63 @@ __global__ void k_adj_kzz_index(int nv, const int *__restrict__ kzz, int lx, int
   idx[x + dx * (y + dy * z)] = i;
 }
 
-// one thread per box entry Q: its (I, J) pairs summed in order of I
-__global__ void k_adj_warp_grad(int nv, const int *__restrict__ kzz, const int *__restrict__ idx, int lx, int ly,
-                                int lz, int dx, int dy, int dz, int w1, int w2, int w3, int cpx,
-                                const double *__restrict__ gr, const double *__restrict__ gi, double *__restrict__ g)
+// The pairs (I, J) of a box entry Q, summed over I.  A block takes 64 entries;
+// its waves take a contiguous slice of I each, and the first wave adds the
+// slices in a fixed order.  Bound by latency: one thread walking all I has one
+// chain of three dependent loads (KZZ, index, Gamma) per I and a box of some
+// thousand entries fills a fraction of the CUs.  With slices and four I in
+// flight per thread: N = 216 83 -> 11 us, 1950 1107 -> 114, 5695 2901 -> 563,
+// 10480 (complex) 9.90 -> 2.67 ms.  At the large orders what is left is the
+// reads of Gamma, 8 scattered bytes each: neighbouring entries pair a row with
+// columns that lie anywhere in the basis.
+constexpr int kWarpSlices = 16;
+__global__ void __launch_bounds__(64 * kWarpSlices)
+    k_adj_warp_grad(int nv, const int *__restrict__ kzz, const int *__restrict__ idx, int lx, int ly, int lz, int dx,
+                    int dy, int dz, int w1, int w2, int w3, int cpx, const double *__restrict__ gr,
+                    const double *__restrict__ gi, double *__restrict__ g)
 {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n1 = 2 * w1 + 1, n2 = 2 * w2 + 1, n3 = 2 * w3 + 1;
-  if (b >= n1 * n2 * n3) return;
-  const int qx = b % n1 - w1, qy = (b / n1) % n2 - w2, qz = b / (n1 * n2) - w3;
+  __shared__ double sr[kWarpSlices][64], si[kWarpSlices][64];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int n1 = 2 * w1 + 1, n2 = 2 * w2 + 1, n3 = 2 * w3 + 1, nbox = n1 * n2 * n3;
+  const int b = blockIdx.x * 64 + lane, q = b < nbox ? b : nbox - 1;
+  const int qx = q % n1 - w1 - lx, qy = (q / n1) % n2 - w2 - ly, qz = q / (n1 * n2) - w3 - lz;
+  const int per = (nv + kWarpSlices - 1) / kWarpSlices, i0 = w * per, i1 = min(i0 + per, nv);
   double ar = 0.0, ai = 0.0;
-  for (int I = 0; I < nv; I++) {
-    const int x = kzz[3 * I] + qx - lx, y = kzz[3 * I + 1] + qy - ly, z = kzz[3 * I + 2] + qz - lz;
-    if (x < 0 || y < 0 || z < 0 || x >= dx || y >= dy || z >= dz) continue;
-    const int J = idx[x + dx * (y + dy * z)];
-    if (J < 0 || J > I) continue;
-    const size_t o = (size_t)I + (size_t)nv * J;
-    if (J < I) {
-      ar += 2.0 * gr[o];
-      if (cpx) ai -= 2.0 * gi[o];
-    } else {
-      ar += gr[o];  // diagonal: the solver reads its real part only
+  for (int i = i0; i < i1; i += 4) {
+    int J[4];
+    double vr[4], vi[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int I = min(i + u, nv - 1);
+      const int x = kzz[3 * I] + qx, y = kzz[3 * I + 1] + qy, z = kzz[3 * I + 2] + qz;
+      const bool in = x >= 0 && y >= 0 && z >= 0 && x < dx && y < dy && z < dz && i + u < i1;
+      const int k = idx[in ? x + dx * (y + dy * z) : 0];
+      J[u] = in && k <= I ? k : -1;
     }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const size_t o = J[u] >= 0 ? (size_t)(i + u) + (size_t)nv * J[u] : 0;
+      vr[u] = J[u] >= 0 ? gr[o] : 0.0;
+      vi[u] = cpx && J[u] >= 0 ? gi[o] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (J[u] < 0) continue;
+      if (J[u] < i + u) {
+        ar += 2.0 * vr[u];
+        ai -= 2.0 * vi[u];
+      } else {
+        ar += vr[u];  // diagonal: the solver reads its real part only
+      }
+    }
+  }
+  sr[w][lane] = ar;
+  si[w][lane] = ai;
+  __syncthreads();
+  if (w != 0 || b >= nbox) return;
+  for (int k = 1; k < kWarpSlices; k++) {
+    ar += sr[k][lane];
+    ai += si[k][lane];
   }
   g[2 * b] = ar;
   g[2 * b + 1] = ai;
@@ -173,7 +208,7 @@ int adjoint_warp_box(Ctx &c, const double *f_host, double *e_band, const double 
                      dy, c.w_int.p);
   W2K_STAGE(s, "k_adj_kzz_index");
   if ((rc = c.w_c.alloc(2 * nbox))) return rc;
-  hipLaunchKernelGGL(k_adj_warp_grad, dim3((unsigned)((nbox + 127) / 128)), dim3(128), 0, s, nv, c.d_kzz.p,
+  hipLaunchKernelGGL(k_adj_warp_grad, dim3((unsigned)((nbox + 63) / 64)), dim3(64 * kWarpSlices), 0, s, nv, c.d_kzz.p,
                      c.w_int.p, lo[0], lo[1], lo[2], dx, dy, dz, w1, w2, w3, cpx, Gr, cpx ? Gi : Gr, c.w_c.p);
   W2K_STAGE(s, "k_adj_warp_grad");
   *d_box = c.w_c.p;
