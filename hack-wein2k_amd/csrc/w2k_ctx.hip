@@ -20,6 +20,8 @@
 // the process).  Host code never names it except to look up its device
 // address once per device (noalloc_scratch_init); the kernels receive that
 // address through the workspaces carved from it.
+// The two-stage tridiagonalisation's work rows, operands and blocked vectors
+// bring a complex order of 768 with all its vectors to 145 MB (noalloc_bytes).
 static __device__ __align__(256) unsigned char scratch[W2K_NOALLOC_SCRATCH_BYTES];
 
 namespace w2k {
