@@ -51,17 +51,23 @@ __device__ __forceinline__ int chol_leaf(Leaf<CX> &s, OK ok)
 #pragma unroll 1
   for (int kb = 0; kb < 4; kb++) {
     const int r0 = 16 * kb;
+    // lanes base .. base + 15 hold the diagonal block's columns
+    const int base = w == 0 ? r0 : 0;
+    double v[16], vi[CX ? 16 : 1];
     if (w < 2) {
-      // lanes base .. base + 15 hold the diagonal block's columns
-      const int base = w == 0 ? r0 : 0, col = w == 0 ? lane : r0 + l16;
+      const int col = w == 0 ? lane : r0 + l16;
       const bool unit = w == 1 && lane >= 16;
-      double v[16], vi[CX ? 16 : 1];
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const double a = s.m[0][r0 + r][col], b = CX ? s.m[CP - 1][r0 + r][col] : 0.0;
         v[r] = unit ? (r == l16 ? 1.0 : 0.0) : a;
         if (CX) vi[r] = unit ? 0.0 : b;
       }
+    }
+    // the second wave has its copy of the diagonal block before the first one
+    // puts U over it
+    __syncthreads();
+    if (w < 2) {
 #pragma unroll
       for (int j = 0; j < 16; j++) {
         const double ajj = lane_value(v[j], base + j);

@@ -117,7 +117,7 @@ __device__ __forceinline__ void wave_trtri(const double *sm, const double *dinv,
 // the inverse of its factor: U over the block of a, U^-1 into the same block
 // of w (zeros below the diagonal).  A non-positive pivot sets *info = k0 + j +
 // 1 for the first such j (DPOTRF's INFO) and is taken as 1 so that the
-// arithmetic stays finite.  38 -> 20 us.
+// arithmetic stays finite.  38 -> 21 us.
 __global__ __launch_bounds__(256) void k_chol_diag(int n, int k0, int kb, double *__restrict__ a,
                                                    double *__restrict__ w, int *__restrict__ info)
 {

@@ -5,7 +5,11 @@
 // has returned.  A wave operation runs once every live lane of the wave waits
 // at it (lanes that returned do not take part, like lanes outside EXEC); a
 // barrier releases once every live work-item of the block waits at it.  A
-// block in which neither can happen is reported as a deadlock.
+// block in which neither can happen is reported as a deadlock.  The waves of a
+// block go in step by default; with W2K_EMU_WAVES=up (down) each runs as far as
+// it can, to a barrier or its end, before the wave after (before) it starts, so
+// that LDS or memory that waves share with no barrier between them holds what
+// the one that ran ahead left.
 //
 // Device memory: every allocation gets its own mapping, with the buffer placed
 // against a PROT_NONE guard page (its end by default, its start with
@@ -302,38 +306,64 @@ void do_waveop(BlockRun &b, int w0, int wn)
     if (L[q]) L[q]->state = READY;
 }
 
+// every ready work-item of [t0, t1) runs until it waits or returns
+void run_ready(BlockRun &b, int t0, int t1)
+{
+  for (int t = t0; t < t1; t++) {
+    Fiber &f = b.f[t];
+    if (f.state != READY) continue;
+    b.running = &f;
+    cur = &f.item;
+    g_fault_tid[0] = f.item.tid.x;
+    g_fault_tid[1] = f.item.tid.y;
+    g_fault_tid[2] = f.item.tid.z;
+    emu_switch(&b.sched_sp, f.sp);
+  }
+  b.running = nullptr;
+  cur = nullptr;
+}
+
+// the wave operation of the wave at w0, if its live lanes all wait at one
+bool run_waveop(BlockRun &b, int w0)
+{
+  const int wn = std::min(64, b.nthreads - w0);
+  int live = 0, wait = 0;
+  for (int q = 0; q < wn; q++) {
+    const int s = b.f[w0 + q].state;
+    if (s != DONE) live++;
+    if (s == WAVEOP) wait++;
+  }
+  if (live == 0 || wait != live) return false;
+  do_waveop(b, w0, wn);
+  return true;
+}
+
+// order of a block's waves between barriers: 0 in step, 1 up, -1 down
+int wave_order()
+{
+  static const int o = [] {
+    const char *e = getenv("W2K_EMU_WAVES");
+    return !e ? 0 : strcmp(e, "up") == 0 ? 1 : strcmp(e, "down") == 0 ? -1 : 0;
+  }();
+  return o;
+}
+
 void run_block(BlockRun &b)
 {
+  const int order = wave_order(), nwave = (b.nthreads + 63) / 64;
   for (;;) {
-    // every ready work-item runs until it waits or returns
-    for (int t = 0; t < b.nthreads; t++) {
-      Fiber &f = b.f[t];
-      if (f.state != READY) continue;
-      b.running = &f;
-      cur = &f.item;
-      g_fault_tid[0] = f.item.tid.x;
-      g_fault_tid[1] = f.item.tid.y;
-      g_fault_tid[2] = f.item.tid.z;
-      emu_switch(&b.sched_sp, f.sp);
-    }
-    b.running = nullptr;
-    cur = nullptr;
-    // wave operations whose live lanes all wait at them
-    bool op_done = false;
-    for (int w0 = 0; w0 < b.nthreads; w0 += 64) {
-      const int wn = std::min(64, b.nthreads - w0);
-      int live = 0, wait = 0;
-      for (int q = 0; q < wn; q++) {
-        const int s = b.f[w0 + q].state;
-        if (s != DONE) live++;
-        if (s == WAVEOP) wait++;
+    if (order != 0) {
+      for (int q = 0; q < nwave; q++) {
+        const int w0 = 64 * (order > 0 ? q : nwave - 1 - q);
+        do run_ready(b, w0, std::min(w0 + 64, b.nthreads));
+        while (run_waveop(b, w0));
       }
-      if (live > 0 && wait == live) {
-        do_waveop(b, w0, wn);
-        op_done = true;
-      }
+    } else {
+      run_ready(b, 0, b.nthreads);
+      bool op_done = false;
+      for (int w0 = 0; w0 < b.nthreads; w0 += 64) op_done |= run_waveop(b, w0);
+      if (op_done) continue;
     }
-    if (op_done) continue;
     int alive = 0, at_bar = 0;
     for (int t = 0; t < b.nthreads; t++) {
       if (b.f[t].state != DONE) alive++;
