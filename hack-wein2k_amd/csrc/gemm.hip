@@ -11,7 +11,8 @@
 // 32x32 block of four 16x16 MFMA accumulators.  Operands staged through LDS
 // k-major so that the MFMA operand reads (lane l -> row l%16, k l/16) are
 // bank-conflict free; LDS double-buffered so the next k-slab's global loads
-// overlap the current slab's MFMAs.
+// overlap the current slab's MFMAs.  No MFMA of these kernels accumulates onto
+// the one just before it, so that their results need no mfma_settle().
 #include <algorithm>
 #include <cstdlib>
 #include <map>

@@ -103,11 +103,11 @@ __device__ __forceinline__ void hns_alm(const HnsArgs &g, int i, int e, int a, F
 // fourth tile for all 64 rows.  Bound by the operands' stores at large sizes,
 // by the chain (Y_lm, then 25 dependent steps) at small ones; one work-item
 // per row and atom spent LINDEX NNSL^2 36 multiply-adds on scalar loads: N =
-// 3861, 100 atoms 3.25 -> 0.68 ms (0.9 GB stored), one atom 0.24 -> 0.03 ms.
+// 3861, 100 atoms 3.25 -> 0.56 ms (0.9 GB stored), one atom 0.24 -> 0.03 ms.
 constexpr int HP_ROWS = 64, HP_LD = HP_ROWS + 16;  // row length: the four parts' rows two by two on other banks
 
 template <bool CPX>
-__global__ __launch_bounds__(256) void k_hns_prep(HnsArgs g)
+__global__ __launch_bounds__(256, 2) void k_hns_prep(HnsArgs g)
 {
   __shared__ double za[W2K_NSL2][2][HP_LD];      // t of a row and lm
   __shared__ double zf[W2K_NSLMAX][3][HP_LD];    // AL, BL, CL of a row and l

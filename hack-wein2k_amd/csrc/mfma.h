@@ -7,15 +7,28 @@ namespace w2k {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-// Before FP64 MFMA results are read by another instruction: 64 clocks more
-// than the compiler leaves after the last MFMA.  It leaves 19 wait
-// states (16 passes + 3) after its issue; where that MFMA accumulates onto the
-// one just before it, whose end it has to wait for, item 3 of the result was
-// read three passes early.
+// To stand between an FP64 MFMA that accumulates onto the one just before it and
+// the first other instruction that reads its result.  The compiler leaves 19
+// wait states there (the MFMA's 16 passes and 3), counted from its issue; but it
+// may have had to wait for the one before: read 19 wait states after its issue,
+// item 3 of a result was three passes old.  36 wait states by count cover 16
+// passes of the one before, its own 16 and 3; they are enough whether or not
+// the compiler adds its own.
+//
+// An accumulator in AGPRs is copied out in front of whatever stands here: the
+// block Cholesky read its sums 19 wait states after a chain's end that way.  A
+// kernel whose launch bounds ask for two waves a SIMD (up to 256 registers a
+// lane) has its accumulators in VGPRs, if its LDS leaves room for two
+// work-groups; where it does not, the chains of two accumulators alternate.
+// Neither is the source's to promise: tests/test_mfma_waits.py checks the
+// assembly of every kernel, also of those that alternate accumulators and do
+// without this (gemm.hip).
 __device__ __forceinline__ void mfma_settle()
 {
   __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_sleep(1);
+#ifdef __AMDGCN__
+  asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 3");
+#endif
   __builtin_amdgcn_sched_barrier(0);
 }
 

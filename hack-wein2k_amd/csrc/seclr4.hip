@@ -118,7 +118,7 @@ __device__ __forceinline__ void wave_trtri(const double *sm, const double *dinv,
 // of w (zeros below the diagonal).  A non-positive pivot sets *info = k0 + j +
 // 1 for the first such j (DPOTRF's INFO) and is taken as 1 so that the
 // arithmetic stays finite.  38 -> 21 us.
-__global__ __launch_bounds__(256) void k_chol_diag(int n, int k0, int kb, double *__restrict__ a,
+__global__ __launch_bounds__(256, 2) void k_chol_diag(int n, int k0, int kb, double *__restrict__ a,
                                                    double *__restrict__ w, int *__restrict__ info)
 {
   __shared__ Leaf<false> s;
@@ -772,7 +772,7 @@ __global__ __launch_bounds__(256) void k_larft_inv(int nb, const double *__restr
 // set when G is not numerically positive definite (a non-positive or
 // non-finite pivot, taken as 1 so that the arithmetic stays finite).  39 ->
 // 18 us.
-__global__ __launch_bounds__(256) void k_chol_rinv(int cw, const double *__restrict__ g, double *__restrict__ rinv,
+__global__ __launch_bounds__(256, 2) void k_chol_rinv(int cw, const double *__restrict__ g, double *__restrict__ rinv,
                                                    int *__restrict__ fail)
 {
   __shared__ Leaf<false> s;

@@ -168,7 +168,7 @@ __global__ void k_zprep(int n, const double *__restrict__ hs, const double *__re
 
 // Cholesky S = U^H U of the kb x kb diagonal block at k0 (over S) and U^-1 into
 // the same block of W (zero below the diagonal); INFO as k_chol_diag.  91 + 32
-// us as two kernels -> 36 us.
+// us as two kernels -> 37 us.
 __global__ __launch_bounds__(256) void k_zchol_diag(int n, int k0, int kb, double *__restrict__ Ur,
                                                     double *__restrict__ Ui, double *__restrict__ Wr,
                                                     double *__restrict__ Wi, int *__restrict__ info)
