@@ -876,7 +876,8 @@ int tridiag_eigen(Ctx &c, Seclr4Bufs &B, double el, double eu, int nume, double 
   W2K_STAGE(s, "k_fill");
   // factor planes of rows 0 .. n in row pairs (16-byte aligned: m pairs per row pair)
   const size_t zp = (size_t)((n + 2) / 2) * 2 * m;
-  if ((rc = c.w_fac.alloc((size_t)5 * zp)) || (rc = c.w_piv.alloc(zp))) return rc;
+  // also room for the application of Q2, which follows
+  if ((rc = c.w_fac.alloc(std::max((size_t)5 * zp, sb_q2_doubles(n, m, B.cplx)))) || (rc = c.w_piv.alloc(zp))) return rc;
   {
     // W2K_TEST_STEIN_FAIL=1 (tests only) raises DSTEIN's growth threshold
     // out of reach, so that every vector takes the non-convergence path

@@ -25,15 +25,15 @@ struct SbArgs {
   double *tau2 = nullptr;                   // their scalars, [step][sweep]
   size_t ntau2 = 0;
   int *prog = nullptr;                      // finished steps per sweep; entry n: the next sweep
-  double *frag = nullptr;                   // operands of the Q2 blocks
+  double *frag = nullptr;                   // operands of the Q2 blocks of some groups
   double *zb = nullptr;                     // vectors between the groups of Q2, 16 columns side by side
   int *q2sync = nullptr;                    // ticket and progress of their application
 };
 
-// doubles (and ints) of the work buffers that sb_buffers carves; of the blocks
-// of Q2
+// doubles (and ints) of the work buffers that sb_buffers carves; doubles that
+// sb_apply_q2 wants in Ctx::w_fac
 size_t sb_doubles(int n, int cplx, size_t *ints);
-size_t sb_frag_doubles(int n, size_t m, int cplx);
+size_t sb_q2_doubles(int n, size_t m, int cplx);
 int sb_buffers(Ctx &c, SbArgs &g, int n, int cplx);
 // A -> tridiagonal (d, e); A keeps Q1's reflectors: column i holds v_i from
 // row i + BND + 1 on (v_i(i + BND) = 1), tau_i in taur/taui, i < n - BND - 1
@@ -41,7 +41,7 @@ int sb_reduce(Ctx &c, hipStream_t s, SbArgs &g, int cplx);
 // while kernel timing is on: the summed time of the products of the panels
 // with the trailing matrix and their number, into the context's timings
 int sb_take_times(Ctx &c, hipStream_t s, int n);
-// Z <- Q2 Z (n x m)
+// Z <- Q2 Z (n x m); overwrites the inverse iteration's factors
 int sb_apply_q2(Ctx &c, hipStream_t s, SbArgs &g, int cplx, int m, double *Zr, double *Zi, int ldz);
 
 }  // namespace w2k

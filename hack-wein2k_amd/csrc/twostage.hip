@@ -21,6 +21,7 @@
 // 1018 -> 325 (+ 84).
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 
 #include <hip/hip_ext.h>
 
@@ -1135,22 +1136,25 @@ __global__ __launch_bounds__(256 * K) void k_sb_chase(SbArgs g)
 // ------------------------------------------------------------------ 3. Q2 times vectors
 // The reflectors of BND consecutive sweeps at one step are a block I - V T V^H
 // on 2 BND - 1 rows (V a parallelogram): k_sb_frag forms V and -V T of every
-// block in the order in which k_sb_q2's lanes read them as MFMA operands.
-// Block (group, t) of ntg groups: groups 0..gr-1 have ntg, ntg - 1, .. blocks.
-__device__ __forceinline__ size_t frag_block(int ntg, int gr, int t)
+// block in the order in which k_sb_q2's lanes read them as MFMA operands.  The
+// groups are counted from the last one, which is applied first: group gi has
+// gi + 1 blocks, and those of the groups from ga on are held at a time.
+__host__ __device__ constexpr size_t frag_block(int ga, int gi, int t)
 {
-  return (size_t)gr * ntg - (size_t)gr * (gr - 1) / 2 + t;
+  return ((size_t)gi * (gi + 1) - (size_t)ga * (ga + 1)) / 2 + t;
 }
 constexpr int FRAG = 4096;  // doubles of a block per plane: 32 + 32 operand fragments of 64
 
 template <bool CX>
-__global__ __launch_bounds__(256) void k_sb_frag(SbArgs g, int ntg, int nsync)
+__global__ __launch_bounds__(256) void k_sb_frag(SbArgs g, int ntg, int ga, int nsync)
 {
   __shared__ double v[CX ? 2 : 1][64][BND + 1], gm[CX ? 2 : 1][BND][BND + 1], tm[CX ? 2 : 1][BND][BND + 1];
-  const int gr = blockIdx.y, t = blockIdx.x, tid = threadIdx.x, n = g.n;
+  const int gi = ga + blockIdx.y, gr = ntg - 1 - gi, t = blockIdx.x, tid = threadIdx.x, n = g.n;
   // the ticket and progress words of k_sb_q2
-  for (int i = (gr * ntg + t) * 256 + tid; i < nsync; i += ntg * ntg * 256) g.q2sync[i] = 0;
-  if (gr + t >= ntg) return;
+  for (size_t i = ((size_t)blockIdx.y * gridDim.x + t) * 256 + tid; i < (size_t)nsync;
+       i += (size_t)gridDim.y * gridDim.x * 256)
+    g.q2sync[i] = 0;
+  if (t > gi) return;
   const int s0 = gr * BND, w0 = s0 + 1 + BND * t;
   for (int e = tid; e < 64 * BND; e += 256) {
     const int x = e & 63, i = e >> 6;
@@ -1214,7 +1218,7 @@ __global__ __launch_bounds__(256) void k_sb_frag(SbArgs g, int ntg, int nsync)
     }
   }
   __syncthreads();
-  double *out = g.frag + frag_block(ntg, gr, t) * FRAG * (CX ? 2 : 1);
+  double *out = g.frag + frag_block(ga, gi, t) * FRAG * (CX ? 2 : 1);
   // V: fragment (w, mt, k): lane (l, q) holds row 16 w + 4 q + k, column 16 mt + l
   for (int e = tid; e < 2048; e += 256) {
     const int lane = e & 63, f = e >> 6, k = f & 3, mt = (f >> 2) & 1, w = f >> 3;
@@ -1242,7 +1246,7 @@ __global__ __launch_bounds__(256) void k_sb_frag(SbArgs g, int ntg, int nsync)
 // rows of the blocked copy of Z (the last window reaches past the matrix)
 __host__ __device__ constexpr size_t q2_rows(int n) { return (size_t)n + 2 * BND; }
 
-// Z <- Q2 Z.  A task is one group of sweeps on a slab of 16 columns of Z: its
+// Z <- Q2 Z for the groups ga .. gb - 1.  A task is one group of sweeps on a slab of 16 columns of Z: its
 // blocks slide down the rows.  A wave holds 16 of the window's 64 rows as MFMA
 // accumulators (lane (l, q): column l, rows 4 q + k in item k), which are at
 // once the operand of V^H Z; the four partial V^H Z meet in LDS.  Between the
@@ -1266,15 +1270,15 @@ constexpr int Q2_FLAG = 4;
 constexpr int Q2_WIDE = 512;
 
 template <bool CX, int NC>
-__global__ __launch_bounds__(256, 2) void k_sb_q2(SbArgs g, int ntg, int mcol, double *__restrict__ Zr,
-                                                           double *__restrict__ Zi, int ldz)
+__global__ __launch_bounds__(256, 2) void k_sb_q2(SbArgs g, int ntg, int ga, int gb, int mcol,
+                                                  double *__restrict__ Zr, double *__restrict__ Zi, int ldz)
 {
   constexpr int CP = CX ? 2 : 1;
   __shared__ double yp[2][CP][NC][4][8][64];
   __shared__ int tick;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l = lane & 15, q4 = lane >> 4;
-  const int n = g.n, nslab = (mcol + 16 * NC - 1) / (16 * NC), ntask = nslab * ntg;
-  int *const done = g.q2sync + 1;  // steps done of (group from the last, slab)
+  const int n = g.n, nslab = (mcol + 16 * NC - 1) / (16 * NC), ntask = nslab * (gb - ga);
+  int *const done = g.q2sync + 1;  // steps done of (group from ga, slab)
   const size_t zrows = q2_rows(n), zplane = zrows * (size_t)nslab * NC * 16;
   const int zo = 64 * q4 + l;  // this lane's place in four rows, 4 q4 rows on
   auto ticket = [&]() { return __hip_atomic_fetch_add(g.q2sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
@@ -1282,13 +1286,13 @@ __global__ __launch_bounds__(256, 2) void k_sb_q2(SbArgs g, int ntg, int mcol, d
   __syncthreads();
   int task = __builtin_amdgcn_readfirstlane(tick);
   while (task < ntask) {
-    const int gi = task / nslab, slab = task - gi * nslab, gr = ntg - 1 - gi, nt = gi + 1;
+    const int q = task / nslab, slab = task - q * nslab, gi = ga + q, gr = ntg - 1 - gi, nt = gi + 1;
     double *const zb = g.zb + (size_t)slab * NC * 16 * zrows;
-    int seen = gi == 0 ? CHASE_DONE : 0;
+    int seen = q == 0 ? CHASE_DONE : 0;
     // rows of window t are final once the group after this one has done step
     // t; its progress is read a step ahead
     int peek = 0;
-    auto progress = [&]() { return gi > 0 ? agent_ld(done + (size_t)(gi - 1) * nslab + slab) : CHASE_DONE; };
+    auto progress = [&]() { return q > 0 ? agent_ld(done + (size_t)(q - 1) * nslab + slab) : CHASE_DONE; };
     auto ready = [&](int t) {
       while (seen < t + 1) {
         seen = __builtin_amdgcn_readfirstlane(progress());
@@ -1354,7 +1358,7 @@ __global__ __launch_bounds__(256, 2) void k_sb_q2(SbArgs g, int ntg, int mcol, d
       double a[8], t[8], ai[CX ? 8 : 1], ti[CX ? 8 : 1];
     };
     auto fetch = [&](Ops &o, int t, int role) {
-      const double *f = g.frag + frag_block(ntg, gr, t) * FRAG * CP + (size_t)role * 512 + lane;
+      const double *f = g.frag + frag_block(ga, gi, t) * FRAG * CP + (size_t)role * 512 + lane;
 #pragma unroll
       for (int k = 0; k < 8; k++) {
         o.a[k] = f[k * 64];
@@ -1427,7 +1431,7 @@ __global__ __launch_bounds__(256, 2) void k_sb_q2(SbArgs g, int ntg, int mcol, d
       const bool flag = t % Q2_FLAG == Q2_FLAG - 1;
       if (flag) vm_drain();  // the tiles of the steps before this one are stored
       __syncthreads();
-      if (flag && tid == 0) agent_st(done + (size_t)gi * nslab + slab, t);
+      if (flag && tid == 0) agent_st(done + (size_t)q * nslab + slab, t);
       // Z -= (V T) (V^H Z), for one real set of columns in two accumulator chains
       constexpr bool TWO = !CX && NC == 1;
       d4 z2 = d4{0.0, 0.0, 0.0, 0.0};
@@ -1478,7 +1482,7 @@ __global__ __launch_bounds__(256, 2) void k_sb_q2(SbArgs g, int ntg, int mcol, d
     vm_drain();
     __syncthreads();
     if (tid == 0) {
-      agent_st(done + (size_t)gi * nslab + slab, CHASE_DONE);
+      agent_st(done + (size_t)q * nslab + slab, CHASE_DONE);
       tick = ticket();
     }
     __syncthreads();
@@ -1507,14 +1511,38 @@ size_t sb_doubles(int n, int cplx, size_t *ints)
          up32((size_t)n * (ntg + 1) * cp);
 }
 
-static size_t q2_words(int n, size_t m) { return (m + 15) / 16 * ((n - 1 + BND - 1) / BND) + 1; }
+// Application of Q2: its workspace holds the vectors in their blocked order, the
+// ticket and progress words, and the operands of as many groups as find room.
+// All operands together take 2 n^2 elements, as much as two matrices; so where
+// they are more than Q2_OPS, a range of groups at a time is formed and applied
+// (every range waits for the one before).  The workspace is the inverse
+// iteration's (5 n m doubles), whose factors are dead by then.  1 GiB: all at
+// once, 1, 1/2 and 1/4 GiB take 84, 86, 89, 91 ms at complex N = 10880, m =
+// 2176 (3.8 GB of operands), 20.0, 20.8, 21.3, 21.8 ms at N = 6559, m = 1311
+// and 5.7, 5.7, 6.0, 6.1 ms at real N = 5951, m = 1190.
+constexpr size_t Q2_OPS = (size_t)1 << 27;  // doubles
 
-static size_t q2_cols(size_t m) { return (m + 31) / 32 * 32; }
-
-size_t sb_frag_doubles(int n, size_t m, int cplx)
+struct Q2Space {
+  size_t zb, words, group, all;  // vectors, words (in doubles), operands of the longest group and of all
+};
+static Q2Space q2_space(int n, size_t m, int cplx)
 {
-  const size_t ntg = (n - 1 + BND - 1) / BND;
-  return (ntg * (ntg + 1) / 2 * FRAG + q2_rows(n) * q2_cols(m)) * (cplx ? 2 : 1) + (q2_words(n, m) + 1) / 2;
+  const size_t ntg = (n - 1 + BND - 1) / BND, cp = cplx ? 2 : 1;
+  return {q2_rows(n) * ((m + 31) / 32 * 32) * cp, up32((m + 15) / 16 * ntg / 2 + 1), ntg * FRAG * cp,
+          ntg * (ntg + 1) / 2 * FRAG * cp};
+}
+// doubles that the operands may take; W2K_TEST_Q2_OPERANDS (tests only) sets fewer
+static size_t q2_ops(const Q2Space &q, size_t room)
+{
+  const char *e = std::getenv("W2K_TEST_Q2_OPERANDS");
+  if (e) room = std::min(room, (size_t)std::atoll(e));
+  return std::min(q.all, std::max(q.group, room));
+}
+
+size_t sb_q2_doubles(int n, size_t m, int cplx)
+{
+  const Q2Space q = q2_space(n, m, cplx);
+  return q.zb + q.words + q2_ops(q, Q2_OPS);
 }
 
 int sb_buffers(Ctx &c, SbArgs &g, int n, int cplx)
@@ -1631,29 +1659,33 @@ int sb_reduce(Ctx &c, hipStream_t s, SbArgs &g, int cplx)
 }
 
 template <bool CX>
-static int apply_q2(hipStream_t s, SbArgs &g, int m, double *Zr, double *Zi, int ldz)
+static int apply_q2(hipStream_t s, SbArgs &g, const Q2Space &q, size_t ops, int m, double *Zr, double *Zi, int ldz)
 {
-  const int ntg = (g.n - 1 + BND - 1) / BND;
-  if (ntg == 0 || m == 0) return 0;
-  const size_t words = q2_words(g.n, m);
-  hipLaunchKernelGGL((k_sb_frag<CX>), dim3(ntg, ntg), dim3(256), 0, s, g, ntg, (int)words);
-  W2K_STAGE(s, "k_sb_frag");
-  const int nwg = (int)std::min(words - 1, (size_t)(m >= Q2_WIDE ? 512 : 256));
-  if (!CX && m >= Q2_WIDE) hipLaunchKernelGGL((k_sb_q2<false, 2>), dim3(nwg), dim3(256), 0, s, g, ntg, m, Zr, Zi, ldz);
-  else hipLaunchKernelGGL((k_sb_q2<CX, 1>), dim3(nwg), dim3(256), 0, s, g, ntg, m, Zr, Zi, ldz);
-  W2K_STAGE(s, "k_sb_q2");
+  const int ntg = (g.n - 1 + BND - 1) / BND, nc = !CX && m >= Q2_WIDE ? 2 : 1, nslab = (m + 16 * nc - 1) / (16 * nc);
+  for (int ga = 0, gb; ga < ntg; ga = gb) {
+    gb = ga + 1;
+    while (gb < ntg && frag_block(ga, gb + 1, 0) * FRAG * (CX ? 2 : 1) <= ops) gb++;
+    const int ntask = nslab * (gb - ga), nwg = std::min(ntask, m >= Q2_WIDE ? 512 : 256);
+    hipLaunchKernelGGL((k_sb_frag<CX>), dim3(gb, gb - ga), dim3(256), 0, s, g, ntg, ga, ntask + 1);
+    W2K_STAGE(s, "k_sb_frag");
+    if (nc == 2)
+      hipLaunchKernelGGL((k_sb_q2<false, 2>), dim3(nwg), dim3(256), 0, s, g, ntg, ga, gb, m, Zr, Zi, ldz);
+    else hipLaunchKernelGGL((k_sb_q2<CX, 1>), dim3(nwg), dim3(256), 0, s, g, ntg, ga, gb, m, Zr, Zi, ldz);
+    W2K_STAGE(s, "k_sb_q2");
+  }
   return 0;
 }
 
 int sb_apply_q2(Ctx &c, hipStream_t s, SbArgs &g, int cplx, int m, double *Zr, double *Zi, int ldz)
 {
-  int rc;
-  if ((rc = c.w_frag.alloc(sb_frag_doubles(g.n, m, cplx)))) return rc;
-  g.frag = c.w_frag.p;
-  const size_t ntg = (g.n - 1 + BND - 1) / BND;
-  g.zb = g.frag + ntg * (ntg + 1) / 2 * FRAG * (cplx ? 2 : 1);
-  g.q2sync = reinterpret_cast<int *>(g.zb + q2_rows(g.n) * q2_cols(m) * (cplx ? 2 : 1));
-  return cplx ? apply_q2<true>(s, g, m, Zr, Zi, ldz) : apply_q2<false>(s, g, m, Zr, Zi, ldz);
+  if (g.n < 2 || m == 0) return 0;
+  const Q2Space q = q2_space(g.n, m, cplx);
+  if (c.w_fac.n < sb_q2_doubles(g.n, m, cplx)) return W2K_ESTATE;
+  g.zb = c.w_fac.p;
+  g.q2sync = reinterpret_cast<int *>(g.zb + q.zb);
+  g.frag = g.zb + q.zb + q.words;
+  const size_t ops = q2_ops(q, c.w_fac.n - q.zb - q.words);
+  return cplx ? apply_q2<true>(s, g, q, ops, m, Zr, Zi, ldz) : apply_q2<false>(s, g, q, ops, m, Zr, Zi, ldz);
 }
 
 }  // namespace w2k

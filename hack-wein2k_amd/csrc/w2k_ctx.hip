@@ -20,8 +20,6 @@
 // the process).  Host code never names it except to look up its device
 // address once per device (noalloc_scratch_init); the kernels receive that
 // address through the workspaces carved from it.
-// The two-stage tridiagonalisation's work rows, operands and blocked vectors
-// bring a complex order of 768 with all its vectors to 145 MB (noalloc_bytes).
 static __device__ __align__(256) unsigned char scratch[W2K_NOALLOC_SCRATCH_BYTES];
 
 namespace w2k {
@@ -425,7 +423,7 @@ void drop_kpoint_state(Ctx &c)
   DBuf<double> *bufs[] = {&c.d_kvec, &c.d_hs, &c.d_hsdiag, &c.d_al, &c.d_bl, &c.d_cs, &c.d_theta, &c.d_colcoef,
                           &c.d_hnsL, &c.d_hnsR, &c.h_small, &c.h_re, &c.h_im, &c.d_eig, &c.d_z, &c.w_a,
                           &c.w_b, &c.w_c, &c.w_v, &c.w_x, &c.w_small, &c.w_fac, &c.w_bt, &c.w_cl, &c.w_gk, &c.w_3m,
-                          &c.w_sb, &c.w_frag};
+                          &c.w_sb};
   for (DBuf<double> *b : bufs) b->release();
   for (DBuf<double> &b : c.at_d) b.release();
   for (DBuf<int> &b : c.at_i) b.release();
@@ -574,12 +572,12 @@ static size_t noalloc_bytes(size_t n, size_t m, int cplx)
   b += r((6 * n + 32 + 1) / 2);                                              // ints
   b += r(m + 1);                                                             // eigenvalues
   const size_t zp = ((n + 2) / 2) * 2 * m;
-  b += r(5 * zp) + r((zp + 1) / 2);                                          // inverse iteration
+  b += r(std::max(5 * zp, sb_q2_doubles((int)n, m, cplx))) + r((zp + 1) / 2);  // inverse iteration, Q2
   b += r(2 * n * 64 + 2 * 64 * 64 + m * 64 + m + 1);                         // clusters
   b += r(z * n * (m + 1));                                                   // Z
   b += cplx ? r(2 * (2 * n + 3 * 64 + 2 * m) * 64 + 64 * 64 * 64) : r((2 * n + 2 * m + 3 * 128) * 128 + 32 * 128 * 128);
   size_t nint = 0;
-  b += r(sb_doubles((int)n, cplx, &nint)) + r(sb_frag_doubles((int)n, m, cplx));   // two-stage tridiagonalisation
+  b += r(sb_doubles((int)n, cplx, &nint));                                   // two-stage tridiagonalisation
   b += r((nint + 1) / 2);
   return b;
 }
@@ -757,7 +755,7 @@ int w2k_seclr4_noalloc(w2k_ctx *x, int n, double *hs, double *hsdiag, double el,
   // and restored afterwards; HS/HSDIAG are the caller's buffers, every
   // workspace and the eigenpairs come from the scratch
   DBuf<double> *dbufs[] = {&c.d_hs, &c.d_hsdiag, &c.d_eig, &c.d_z, &c.w_a, &c.w_b, &c.w_c, &c.w_v, &c.w_x,
-                           &c.w_small, &c.w_fac, &c.w_bt, &c.w_cl, &c.w_gk, &c.w_sb, &c.w_frag};
+                           &c.w_small, &c.w_fac, &c.w_bt, &c.w_cl, &c.w_gk, &c.w_sb};
   DBuf<int> *ibufs[] = {&c.w_int, &c.w_piv, &c.w_sbi};
   constexpr int ND = sizeof(dbufs) / sizeof(dbufs[0]), NI = sizeof(ibufs) / sizeof(ibufs[0]);
   DBuf<double> dsave[ND];

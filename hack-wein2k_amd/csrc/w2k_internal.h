@@ -177,7 +177,7 @@ struct Ctx {
   DBuf<double> w_a, w_b, w_c, w_v, w_x;
   DBuf<double> w_small;
   DBuf<int> w_int;
-  DBuf<double> w_fac;   // inverse-iteration factors, [plane][row][eigenvalue]
+  DBuf<double> w_fac;   // inverse-iteration factors, [plane][row][eigenvalue]; then Q2's operands and blocked vectors
   DBuf<int> w_piv;      // inverse-iteration pivots
   DBuf<double> w_bt;    // back-transform panel work
   DBuf<double> w_cl;    // cluster orthogonalisation work
@@ -188,7 +188,6 @@ struct Ctx {
   // LO flags, coupling triples
   DBuf<double> at_d[8];
   DBuf<int> at_i[2];
-  DBuf<double> w_frag;  // operands of the second stage's reflector blocks
   DBuf<double> w_3m;    // three-product complex GEMM: Re + Im of both operands, one real product
   // launch mode of the tridiagonalisation, chosen per shape by measurement:
   // direct launches or one captured HIP graph replayed (seclr4.hip)

@@ -167,7 +167,7 @@ int w2k_seclr4(w2k_ctx *ctx, double el, double eu, int nume, int *ne, int *nbelw
  * device shares that device's scratch, so calls that overlap on one device
  * (from different threads or contexts) race; calls on one context are
  * serial.  The context's own HS and eigenpairs are left untouched. */
-#define W2K_NOALLOC_SCRATCH_BYTES (160u << 20)
+#define W2K_NOALLOC_SCRATCH_BYTES (128u << 20)
 #define W2K_NOALLOC_MAXN 768
 int w2k_seclr4_noalloc(w2k_ctx *ctx, int n, double *hs, double *hsdiag, double el, double eu, int nume,
                        int *ne, int *nbelw, double *eigval, double *z, int ldz);
