@@ -19,6 +19,7 @@ struct SbArgs {
   double *taur = nullptr, *taui = nullptr;  // reflector scalars of Q1, n
   double *exch = nullptr;                   // sums exchanged within a panel's QR
   int *sync = nullptr;
+  int qr_cap = 1 << 30;                     // most work-groups that share a panel (tests set fewer)
   double *ab = nullptr;                     // band, 2 BND x n
   double *d = nullptr, *e = nullptr;        // tridiagonal matrix
   double *V2r = nullptr, *V2i = nullptr;    // reflectors of Q2: sweep s in column s, n x n

@@ -395,12 +395,12 @@ __global__ __launch_bounds__(QR_ROWS) void k_sb_qr(SbArgs g, int j0)
     if (tid == 0) {
       const int old = __hip_atomic_fetch_add(g.sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       int me = old, cnt = 0;
-      if (old & SB_CLOSED) {
+      if (old & SB_CLOSED || old >= g.qr_cap) {
         me = -1;
       } else if (old == 0) {
         const long long t0 = wall_clock64();
         while (agent_ld(g.sync) < nblk && wall_clock64() - t0 < QR_WAIT) __builtin_amdgcn_s_sleep(1);
-        cnt = __hip_atomic_fetch_or(g.sync, SB_CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        cnt = min(__hip_atomic_fetch_or(g.sync, SB_CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), g.qr_cap);
         agent_st(g.sync + 1, cnt);
       } else {
         while ((cnt = agent_ld(g.sync + 1)) == 0) __builtin_amdgcn_s_sleep(1);
@@ -1655,6 +1655,10 @@ static int reduce(Ctx &c, hipStream_t s, SbArgs &g)
 
 int sb_reduce(Ctx &c, hipStream_t s, SbArgs &g, int cplx)
 {
+  // W2K_TEST_QR_GROUPS (tests only): that many work-groups share a panel, as if
+  // the others had come late
+  const char *cap = std::getenv("W2K_TEST_QR_GROUPS");
+  if (cap) g.qr_cap = std::max(1, std::atoi(cap));
   return cplx ? reduce<true>(c, s, g) : reduce<false>(c, s, g);
 }
 
