@@ -333,12 +333,12 @@ def measure(L, run, basis, kd, args, label: str, workload: str, full_checks: boo
         "k_hamilt_pw": ("valu", f_hamilt, t["hamilt_pw_kernel"], 1),
         "k_dgemm (HNS rank-K)": ("mfma", f_hns, t["hns_gemm"], 1),
     }
-    if tk is not None and tk["tri_symv_launches"] > 0:
+    if tk is not None and tk["tri_panel_launches"] > 0:
         # the products A V of the band reduction: order m = n - 32 p of the
         # trailing matrix, 32 columns of V
-        npan = int(tk["tri_symv_launches"])
+        npan = int(tk["tri_panel_launches"])
         av_flops = sum(cx * 2.0 * 32 * float(n - 32 * p) ** 2 for p in range(1, npan + 1))
-        kernels["k_sb_av"] = ("mfma", av_flops, tk["tri_symv_total"], npan)
+        kernels["k_sb_av"] = ("mfma", av_flops, tk["tri_panel_total"], npan)
     kname, (bound, work, kms, nl) = max(kernels.items(), key=lambda kv: kv[1][2])
 
     def rate(bd, wk, ms_):

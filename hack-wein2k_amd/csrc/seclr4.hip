@@ -7,7 +7,7 @@
 // Stages (all on the context stream):
 //   1. Cholesky S = U^T U (POTRF 'U', seclr4.F:196) together with
 //      W = U^-1: recursive halving on 64-column boundaries, 64x64 leaves
-//      factored and inverted by one wave in registers, the TRSM as a GEMM
+//      factored and inverted by one work-group each (chol_leaf.h), the TRSM as a GEMM
 //      with the leading half's inverse, the SYRK as an MFMA GEMM on the upper
 //      triangle, W12 = -(W11 U12) W22.
 //   2. Reduction to standard form C = U^-T H U^-1 (DSCGST, dscgst.f:99-142):
@@ -831,10 +831,9 @@ int seclr4_buffers(Ctx &c, int n, int cplx, Seclr4Bufs &B)
   B.P = take(z * 3 * (size_t)n * BND);
   B.bgl = take(n); B.bgu = take(n); B.batol = take(n); B.bnrm = take(n); B.xs = take(n);
   B.pivmin = take(1);
-  // ints: [0,4) INFO, [4,12) counts, [12,16) grid-reduction tickets, then task arrays
+  // ints: [0,4) INFO, [4,12) counts, then from 16 on task arrays
   B.info = c.w_int.p;
   B.cnt = B.info + 4;
-  B.ticket = B.info + 12;
   B.tblk = B.info + 16;
   B.tidx = B.tblk + n;
   B.bstart = B.tidx + n;
@@ -1115,7 +1114,7 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
   // on 64-column boundaries: factor the leading half (U11, W11), form
   // U12 = W11^T S12 and S22 -= U12^T U12 (upper triangle), factor the
   // trailing half (U22, W22), then W12 = -(W11 U12) W22.  The 64x64 leaves
-  // are factored and inverted by one wave each; the products at the top
+  // are factored and inverted by one work-group each; the products at the top
   // levels are square.  W is zero below the diagonal.
   {
     hipLaunchKernelGGL(k_fill, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, nn, W, 0.0);
@@ -1232,7 +1231,7 @@ static int seclr4_real(Ctx &c, double el, double eu, int nume, int *ne_out, int 
     for (int q = 0; q < nblk; q++) {
       const int u = q & 1, p0 = p0_of(q), nb = std::min(BTNB, nref - p0);
       W2K_HIP(hipStreamWaitEvent(s, c.bt_ready[u], 0));
-      const int o = (p0 + BND) & ~15, nr = n - o;  // the block's reflectors are zero above row p0+1
+      const int o = (p0 + BND) & ~15, nr = n - o;  // the block's reflectors are zero above row p0+BND
       if ((rc = dgemm(s, 'T', 'N', nb, m, nr, 1.0, vbuf[u] + o, n, Zt + o, n, 0.0, y1, nb, 0, 0, 0, c.w_gk.p,
                       c.w_gk.n)))
         return rc;

@@ -113,7 +113,7 @@ struct Seclr4Bufs {
   double *wv;               // eigenvalues (block order, then sorted)
   double *P;                // panel buffer n x 3 BND (complex: twice)
   double *bgl, *bgu, *batol, *bnrm, *xs, *pivmin;
-  int *info, *cnt, *ticket, *tblk, *tidx, *bstart, *bend, *cstart, *perm;
+  int *info, *cnt, *tblk, *tidx, *bstart, *bend, *cstart, *perm;
 };
 
 // doubles of those buffers

@@ -20,12 +20,12 @@ struct SbArgs {
   double *exch = nullptr;                   // sums exchanged within a panel's QR
   int *sync = nullptr;
   int qr_cap = 1 << 30;                     // most work-groups that share a panel (tests set fewer)
-  double *ab = nullptr;                     // band, 2 BND x n
+  double *ab = nullptr;                     // band, 2 BND x (n + 4 BND): columns of zeros past the last
   double *d = nullptr, *e = nullptr;        // tridiagonal matrix
   double *V2r = nullptr, *V2i = nullptr;    // reflectors of Q2: sweep s in column s, n x n
   double *tau2 = nullptr;                   // their scalars, [step][sweep]
   size_t ntau2 = 0;
-  int *prog = nullptr;                      // finished steps per sweep; entry n: the next sweep
+  int *prog = nullptr;                      // finished steps per group of sweeps; entry n: the next group
   double *frag = nullptr;                   // operands of the Q2 blocks of some groups
   double *zb = nullptr;                     // vectors between the groups of Q2, 16 columns side by side
   int *q2sync = nullptr;                    // ticket and progress of their application

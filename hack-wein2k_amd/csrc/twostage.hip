@@ -817,11 +817,12 @@ constexpr int CNC = 4;  // columns per lane of a sweep's four waves
 // of D v and C v and their sums, and before the next sweep reads; what follows
 // the sums is done by every wave for itself.  The band has columns of zeros
 // after the last one, and sweeps and steps past the matrix' end run on those:
-// no step has an edge.  Reduction as a whole with one sweep per work-group and
-// three barriers a step -> as here: real N = 731 7.4 -> 5.3 ms, N = 5951 79 ->
-// 64; complex N = 251 2.9 -> 2.6, N = 1950 28.2 -> 25.8.  K = 2, 3, 4 take
-// 5.5, 5.3, 5.5 (N = 731) and 69, 64, 63 ms (N = 5951), complex K = 1, 2, 3
-// 3.2, 2.6, 2.5 (N = 251) and 30.8, 25.8, 26.4 ms (N = 1950).
+// no step has an edge.  Measured on the reduction as a whole (whose products took
+// up to 4 ms more then than now), one sweep per work-group and three barriers a
+// step -> as here: real N = 731 7.4 -> 5.3 ms, N = 5951 79 -> 64; complex N =
+// 251 2.9 -> 2.6, N = 1950 28.2 -> 25.8.  K = 2, 3, 4 took 5.5, 5.3, 5.5 (N =
+// 731) and 69, 64, 63 ms (N = 5951), complex K = 1, 2, 3 3.2, 2.6, 2.5 (N =
+// 251) and 30.8, 25.8, 26.4 ms (N = 1950).
 //
 // A work-group takes groups of sweeps in order from a ticket: the oldest
 // unfinished group always has a running work-group and waits for nothing, so

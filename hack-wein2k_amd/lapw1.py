@@ -526,12 +526,12 @@ class Lapw1:
         return ev[:ne], z[:, :ne]
 
     TIMING_NAMES = ("hamilt", "hns", "seclr4", "cholesky", "reduction", "tridiag", "bisect_invit",
-                    "backtransform", "hamilt_pw_kernel", "hns_gemm", "tri_symv_total", "tri_symv_launches",
+                    "backtransform", "hamilt_pw_kernel", "hns_gemm", "tri_panel_total", "tri_panel_launches",
                     "tri_launch_mode")
 
     def set_kernel_timing(self, on: bool):
         """Per-launch events around the tridiagonalisation's products of the
-        trailing matrix with a panel (the tri_symv timings)."""
+        trailing matrix with a panel (the tri_panel timings)."""
         self._chk("w2k_set_kernel_timing", self.lib.w2k_set_kernel_timing(self.ctx, int(bool(on))))
 
     def set_graphs(self, on: bool):
