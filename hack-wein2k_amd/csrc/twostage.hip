@@ -18,7 +18,7 @@
 // two steps per sweep.  Whole reduction, before -> now (Q2's application in
 // brackets): real N = 221 3.1 -> 1.3 ms, N = 731 10.7 -> 5.3, N = 5951 135 ->
 // 60 (+ 6); complex N = 251 5.4 -> 2.5, N = 1950 47 -> 25 (+ 2), N = 10880
-// 1018 -> 325 (+ 84).
+// 1018 -> 326 (+ 86).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
